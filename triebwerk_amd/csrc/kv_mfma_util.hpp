@@ -60,6 +60,49 @@ constexpr int kStreamNorms = 0;
 // compute units of the current device (cached; kv_attention_mfma.hip)
 int compute_units();
 
+// The forms of the two flash prefill kernels, and the rule that picks one.  A workgroup of `waves` waves in `groups` groups takes
+// 16 * nq * (waves / groups) / R query tokens of one KV head; the groups take turns with the context's tiles.
+// With causal rows the last block's chain of tiles is twice the average, so what a launch takes is the larger of its longest
+// chain (at the pace of a workgroup that has its compute unit for itself) and of the steps all workgroups make (at the pace of
+// a full compute unit): estimate = fixed + max(alone * longest, loaded * steps per unit) + per_wg * workgroups per unit
+//                                 + both * min(longest, steps per unit), in us.
+// The figures are fitted to launches of 31 to 8200 tokens with 8, 16 and 32 heads over 2 and 8 KV heads on MI355X (256 compute
+// units): within 15 % everywhere, and the form with the smallest estimate is the fastest measured one or within 3 %
+// of it in 41 of 42 cases (the other: 5 %).
+struct PrefillForm { int id, waves, nq, groups; double fixed, alone, loaded, per_wg, both; };
+struct PrefillChoice { int id, waves, nq, groups; bool mirror; int blocks; };
+
+inline PrefillChoice choose_prefill_form(const PrefillForm* forms, int nforms, double mirror_fill, int T, int R, int num_kv_heads, int forced) {
+    const double cus = compute_units();
+    PrefillChoice best{};
+    double best_us = 0.0;
+    for (int i = 0; i < nforms; i++) {
+        const PrefillForm& f = forms[i];
+        const int tpw = 16 * f.nq * (f.waves / f.groups) / R, blocks = (T + tpw - 1) / tpw;
+        const double longest = ((T + 31) / 32 + f.groups - 1) / f.groups;
+        const double shortest = (tpw + 31) / 32 > f.groups ? (double)((tpw + 31) / 32) / f.groups : 1.0;
+        const double per_unit = blocks * (longest + shortest) * 0.5 * num_kv_heads / cus;
+        double us = f.fixed + (f.alone * longest > f.loaded * per_unit ? f.alone * longest : f.loaded * per_unit) +
+                    f.per_wg * blocks * num_kv_heads / cus + f.both * (longest < per_unit ? longest : per_unit);
+        // Blocks in pairs, each with its mirror image from the other end, when the pairs fill whole rounds of one workgroup
+        // per compute unit (a single round: by mirror_fill): every workgroup then does the same work and none starts late
+        // (8192 tokens: 0.266 against 0.271 ms on the fp16 cache, 0.498 against 0.511 at 4 bit; 6400 tokens, a round 3/4 full: 0.186
+        // against 0.192, but 0.392 against 0.364 at 4 bit).  A pair too many costs a second round (8200 tokens: 0.310 against
+        // 0.275 and 0.605 against 0.524), so otherwise the blocks are workgroups of their own, longest first: a compute
+        // unit that is done takes the next shorter one, which pairs them just as well.
+        const double pairs = (double)((blocks + 1) / 2) * num_kv_heads, rounds = (double)(long long)((pairs + cus - 1) / cus);
+        bool mirror = f.waves == 8 && f.groups == 1 && pairs >= (rounds > 1.0 ? 0.97 : mirror_fill) * rounds * cus;
+        if (mirror) us *= 0.97;
+        // forced by a test: 5 and 6 in pairs, 7 and 8 the same forms unpaired, 1 to 3 (never in pairs) as they are
+        if (f.id == forced || f.id + 2 == forced) {
+            if (f.id >= 5) { us = -1.0; mirror = f.id == forced; }
+            else if (f.id == forced) us = -1.0;
+        }
+        if (i == 0 || us < best_us) { best_us = us; best = PrefillChoice{f.id, f.waves, f.nq, f.groups, mirror, blocks}; }
+    }
+    return best;
+}
+
 // The dequantization table of the MFMA scans, built by the nthreads threads of a workgroup: entry e (a cache byte)
 // fills 256 bytes with replicas of its centroids as fp16 -- 4 bit: 64 replicas of (low code, high code); 2 bit: 32
 // replicas of the byte's four codes, in their own order (NATURAL) or as 0, 2, 1, 3.  The centroids come out of a

@@ -23,9 +23,8 @@
 // consecutive tokens and writes 8 dwords).  The loop is a pipeline, one barrier per tile, a tile
 // taking five steps through it: global loads issued; written to LDS; K operands read into registers; score
 // MFMAs (with the previous tile's exponentials between them) and maxima; exponentials and P.V MFMAs (with the
-// next tile's maxima between them).  Two K buffers, four V buffers; the loop says which step does what.  For long prompts a workgroup does a token block and then its
-// mirror image from the other end of the sequence, so causal rows cost every workgroup the same; short
-// prompts take one block each, longest first.  The workgroups of a KV head run on one XCD, so the head's
+// next tile's maxima between them).  Two K buffers, four V buffers; the loop says which step does what.  choose_prefill_form (kv_mfma_util.hpp) says
+// which form a prompt takes and when a workgroup does a token block together with its mirror image from the other end.  The workgroups of a KV head run on one XCD, so the head's
 // rows come out of one L2.
 
 #include "kv_common.hpp"
@@ -40,6 +39,9 @@ namespace {
 constexpr int kPfKRow = 2 * kHeadDim + 32;   // bytes per K row in LDS: with 288 the operand reads (16 rows x 4 column groups of 16 bytes) run at the LDS's full rate, with 272 at 53 % of it (measured)
 constexpr int kPfVRow = 2 * 32 + 32;         // bytes per V^T row (32 token slots) in LDS: 96 at the full rate, 80 at 54 %
 
+// a masked score: below the initial maximum by more than the exponent's range, also when a group's first tile is all masked
+constexpr float kMasked = -3.0e38f;
+
 template <bool B> struct Flag { static constexpr bool value = B; };
 
 // column of a tile's token in the V^T rows: the contraction slot order of the second MFMA
@@ -47,19 +49,25 @@ __device__ __forceinline__ int vt_slot(int token) { return 8 * ((token & 15) >> 
 
 }  // namespace
 
-// NQ: 16-row query blocks per wave (every K and V operand read feeds NQ MFMAs).  MIRROR: a workgroup does a
-// token block and then its mirror image from the other end of the sequence.
-// W: waves per workgroup, 4 (two workgroups per CU) or 8 (one: a tile is brought into LDS once for twice the queries).
-template <int R, int NQ, bool MIRROR, int W>
+// W: waves per workgroup, 4 (two workgroups per CU) or 8 (one).  NQ: 16-row query blocks per wave (every K and V operand read
+// feeds NQ MFMAs).  KS: groups the waves form.  With one group a tile is brought into LDS once for all query rows of the
+// workgroup; with two, each group takes every other tile of the context for the same query rows (twice the
+// LDS, half the chain of steps) and their sums meet in LDS at the end.  MIRROR: a workgroup does a token block and then its
+// mirror image from the other end of the sequence.
+template <int R, int NQ, int W, int KS, bool MIRROR>
 __global__ void __launch_bounds__(W* kWave, W == 4 ? 2 : 1)  // two waves per SIMD either way (three would spill)
 prefill_f16_mfma_kernel(AttnArgs a, int T) {
-    static_assert(W == 4 || W == 8, "the staging maps are written for 256 and 512 threads");
-    constexpr int TPW = 16 * NQ * W / R;                   // query tokens per workgroup pass
-    __shared__ __attribute__((aligned(16))) char k_s[2][32 * kPfKRow];
-    __shared__ __attribute__((aligned(16))) char v_s[4][kHeadDim * kPfVRow];
+    constexpr int GW = W / KS;                             // waves per group
+    static_assert(GW == 4 || GW == 8, "the staging maps are written for 256 and 512 threads");
+    constexpr int TPW = 16 * NQ * GW / R;                  // query tokens per workgroup pass
+    __shared__ __attribute__((aligned(16))) char k_all[KS][2][32 * kPfKRow];
+    __shared__ __attribute__((aligned(16))) char v_all[KS][4][kHeadDim * kPfVRow];
 
-    const int tid = threadIdx.x;
-    const int wave = uniform(tid / kWave), lane = tid % kWave;
+    const int wave_wg = uniform((int)threadIdx.x / kWave), lane = threadIdx.x % kWave;
+    const int grp = KS == 1 ? 0 : wave_wg / GW, wave = KS == 1 ? wave_wg : wave_wg % GW;
+    const int tid = wave * kWave + lane;                   // within the group
+    auto& k_s = k_all[grp];
+    auto& v_s = v_all[grp];
     const int ln = lane & 15, kg = lane >> 4;
     const int nblk = (T + TPW - 1) / TPW;
     // Workgroups are dealt to the 8 XCDs in turn (linear id % 8), each with an L2 of its own.  The workgroups of a
@@ -96,12 +104,13 @@ prefill_f16_mfma_kernel(AttnArgs a, int T) {
     const __amdgpu_buffer_rsrc_t krs = make_rsrc(reinterpret_cast<const char*>(kbase), T * kv_dim * 2 - kvh * kHeadDim * 2);
     const __amdgpu_buffer_rsrc_t vrs = make_rsrc(reinterpret_cast<const char*>(vbase), T * kv_dim * 2 - kvh * kHeadDim * 2);
     const int koff0 = (sr * kv_dim + 8 * sc) * 2, koff1 = koff0 + 16 * kv_dim * 2;
-    const int voff0 = (2 * vr_ * kv_dim + (W == 4 ? 8 : 4) * vc_) * 2, voff1 = voff0 + kv_dim * 2;
+    const int voff0 = (2 * vr_ * kv_dim + (GW == 4 ? 8 : 4) * vc_) * 2, voff1 = voff0 + kv_dim * 2;
+    const int last_tile = (T - 1) & ~31;                   // a tile past the end is this one again (and masked)
     auto load_tile = [&](int tile, uint4 (&kr)[2], uint4 (&vr)[2]) {
-        const int toff = tile * kv_dim * 2;
+        const int toff = min(tile, last_tile) * kv_dim * 2;
         const uint32x4_t k0 = __builtin_amdgcn_raw_buffer_load_b128(krs, koff0, toff, 0);
         kr[0] = uint4{k0[0], k0[1], k0[2], k0[3]};
-        if constexpr (W == 4) {
+        if constexpr (GW == 4) {
             const uint32x4_t k1 = __builtin_amdgcn_raw_buffer_load_b128(krs, koff1, toff, 0);
             const uint32x4_t v0 = __builtin_amdgcn_raw_buffer_load_b128(vrs, voff0, toff, 0);
             const uint32x4_t v1 = __builtin_amdgcn_raw_buffer_load_b128(vrs, voff1, toff, 0);
@@ -118,26 +127,27 @@ prefill_f16_mfma_kernel(AttnArgs a, int T) {
     const int vcol = 2 * vt_slot(2 * vr_);                  // byte column of the token pair in a V^T row
     auto stash = [&](int buf, int vbuf, const uint4 (&kr)[2], const uint4 (&vr)[2]) {
         *reinterpret_cast<uint4*>(&k_s[buf][sr * kPfKRow + 16 * sc]) = kr[0];
-        if constexpr (W == 4) *reinterpret_cast<uint4*>(&k_s[buf][(sr + 16) * kPfKRow + 16 * sc]) = kr[1];
+        if constexpr (GW == 4) *reinterpret_cast<uint4*>(&k_s[buf][(sr + 16) * kPfKRow + 16 * sc]) = kr[1];
         const uint32_t va[4] = {vr[0].x, vr[0].y, vr[0].z, vr[0].w};
         const uint32_t vb[4] = {vr[1].x, vr[1].y, vr[1].z, vr[1].w};
-        char* dst = &v_s[vbuf][((W == 4 ? 8 : 4) * vc_) * kPfVRow + vcol];
+        char* dst = &v_s[vbuf][((GW == 4 ? 8 : 4) * vc_) * kPfVRow + vcol];
 #pragma unroll
-        for (int i = 0; i < (W == 4 ? 4 : 2); i++) {       // dims 8c + 2i (low halves) and 8c + 2i + 1 (high halves); 512 threads: 4c + ...
+        for (int i = 0; i < (GW == 4 ? 4 : 2); i++) {       // dims 8c + 2i (low halves) and 8c + 2i + 1 (high halves); 512 threads: 4c + ...
             *reinterpret_cast<uint32_t*>(dst + (2 * i) * kPfVRow) = __builtin_amdgcn_perm(vb[i], va[i], 0x05040100u);
             *reinterpret_cast<uint32_t*>(dst + (2 * i + 1) * kPfVRow) = __builtin_amdgcn_perm(vb[i], va[i], 0x07060302u);
         }
     };
 
-    // A workgroup takes token block blockIdx.x and its mirror image from the other end, one after the
-    // other: with causal rows the two together cost the same for every workgroup.
+    // MIRROR: a workgroup takes a token block and its mirror image from the other end, one after the other: with causal
+    // rows the two together cost the same for every workgroup.
     const int first = blk, second = nblk - 1 - blk;   // without MIRROR: longest blocks first
     for (int pass = 0; pass < (MIRROR ? 2 : 1); pass++) {
         if (pass == 1 && second == first) break;           // the middle block of an odd count
         const int tb = pass == 0 ? second : first;         // the long one first
         const int q0 = tb * TPW + 16 * NQ * (wave / R);    // this wave's 16 NQ query tokens
         const int wg_last = min(T, (tb + 1) * TPW) - 1;    // last query token of the pass
-        const int ntiles = (wg_last >> 5) + 1;
+        const int ntiles = ((wg_last >> 5) + KS) / KS;     // steps: a group's tiles are grp, grp + KS, ...
+        auto first_token = [&](int u) -> int { return 32 * (KS * u + grp); };
 
         // ---- B operands of the first MFMA: Q[q0 + 16 nq + ln][32j + 8kg .. +7], j = 0..3
         half8_t qb[NQ][4];
@@ -186,10 +196,10 @@ prefill_f16_mfma_kernel(AttnArgs a, int T) {
         uint4 kr[2], vr[2];
         {
             uint4 kr1[2], vr1[2];                          // tiles 0, 1 and 2 are asked for together: one trip to memory, not three
-            load_tile(0, kr, vr);
-            if (ntiles > 1) load_tile(32, kr1, vr1);
+            load_tile(first_token(0), kr, vr);
+            if (ntiles > 1) load_tile(first_token(1), kr1, vr1);
             stash(0, 0, kr, vr);
-            if (ntiles > 2) load_tile(64, kr, vr);
+            if (ntiles > 2) load_tile(first_token(2), kr, vr);
             if (ntiles > 1) stash(1, 1, kr1, vr1);
         }
         __syncthreads();
@@ -199,11 +209,12 @@ prefill_f16_mfma_kernel(AttnArgs a, int T) {
 
         float x[NQ][8];                                    // raw scores of the tile whose exponentials come next
         bool have_x = false;
-        const int n_below = q0 < T ? (q0 + 1) >> 5 : 0;    // tiles wholly below this wave's diagonal
+        // tiles of this group wholly below the wave's diagonal
+        const int n_below = q0 < T ? (((q0 + 1) >> 5) + KS - 1 - grp) / KS : 0;
 
         auto step = [&](auto steady_c, int t) {
             constexpr bool STEADY = decltype(steady_c)::value;
-            const int tile1 = 32 * (t + 1);                // first token of tile t + 1
+            const int tile1 = first_token(t + 1);
             const bool do_s = STEADY || (t + 1 < ntiles && tile1 <= q0 + 16 * NQ - 1 && q0 < T);   // tile t + 1 reaches this wave's queries
             const bool do_p = STEADY || have_x;
             // ---- phase 1 (the wave's priority falls through the step: of the two waves of a SIMD the one in its score
@@ -259,7 +270,7 @@ prefill_f16_mfma_kernel(AttnArgs a, int T) {
             }
             if (STEADY || t + 2 < ntiles) read_k(t & 1, kf);                           // tile t + 2
             if (STEADY || t + 3 < ntiles) stash((t + 1) & 1, (t + 3) & 3, kr, vr);      // tile t + 3
-            if (STEADY || t + 4 < ntiles) load_tile(32 * (t + 4), kr, vr);              // STEADY: rows past the cache read as zeros
+            if (STEADY || t + 4 < ntiles) load_tile(first_token(t + 4), kr, vr);              // STEADY: rows past the cache read as zeros
             if (do_s) {
                 // maxima of tile t + 1 per query: this lane holds kv tokens tile1 + 16 sub + 4kg + i
 #pragma unroll
@@ -275,7 +286,7 @@ prefill_f16_mfma_kernel(AttnArgs a, int T) {
                         for (int sub = 0; sub < 2; sub++) {
 #pragma unroll
                             for (int i = 0; i < 4; i++) {
-                                if (tile1 + 16 * sub + 4 * kg + i > tq) x[nq][4 * sub + i] = kNegBig;
+                                if (tile1 + 16 * sub + 4 * kg + i > tq) x[nq][4 * sub + i] = kMasked;
                             }
                         }
                     }
@@ -311,23 +322,82 @@ prefill_f16_mfma_kernel(AttnArgs a, int T) {
 #pragma clang loop unroll(disable)
         for (; t < ntiles; t++) step(Flag<false>{}, t);
 
-        // ---- normalise (kernels.cu:1146: 1 / (sum + 1e-8)) and store; accumulator register i is query 4kg + i
+        // ---- the groups' sums meet in LDS: with two query blocks group s finishes block s, with one it finishes the
+        // dims 64 s .. 64 s + 63
+        float l_sum[NQ];
 #pragma unroll
         for (int nq = 0; nq < NQ; nq++) {
             float l = l_run[nq];
             l += __shfl_xor(l, 16, 64);
             l += __shfl_xor(l, 32, 64);
-            const float inv = 1.0f / (l + 1e-8f);
+            l_sum[nq] = l;
+        }
+        constexpr int NF = KS == 2 && NQ == 2 ? 1 : NQ;    // query blocks this wave finishes
+        constexpr int NJ = KS == 2 && NQ == 1 ? 4 : 8;     // 16-dim blocks of each
+        const int nq_first = KS == 2 && NQ == 2 ? grp : 0, j_first = KS == 2 && NQ == 1 ? 4 * grp : 0;
+        float4_t of[NF][NJ];
+        float lf[NF];
+        if constexpr (KS == 2) {
+            constexpr int NG = NQ == 2 ? 8 : 4;            // 16-dim blocks that change hands
+            float4_t* ex = reinterpret_cast<float4_t*>(&v_all[0][0][0]);                              // [wave of the workgroup][NG][lane]
+            static_assert(W * kWave * (NG * 16 + 8) <= (int)sizeof(v_all), "the sums fit the V tiles");
+            float2* exml = reinterpret_cast<float2*>(&v_all[0][0][0] + W * NG * kWave * 16);          // [wave][lane]: maximum, sum
+            __syncthreads();                               // every wave is done with the tiles
+            // what the partner finishes, and what this wave keeps (grp is uniform: scalar branches)
+            if (grp == 0) {
+#pragma unroll
+                for (int j = 0; j < NG; j++) {
+                    ex[(wave_wg * NG + j) * kWave + lane] = NQ == 2 ? o[NQ - 1][j] : o[0][4 + (j & 3)];
+                    of[0][j] = o[0][j];
+                }
+                exml[wave_wg * kWave + lane] = float2{m_run[NQ - 1], l_sum[NQ - 1]};
+            } else {
+#pragma unroll
+                for (int j = 0; j < NG; j++) {
+                    ex[(wave_wg * NG + j) * kWave + lane] = o[0][j];
+                    of[0][j] = NQ == 2 ? o[NQ - 1][j] : o[0][4 + (j & 3)];
+                }
+                exml[wave_wg * kWave + lane] = float2{m_run[0], l_sum[0]};
+            }
+            const float m_own = grp == 0 ? m_run[0] : m_run[NQ - 1], l_own = grp == 0 ? l_sum[0] : l_sum[NQ - 1];
+            __syncthreads();
+            const int other = wave_wg ^ GW;
+            const float2 ml = exml[other * kWave + lane];
+            const float m_new = fmaxf(m_own, ml.x);
+            const float f_own = __builtin_amdgcn_exp2f(m_own - m_new), f_oth = __builtin_amdgcn_exp2f(ml.x - m_new);
+            lf[0] = l_own * f_own + ml.y * f_oth;
+            float fo[4], ft[4];
+#pragma unroll
+            for (int i = 0; i < 4; i++) { fo[i] = __shfl(f_own, 4 * kg + i, 64); ft[i] = __shfl(f_oth, 4 * kg + i, 64); }
+#pragma unroll
+            for (int j = 0; j < NG; j++) {
+                const float4_t p = ex[(other * NG + j) * kWave + lane];
+#pragma unroll
+                for (int i = 0; i < 4; i++) of[0][j][i] = of[0][j][i] * fo[i] + p[i] * ft[i];
+            }
+        } else {
+#pragma unroll
+            for (int nq = 0; nq < NQ; nq++) {
+                lf[nq] = l_sum[nq];
+#pragma unroll
+                for (int j = 0; j < 8; j++) of[nq][j] = o[nq][j];
+            }
+        }
+
+        // ---- normalise (kernels.cu:1146: 1 / (sum + 1e-8)) and store; accumulator register i is query 4kg + i
+#pragma unroll
+        for (int nf = 0; nf < NF; nf++) {
+            const float inv = 1.0f / (lf[nf] + 1e-8f);
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const float inv_i = __shfl(inv, 4 * kg + i, 64);
-                const int t = q0 + 16 * nq + 4 * kg + i;
+                const int t = q0 + 16 * (nq_first + nf) + 4 * kg + i;
                 if (t < T) {
-                    const long long col = (long long)head * kHeadDim + ln;
+                    const long long col = (long long)head * kHeadDim + 16 * j_first + ln;
                     half_t* orow = a.out + (long long)t * a.q_stride + col;
 #pragma unroll
-                    for (int j = 0; j < 8; j++) {
-                        half_t h = (half_t)(o[nq][j][i] * inv_i);
+                    for (int j = 0; j < NJ; j++) {
+                        half_t h = (half_t)(of[nf][j][i] * inv_i);
                         if (a.gate) h = gated(h, a.gate[(long long)t * a.gate_stride + col + 16 * j]);
                         orow[16 * j] = h;
                     }
@@ -351,31 +421,19 @@ bool prefill_f16_mfma_usable(const AttnArgs& a) {
 void launch_prefill_f16_mfma(const AttnArgs& a, hipStream_t s, int form) {
     const int R = a.num_heads / a.num_kv_heads;
     const int T = a.G;
-    // Long prompts: eight waves per workgroup, two query blocks per wave and mirrored block pairs (a tile is brought
-    // into LDS once for 256 query rows, every operand read feeds two MFMAs, equal work per workgroup).  Shorter ones
-    // do not fill the GPU that way and take one query block per wave, then four waves, then unpaired workgroups.
-    // Measured with 16 heads over 8 KV heads: the eight-wave forms win from three workgroups per four CUs upwards
-    // (6144 tokens: 0.196 against 0.203 ms; 4096: 0.090 against 0.098; 3072: 0.065 against 0.072; at one per two CUs
-    // they lose, 2048 tokens: 0.047 against 0.038), the four-wave ones from one per CU.
-    const int cus = compute_units();
-    auto pairs = [&](int waves, int nq) { const int tpw = 16 * nq * waves / R; return ((T + tpw - 1) / tpw + 1) / 2 * a.num_kv_heads; };
-    int mode = 1;
-    if (4 * pairs(8, 2) >= 3 * cus) mode = 6;
-    else if (4 * pairs(8, 1) >= 3 * cus) mode = 5;
-    else if (pairs(4, 1) >= cus) mode = 2;
-    if ((form >= 1 && form <= 3) || form == 5 || form == 6) mode = form;    // forced by a test (4 is the compressed cache's other kernel)
-    const int waves = mode >= 5 ? 8 : 4;
-    const int nq = (mode == 3 || mode == 6) ? 2 : 1;
-    const bool mirror = mode != 1;
-    const int tpw = 16 * nq * waves / R;
-    const int nblk = (T + tpw - 1) / tpw;
-    const dim3 grid(mirror ? (nblk + 1) / 2 : nblk, a.num_kv_heads), block(waves * kWave);
+    // id: the number the test hook forces the form by
+    static constexpr PrefillForm kForms[] = {
+        {1, 4, 1, 1, 8.3, 0.314, 0.297, 0.0, 0.158}, {2, 8, 1, 2, 9.0, 0.470, 0.758, 0.73, 0.067}, {3, 8, 2, 2, 8.9, 0.878, 1.132, 4.8, 0.0},
+        {5, 8, 1, 1, 7.8, 0.453, 0.582, 0.0, 0.099}, {6, 8, 2, 1, 7.4, 0.800, 0.962, 4.9, 0.021}};
+    const PrefillChoice c = choose_prefill_form(kForms, 5, 0.7, T, R, a.num_kv_heads, form);
+    const dim3 grid(c.mirror ? (c.blocks + 1) / 2 : c.blocks, a.num_kv_heads), block(c.waves * kWave);
     note_scan_kernel("prefill_f16_mfma_kernel");
-#define TW_PF_LAUNCH(RR, NN, MM, WW) launch_scan_kernel(prefill_f16_mfma_kernel<RR, NN, MM, WW>, grid, block, s, a, T)
+#define TW_PF_LAUNCH(RR, NN, WW, KK, MM) launch_scan_kernel(prefill_f16_mfma_kernel<RR, NN, WW, KK, MM>, grid, block, s, a, T)
 #define TW_PF_MODES(RR) \
-    do { if (mode == 1) TW_PF_LAUNCH(RR, 1, false, 4); else if (mode == 2) TW_PF_LAUNCH(RR, 1, true, 4); \
-         else if (mode == 3) TW_PF_LAUNCH(RR, 2, true, 4); else if (mode == 5) TW_PF_LAUNCH(RR, 1, true, 8); \
-         else TW_PF_LAUNCH(RR, 2, true, 8); } while (0)
+    do { if (c.id == 1) TW_PF_LAUNCH(RR, 1, 4, 1, false); else if (c.id == 2) TW_PF_LAUNCH(RR, 1, 8, 2, false); \
+         else if (c.id == 3) TW_PF_LAUNCH(RR, 2, 8, 2, false); \
+         else if (c.id == 5) { if (c.mirror) TW_PF_LAUNCH(RR, 1, 8, 1, true); else TW_PF_LAUNCH(RR, 1, 8, 1, false); } \
+         else { if (c.mirror) TW_PF_LAUNCH(RR, 2, 8, 1, true); else TW_PF_LAUNCH(RR, 2, 8, 1, false); } } while (0)
     if (R == 1) TW_PF_MODES(1); else if (R == 2) TW_PF_MODES(2); else TW_PF_MODES(4);
 #undef TW_PF_MODES
 #undef TW_PF_LAUNCH

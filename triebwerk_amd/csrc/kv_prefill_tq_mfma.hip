@@ -29,31 +29,42 @@ constexpr int kPtVTile = kHeadDim * kPtVRow; // bytes of a V^T tile
 constexpr int kPtVBytes = 3 * kPtVTile;      // 3 tiles, and room for the 128 x 128 fp16 rotation
 static_assert(kPtVBytes >= 2 * kHeadDim * kHeadDim, "the rotation fits");
 
+// a masked score: below the initial maximum by more than the exponent's range, also when a group's first tile is all masked
+constexpr float kMasked = -3.0e38f;
+
 // column of a tile's token in the V^T rows: the contraction slot order of the second MFMA
 __device__ __forceinline__ int vt_slot(int token) { return 8 * ((token & 15) >> 2) + 4 * (token >> 4) + (token & 3); }
 
 }  // namespace
 
-// NQ: 16-row query blocks per wave (every K and V operand read feeds NQ MFMAs).  MIRROR: a workgroup does a
-// token block and then its mirror image from the other end of the sequence.
-// W: waves per workgroup, 4 (two workgroups per CU) or 8 (one: a tile is expanded once for twice the queries).
-template <int R, int BITS, int NQ, bool MIRROR, int W>
+// W: waves per workgroup, 4 (two workgroups per CU) or 8 (one).  NQ: 16-row query blocks per wave (every K and V operand read
+// feeds NQ MFMAs).  KS: groups the waves form.  With one group a tile is brought into LDS once for all query rows of the
+// workgroup; with two, each group takes every other tile of the context for the same query rows (twice the
+// LDS, half the chain of steps) and their sums meet in LDS at the end.  mirror: a workgroup does a token block and then its
+// mirror image from the other end of the sequence.
+template <int R, int BITS, int NQ, int W, int KS>
 __global__ void __launch_bounds__(W* kWave, W == 4 ? 2 : 1)  // two waves per SIMD either way: at most 256 registers per lane
-prefill_tq_mfma_kernel(AttnArgs a, int T) {
-    static_assert(W == 4 || W == 8, "the staging maps are written for 256 and 512 threads");
-    constexpr int TPW = 16 * NQ * W / R;                   // query tokens per workgroup pass
+prefill_tq_mfma_kernel(AttnArgs a, int T, int mirror) {
+    constexpr int GW = W / KS;                             // waves per group
+    static_assert(GW == 4 || GW == 8, "the staging maps are written for 256 and 512 threads");
+    constexpr int TPW = 16 * NQ * GW / R;                  // query tokens per workgroup pass
     constexpr float kAlpha = BITS == 4 ? kAlpha4 : kAlpha2;
     constexpr float kQScale = kLog2e * kInvSqrtD / kAlpha;   // score scale of kernels.cu:1707 in base 2, table scale undone
     constexpr int kHeadBytes = BITS * 16;                  // bytes of one head in a cache row
     constexpr int kEntryDwords = BITS == 4 ? 1 : 2;        // a byte holds 2 (4) codes -> 2 (4) halves
     constexpr int kPtReplicas = BITS == 4 ? 16 : 8;        // copies of the byte -> centroids table (16 KB either way): fewer bank conflicts in the expansion
-    __shared__ __attribute__((aligned(16))) char k_s[2][32 * kPtKRow];
-    __shared__ __attribute__((aligned(16))) char v_s[kPtVBytes];           // 3 V^T tiles; in the epilogue the rotation
-    __shared__ __attribute__((aligned(16))) float n_s[3][2][32];          // [buffer][k | v][token]
+    __shared__ __attribute__((aligned(16))) char k_all[KS][2][32 * kPtKRow];
+    __shared__ __attribute__((aligned(16))) char v_all[KS][kPtVBytes];    // 3 V^T tiles; in the epilogue the rotation, or the groups' sums
+    __shared__ __attribute__((aligned(16))) float n_all[KS][3][2][32];    // [group][buffer][k | v][token]
     __shared__ __attribute__((aligned(8))) uint32_t tab_s[256 * kPtReplicas * kEntryDwords];
 
-    const int tid = threadIdx.x;
-    const int wave = uniform(tid / kWave), lane = tid % kWave;
+    const int tid_wg = threadIdx.x;
+    const int wave_wg = uniform(tid_wg / kWave), lane = tid_wg % kWave;
+    const int grp = KS == 1 ? 0 : wave_wg / GW, wave = KS == 1 ? wave_wg : wave_wg % GW;
+    const int tid = wave * kWave + lane;                   // within the group
+    auto& k_s = k_all[grp];
+    auto& v_s = v_all[grp];
+    float (*n_s)[2][32] = n_all[grp];
     const int ln = lane & 15, kg = lane >> 4;
     const int nblk = (T + TPW - 1) / TPW;
     // Workgroups are dealt to the 8 XCDs in turn (linear id % 8), each with an L2 of its own.  The workgroups of a
@@ -77,7 +88,7 @@ prefill_tq_mfma_kernel(AttnArgs a, int T) {
     constexpr float kRaise = 5.0f;
 
     // ---- table: byte -> its codes' centroids (low field first) as fp16(alpha c), kPtReplicas copies
-    for (int i = tid; i < 256 * kPtReplicas; i += W * kWave) {
+    for (int i = tid_wg; i < 256 * kPtReplicas; i += W * kWave) {
         const int e = i / kPtReplicas;
         if constexpr (BITS == 4) {
             half2_t p = {(half_t)(kAlpha * kCentroids4[e & 15]), (half_t)(kAlpha * kCentroids4[e >> 4])};
@@ -134,7 +145,7 @@ prefill_tq_mfma_kernel(AttnArgs a, int T) {
     const __amdgpu_buffer_rsrc_t knrs = make_rsrc(reinterpret_cast<const char*>(a.k_norms) + kvh * 2, T * nrow_bytes - kvh * 2);
     const __amdgpu_buffer_rsrc_t vnrs = make_rsrc(reinterpret_cast<const char*>(a.v_norms) + kvh * 2, T * nrow_bytes - kvh * 2);
     const int koff0 = sr * row_bytes + kPiece * sc, koff1 = koff0 + 16 * row_bytes;
-    const int voff0 = 2 * vr_ * row_bytes + (W == 4 ? kPiece : kPiece / 2) * vc_, voff1 = voff0 + row_bytes;
+    const int voff0 = 2 * vr_ * row_bytes + (GW == 4 ? kPiece : kPiece / 2) * vc_, voff1 = voff0 + row_bytes;
     const int noff = (tid & 31) * nrow_bytes;
     const __amdgpu_buffer_rsrc_t nrs = (wave & 1) ? vnrs : knrs;     // wave-uniform: a scalar choice
     auto load_codes = [&](__amdgpu_buffer_rsrc_t rs, int voff, int soff) -> uint32_t {
@@ -145,10 +156,12 @@ prefill_tq_mfma_kernel(AttnArgs a, int T) {
         if constexpr (BITS == 4) return __builtin_amdgcn_raw_buffer_load_b16(rs, voff, soff, 0);
         else return __builtin_amdgcn_raw_buffer_load_b8(rs, voff, soff, 0);
     };
+    const int last_tile = (T - 1) & ~31;                   // a tile past the end is this one again (and masked)
     auto load_tile = [&](int tile, Staged& st) {
+        tile = min(tile, last_tile);
         const int toff = tile * row_bytes;
         st.k[0] = load_codes(krs, koff0, toff);
-        if constexpr (W == 4) {
+        if constexpr (GW == 4) {
             st.k[1] = load_codes(krs, koff1, toff);
             st.v[0] = load_codes(vrs, voff0, toff);
             st.v[1] = load_codes(vrs, voff1, toff);
@@ -167,21 +180,21 @@ prefill_tq_mfma_kernel(AttnArgs a, int T) {
         uint32_t e[4];
         expand8(st.k[0], e);
         *reinterpret_cast<uint4*>(&k_s[buf][sr * kPtKRow + 16 * sc]) = uint4{e[0], e[1], e[2], e[3]};
-        if constexpr (W == 4) {
+        if constexpr (GW == 4) {
             expand8(st.k[1], e);
             *reinterpret_cast<uint4*>(&k_s[buf][(sr + 16) * kPtKRow + 16 * sc]) = uint4{e[0], e[1], e[2], e[3]};
         }
         uint32_t va[4], vb[4];
-        if constexpr (W == 4) {
+        if constexpr (GW == 4) {
             expand8(st.v[0], va);
             expand8(st.v[1], vb);
         } else {
             expand4(st.v[0], va);
             expand4(st.v[1], vb);
         }
-        char* dst = &v_s[vbuf * kPtVTile + ((W == 4 ? 8 : 4) * vc_) * kPtVRow + vcol];
+        char* dst = &v_s[vbuf * kPtVTile + ((GW == 4 ? 8 : 4) * vc_) * kPtVRow + vcol];
 #pragma unroll
-        for (int i = 0; i < (W == 4 ? 4 : 2); i++) {       // dims 8c + 2i (low halves) and 8c + 2i + 1 (high halves); 512 threads: 4c + ...
+        for (int i = 0; i < (GW == 4 ? 4 : 2); i++) {       // dims 8c + 2i (low halves) and 8c + 2i + 1 (high halves); 512 threads: 4c + ...
             *reinterpret_cast<uint32_t*>(dst + (2 * i) * kPtVRow) = __builtin_amdgcn_perm(vb[i], va[i], 0x05040100u);
             *reinterpret_cast<uint32_t*>(dst + (2 * i + 1) * kPtVRow) = __builtin_amdgcn_perm(vb[i], va[i], 0x07060302u);
         }
@@ -189,15 +202,15 @@ prefill_tq_mfma_kernel(AttnArgs a, int T) {
     };
     __syncthreads();                                       // the table is there
 
-    // A workgroup takes token block blockIdx.x and its mirror image from the other end, one after the
-    // other: with causal rows the two together cost the same for every workgroup.
-    const int first = blk, second = nblk - 1 - blk;   // without MIRROR: longest blocks first
-    for (int pass = 0; pass < (MIRROR ? 2 : 1); pass++) {
+    // mirror: a workgroup takes a token block and its mirror image from the other end, one after the other: with causal
+    // rows the two together cost the same for every workgroup.
+    const int first = blk, second = nblk - 1 - blk;   // without mirror: longest blocks first
+    for (int pass = 0; pass < (W == 8 && KS == 1 ? 1 + mirror : 1); pass++) {
         if (pass == 1 && second == first) break;           // the middle block of an odd count
         const int tb = pass == 0 ? second : first;         // the long one first
         const int q0 = tb * TPW + 16 * NQ * (wave / R);    // this wave's 16 NQ query tokens
         const int wg_last = min(T, (tb + 1) * TPW) - 1;    // last query token of the pass
-        const int ntiles = (wg_last >> 5) + 1;
+        const int ntiles = ((wg_last >> 5) + KS) / KS;     // steps: a group's tiles are grp, grp + KS, ...
 
         // ---- B operands of the first MFMA: q_rot[q0 + 16 nq + ln][32j + 8kg .. +7], j = 0..3, as an fp16 value
         // and what its rounding left over (scores reach tens of base-2 units on caches with outlier channels,
@@ -272,7 +285,7 @@ prefill_tq_mfma_kernel(AttnArgs a, int T) {
         // than the 226 this kernel already uses with its second set of operands.)
         __syncthreads();                                   // a previous pass may still be reading its last V tile
         Staged st;
-        load_tile(0, st);
+        load_tile(32 * grp, st);
         stash(0, 0, st);
         __syncthreads();
 
@@ -280,12 +293,12 @@ prefill_tq_mfma_kernel(AttnArgs a, int T) {
         bool have_prev = false;
         for (int it = 0; it < ntiles; it++) {
             const int buf = it & 1, nbuf = it % 3;
-            const int tile = 32 * it;
+            const int tile = 32 * (KS * it + grp);
             const bool more = it + 1 < ntiles;
             // the wave's priority falls through the tile (scores 3, P.V 2, softmax 1, hand-over 0): of the two waves of a
             // SIMD the one earlier in its tile goes first; 1.5 % at 8192 tokens, 3 % at 4096
             __builtin_amdgcn_s_setprio(3);
-            if (more) load_tile(tile + 32, st);
+            if (more) load_tile(tile + 32 * KS, st);
 
             const bool active = tile <= q0 + 16 * NQ - 1 && q0 < T;      // the tile reaches this wave's queries (uniform over the wave)
             float4_t s[NQ][2];
@@ -332,7 +345,7 @@ prefill_tq_mfma_kernel(AttnArgs a, int T) {
                         for (int sub = 0; sub < 2; sub++) {
 #pragma unroll
                             for (int i = 0; i < 4; i++) {
-                                if (tile + 16 * sub + 4 * kg + i > tq) x[4 * sub + i] = kNegBig;
+                                if (tile + 16 * sub + 4 * kg + i > tq) x[4 * sub + i] = kMasked;
                             }
                         }
                     }
@@ -374,13 +387,52 @@ prefill_tq_mfma_kernel(AttnArgs a, int T) {
         // out^T = R^T . O^T.  The rotation goes into the V buffers in operand order: 16-byte entry
         // (db * 4 + t) * 64 + lane holds R[k][16 db + ln] for the 8 k that lane (ln, kg) carries in step t,
         // k = 32t + 16 (e / 4) + 4kg + e % 4 -- the dims its accumulators o[.][2t + e / 4][e % 4] belong to.
-        __syncthreads();                                   // every wave is done with the V tiles
+        __syncthreads();                                   // every wave is done with the tiles
+        // two groups: their sums change hands through the V tiles -- with two query blocks group s finishes block s, with one
+        // query block both groups merge the whole of it and each rotates half of the dims -- and the rotation takes the K tiles
+        char* rot_s = KS == 2 ? &k_all[0][0][0] : &v_all[0][0];
+        static_assert(KS == 1 || (sizeof(k_all) >= 2 * kHeadDim * kHeadDim && (int)sizeof(v_all) >= W * kWave * (8 * 16 + 8)), "both fit");
+        float4_t* ex = reinterpret_cast<float4_t*>(&v_all[0][0]);                                  // [wave of the workgroup][8][lane]
+        float2* exml = reinterpret_cast<float2*>(&v_all[0][0] + W * 8 * kWave * 16);               // [wave][lane]: maximum, sum
+        constexpr int NF = KS == 2 ? 1 : NQ;               // query blocks this wave finishes
+        constexpr int NDB = KS == 2 && NQ == 1 ? 4 : 8;    // 16-dim blocks of each
+        const int nq_first = KS == 2 && NQ == 2 ? grp : 0, db_first = KS == 2 && NQ == 1 ? 4 * grp : 0;
+        float lsum[NQ];
+#pragma unroll
+        for (int nq = 0; nq < NQ; nq++) {
+            float l = l_run[nq];
+            l += __shfl_xor(l, 16, 64);
+            l += __shfl_xor(l, 32, 64);
+            lsum[nq] = l;
+        }
+        float4_t of[NF][8];
+        float lf[NF], m_own = 0.0f;
+        if constexpr (KS == 2) {
+            if (grp == 0) {                                // grp is uniform: scalar branches
+#pragma unroll
+                for (int j = 0; j < 8; j++) { ex[(wave_wg * 8 + j) * kWave + lane] = o[NQ - 1][j]; of[0][j] = o[0][j]; }
+                exml[wave_wg * kWave + lane] = float2{m_run[NQ - 1], lsum[NQ - 1]};
+                m_own = m_run[0]; lf[0] = lsum[0];
+            } else {
+#pragma unroll
+                for (int j = 0; j < 8; j++) { ex[(wave_wg * 8 + j) * kWave + lane] = o[0][j]; of[0][j] = o[NQ - 1][j]; }
+                exml[wave_wg * kWave + lane] = float2{m_run[0], lsum[0]};
+                m_own = m_run[NQ - 1]; lf[0] = lsum[NQ - 1];
+            }
+        } else {
+#pragma unroll
+            for (int nq = 0; nq < NQ; nq++) {
+                lf[nq] = lsum[nq];
+#pragma unroll
+                for (int j = 0; j < 8; j++) of[nq][j] = o[nq][j];
+            }
+        }
         {
             // thread -> rows k = 16r + tid / 16, r = 0..7, columns 8c .. 8c + 7 with c = tid % 16; of k only r is
             // not fixed per thread, and r moves the destination by whole steps t = r / 2 and halves 4 (r % 2)
-            const uint4* rsrc = reinterpret_cast<const uint4*>(a.rotation) + tid;
-            const int krow = tid >> 4, c = tid & 15;       // 512 threads: rows k = 32r + tid / 16, r = 0..3
-            char* dst0 = &v_s[(c >> 1) * 4096 + ((krow >> 2) & 3) * 256 + (c & 1) * 128 + 2 * (krow & 3) + (W == 8 ? 8 * (krow >> 4) : 0)];
+            const uint4* rsrc = reinterpret_cast<const uint4*>(a.rotation) + tid_wg;
+            const int krow = tid_wg >> 4, c = tid_wg & 15;       // 512 threads: rows k = 32r + tid / 16, r = 0..3
+            char* dst0 = &rot_s[(c >> 1) * 4096 + ((krow >> 2) & 3) * 256 + (c & 1) * 128 + 2 * (krow & 3) + (W == 8 ? 8 * (krow >> 4) : 0)];
 #pragma unroll
             for (int r = 0; r < 32 / W; r++) {
                 const uint4 rp = rsrc[r * (W * kWave)];
@@ -392,45 +444,56 @@ prefill_tq_mfma_kernel(AttnArgs a, int T) {
             }
         }
         __syncthreads();
-        half8_t oh[NQ][4], ol[NQ][4];
+        if constexpr (KS == 2) {                           // a lane's accumulators all belong to query ln, its maximum and sum too
+            const int other = wave_wg ^ GW;
+            const float2 ml = exml[other * kWave + lane];
+            const float m_new = fmaxf(m_own, ml.x);
+            const float f_own = __builtin_amdgcn_exp2f(m_own - m_new), f_oth = __builtin_amdgcn_exp2f(ml.x - m_new);
+            lf[0] = lf[0] * f_own + ml.y * f_oth;
 #pragma unroll
-        for (int nq = 0; nq < NQ; nq++) {
-            float l = l_run[nq];
-            l += __shfl_xor(l, 16, 64);
-            l += __shfl_xor(l, 32, 64);
-            const float inv = (1.0f / kAlpha) / (l + 1e-8f);
+            for (int j = 0; j < 8; j++) {
+                const float4_t p = ex[(other * 8 + j) * kWave + lane];
+#pragma unroll
+                for (int i = 0; i < 4; i++) of[0][j][i] = of[0][j][i] * f_own + p[i] * f_oth;
+            }
+        }
+        half8_t oh[NF][4], ol[NF][4];
+#pragma unroll
+        for (int nf = 0; nf < NF; nf++) {
+            const float inv = (1.0f / kAlpha) / (lf[nf] + 1e-8f);
 #pragma unroll
             for (int t = 0; t < 4; t++) {
 #pragma unroll
                 for (int e = 0; e < 8; e++) {
-                    const float x = o[nq][2 * t + (e >> 2)][e & 3] * inv;
+                    const float x = of[nf][2 * t + (e >> 2)][e & 3] * inv;
                     const half_t hi = (half_t)x;
-                    oh[nq][t][e] = hi;
-                    ol[nq][t][e] = (half_t)(x - (float)hi);
+                    oh[nf][t][e] = hi;
+                    ol[nf][t][e] = (half_t)(x - (float)hi);
                 }
             }
         }
 #pragma unroll
-        for (int db = 0; db < 8; db++) {
-            float4_t y[NQ];
+        for (int d = 0; d < NDB; d++) {
+            const int db = db_first + d;
+            float4_t y[NF];
 #pragma unroll
-            for (int nq = 0; nq < NQ; nq++) y[nq] = float4_t{0.f, 0.f, 0.f, 0.f};
+            for (int nf = 0; nf < NF; nf++) y[nf] = float4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int t = 0; t < 4; t++) {
-                const half8_t ra = *reinterpret_cast<const half8_t*>(&v_s[((db * 4 + t) * 64 + lane) * 16]);
+                const half8_t ra = *reinterpret_cast<const half8_t*>(&rot_s[((db * 4 + t) * 64 + lane) * 16]);
 #pragma unroll
-                for (int nq = 0; nq < NQ; nq++) {
-                    y[nq] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ra, oh[nq][t], y[nq], 0, 0, 0);
-                    y[nq] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ra, ol[nq][t], y[nq], 0, 0, 0);
+                for (int nf = 0; nf < NF; nf++) {
+                    y[nf] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ra, oh[nf][t], y[nf], 0, 0, 0);
+                    y[nf] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ra, ol[nf][t], y[nf], 0, 0, 0);
                 }
             }
             // lane holds out[tq][head][16 db + 4kg + i], i = 0..3, of its query token tq
 #pragma unroll
-            for (int nq = 0; nq < NQ; nq++) {
-                const int tq = q0 + 16 * nq + ln;
+            for (int nf = 0; nf < NF; nf++) {
+                const int tq = q0 + 16 * (nq_first + nf) + ln;
                 if (tq < T) {
                     const long long col = (long long)head * kHeadDim + 16 * db + 4 * kg;
-                    half_t h[4] = {(half_t)y[nq][0], (half_t)y[nq][1], (half_t)y[nq][2], (half_t)y[nq][3]};
+                    half_t h[4] = {(half_t)y[nf][0], (half_t)y[nf][1], (half_t)y[nf][2], (half_t)y[nf][3]};
                     *reinterpret_cast<uint2*>(a.out + (long long)tq * a.q_stride + col) = *reinterpret_cast<const uint2*>(h);
                 }
             }
@@ -454,27 +517,17 @@ bool prefill_tq_mfma_usable(const AttnArgs& a) {
 void launch_prefill_tq_mfma(const AttnArgs& a, hipStream_t s, int form) {
     const int R = a.num_heads / a.num_kv_heads;
     const int T = a.G;
-    // forms as for the fp16 prefill kernel: long prompts take eight waves per workgroup, two query blocks per wave and
-    // mirrored block pairs; shorter ones one query block per wave, then four waves, then unpaired workgroups
-    const int cus = compute_units();
-    auto pairs = [&](int waves, int nq) { const int tpw = 16 * nq * waves / R; return ((T + tpw - 1) / tpw + 1) / 2 * a.num_kv_heads; };
-    int mode = 1;
-    if (4 * pairs(8, 2) >= 3 * cus) mode = 6;
-    else if (4 * pairs(8, 1) >= 3 * cus) mode = 5;
-    else if (pairs(4, 1) >= cus) mode = 2;
-    if ((form >= 1 && form <= 3) || form == 5 || form == 6) mode = form;    // forced by a test
-    const int waves = mode >= 5 ? 8 : 4;
-    const int nq = (mode == 3 || mode == 6) ? 2 : 1;
-    const bool mirror = mode != 1;
-    const int tpw = 16 * nq * waves / R;
-    const int nblk = (T + tpw - 1) / tpw;
-    const dim3 grid(mirror ? (nblk + 1) / 2 : nblk, a.num_kv_heads), block(waves * kWave);
+    static constexpr PrefillForm kForms[] = {
+        {1, 4, 1, 1, 12.7, 0.785, 0.583, 3.0, 0.242}, {2, 8, 1, 2, 16.6, 0.917, 1.449, 8.8, 0.080}, {3, 8, 2, 2, 18.8, 1.702, 2.150, 6.8, 0.043},
+        {5, 8, 1, 1, 16.3, 0.946, 1.154, 5.5, 0.032}, {6, 8, 2, 1, 18.5, 1.657, 1.869, 7.9, 0.0}};
+    const PrefillChoice c = choose_prefill_form(kForms, 5, 0.97, T, R, a.num_kv_heads, form);
+    const int mirror = c.mirror ? 1 : 0;
+    const dim3 grid(mirror ? (c.blocks + 1) / 2 : c.blocks, a.num_kv_heads), block(c.waves * kWave);
     note_scan_kernel("prefill_tq_mfma_kernel");
-#define TW_PT_LAUNCH(RR, BB, NN, MM, WW) launch_scan_kernel(prefill_tq_mfma_kernel<RR, BB, NN, MM, WW>, grid, block, s, a, T)
+#define TW_PT_LAUNCH(RR, BB, NN, WW, KK) launch_scan_kernel(prefill_tq_mfma_kernel<RR, BB, NN, WW, KK>, grid, block, s, a, T, mirror)
 #define TW_PT_MODES(RR, BB) \
-    do { if (mode == 1) TW_PT_LAUNCH(RR, BB, 1, false, 4); else if (mode == 2) TW_PT_LAUNCH(RR, BB, 1, true, 4); \
-         else if (mode == 3) TW_PT_LAUNCH(RR, BB, 2, true, 4); else if (mode == 5) TW_PT_LAUNCH(RR, BB, 1, true, 8); \
-         else TW_PT_LAUNCH(RR, BB, 2, true, 8); } while (0)
+    do { if (c.id == 1) TW_PT_LAUNCH(RR, BB, 1, 4, 1); else if (c.id == 2) TW_PT_LAUNCH(RR, BB, 1, 8, 2); \
+         else if (c.id == 3) TW_PT_LAUNCH(RR, BB, 2, 8, 2); else if (c.id == 5) TW_PT_LAUNCH(RR, BB, 1, 8, 1); else TW_PT_LAUNCH(RR, BB, 2, 8, 1); } while (0)
 #define TW_PT_BITS(RR) do { if (a.bits == 4) TW_PT_MODES(RR, 4); else TW_PT_MODES(RR, 2); } while (0)
     if (R == 1) TW_PT_BITS(1); else if (R == 2) TW_PT_BITS(2); else TW_PT_BITS(4);
 #undef TW_PT_BITS
