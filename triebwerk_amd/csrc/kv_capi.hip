@@ -337,7 +337,7 @@ int tw_kv_broadcast_rows(void* const* bases, const size_t* seq_bytes, const size
         return -1;
     }
     BroadcastArgs b{};
-    b.src = src; b.dst_begin = dst_begin; b.dst_end = dst_end;
+    b.src = src; b.dst_begin = dst_begin; b.dst_end = dst_end; b.layers = 1;
     for (int i = 0; i < narrays; i++) {
         if (!bases[i] || bytes[i] > seq_bytes[i] || ((reinterpret_cast<uintptr_t>(bases[i]) | seq_bytes[i] | bytes[i]) & 1u)) {
             set_error(1, "tw_kv_broadcast_rows: arrays must be fp16-aligned and T rows must fit a sequence");

@@ -24,6 +24,7 @@
 #include <vector>
 
 #include "../../include/triebwerk_kv.h"
+#include "kv_kernels.hpp"
 
 namespace {
 constexpr int kMaxLayers = 128;  // model.h:9
@@ -766,27 +767,25 @@ int tw_kv_set_trace_ranges(int on) {
 int tw_engine_broadcast_prefix(tw_engine* e, int src, int dst_begin, int dst_end, int T, hipStream_t s) {
     if (!e->arena || src < 0 || src >= e->G || dst_begin < 0 || dst_end > e->G || T < 0 || T > e->batch_msl)
         return -1;
+    if (dst_end < dst_begin) return -2;
     s = pick(e, s);
     e->note_step(s);
+    // one launch: every layer, array and destination (carve() lays the layers out at equal distances)
     const size_t msl = (size_t)e->batch_msl;
-    for (int l = 0; l < e->shape.num_layers; l++) {
-        void* bases[4];
-        size_t seq_bytes[4], bytes[4];
-        int n = 0;
-        for (int which = 0; which < 4; which++) {
-            if (!e->cache[l][which]) continue;
-            size_t row_bytes;
-            if (e->kv_bits == 0) row_bytes = (size_t)e->kv_dim() * 2;
-            else row_bytes = which < 2 ? e->kv_dim_packed() : (size_t)e->shape.num_kv_heads * 2;
-            bases[n] = e->cache[l][which];
-            seq_bytes[n] = msl * row_bytes;
-            bytes[n] = (size_t)T * row_bytes;
-            n++;
-        }
-        // one launch per layer: every array, every destination
-        if (tw_kv_broadcast_rows(bases, seq_bytes, bytes, n, src, dst_begin, dst_end, s) != 0) return -2;
+    twkv::BroadcastArgs b{};
+    b.src = src; b.dst_begin = dst_begin; b.dst_end = dst_end;
+    b.layers = e->shape.num_layers;
+    b.layer_bytes = b.layers > 1 ? (size_t)((char*)e->cache[1][0] - (char*)e->cache[0][0]) : 0;
+    for (int which = 0; which < 4; which++) {
+        if (!e->cache[0][which]) continue;
+        const size_t row_bytes = cache_row_bytes(e, which);
+        b.base[b.narrays] = (char*)e->cache[0][which];
+        b.seq_bytes[b.narrays] = msl * row_bytes;
+        b.bytes[b.narrays] = (size_t)T * row_bytes;
+        b.narrays++;
     }
-    return 0;
+    if (T > 0) twkv::launch_broadcast_rows(b, s);
+    return hipGetLastError() == hipSuccess ? 0 : -2;
 }
 
 }  // extern "C"

@@ -52,10 +52,13 @@ void launch_increment(int* positions, int G, hipStream_t s);
 
 // Rows [0, T) of sequence `src` copied to sequences [dst_begin, dst_end) (src itself skipped) in up to four
 // arrays that are laid out (sequence, row, ...): bytes = T * row bytes, seq_bytes = rows per sequence * row bytes.
+// The same for `layers` layers whose arrays lie layer_bytes apart (one layer: any distance).
 struct BroadcastArgs {
     char* base[4];
     size_t seq_bytes[4];
     size_t bytes[4];
+    int layers;
+    size_t layer_bytes;
     int narrays;
     int src, dst_begin, dst_end;
 };
