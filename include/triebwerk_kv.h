@@ -200,12 +200,13 @@ const char* tw_kv_debug_last_scan_kernel(void);
  * Alignment of the buffers, which the entry point also checks, is not part of it. */
 int tw_kv_decode_step_plan(int G, int num_heads, int num_kv_heads, int bits, int max_seq_len, int ctx_min, int ctx_max);
 /* The same for a caller that hands the step tickets (tw_layer_step_args::tickets; can_share != 0): the one launch may
- * then give a sequence's context to up to eight workgroups where the batch alone leaves compute units idle, which
- * makes it the choice for small batches of long sequences too (16 sequences of 4096 or 8192 tokens). */
+ * then give a sequence's context to up to 64 workgroups where the batch alone leaves compute units idle, which
+ * makes it the choice for small batches of long sequences too (1 sequence of 16000 tokens, 16 of 4096 or 8192), also
+ * ragged ones. */
 int tw_kv_decode_step_plan2(int G, int num_heads, int num_kv_heads, int bits, int max_seq_len, int ctx_min, int ctx_max,
                             int can_share);
 /* Test hook: KV heads per workgroup (0 = automatic; 1, 2, 4, 8) and workgroups per sequence and head group (0 =
- * automatic; 1, 2, 4 -- more than 1 only where the call has tickets) of the one-launch decode step. */
+ * automatic; a power of two up to 64 -- more than 1 only where the call has tickets) of the one-launch decode step. */
 void tw_kv_debug_set_fused_shape(int hkw, int shares);
 /* Layer steps that took the one-launch kernel since the library was loaded (launches issued or recorded into a
  * graph under capture): lets a benchmark say which kernel its figures belong to. */

@@ -232,10 +232,10 @@ void tw_kv_debug_set_num_splits(int n) { g_nsplit_override.store(n); }
 void tw_kv_debug_set_prefill_form(int form) { g_prefill_form.store(form); }
 void tw_kv_debug_set_decode_fused(int mode) { g_decode_fused.store(mode); }
 
-// shares' sums that fit the attention scratch (max_seq_len floats per sequence and head): a power of two up to 8
+// shares' sums that fit the attention scratch (max_seq_len floats per sequence and head): a power of two up to 64
 static int shares_that_fit(int max_seq_len) {
     int n = 1;
-    while (n < 8 && 2 * n * kPartialFloats <= max_seq_len) n *= 2;
+    while (n < 64 && 2 * n * kPartialFloats <= max_seq_len) n *= 2;
     return n;
 }
 
@@ -250,14 +250,19 @@ int tw_kv_decode_step_plan2(int G, int num_heads, int num_kv_heads, int bits, in
     const bool known = ctx_max > 0;
     const int bound = known ? ctx_max : max_seq_len;
     if (bound <= 256 * split) return 1;                           // at most 8 tiles of 32 tokens per wave
-    if (!known || (long long)(ctx_max - ctx_min) * 8 > ctx_max) return 0;   // lengths unknown or ragged: the balanced walk
-    // Equal lengths: the cheaper of the two by estimates fitted to measured launches (microseconds per layer; the
+    if (!known) return 0;                                         // lengths unknown: the balanced walk
+    const bool ragged = (long long)(ctx_max - ctx_min) * 8 > ctx_max;
+    // The cheaper of the two by estimates fitted to measured launches (microseconds per layer; the
     // figures live in one table, plan_constants): one launch as decode_fused_shape counts it (with a sequence's context
     // shared by workgroups where the caller can hand over tickets and the batch alone leaves compute units idle), three
-    // launches as decode_three_estimate_us does.
+    // launches as decode_three_estimate_us does.  Ragged batches take the balanced walk of the three launches, except
+    // small ones whose longest sequence is shared by enough workgroups: that one decides how long the one launch takes,
+    // the mean length the walk.
     const int max_shares = can_share != 0 ? shares_that_fit(max_seq_len) : 1;
-    const double one = decode_fused_shape(G, num_heads, num_kv_heads, bits, allow_pairs, max_shares, ctx_max).us;
-    const double three = decode_three_estimate_us(G, num_kv_heads, bits, ctx_max);
+    const FusedShape shape = decode_fused_shape(G, num_heads, num_kv_heads, bits, allow_pairs, max_shares, ctx_max);
+    if (ragged && shape.shares == 1) return 0;
+    const double one = shape.us;
+    const double three = decode_three_estimate_us(G, num_heads, num_kv_heads, bits, ragged ? 0.5 * (ctx_min + ctx_max) : ctx_max);
     return one <= three ? 1 : 0;
 }
 int tw_kv_decode_step_plan(int G, int num_heads, int num_kv_heads, int bits, int max_seq_len, int ctx_min, int ctx_max) {
@@ -644,7 +649,7 @@ static bool try_decode_fused(const AttnArgs& a, const FusedArgs& f_in, int msl, 
     f.ctx_bound = t_ctx_max > 0 ? (t_ctx_max < msl ? t_ctx_max : msl) : msl;
     if (mode == 2 || g_variant.load() == 1) return false;
     if (!decode_fused_usable(a, f)) return false;
-    // shares: the caller's tickets, and the attention scratch (G * num_heads * msl floats) for up to four shares' sums
+    // shares: the caller's tickets, and the attention scratch (G * num_heads * msl floats) for the shares' sums
     const bool can_share = t_tickets != nullptr && a.ws != nullptr && shares_that_fit(msl) >= 2 &&
                            (reinterpret_cast<uintptr_t>(a.ws) & 3u) == 0;
     f.max_shares = 1;

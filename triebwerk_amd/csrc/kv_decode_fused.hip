@@ -59,7 +59,8 @@ constexpr unsigned kPairTileShare = 32;        // the same with eight waves in a
 constexpr int kFusedMaxQ = 32;                 // query heads of a unit: HKW * R <= 8 * 4
 constexpr int kRowFloats = kHeadDim + 4;       // LDS row of a vector: conflict-free 16-byte accesses
 constexpr int kStageStride = 2 * kHeadDim + 16;   // bytes per staged fp16 vector
-constexpr int kMaxShares = 8;                  // workgroups that may share one sequence's context
+constexpr int kMaxShares = 64;                 // workgroups that may share one sequence's context
+constexpr int kDeviceScope = 16;               // the sc1 bit of a raw buffer access: device scope
 static_assert(8 * (2 + 4) * kStageStride <= kFusedMaxQ * kRowFloats * 4, "staged vectors fit the output rows");
 
 }  // namespace
@@ -67,14 +68,17 @@ static_assert(8 * (2 + 4) * kStageStride <= kFusedMaxQ * kRowFloats * 4, "staged
 // EARLY (PAIR only): waves ask for their first tile in the middle of the prologue; for launches whose waves have few
 // tiles (the host decides from what it knows of the context lengths).  A template parameter because the mere presence
 // of that path, never taken, made the long-context launch 2 us slower.
-// SHARES: f.shares (2, 4 or 8) workgroups share the context of a unit -- for batches whose units alone leave compute units
-// idle.  Share c scans the c-th of f.shares even runs of the sequence's tiles; the last share appends the new row.  Each
+// SHARES: f.shares (a power of two up to 64) workgroups share the context of a unit -- for batches whose units alone leave
+// compute units idle.  Share c scans the c-th of f.shares even runs of the sequence's tiles; the last share appends the new row.  Each
 // leaves its unnormalised sums in memory, draws a ticket, and the workgroup with the last ticket merges all of them (in
 // share order, all read back from memory: the result does not depend on who was last) and finishes the unit.  The
 // hand-over uses device-scope accesses only where they are needed -- the partial sums and the ticket -- and no
 // cache-wide fence: stores with device scope are written through to where every compute unit's device-scope loads look
-// (a release / acquire pair at device scope writes back and invalidates a whole L2 and costs 20 us per launch where this
-// costs 4-9 us with every workgroup of a full-size launch taking part, measured with a stand-alone probe).
+// (a release / acquire pair at device scope writes back and invalidates a whole L2 and costs 20 us per launch; this costs
+// 2.9 us with 2 shares, 3.4 with 8, 4.9 with 32: what 1 sequence of 16001 tokens, 4 bit, 16 heads over 8 KV heads, pays to have
+// 128 workgroups instead of 64 single chunks, a merge launch and a rotation launch -- 19 us per layer against 38; 4 sequences
+// of 8192 tokens 20.9 against 25.3 with 8 shares merged one after the other).
+// (Tried with SHARES: the first tile requested in the middle of the prologue as in EARLY: 4 bit within 1 %, 2 bit 5 % slower.)
 template <int R, int BITS, bool PROD, bool PAIR, bool EARLY, bool SHARES = false>
 __global__ void __launch_bounds__((PAIR ? kPairWaves : kFusedWaves) * kWave)
 decode_fused_kernel(AttnArgs a, FusedArgs f) {
@@ -758,16 +762,20 @@ decode_fused_kernel(AttnArgs a, FusedArgs f) {
             }
         }
         if constexpr (SHARES) {
-            // this share's sums to memory (device scope: written through), then the ticket
+            // this share's sums to memory (device scope: written through), then the ticket.  16-byte accesses with the sc1
+            // bit of device scope; a row of the sums is 128 values, then maximum and sum (and two spare words).
             __shared__ unsigned last_s;
             const long long unit = (long long)g * nhg + hg;
-            auto slot = [&](int sh) -> float* { return f.share_ws + ((unit * nshares + sh) * nv + vec) * kRowFloats; };
-            auto put = [](float* p, float x) { __hip_atomic_store(p, x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
-            auto get = [](const float* p) -> float { return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT); };
+            const __amdgpu_buffer_rsrc_t rs = make_rsrc(reinterpret_cast<const char*>(f.share_ws + unit * nshares * nv * kRowFloats),
+                                                        nshares * nv * kRowFloats * 4);
+            auto row_bytes = [&](int sh, int v) -> int { return (sh * nv + v) * (kRowFloats * 4); };
+            auto bits4 = [](const float4& x) -> uint32x4_t {
+                return uint32x4_t{__float_as_uint(x.x), __float_as_uint(x.y), __float_as_uint(x.z), __float_as_uint(x.w)};
+            };
             if (vec < nv) {
-                float* mine = slot(share);
-                put(mine + k4, av.x); put(mine + k4 + 1, av.y); put(mine + k4 + 2, av.z); put(mine + k4 + 3, av.w);
-                if (k4 == 0) { put(mine + kHeadDim, mg); put(mine + kHeadDim + 1, lsum); }
+                __builtin_amdgcn_raw_buffer_store_b128(bits4(av), rs, row_bytes(share, vec) + 4 * k4, 0, kDeviceScope);
+                if (k4 == 0)
+                    __builtin_amdgcn_raw_buffer_store_b128(bits4(float4{mg, lsum, 0.f, 0.f}), rs, row_bytes(share, vec) + 4 * kHeadDim, 0, kDeviceScope);
             }
             __builtin_amdgcn_s_waitcnt(0);          // every store of this wave has been acknowledged
             __syncthreads();
@@ -778,26 +786,61 @@ decode_fused_kernel(AttnArgs a, FusedArgs f) {
             __syncthreads();
             if (!last_s) return;                    // uniform over the workgroup: the last share finishes the unit
             if (tid == 0) __hip_atomic_store(f.tickets + unit, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // for the next launch
-            if (vec < nv) {
-                float ms[kMaxShares], ls[kMaxShares];
-                float4 as[kMaxShares];
-                mg = kNegBig;
-                for (int sh = 0; sh < nshares; sh++) {
-                    const float* p = slot(sh);
-                    as[sh] = float4{get(p + k4), get(p + k4 + 1), get(p + k4 + 2), get(p + k4 + 3)};
-                    ms[sh] = get(p + kHeadDim);
-                    ls[sh] = get(p + kHeadDim + 1);
-                    mg = fmaxf(mg, ms[sh]);
+            // The slots of 32 threads that the unit's vectors leave free take a part of the shares each (slot = (part, vector),
+            // shares part, part + nsub, ...), eight shares' loads in flight at a time -- one share after the other costs
+            // a trip to memory each -- and the parts meet in LDS, where the waves' partial sums were.  All orders
+            // are fixed by the shape alone.
+            constexpr int kSlots = NW * kWave / 32;
+            const int nsub = min(kSlots, kParts * R) / nv;                 // nv is a power of two, at most both
+            const int mv = vec & (nv - 1), msub = vec / nv;
+            float (*sum_s)[kRowFloats] = &part_s[0][0];
+            if (msub < nsub) {
+                float m = kNegBig, l = 0.0f;
+                float4 acc = {0.f, 0.f, 0.f, 0.f};
+                for (int s0 = msub; s0 < nshares; s0 += 8 * nsub) {
+                    uint32x4_t ml[8], x[8];
+#pragma unroll
+                    for (int j = 0; j < 8; j++) {
+                        const int at = row_bytes(min(s0 + j * nsub, nshares - 1), mv);
+                        ml[j] = __builtin_amdgcn_raw_buffer_load_b128(rs, at + 4 * kHeadDim, 0, kDeviceScope);
+                        x[j] = __builtin_amdgcn_raw_buffer_load_b128(rs, at + 4 * k4, 0, kDeviceScope);
+                    }
+                    float mb = m;
+#pragma unroll
+                    for (int j = 0; j < 8; j++) {
+                        if (s0 + j * nsub >= nshares) ml[j] = uint32x4_t{__float_as_uint(kNegBig), 0u, 0u, 0u};
+                        mb = fmaxf(mb, __uint_as_float(ml[j][0]));
+                    }
+                    const float fo = __builtin_amdgcn_exp2f(m - mb);
+                    l *= fo; acc.x *= fo; acc.y *= fo; acc.z *= fo; acc.w *= fo;
+                    m = mb;
+#pragma unroll
+                    for (int j = 0; j < 8; j++) {
+                        const float fs = s0 + j * nsub < nshares ? __builtin_amdgcn_exp2f(__uint_as_float(ml[j][0]) - m) : 0.0f;
+                        l = __builtin_fmaf(__uint_as_float(ml[j][1]), fs, l);
+                        acc.x = __builtin_fmaf(__uint_as_float(x[j][0]), fs, acc.x);
+                        acc.y = __builtin_fmaf(__uint_as_float(x[j][1]), fs, acc.y);
+                        acc.z = __builtin_fmaf(__uint_as_float(x[j][2]), fs, acc.z);
+                        acc.w = __builtin_fmaf(__uint_as_float(x[j][3]), fs, acc.w);
+                    }
                 }
-                lsum = 0.0f;
+                *reinterpret_cast<float4*>(&sum_s[vec][k4]) = acc;
+                if (k4 == 0) { sum_s[vec][kHeadDim] = m; sum_s[vec][kHeadDim + 1] = l; }
+            }
+            lds_barrier();
+            if (vec < nv) {
+                mg = kNegBig; lsum = 0.0f;
                 av = float4{0.f, 0.f, 0.f, 0.f};
-                for (int sh = 0; sh < nshares; sh++) {
-                    const float fs = __builtin_amdgcn_exp2f(ms[sh] - mg);
-                    lsum = __builtin_fmaf(ls[sh], fs, lsum);
-                    av.x = __builtin_fmaf(as[sh].x, fs, av.x);
-                    av.y = __builtin_fmaf(as[sh].y, fs, av.y);
-                    av.z = __builtin_fmaf(as[sh].z, fs, av.z);
-                    av.w = __builtin_fmaf(as[sh].w, fs, av.w);
+                for (int u = 0; u < nsub; u++) mg = fmaxf(mg, sum_s[u * nv + vec][kHeadDim]);
+                for (int u = 0; u < nsub; u++) {
+                    const float* pr = &sum_s[u * nv + vec][0];
+                    const float fs = __builtin_amdgcn_exp2f(pr[kHeadDim] - mg);
+                    const float4 c = *reinterpret_cast<const float4*>(pr + k4);
+                    lsum = __builtin_fmaf(pr[kHeadDim + 1], fs, lsum);
+                    av.x = __builtin_fmaf(c.x, fs, av.x);
+                    av.y = __builtin_fmaf(c.y, fs, av.y);
+                    av.z = __builtin_fmaf(c.z, fs, av.z);
+                    av.w = __builtin_fmaf(c.w, fs, av.w);
                 }
             }
         }
@@ -855,11 +898,13 @@ static bool pairs_fit(int bits, int R, int hkw) {
 }
 bool decode_fused_pairs(const AttnArgs& a, int hkw) { return pairs_fit(a.bits, a.num_heads / a.num_kv_heads, hkw); }
 
-// The measured figures behind the estimates below.  MI355X: launches at batches 8 to 256 and contexts 1k to 8k
-// reproduce within 5 %; hand-over costs from a probe in which all 512 workgroups of a streaming launch take part.
+// The measured figures behind the estimates below, fitted to 390 launches on MI355X (batches 1 to 256, contexts 300 to 16001, all
+// shapes of a launch, 1 to 64 shares): 4.6 % root mean square.  The shape with the smallest estimate is the fastest
+// measured one or within 3 % of it in 31 of 36 cases (the others within 7.5 %).
 namespace {
 constexpr PlanConstants kPlanTable[] = {
-    {"gfx950", 12.0, {3.08, 2.72}, 2.45, {5.95, 4.68}, {7200.0, 5500.0}, {27.0, 25.0}, {7.2e6, 5.4e6}, {0.0, 3.7, 5.4, 8.7}},
+    {"gfx950", {10.8, 11.3}, {{{1.60, 1.93, 3.02}, {0.80, 1.25, 1.65}}, {{1.73, 2.11, 2.91}, {2.03, 1.58, 2.17}}},
+     {{7.4e6, 5.1e6}, {4.9e6, 3.4e6}}, {0.0, 2.9, 3.2, 3.4, 4.1, 4.9, 6.5}, {27.0, 25.0}, 2.5, {7.0e6, 5.4e6}},
 };
 }  // namespace
 const PlanConstants& plan_constants() {
@@ -879,31 +924,30 @@ const PlanConstants& plan_constants() {
     return *chosen;
 }
 
-// Microseconds one launch takes for G sequences of ctx tokens with hkw KV heads per workgroup, by a count fitted to
-// measured launches (plan_constants): the workgroups run in rounds of one per CU; a round costs its fixed part and,
-// per token of context, the cube-root sum of what one CU sustains for the workgroup's heads (a workgroup whose waves
-// scan one head each moves its bytes at about half the rate of one whose waves scan two) and of the whole chip's rate
-// for all the workgroups of the round.
+// Microseconds one launch takes for G sequences of ctx tokens with hkw KV heads per workgroup: the workgroups run in
+// rounds of one per CU, and a round costs its fixed part and the cube-root sum of its waves' tiles, one after the other,
+// and of all its bytes at the rate the chip streams them in this pattern (waves with one head each: half lines).
 double decode_fused_estimate_us(int G, int num_heads, int Hk, int bits, bool allow_pairs, int hkw, double ctx) {
     const PlanConstants& pc = plan_constants();
     const double cus = compute_units();
     const int R = Hk > 0 ? num_heads / Hk : 1;
-    const int w = bits == 4 ? 0 : 1;
+    const int w = bits == 4 ? 0 : 1, r = R >= 4 ? 2 : R >= 2 ? 1 : 0;
     const double bpt = bits == 4 ? 132.0 : 68.0;                  // bytes per token and KV head: K and V codes and norms
     const double units = (double)G * (Hk / hkw);
     const double rounds = std::ceil(units / cus), active = units < cus ? units : cus;
     const bool pair = allow_pairs && pairs_fit(bits, R, hkw);
-    const double per_head_ns = pair ? (bits == 2 && hkw >= 4 ? pc.pair_wide2_ns : pc.pair_ns[w]) : pc.single_ns[w];
-    const double k_cu = hkw * per_head_ns, k_bw = active * hkw * bpt / pc.one_bw[w];   // ns per token
-    return rounds * (pc.one_fixed_us + ctx * 1e-3 * std::cbrt(k_cu * k_cu * k_cu + k_bw * k_bw * k_bw));
+    const int parts = (pair ? 2 * kPairWaves : kFusedWaves) / hkw;          // waves that share a head's tiles
+    const double tiles = std::ceil(std::ceil(ctx / 32.0) / parts) * pc.tile_us[pair ? 0 : 1][w][r];
+    const double bytes = active * hkw * bpt * ctx / pc.one_bw[pair ? 0 : 1][w];
+    return rounds * (pc.one_fixed_us[pair ? 0 : 1] + std::cbrt(tiles * tiles * tiles + bytes * bytes * bytes));
 }
 
 // Three launches (rotation, scan, merge) for the same step: their fixed cost and the scan at its rate.
-double decode_three_estimate_us(int G, int Hk, int bits, double ctx) {
+double decode_three_estimate_us(int G, int num_heads, int Hk, int bits, double ctx) {
     const PlanConstants& pc = plan_constants();
     const int w = bits == 4 ? 0 : 1;
     const double bpt = bits == 4 ? 132.0 : 68.0;
-    return pc.three_fixed_us[w] + (double)G * Hk * bpt * ctx / pc.three_bw[w];
+    return pc.three_fixed_us[w] + (num_heads >= 4 * Hk ? pc.three_gqa4_us : 0.0) + (double)G * Hk * bpt * ctx / pc.three_bw[w];
 }
 
 // KV heads per workgroup (8, 4, 2 or 1): the choice with the smallest estimate at a context of 4096 tokens (the order

@@ -200,7 +200,7 @@ struct FusedArgs {
     int hkw;                // KV heads per workgroup (launch_decode_fused fills this in)
     float q_scale;          // likewise
     // A unit's context shared by several workgroups, for batches whose units alone leave compute units idle:
-    int shares;             // 1, 2, 4 or 8 (launch_decode_fused fills this in; > 1 only with the three below)
+    int shares;             // a power of two up to 64 (launch_decode_fused fills this in; > 1 only with the three below)
     int max_shares;         // as many shares as share_ws has room for (1: none)
     float* share_ws;        // G * num_heads * max_shares * (kHeadDim + 4) floats for the shares' unnormalised sums
     unsigned* tickets;      // one word per (sequence, KV head): zero before the first launch, left zero by every launch
@@ -219,14 +219,14 @@ struct FusedArgs {
 // use that number; tests/test_gpu_plan.py checks on the GPU at hand that the automatic choice is the faster form.
 struct PlanConstants {
     const char* device;         // substring of hipDeviceProp_t::gcnArchName
-    double one_fixed_us;        // one launch: prologue, first tile, epilogue, launch and drain
-    double pair_ns[2];          // ns per token and KV head one compute unit sustains, waves with two heads: [4 bit, 2 bit]
-    double pair_wide2_ns;       // the same at 2 bit with four or more heads per workgroup
-    double single_ns[2];        // waves with one head each
-    double one_bw[2];           // bytes per us the whole chip streams in the one-launch pattern
+    // one launch; first index: waves that scan two KV heads, one head
+    double one_fixed_us[2];     // prologue, first tile, epilogue, launch and drain
+    double tile_us[2][2][3];    // a wave's tile of 32 tokens, the waves of a compute unit side by side: [4 bit, 2 bit][GQA group 1, 2, 4]
+    double one_bw[2][2];        // bytes per us the whole chip streams: [4 bit, 2 bit]
+    double handover_us[7];      // shares' sums through memory, by log2(shares)
     double three_fixed_us[2];   // three launches: rotation, merge, launches and the scan's start and end
+    double three_gqa4_us;       // more with four query heads per KV head
     double three_bw[2];         // bytes per us of the scan
-    double handover_us[4];      // shares' sums through memory, by log2(shares)
 };
 const PlanConstants& plan_constants();
 bool decode_fused_usable(const AttnArgs& a, const FusedArgs& f);
@@ -234,7 +234,7 @@ int decode_fused_heads_per_workgroup(int G, int num_heads, int num_kv_heads, int
 // estimated microseconds of one launch with hkw KV heads per workgroup, all sequences at ctx tokens
 double decode_fused_estimate_us(int G, int num_heads, int num_kv_heads, int bits, bool allow_pairs, int hkw, double ctx);
 // estimated microseconds of the same step as three launches (rotation, scan, merge)
-double decode_three_estimate_us(int G, int num_kv_heads, int bits, double ctx);
+double decode_three_estimate_us(int G, int num_heads, int num_kv_heads, int bits, double ctx);
 // The launch's shape when a unit's context may be shared by up to max_shares workgroups (1: the caller has no tickets
 // or no room for the shares' sums): KV heads per workgroup, shares, and the estimate for sequences of ctx tokens.
 struct FusedShape { int hkw, shares; double us; };
