@@ -22,6 +22,7 @@ ORACLE_LIB = ORACLE_DIR / "libkv_oracle.so"
 
 SOURCES = [
     "kv_append.hip",
+    "kv_append_tokens.hip",
     "kv_attention_valu.hip",
     "kv_attention_mfma.hip",
     "kv_attention_pair.hip",

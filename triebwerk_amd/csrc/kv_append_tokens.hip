@@ -1,0 +1,263 @@
+// kv_append_tokens.hip -- the compressed append of a prompt's rows (turbo_kv_quantize_kernel, kernels.cu:1482-1559), with
+// the producers of q and k on the way (qk_norm_batch, rope_batch, 880-961), in one launch (gfx950).
+//
+// rotate_kernel (kv_rotate.hip) gives every wave 16 output coordinates of its vectors and nothing to share: right for the
+// few vectors of a decode step, but each vector is then fetched, transformed, measured and regrouped eight times.  Here a
+// workgroup of four waves takes a tile of 16 vectors at a time, once:
+//   - 16 lanes to a vector, 16 bytes each: RMSNorm and rotation (K), the norm, and the unit vector into LDS as fp32,
+//     regrouped for the matrix cores (coordinate 4s + kk at kk * 32 + s); K goes back to its row as the producers leave it;
+//   - wave w rotates the tile for output coordinates 16w .. 16w + 15 and 64 + 16w ...: two chains of
+//     v_mfma_f32_16x16x4_f32 in rotate_kernel's order of k, hence its bits; codes meet in LDS and leave 16 lanes to a vector.
+// One barrier per tile: tile i is rotated while tile i + 1 is transformed and the codes of tile i - 1 are stored.
+// The matrix cores bound it: 16 x 128 x 128 products per tile at 256 fp32 operations per cycle and compute unit, 14 us for
+// the 65776 vectors of 4111 tokens and 8 KV heads.  Other workgroups of the same launch transform the queries, a
+// matter of memory alone, beside them.
+// 8192 tokens, 8 KV heads, 4 bit: 47.4 us against rotate_kernel's 79.7 (2 bit 47.4 against 70.6); 4111 tokens 28.6 against 43.
+
+#include <algorithm>
+
+#include "kv_common.hpp"
+#include "kv_kernels.hpp"
+#include "kv_mfma_util.hpp"
+#include "kv_producer_rows.hpp"
+#include "kv_rotate_util.hpp"
+
+namespace twkv {
+
+namespace {
+
+constexpr int kTileVecs = 16;
+constexpr int kUnitRow = kHeadDim + 4;         // floats per unit vector in LDS: 16 lanes' 16-byte reads touch every bank once
+constexpr int kAppendWaves = 4;
+static_assert(kAppendWaves * kWave == kProducerThreads && 2 * kTileVecs * kUnitRow >= kAppendWaves * kOperandTileDwords,
+              "the space of the unit vectors first holds a wave's 16 rows of R each");
+
+// Decision boundaries of turbo_quantize (kernels.cu:1448-1473) and their buckets: boundary i lies in a bucket of its own, at
+// least 0.15 bucket widths from the bucket's edges, far more than bucket_of rounds.
+constexpr float kEdges4[15] = {-0.21224f, -0.16299f, -0.12701f, -0.09715f, -0.07068f, -0.04619f, -0.02284f, 0.00000f,
+                                0.02284f,  0.04619f,  0.07068f,  0.09715f,  0.12701f,  0.16299f,  0.21224f};
+constexpr int kBuckets = 32;
+constexpr float kBucketScale = 72.30f, kBucketShift = 16.50f;
+// (the smaller bound comes last: a NaN ends up in the last bucket)
+__host__ __device__ __forceinline__ int bucket_of(float x) {
+    return (int)fmaxf(fminf(__builtin_fmaf(x, kBucketScale, kBucketShift), (float)(kBuckets - 1)), 0.0f);
+}
+
+}  // namespace
+
+template <int BITS, bool PROD>
+__global__ void __launch_bounds__(kAppendWaves* kWave, 3)
+append_tokens_kernel(AppendTokensArgs a) {
+    constexpr int kHeadBytes = kHeadDim * BITS / 8;
+    constexpr int kCodeRow = kHeadBytes + 4;           // bytes per vector of codes in LDS
+    __shared__ __attribute__((aligned(16))) float u_s[2][kTileVecs][kUnitRow];
+    __shared__ __attribute__((aligned(8))) float2 bucket_s[kBuckets];
+    __shared__ __attribute__((aligned(16))) char code_s[2][kTileVecs][kCodeRow];
+
+    // workgroups in turn: a tile run of K and V, a run of queries, until one kind is used up
+    int b = (int)blockIdx.x;
+    if (PROD) {
+        const int both = min(a.kv_blocks, a.q_blocks);
+        const bool is_q = b < 2 * both ? (b & 1) != 0 : a.q_blocks > a.kv_blocks;
+        b = b < 2 * both ? b >> 1 : b - both;
+        if (is_q) {
+            producer_rows(a.p, (long long)b * kProducerVecs, a.p.num_heads);
+            return;
+        }
+    }
+    const int tid = threadIdx.x;
+    const int wave = uniform(tid / kWave), lane = tid % kWave;
+    const int i16 = lane & 15, kk = lane >> 4;
+    const int vl = tid >> 4, c = tid & 15;             // vector of the tile and piece of it this thread carries
+    const int Hk = a.p.num_kv_heads;
+    const unsigned per_row = (unsigned)(Hk * a.nstreams);
+    const int nvec = a.p.rows * (int)per_row;
+    const int tile0 = b * a.nper, ntiles = min(a.nper, (nvec + kTileVecs - 1) / kTileVecs - tile0);
+    const bool normed = PROD && a.p.norm, roped = PROD && a.p.cos_table != nullptr;
+
+    // The vector a thread carries, tile by tile: 16 vectors on is q16 rows and r16 heads on.  Past the end: the last row, not stored.
+    struct Vec { int row, h, v; };
+    const int q16 = kTileVecs / (int)per_row, r16 = kTileVecs % (int)per_row;
+    auto advance = [&](const Vec& x) -> Vec {
+        Vec r = {x.row + q16, x.h + r16, x.v + kTileVecs};
+        if (r.h >= (int)per_row) { r.h -= (int)per_row; r.row++; }
+        return r;
+    };
+    const int end_v = min(nvec, (tile0 + ntiles) * kTileVecs);
+    auto row_of = [&](const Vec& x) -> int { return min(x.row, a.p.rows - 1); };
+    // Requests run ahead of their use: the position three tiles, the vector and its table rows two.
+    struct Request { uint4 x, cp, sp; };
+    auto request_pos = [&](const Vec& x) -> int { return a.p.positions[row_of(x)]; };
+    auto request = [&](const Vec& x, int pos) -> Request {
+        Request q{};
+        const half_t* src = (x.h >= Hk ? a.p.v - (long long)Hk * kHeadDim : a.p.k) + (long long)row_of(x) * a.p.kv_stride + x.h * kHeadDim;
+        q.x = reinterpret_cast<const uint4*>(src)[c];
+        if (roped && x.h < Hk) {
+            const long long at = (long long)pos * (a.p.rope_dim >> 4) + rope_piece16(c, a.p.rope_dim);
+            q.cp = reinterpret_cast<const uint4*>(a.p.cos_table)[at];
+            q.sp = reinterpret_cast<const uint4*>(a.p.sin_table)[at];
+        }
+        return q;
+    };
+
+    Vec x0;
+    x0.v = tile0 * kTileVecs + vl;
+    x0.row = (int)((unsigned)x0.v / per_row);
+    x0.h = (int)((unsigned)x0.v - (unsigned)x0.row * per_row);
+    Vec x1 = advance(x0), x2 = advance(x1);
+    int pos0 = request_pos(x0), pos1 = request_pos(x1), pos2 = request_pos(x2);
+    // 4 bit: a value's code from its bucket -- the buckets are narrower than the gaps between the decision boundaries, so at most
+    // one boundary lies in each -- instead of 15 comparisons: {boundary, codes below it} of bucket tid
+    if (BITS == 4 && tid < kBuckets) {
+        float lim = 3.0e38f;
+        int below = 0;
+#pragma unroll
+        for (int i = 0; i < 15; i++) {
+            if (bucket_of(kEdges4[i]) == tid) lim = kEdges4[i];
+            if (bucket_of(kEdges4[i]) < tid) below++;
+        }
+        bucket_s[tid] = float2{lim, __builtin_bit_cast(float, below)};
+    }
+    uint4 rraw[2][4];
+#pragma unroll
+    for (int d = 0; d < 2; d++)
+#pragma unroll
+        for (int j = 0; j < 4; j++)
+            rraw[d][j] = reinterpret_cast<const uint4*>(a.rotation + (wave + 4 * d) * 16 * kHeadDim)[j * kWave + lane];
+    uint4 kw{};
+    if (normed) kw = reinterpret_cast<const uint4*>(a.p.k_weight)[c];
+    Request cur = request(x0, pos0);
+    float rv[2][32];                                   // R[16 * (wave + 4 d) + i16][4s + kk]
+    {
+        uint32_t* mine = reinterpret_cast<uint32_t*>(&u_s[0][0][0]) + wave * kOperandTileDwords;
+#pragma unroll
+        for (int d = 0; d < 2; d++) {
+            stage_operand_tile(mine, rraw[d], lane);
+            lds_barrier();
+            read_operand_tile(mine, lane, rv[d]);
+            lds_barrier();
+        }
+    }
+
+    // transform, measure and regroup the vector piece of tile i
+    auto fill = [&](int buf, const Vec& r, int pos, const Request& q) {
+        float x[8], t[8];
+        unpack_halves(q.x, x);
+        const bool live = r.v < end_v, is_v = r.h >= Hk;
+        if (PROD && !is_v) {                           // the same for the 16 lanes of a vector
+            if (normed) norm_head16(x, kw, a.p.eps, a.p.biased);
+            if (roped) rope_head16(x, q.cp, q.sp, c, a.p.rope_dim, 0);
+            if (live) reinterpret_cast<uint4*>(a.p.k + (long long)r.row * a.p.kv_stride + r.h * kHeadDim)[c] = pack_halves(x);
+        }
+#pragma unroll
+        for (int e = 0; e < 8; e++) t[e] = x[e] * x[e];                // exact: fp16 values
+        const float norm = sqrtf(head_tree_sum16(t) + 1e-12f);
+        const float inv = 1.0f / norm;
+        float* dst = &u_s[buf][vl][2 * c];
+#pragma unroll
+        for (int e = 0; e < 4; e++) *reinterpret_cast<float2*>(dst + 32 * e) = float2{x[e] * inv, x[e + 4] * inv};
+        if (live && c == 0) {
+            const long long crow = (long long)r.row * a.seq_stride_rows + pos;
+            (is_v ? a.norms[1] : a.norms[0])[crow * Hk + (is_v ? r.h - Hk : r.h)] = (half_t)norm;
+        }
+    };
+    auto store_codes = [&](int buf, const Vec& r, int pos) {
+        if (r.v >= end_v) return;
+        const bool is_v = r.h >= Hk;
+        const long long crow = (long long)r.row * a.seq_stride_rows + pos;
+        uint8_t* dst = (is_v ? a.codes[1] : a.codes[0]) + (crow * Hk + (is_v ? r.h - Hk : r.h)) * kHeadBytes + c * BITS;
+        const char* src = &code_s[buf][vl][c * BITS];
+        if (BITS == 4) *reinterpret_cast<uint32_t*>(dst) = *reinterpret_cast<const uint32_t*>(src);
+        else *reinterpret_cast<uint16_t*>(dst) = *reinterpret_cast<const uint16_t*>(src);
+    };
+    auto quantize = [&](float val) -> uint32_t {
+        if constexpr (BITS == 4) {                     // (a NaN takes the last bucket, whose comparison it passes: 15, as turbo_quantize)
+            const float2 e = bucket_s[bucket_of(val)];
+            return __builtin_bit_cast(uint32_t, e.y) + (!(val < e.x) ? 1u : 0u);
+        } else {
+            return (uint32_t)turbo_quantize(val, 2);
+        }
+    };
+
+    Request next = request(x1, pos1);
+    fill(0, x0, pos0, cur);
+    Vec xs = x0, xf = x0;                              // whose codes are stored next; whose piece was filled in last
+    int ps = pos0, pf = pos0;
+    for (int i = 0;; i++) {
+        lds_barrier();      // tile i and the codes of tile i - 1 are complete; tile i - 1 and the codes of i - 2 have been read
+        if (i > 0) store_codes((i - 1) & 1, xs, ps);
+        if (i == ntiles) break;
+        xs = xf; ps = pf;
+        if (i + 1 < ntiles) {
+            const Request now = next;
+            xf = x1; pf = pos1;
+            next = request(x2, pos2);
+            x1 = x2; pos1 = pos2;
+            x2 = advance(x2);
+            pos2 = request_pos(x2);
+            fill((i + 1) & 1, xf, pf, now);
+        }
+        float4_t acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+        const float* urow = &u_s[i & 1][i16][32 * kk];
+#pragma unroll
+        for (int t = 0; t < 8; t++) {
+            const float4 u = *reinterpret_cast<const float4*>(urow + 4 * t);
+            const float uv[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+#pragma unroll
+                for (int d = 0; d < 2; d++) acc[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(rv[d][4 * t + j], uv[j], acc[d], 0, 0, 0);
+        }
+#pragma unroll
+        for (int d = 0; d < 2; d++) {                  // lane: coordinates 16 (wave + 4d) + 4kk .. + 3 of vector i16
+            uint32_t packed = 0;
+#pragma unroll
+            for (int r = 0; r < 4; r++) packed |= quantize(acc[d][r]) << (r * BITS);
+            char* dst = &code_s[i & 1][i16][((wave + 4 * d) * 4 + kk) * (BITS / 2)];
+            if (BITS == 4) *reinterpret_cast<uint16_t*>(dst) = (uint16_t)packed;
+            else *reinterpret_cast<uint8_t*>(dst) = (uint8_t)packed;
+        }
+    }
+}
+
+bool append_tokens_usable(const AppendTokensArgs& a) {
+    auto ok = [](const void* p, unsigned m) { return (reinterpret_cast<uintptr_t>(p) & m) == 0; };
+    const bool prod = a.p.norm || a.p.cos_table;
+    if (prod && !producer_rows_usable(a.p)) return false;
+    for (int s = 0; s < a.nstreams; s++)
+        if (!ok(a.codes[s], 3u) || !ok(a.norms[s], 1u)) return false;
+    return ok(a.p.k, 15u) && (a.nstreams < 2 || ok(a.p.v, 15u)) && ok(a.rotation, 15u) && (a.p.kv_stride & 7) == 0 &&
+           (long long)a.p.rows * a.p.num_kv_heads * a.nstreams < (1LL << 30) && (long long)a.p.rows * a.p.num_heads < (1LL << 31);
+}
+
+void launch_append_tokens(const AppendTokensArgs& args, int bits, hipStream_t s) {
+    AppendTokensArgs a = args;
+    const bool prod = a.p.norm || a.p.cos_table;
+    const int tiles = (a.p.rows * a.p.num_kv_heads * a.nstreams + kTileVecs - 1) / kTileVecs;
+    if (tiles <= 0) return;
+    // One tile per workgroup while there are fewer than four workgroups per compute unit, then up to four: a workgroup's start
+    // (R, the first loads) is worth a tile, but a few workgroups more than four rounds' worth cost a whole round
+    // (2000 tiles, 4 bit: 17.0, 15.2, 16.4 us with 1, 2, 3 tiles each; 4111: 32.5, 29.7, 28.6, 31.3 with 1 to 4; 8192: 57, 49.5, 49.5,
+    // 47.4, and 47.6 with 8).
+    a.nper = std::max(1, std::min(4, (tiles + 1023) / 1365));
+    a.kv_blocks = (tiles + a.nper - 1) / a.nper;
+    a.q_blocks = prod ? (int)(((long long)a.p.rows * a.p.num_heads + kProducerVecs - 1) / kProducerVecs) : 0;
+    // queries beside the tiles while everything runs at once; beyond that the low occupancy of this kernel costs them more than
+    // a launch of their own
+    if (prod && a.kv_blocks + a.q_blocks > 3 * compute_units()) {
+        ProducerArgs q = a.p;
+        q.num_kv_heads = 0;
+        launch_producer(q, s);
+        a.q_blocks = 0;
+    }
+    const dim3 grid(a.kv_blocks + a.q_blocks), block(kAppendWaves * kWave);
+    if (bits == 4) {
+        if (prod) hipLaunchKernelGGL((append_tokens_kernel<4, true>), grid, block, 0, s, a);
+        else hipLaunchKernelGGL((append_tokens_kernel<4, false>), grid, block, 0, s, a);
+    } else {
+        if (prod) hipLaunchKernelGGL((append_tokens_kernel<2, true>), grid, block, 0, s, a);
+        else hipLaunchKernelGGL((append_tokens_kernel<2, false>), grid, block, 0, s, a);
+    }
+}
+
+}  // namespace twkv

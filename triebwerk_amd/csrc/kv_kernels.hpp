@@ -91,6 +91,20 @@ struct ProducerArgs {
     long long seq_stride_rows;
 };
 void launch_producer(const ProducerArgs& a, hipStream_t s);
+bool producer_rows_usable(const ProducerArgs& a);   // pointers and strides admit 16-byte accesses
+
+// Compressed append of many rows, optionally with the producers of q and k (kv_append_tokens.hip)
+struct AppendTokensArgs {
+    ProducerArgs p;          // p.k, p.v: the rows of streams 0 and 1; p.norm / p.cos_table: q and k transformed in place
+    int nstreams;
+    uint8_t* codes[2];
+    half_t* norms[2];
+    const half_t* rotation;
+    long long seq_stride_rows;   // row r goes to cache row r * seq_stride_rows + positions[r]
+    int nper, kv_blocks, q_blocks;   // launch_append_tokens fills these in
+};
+bool append_tokens_usable(const AppendTokensArgs& a);
+void launch_append_tokens(const AppendTokensArgs& a, int bits, hipStream_t s);
 // data[r][i] = half(data[r][i] / (1 + exp(-gate[r][i]))), rows of `dim` halves with their own strides
 void launch_sigmoid_gate(half_t* data, long long data_stride, const half_t* gate, long long gate_stride, int dim,
                          int rows, hipStream_t s);

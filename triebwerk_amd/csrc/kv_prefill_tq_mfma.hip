@@ -56,7 +56,7 @@ prefill_tq_mfma_kernel(AttnArgs a, int T, int mirror) {
     __shared__ __attribute__((aligned(16))) char k_all[KS][2][32 * kPtKRow];
     __shared__ __attribute__((aligned(16))) char v_all[KS][kPtVBytes];    // 3 V^T tiles; in the epilogue the rotation, or the groups' sums
     __shared__ __attribute__((aligned(16))) float n_all[KS][3][2][32];    // [group][buffer][k | v][token]
-    __shared__ __attribute__((aligned(8))) uint32_t tab_s[256 * kPtReplicas * kEntryDwords];
+    __shared__ __attribute__((aligned(16))) uint32_t tab_s[256 * kPtReplicas * kEntryDwords];
 
     const int tid_wg = threadIdx.x;
     const int wave_wg = uniform(tid_wg / kWave), lane = tid_wg % kWave;
@@ -88,16 +88,24 @@ prefill_tq_mfma_kernel(AttnArgs a, int T, int mirror) {
     constexpr float kRaise = 5.0f;
 
     // ---- table: byte -> its codes' centroids (low field first) as fp16(alpha c), kPtReplicas copies
-    for (int i = tid_wg; i < 256 * kPtReplicas; i += W * kWave) {
-        const int e = i / kPtReplicas;
-        if constexpr (BITS == 4) {
-            half2_t p = {(half_t)(kAlpha * kCentroids4[e & 15]), (half_t)(kAlpha * kCentroids4[e >> 4])};
-            tab_s[i] = *reinterpret_cast<uint32_t*>(&p);
-        } else {
-            half2_t p0 = {(half_t)(kAlpha * kCentroids2[e & 3]), (half_t)(kAlpha * kCentroids2[(e >> 2) & 3])};
-            half2_t p1 = {(half_t)(kAlpha * kCentroids2[(e >> 4) & 3]), (half_t)(kAlpha * kCentroids2[(e >> 6) & 3])};
-            tab_s[2 * i] = *reinterpret_cast<uint32_t*>(&p0);
-            tab_s[2 * i + 1] = *reinterpret_cast<uint32_t*>(&p1);
+    // A thread stores 16 bytes at a time; the centroids come out of a register by wave shuffle (lane c holds centroid c):
+    // an index into the constant array that differs between lanes is a load per look-up, one waiting for the other.
+    {
+        const float cent_lane = kAlpha * (BITS == 4 ? kCentroids4[lane & 15] : kCentroids2[lane & 3]);
+        auto cent = [&](int c) -> half_t { return (half_t)__shfl(cent_lane, c, 64); };
+#pragma unroll
+        for (int i = tid_wg * 4; i < 256 * kPtReplicas * kEntryDwords; i += W * kWave * 4) {
+            const int e = i / (kPtReplicas * kEntryDwords);
+            if constexpr (BITS == 4) {
+                half2_t p = {cent(e & 15), cent(e >> 4)};
+                const uint32_t w = *reinterpret_cast<uint32_t*>(&p);
+                *reinterpret_cast<uint4*>(&tab_s[i]) = uint4{w, w, w, w};
+            } else {
+                half2_t p0 = {cent(e & 3), cent((e >> 2) & 3)};
+                half2_t p1 = {cent((e >> 4) & 3), cent((e >> 6) & 3)};
+                const uint32_t w0 = *reinterpret_cast<uint32_t*>(&p0), w1 = *reinterpret_cast<uint32_t*>(&p1);
+                *reinterpret_cast<uint4*>(&tab_s[i]) = uint4{w0, w1, w0, w1};
+            }
         }
     }
     const int rep = lane & (kPtReplicas - 1);
