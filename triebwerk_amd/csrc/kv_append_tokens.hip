@@ -32,17 +32,6 @@ constexpr int kAppendWaves = 4;
 static_assert(kAppendWaves * kWave == kProducerThreads && 2 * kTileVecs * kUnitRow >= kAppendWaves * kOperandTileDwords,
               "the space of the unit vectors first holds a wave's 16 rows of R each");
 
-// Decision boundaries of turbo_quantize (kernels.cu:1448-1473) and their buckets: boundary i lies in a bucket of its own, at
-// least 0.15 bucket widths from the bucket's edges, far more than bucket_of rounds.
-constexpr float kEdges4[15] = {-0.21224f, -0.16299f, -0.12701f, -0.09715f, -0.07068f, -0.04619f, -0.02284f, 0.00000f,
-                                0.02284f,  0.04619f,  0.07068f,  0.09715f,  0.12701f,  0.16299f,  0.21224f};
-constexpr int kBuckets = 32;
-constexpr float kBucketScale = 72.30f, kBucketShift = 16.50f;
-// (the smaller bound comes last: a NaN ends up in the last bucket)
-__host__ __device__ __forceinline__ int bucket_of(float x) {
-    return (int)fmaxf(fminf(__builtin_fmaf(x, kBucketScale, kBucketShift), (float)(kBuckets - 1)), 0.0f);
-}
-
 }  // namespace
 
 template <int BITS, bool PROD>
@@ -106,18 +95,7 @@ append_tokens_kernel(AppendTokensArgs a) {
     x0.h = (int)((unsigned)x0.v - (unsigned)x0.row * per_row);
     Vec x1 = advance(x0), x2 = advance(x1);
     int pos0 = request_pos(x0), pos1 = request_pos(x1), pos2 = request_pos(x2);
-    // 4 bit: a value's code from its bucket -- the buckets are narrower than the gaps between the decision boundaries, so at most
-    // one boundary lies in each -- instead of 15 comparisons: {boundary, codes below it} of bucket tid
-    if (BITS == 4 && tid < kBuckets) {
-        float lim = 3.0e38f;
-        int below = 0;
-#pragma unroll
-        for (int i = 0; i < 15; i++) {
-            if (bucket_of(kEdges4[i]) == tid) lim = kEdges4[i];
-            if (bucket_of(kEdges4[i]) < tid) below++;
-        }
-        bucket_s[tid] = float2{lim, __builtin_bit_cast(float, below)};
-    }
+    if (BITS == 4 && tid < kBuckets) bucket_s[tid] = bucket_entry(tid);
     uint4 rraw[2][4];
 #pragma unroll
     for (int d = 0; d < 2; d++)
@@ -170,14 +148,7 @@ append_tokens_kernel(AppendTokensArgs a) {
         if (BITS == 4) *reinterpret_cast<uint32_t*>(dst) = *reinterpret_cast<const uint32_t*>(src);
         else *reinterpret_cast<uint16_t*>(dst) = *reinterpret_cast<const uint16_t*>(src);
     };
-    auto quantize = [&](float val) -> uint32_t {
-        if constexpr (BITS == 4) {                     // (a NaN takes the last bucket, whose comparison it passes: 15, as turbo_quantize)
-            const float2 e = bucket_s[bucket_of(val)];
-            return __builtin_bit_cast(uint32_t, e.y) + (!(val < e.x) ? 1u : 0u);
-        } else {
-            return (uint32_t)turbo_quantize(val, 2);
-        }
-    };
+    auto quantize = [&](float val) -> uint32_t { return bucket_quantize<BITS>(bucket_s, val); };
 
     Request next = request(x1, pos1);
     fill(0, x0, pos0, cur);

@@ -11,12 +11,12 @@
 // nothing is handed from one workgroup to another.  Two forms: PAIR (HKW even) -- 8 waves, each scanning two KV heads
 // with the tile of kv_pair_scan.hpp (256 registers per wave, two waves per SIMD either way); otherwise 16 waves with
 // one KV head each, described here:
-//   1. all threads stage the unit's vectors (K heads, V heads, query heads of the new token) in LDS and fill
-//      the centroid table; with producers one wave per K or query vector applies RMSNorm and rotary embedding
-//      there (kernels.cu:880-961).  Waves 0-7 (all 16 when the unit has more than 16 vectors) then rotate the
-//      vectors exactly as rotate_kernel does -- lane i16 = vector, wave = block of 16 output coordinates, the
-//      same v_mfma_f32_16x16x4_f32 chain, so the codes have the same bits -- and store codes and norms in the
-//      cache, the scaled q_rot in LDS;
+//   1. all threads fetch the unit's vectors (K heads, V heads, query heads of the new token), 16 lanes to a vector, and
+//      fill the centroid table meanwhile; the 16 lanes apply the producers' RMSNorm and rotary embedding
+//      (kernels.cu:880-961), measure the vector and leave it in LDS.  Waves 0-7 (all 16 when the unit has more than 16
+//      vectors) then rotate the vectors exactly as rotate_kernel does -- lane i16 = vector, wave = block of 16 output
+//      coordinates, the same v_mfma_f32_16x16x4_f32 chain, so the codes have the same bits -- and store the codes in
+//      the cache, the scaled q_rot in LDS;
 //   2. after the barrier wave w scans every SPLIT-th tile of the context (SPLIT = 16 / HKW, starting at tile
 //      w / HKW) for head w % HKW with the loop of attention_mfma_kernel (the table look-ups, MFMA tiling,
 //      online softmax are described there).  All its loads are issued after the barrier: the new token's row
@@ -58,10 +58,8 @@ constexpr unsigned kFusedShare = 33;           // 64ths of a sequence's tiles th
 constexpr unsigned kPairTileShare = 32;        // the same with eight waves in all: two per SIMD, no upper slots
 constexpr int kFusedMaxQ = 32;                 // query heads of a unit: HKW * R <= 8 * 4
 constexpr int kRowFloats = kHeadDim + 4;       // LDS row of a vector: conflict-free 16-byte accesses
-constexpr int kStageStride = 2 * kHeadDim + 16;   // bytes per staged fp16 vector
 constexpr int kMaxShares = 64;                 // workgroups that may share one sequence's context
 constexpr int kDeviceScope = 16;               // the sc1 bit of a raw buffer access: device scope
-static_assert(8 * (2 + 4) * kStageStride <= kFusedMaxQ * kRowFloats * 4, "staged vectors fit the output rows");
 
 }  // namespace
 
@@ -87,18 +85,22 @@ decode_fused_kernel(AttnArgs a, FusedArgs f) {
     constexpr uint32_t kHeadBytes = BITS * 16;
     constexpr float kAlpha = BITS == 4 ? kAlpha4 : kAlpha2;
     __shared__ __attribute__((aligned(16))) uint32_t tab_s[kTableWords];
-    // the scan's probabilities and partials; before the scan the same space holds R as 8 operand tiles
+    // the scan's probabilities and partials; before the scan the same space holds R as 8 operand tiles, then the unit's vectors
     constexpr int kParts = PAIR ? 2 * NW : NW;                 // (part, head) partials: a wave leaves one per head it scans
     constexpr int kRotGroups = NW / 8;                         // groups of eight waves that rotate (a wave = 16 output coordinates)
     constexpr int kPBytes = NW * 16 * 32 * 2, kPartBytes = kParts * R * kRowFloats * 4;
     constexpr int kRotBytes = 8 * kOperandTileDwords * 4;
-    __shared__ __attribute__((aligned(16))) char scan_s[kPBytes + kPartBytes > kRotBytes ? kPBytes + kPartBytes : kRotBytes];
+    constexpr int kMaxVecs = PAIR ? 4 * NW : 8 * (2 + R);      // vectors of a unit: a thread group of 16 each
+    static_assert(kMaxVecs <= 4 * NW, "a vector per 16 threads");
+    constexpr int kPrologueBytes = kRotBytes + kMaxVecs * kRowFloats * 4;
+    __shared__ __attribute__((aligned(16))) char scan_s[kPBytes + kPartBytes > kPrologueBytes ? kPBytes + kPartBytes : kPrologueBytes];
     half_t (*p_s)[16][32] = reinterpret_cast<half_t (*)[16][32]>(scan_s);
     float (*part_s)[R][kRowFloats] = reinterpret_cast<float (*)[R][kRowFloats]>(scan_s + kPBytes);
     uint32_t* rot_s = reinterpret_cast<uint32_t*>(scan_s);
+    float (*u_s)[kRowFloats] = reinterpret_cast<float (*)[kRowFloats]>(scan_s + kRotBytes);
     __shared__ __attribute__((aligned(16))) float qrot_s[kFusedMaxQ][kHeadDim];
     __shared__ __attribute__((aligned(16))) float o_s[kFusedMaxQ][kRowFloats];
-    __shared__ __attribute__((aligned(16))) half_t prod_s[4][kHeadDim];   // k_weight, q_weight, cos row, sin row
+    __shared__ __attribute__((aligned(8))) float2 bucket_s[kBuckets];
 
     const int tid = threadIdx.x;
     const int wave = uniform(tid / kWave), lane = tid % kWave;
@@ -128,8 +130,8 @@ decode_fused_kernel(AttnArgs a, FusedArgs f) {
     }
     const bool appends = !SHARES || share == nshares - 1;          // the share that holds the sequence's last tile
     // ---- operands of the rotations first: nothing about them depends on the position.  The unit's vectors
-    // (K heads, V heads, query heads) are fetched once by all threads, 16 bytes each, and staged in LDS;
-    // the rotating waves fetch their 16 rows of R.
+    // (K heads, V heads, query heads) are fetched once by all threads, 16 lanes to a vector, 16 bytes each;
+    // waves 0-7 fetch 16 rows of R each.
     const int nvec = HKW * (2 + R);
     const int rot_dblk = wave & 7;
     const bool rotating = wave < 8 * kRotGroups && (wave >> 3) * 16 < nvec;
@@ -145,10 +147,15 @@ decode_fused_kernel(AttnArgs a, FusedArgs f) {
         kind = 2; head = hg * HKW * R + (vc - 2 * HKW);
         return a.q + (long long)g * a.q_stride + (long long)head * kHeadDim;
     };
-    uint4 stage = {0u, 0u, 0u, 0u};                    // piece tid % 16 of vector tid / 16
-    if ((tid >> 4) < nvec) {
-        int kind0, head0;
-        stage = reinterpret_cast<const uint4*>(unit_vector(tid >> 4, kind0, head0))[tid & 15];
+    const int my_vec = tid >> 4, my_piece = tid & 15;  // what this thread carries of the unit's vectors
+    const bool carries = my_vec < nvec;
+    int my_kind, my_head;
+    const half_t* my_src = unit_vector(carries ? my_vec : 0, my_kind, my_head);
+    uint4 stage = {0u, 0u, 0u, 0u}, prod_w = {0u, 0u, 0u, 0u};
+    const bool normed = PROD && f.q_weight != nullptr, roped = PROD && f.cos_table != nullptr;
+    if (carries) {
+        stage = reinterpret_cast<const uint4*>(my_src)[my_piece];
+        if (normed && my_kind != 1) prod_w = reinterpret_cast<const uint4*>(my_kind == 0 ? f.k_weight : f.q_weight)[my_piece];
     }
     // R: wave w < 8 fetches rows 16w .. 16w + 15 (4 KB in a row, 4 fully used pieces per lane) and stages them
     // as an operand tile; the rotating waves read their operand from there
@@ -160,7 +167,7 @@ decode_fused_kernel(AttnArgs a, FusedArgs f) {
     }
 
     // scaled centroid number lane % 16 (4 bit) or lane % 4 (2 bit), for the table build
-    const float cent_lane = kAlpha * (BITS == 4 ? kCentroids4[lane & 15] : kCentroids2[lane & 3]);
+    const float cent_lane = kAlpha * centroid_of<BITS>(lane);
 
     const int pos = uniform(a.positions[g]);
     const int n = pos + 1;
@@ -168,20 +175,12 @@ decode_fused_kernel(AttnArgs a, FusedArgs f) {
     const int hk_local = PAIR ? 2 * (wave % (HKW >> 1)) : wave % HKW, part = PAIR ? wave / (HKW >> 1) : wave / HKW;
     const int h = hg * HKW + hk_local;                 // (first) KV head of this wave
 
-    // producers' operands: the two weight vectors and the table rows of this sequence's position, 16 bytes per thread
-    const bool normed = PROD && f.q_weight != nullptr, roped = PROD && f.cos_table != nullptr;
-    uint4 prod = {0u, 0u, 0u, 0u};
-    const int prod_row = tid >> 4, prod_piece = tid & 15;
-    bool prod_live = false;
-    if (PROD && tid < 64) {
-        if (prod_row < 2 && normed) {
-            prod = reinterpret_cast<const uint4*>(prod_row == 0 ? f.k_weight : f.q_weight)[prod_piece];
-            prod_live = true;
-        } else if (prod_row >= 2 && roped && prod_piece < (f.rope_dim >> 4)) {
-            const half_t* tabrow = (prod_row == 2 ? f.cos_table : f.sin_table) + (long long)pos * (f.rope_dim >> 1);
-            prod = reinterpret_cast<const uint4*>(tabrow)[prod_piece];
-            prod_live = true;
-        }
+    // producers: the pieces of the table rows of this sequence's position that go with this thread's coordinates
+    uint4 prod_c = {0u, 0u, 0u, 0u}, prod_s = {0u, 0u, 0u, 0u};
+    if (roped && carries && my_kind != 1) {
+        const long long at = (long long)pos * (f.rope_dim >> 4) + rope_piece16(my_piece, f.rope_dim);
+        prod_c = reinterpret_cast<const uint4*>(f.cos_table)[at];
+        prod_s = reinterpret_cast<const uint4*>(f.sin_table)[at];
     }
 
     // ---- tiles of 32 tokens this wave scans.  They are dealt round by round: in round r part p takes tile
@@ -346,41 +345,34 @@ decode_fused_kernel(AttnArgs a, FusedArgs f) {
             }
         }
 
-        // the staged vectors: rows of kStageStride bytes (16-byte aligned; a lane group's 2-byte reads below
-        // fall into 32 different banks), in the space the merged outputs will use at the end
-        char* x_s = reinterpret_cast<char*>(o_s);
-        if ((tid >> 4) < nvec) *reinterpret_cast<uint4*>(x_s + (tid >> 4) * kStageStride + (tid & 15) * 16) = stage;
-        if (PROD && prod_live) *reinterpret_cast<uint4*>(&prod_s[prod_row][8 * prod_piece]) = prod;
+        if (BITS == 4 && wave == NW - 1 && lane < kBuckets) bucket_s[lane] = bucket_entry(lane);
         if (wave < 8) stage_operand_tile(rot_s + wave * kOperandTileDwords, rraw, lane);
+        // This thread's piece of its vector: the optional producers (K and queries; each step rounded to fp16 as the
+        // reference's in-place kernels leave it), the norm in the reference's order, and K and V as unit vectors, once for
+        // all waves, into LDS as fp32 regrouped for the matrix cores (coordinate 4s + kk at kk * 32 + s).  (Each rotating wave
+        // doing norm and regrouping for itself, and a wave per vector for the producers: rotations 2.3 us of a launch and
+        // producers 3.5.)
+        if (carries) {                                     // the same for the 16 lanes of a vector
+            float x[8], t[8];
+            unpack_halves(stage, x);
+            if (PROD && my_kind != 1) {
+                if (normed) norm_head16(x, prod_w, f.eps, f.biased);
+                if (roped) rope_head16(x, prod_c, prod_s, my_piece, f.rope_dim, 0);
+            }
+#pragma unroll
+            for (int e = 0; e < 8; e++) t[e] = x[e] * x[e];            // exact: fp16 values
+            const float norm = sqrtf(head_tree_sum16(t) + 1e-12f);
+            const float inv = my_kind == 2 ? 1.0f : 1.0f / norm;
+            float* dst = &u_s[my_vec][2 * my_piece];
+#pragma unroll
+            for (int e = 0; e < 4; e++) *reinterpret_cast<float2*>(dst + 32 * e) = float2{x[e] * inv, x[e + 4] * inv};
+            if (my_kind != 2 && my_piece == 0 && appends)
+                (my_kind == 0 ? f.k_norms : f.v_norms)[((long long)g * a.seq_stride_rows + pos) * Hk + my_head] = (half_t)norm;
+        }
         lds_barrier();
         early();
         float rv[32];                                      // R[16 * rot_dblk + ln][4s + kg]
         if (rotating) read_operand_tile(rot_s + rot_dblk * kOperandTileDwords, lane, rv);
-        if (PROD) {
-            // optional producers on the staged K and query vectors, one vector per wave: per-head RMSNorm
-            // (kernels.cu:880-923), then rotary embedding (927-961), each rounded to fp16 as the reference's
-            // in-place kernels leave it; V vectors stay as they are
-            for (int v = wave; v < nvec; v += NW) {
-                int kind, head;
-                (void)unit_vector(v, kind, head);
-                if (kind == 1) continue;                           // uniform over the wave
-                half_t* row = reinterpret_cast<half_t*>(x_s + v * kStageStride);
-                float x0 = (float)row[lane], x1 = (float)row[lane + 64];
-                HeadXform t;
-                t.weight = normed ? &prod_s[0][0] + (kind == 0 ? 0 : kHeadDim) : nullptr;
-                t.eps = f.eps;
-                t.biased = f.biased;
-                t.cos_row = roped ? prod_s[2] : nullptr;
-                t.sin_row = prod_s[3];
-                t.rope_dim = f.rope_dim;
-                t.single_order = 0;
-                xform_head(x0, x1, lane, t);
-                row[lane] = (half_t)x0;                            // both are fp16 values already
-                row[lane + 64] = (half_t)x1;
-            }
-            lds_barrier();
-        }
-
         for (int vt = wave >> 3; rotating && vt * 16 < nvec; vt += kRotGroups) {  // uniform over the wave
             const int vi = vt * 16 + i16;
             const int vc = vi < nvec ? vi : nvec - 1;              // clamp reads, mask stores
@@ -388,42 +380,28 @@ decode_fused_kernel(AttnArgs a, FusedArgs f) {
             (void)unit_vector(vc, kind, head);
             const bool is_query = kind == 2;
             // B operand: coordinate 4s + kk of vector vc
-            float xv[32];
-            const half_t* xrow = reinterpret_cast<const half_t*>(x_s + vc * kStageStride) + kk;
-#pragma unroll
-            for (int s2 = 0; s2 < 32; s2++) xv[s2] = (float)xrow[4 * s2];
-            const float n2 = rotation_tree_sum_sq(xv);                 // the reference's order, as rotate_kernel
-            if (!is_query) {
-                const float inv = 1.0f / sqrtf(n2 + 1e-12f);
-#pragma unroll
-                for (int s = 0; s < 32; s++) xv[s] *= inv;
-            }
             float4_t acc = {0.f, 0.f, 0.f, 0.f};
+            const float* urow = &u_s[vc][32 * kk];
 #pragma unroll
-            for (int s = 0; s < 32; s++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(rv[s], xv[s], acc, 0, 0, 0);
-
+            for (int t = 0; t < 8; t++) {
+                const float4 u = *reinterpret_cast<const float4*>(urow + 4 * t);
+                const float uv[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+                for (int j = 0; j < 4; j++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(rv[4 * t + j], uv[j], acc, 0, 0, 0);
+            }
             if (is_query && vi < nvec) {
                 float4 o = {acc[0] * f.q_scale, acc[1] * f.q_scale, acc[2] * f.q_scale, acc[3] * f.q_scale};
                 *reinterpret_cast<float4*>(&qrot_s[vc - 2 * HKW][dblk * 16 + 4 * kk]) = o;
             }
-            uint32_t packed = 0;
+            if (appends && vt * 16 < 2 * HKW) {                    // lane: coordinates 16 dblk + 4kk .. + 3
+                uint32_t packed = 0;
 #pragma unroll
-            for (int r = 0; r < 4; r++) packed |= (uint32_t)turbo_quantize(acc[r], BITS) << (r * BITS);
-            constexpr int PB = 4 * BITS;
-            uint32_t p1 = (uint32_t)__shfl((int)packed, i16 + 16, 64);
-            uint32_t p2 = (uint32_t)__shfl((int)packed, i16 + 32, 64);
-            uint32_t p3 = (uint32_t)__shfl((int)packed, i16 + 48, 64);
-            if (kk == 0 && vi < nvec && !is_query && appends) {
-                constexpr int BPH = kHeadDim * BITS / 8;
-                const long long crow = seq_row0 + pos;
-                uint8_t* dst = (kind == 0 ? f.k_codes : f.v_codes) + (crow * Hk + head) * BPH + dblk * (2 * BITS);
-                if (BITS == 4) {
-                    uint2 o = {packed | (p1 << PB), p2 | (p3 << PB)};
-                    *reinterpret_cast<uint2*>(dst) = o;
-                } else {
-                    *reinterpret_cast<uint32_t*>(dst) = packed | (p1 << PB) | (p2 << (2 * PB)) | (p3 << (3 * PB));
+                for (int r = 0; r < 4; r++) packed |= bucket_quantize<BITS>(bucket_s, acc[r]) << (r * BITS);
+                if (vi < nvec && !is_query) {
+                    uint8_t* dst = (kind == 0 ? f.k_codes : f.v_codes) + ((seq_row0 + pos) * Hk + head) * kHeadBytes + (4 * dblk + kk) * (BITS / 2);
+                    if (BITS == 4) *reinterpret_cast<uint16_t*>(dst) = (uint16_t)packed;
+                    else *dst = (uint8_t)packed;
                 }
-                if (dblk == 0) (kind == 0 ? f.k_norms : f.v_norms)[crow * Hk + head] = (half_t)sqrtf(n2 + 1e-12f);
             }
         }
         __syncthreads();        // table, q_rot and the new cache row are in place; R has been read

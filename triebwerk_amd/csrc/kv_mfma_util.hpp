@@ -32,6 +32,22 @@ __device__ __forceinline__ float h2f_bits(uint32_t bits16) {
     return (float)cv.h;
 }
 
+// Centroid number c % 16 (4 bit) or c % 4 (2 bit) by selections between immediates: the values are in a register while the
+// first loads of a kernel are still under way, where a per-lane index into the constant array is one more load to wait for.
+template <int BITS>
+__device__ __forceinline__ float centroid_of(int c) {
+    if constexpr (BITS == 4) {
+        const int k = (c & 7) ^ ((c & 8) ? 0 : 7);                  // the tables are symmetric
+        const float m01 = (k & 1) ? 0.03432f : 0.01135f, m23 = (k & 1) ? 0.08330f : 0.05806f;
+        const float m45 = (k & 1) ? 0.14304f : 0.11099f, m67 = (k & 1) ? 0.24155f : 0.18293f;
+        const float m = (k & 4) ? ((k & 2) ? m67 : m45) : ((k & 2) ? m23 : m01);
+        return (c & 8) ? m : -m;
+    } else {
+        const float m = ((c ^ (c >> 1)) & 1) ? 0.04003f : 0.13351f;
+        return (c & 2) ? m : -m;
+    }
+}
+
 __device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
 
 typedef uint32_t uint32x4_t __attribute__((ext_vector_type(4)));
@@ -112,7 +128,7 @@ inline PrefillChoice choose_prefill_form(const PrefillForm* forms, int nforms, d
 template <int BITS, bool NATURAL>
 __device__ __forceinline__ void build_centroid_table(uint32_t* tab_s, float alpha, int tid, int nthreads) {
     const int lane = tid & 63;
-    const float cent_lane = alpha * (BITS == 4 ? kCentroids4[lane & 15] : kCentroids2[lane & 3]);
+    const float cent_lane = alpha * centroid_of<BITS>(lane);
     auto cent = [&](int c) -> half_t { return (half_t)__shfl(cent_lane, c, 64); };
     for (int i = tid * 4; i < kTableWords; i += nthreads * 4) {
         const int e = i >> 6;

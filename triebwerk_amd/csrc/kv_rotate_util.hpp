@@ -78,4 +78,37 @@ __device__ __forceinline__ float rotation_tree_sum_sq(const float (&xv)[32]) {
     return (sgrp[0] + sgrp[2]) + (sgrp[1] + sgrp[3]);
 }
 
+// Decision boundaries of turbo_quantize (kernels.cu:1448-1473) and their buckets: boundary i lies in a bucket of its own, at
+// least 0.15 bucket widths from the bucket's edges, far more than bucket_of rounds.  A 4-bit code then comes from its
+// bucket -- at most one boundary lies in each -- instead of 15 comparisons.
+constexpr float kEdges4[15] = {-0.21224f, -0.16299f, -0.12701f, -0.09715f, -0.07068f, -0.04619f, -0.02284f, 0.00000f,
+                                0.02284f,  0.04619f,  0.07068f,  0.09715f,  0.12701f,  0.16299f,  0.21224f};
+constexpr int kBuckets = 32;
+constexpr float kBucketScale = 72.30f, kBucketShift = 16.50f;
+// (the smaller bound comes last: a NaN ends up in the last bucket)
+__host__ __device__ __forceinline__ int bucket_of(float x) {
+    return (int)fmaxf(fminf(__builtin_fmaf(x, kBucketScale, kBucketShift), (float)(kBuckets - 1)), 0.0f);
+}
+// {boundary in bucket b, codes below it}
+__device__ __forceinline__ float2 bucket_entry(int b) {
+    float lim = 3.0e38f;
+    int below = 0;
+#pragma unroll
+    for (int i = 0; i < 15; i++) {
+        if (bucket_of(kEdges4[i]) == b) lim = kEdges4[i];
+        if (bucket_of(kEdges4[i]) < b) below++;
+    }
+    return float2{lim, __builtin_bit_cast(float, below)};
+}
+// turbo_quantize by the table of the kBuckets entries (2 bit: its three comparisons, no table)
+template <int BITS>
+__device__ __forceinline__ uint32_t bucket_quantize(const float2* buckets, float val) {
+    if constexpr (BITS == 4) {                     // (a NaN takes the last bucket, whose comparison it passes: 15, as turbo_quantize)
+        const float2 e = buckets[bucket_of(val)];
+        return __builtin_bit_cast(uint32_t, e.y) + (!(val < e.x) ? 1u : 0u);
+    } else {
+        return (uint32_t)turbo_quantize(val, 2);
+    }
+}
+
 }  // namespace twkv
