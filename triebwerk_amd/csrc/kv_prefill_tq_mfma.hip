@@ -27,7 +27,8 @@ constexpr int kPtKRow = 2 * kHeadDim + 32;   // bytes per expanded K row in LDS 
 constexpr int kPtVRow = 2 * 32 + 32;         // bytes per V^T row (32 token slots) in LDS (96: full rate, 80: 54 %)
 constexpr int kPtVTile = kHeadDim * kPtVRow; // bytes of a V^T tile
 constexpr int kPtVBytes = 3 * kPtVTile;      // 3 tiles, and room for the 128 x 128 fp16 rotation
-static_assert(kPtVBytes >= 2 * kHeadDim * kHeadDim, "the rotation fits");
+constexpr int kPtRotBlock = 4 * kWave * 16 + 16;   // bytes per 16 output dims of the rotation in the epilogue: 16 more than the entries, so that its 2-byte writes meet no bank twice
+static_assert(kPtVBytes >= kHeadDim * kPtKRow && kPtVBytes >= 8 * kPtRotBlock, "the rotation fits in both layouts");
 
 // a masked score: below the initial maximum by more than the exponent's range, also when a group's first tile is all masked
 constexpr float kMasked = -3.0e38f;
@@ -90,8 +91,8 @@ prefill_tq_mfma_kernel(AttnArgs a, int T, int mirror) {
     // ---- table: byte -> its codes' centroids (low field first) as fp16(alpha c), kPtReplicas copies
     // A thread stores 16 bytes at a time; the centroids come out of a register by wave shuffle (lane c holds centroid c):
     // an index into the constant array that differs between lanes is a load per look-up, one waiting for the other.
-    {
-        const float cent_lane = kAlpha * (BITS == 4 ? kCentroids4[lane & 15] : kCentroids2[lane & 3]);
+    auto build_table = [&]() {
+        const float cent_lane = kAlpha * centroid_of<BITS>(lane);
         auto cent = [&](int c) -> half_t { return (half_t)__shfl(cent_lane, c, 64); };
 #pragma unroll
         for (int i = tid_wg * 4; i < 256 * kPtReplicas * kEntryDwords; i += W * kWave * 4) {
@@ -107,7 +108,7 @@ prefill_tq_mfma_kernel(AttnArgs a, int T, int mirror) {
                 *reinterpret_cast<uint4*>(&tab_s[i]) = uint4{w0, w1, w0, w1};
             }
         }
-    }
+    };
     const int rep = lane & (kPtReplicas - 1);
     // the 8 halves (4 dwords) of 8 consecutive coordinates from their packed codes (4 bytes at 4 bit, 2 at 2 bit)
     auto expand8 = [&](uint32_t codes, uint32_t (&out)[4]) {
@@ -208,7 +209,12 @@ prefill_tq_mfma_kernel(AttnArgs a, int T, int mirror) {
         }
         if (tid < 2 * kWave && (tid & 32) == 0) n_s[vbuf][tid >> 6][tid & 31] = h2f_bits(st.nb);
     };
-    __syncthreads();                                       // the table is there
+    // The rotation, a piece per thread: rows k = 16r + tid / 16 (512 threads: 32r + tid / 16), columns 8c .. 8c + 7, c = tid % 16
+    auto load_rotation = [&](uint4 (&rp)[32 / W]) {
+        const uint4* rsrc = reinterpret_cast<const uint4*>(a.rotation) + tid_wg;
+#pragma unroll
+        for (int r = 0; r < 32 / W; r++) rp[r] = rsrc[r * (W * kWave)];
+    };
 
     // mirror: a workgroup takes a token block and its mirror image from the other end, one after the other: with causal
     // rows the two together cost the same for every workgroup.
@@ -226,8 +232,16 @@ prefill_tq_mfma_kernel(AttnArgs a, int T, int mirror) {
         // is made here, on the matrix cores: q_rot^T[d][query] = R[d][.] . q^T, 16 rows d at a time, the rows
         // picked so that the result lands where the operand wants it -- accumulator row 4kg + i of block (j, h)
         // is d = 32j + 8kg + 4h + i.  Both factors are exact in fp16 and the sum is kept in fp32.
+        // A pass asks for the rotation, its queries and its first tile at once and builds the table meanwhile (one trip to memory in
+        // front of the tiles instead of three); R goes through the V tiles' space, row d = 32j + 8a + 4h + i at 32j + 16h + 4a + i,
+        // which makes a wave's 16 rows neighbours there.  Before, table, queries, R (each wave its own, in operand order), first tile
+        // and the epilogue's R came one after the other, and that R went to LDS eight lanes to a bank: 28 layers of 16
+        // prompts of 97 to 256 tokens, handed to groups of 8, 12.06 ms against 9.37 now; 4 layers of 4111 tokens 1.01 against 0.90.
         half8_t qb[NQ][4], ql[NQ][4];
+        Staged st;
         {
+            uint4 rp[32 / W];
+            load_rotation(rp);
             half8_t qv[NQ][4];                             // q[query ln][32t + 8kg .. +7]
 #pragma unroll
             for (int nq = 0; nq < NQ; nq++) {
@@ -235,9 +249,18 @@ prefill_tq_mfma_kernel(AttnArgs a, int T, int mirror) {
 #pragma unroll
                 for (int t = 0; t < 4; t++) qv[nq][t] = *reinterpret_cast<const half8_t*>(qsrc + 32 * t);
             }
-            int rrow = 8 * (ln >> 2) + (ln & 3);           // row of R this lane feeds within a block, less 32j + 4h
-            asm volatile("" : "+v"(rrow));                 // per pass: the 32 loads below are not kept across passes
-            const half_t* rsrc = a.rotation + rrow * kHeadDim + 8 * kg;
+            load_tile(32 * grp, st);
+            if (pass == 0) build_table();
+            else lds_barrier();                            // the previous pass's epilogue reads the rotation in the same place
+            {
+                const int krow = tid_wg >> 4, c = tid_wg & 15;
+                char* dst = &v_all[0][(16 * ((krow >> 2) & 1) + 4 * (krow >> 3) + (krow & 3)) * kPtKRow + 16 * c];
+#pragma unroll
+                for (int r = 0; r < 32 / W; r++)
+                    *reinterpret_cast<uint4*>(dst + (W == 4 ? 32 * (r >> 1) + 8 * (r & 1) : 32 * r) * kPtKRow) = rp[r];
+            }
+            lds_barrier();                                 // the table and R are there
+            const char* rrow = &v_all[0][ln * kPtKRow + 16 * kg];
 #pragma unroll
             for (int j = 0; j < 4; j++) {
 #pragma unroll
@@ -247,7 +270,7 @@ prefill_tq_mfma_kernel(AttnArgs a, int T, int mirror) {
                     for (int nq = 0; nq < NQ; nq++) y[nq] = float4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                     for (int t = 0; t < 4; t++) {
-                        const half8_t ra = *reinterpret_cast<const half8_t*>(rsrc + (32 * j + 4 * h) * kHeadDim + 32 * t);
+                        const half8_t ra = *reinterpret_cast<const half8_t*>(rrow + (32 * j + 16 * h) * kPtKRow + 64 * t);
 #pragma unroll
                         for (int nq = 0; nq < NQ; nq++) y[nq] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ra, qv[nq][t], y[nq], 0, 0, 0);
                     }
@@ -291,9 +314,7 @@ prefill_tq_mfma_kernel(AttnArgs a, int T, int mirror) {
         // depend on tile t) ahead of the softmax arithmetic of tile t.  Three V (and norm) buffers, two K buffers.
         // (The fp16 kernel's deeper pipeline -- K operands a tile ahead in registers -- needs 64 registers more
         // than the 226 this kernel already uses with its second set of operands.)
-        __syncthreads();                                   // a previous pass may still be reading its last V tile
-        Staged st;
-        load_tile(32 * grp, st);
+        lds_barrier();                                     // every wave has read R out of the V tiles
         stash(0, 0, st);
         __syncthreads();
 
@@ -389,17 +410,19 @@ prefill_tq_mfma_kernel(AttnArgs a, int T, int mirror) {
             if (more) stash(buf ^ 1, (it + 1) % 3, st);
             __syncthreads();
         }
+        uint4 rot_raw[32 / W];
+        load_rotation(rot_raw);                            // for the epilogue, under the last tile's product
         if (have_prev) pv((ntiles - 1) % 3, pa_prev, pl_prev);
 
         // ---- epilogue: out[q][d] = sum_k R[k][d] o[q][k] / (sum + 1e-8) (kernels.cu:1946-1957) as
         // out^T = R^T . O^T.  The rotation goes into the V buffers in operand order: 16-byte entry
-        // (db * 4 + t) * 64 + lane holds R[k][16 db + ln] for the 8 k that lane (ln, kg) carries in step t,
+        // t * 64 + lane of block db holds R[k][16 db + ln] for the 8 k that lane (ln, kg) carries in step t,
         // k = 32t + 16 (e / 4) + 4kg + e % 4 -- the dims its accumulators o[.][2t + e / 4][e % 4] belong to.
         __syncthreads();                                   // every wave is done with the tiles
         // two groups: their sums change hands through the V tiles -- with two query blocks group s finishes block s, with one
         // query block both groups merge the whole of it and each rotates half of the dims -- and the rotation takes the K tiles
         char* rot_s = KS == 2 ? &k_all[0][0][0] : &v_all[0][0];
-        static_assert(KS == 1 || (sizeof(k_all) >= 2 * kHeadDim * kHeadDim && (int)sizeof(v_all) >= W * kWave * (8 * 16 + 8)), "both fit");
+        static_assert(KS == 1 || (sizeof(k_all) >= 8 * kPtRotBlock && (int)sizeof(v_all) >= W * kWave * (8 * 16 + 8)), "both fit");
         float4_t* ex = reinterpret_cast<float4_t*>(&v_all[0][0]);                                  // [wave of the workgroup][8][lane]
         float2* exml = reinterpret_cast<float2*>(&v_all[0][0] + W * 8 * kWave * 16);               // [wave][lane]: maximum, sum
         constexpr int NF = KS == 2 ? 1 : NQ;               // query blocks this wave finishes
@@ -438,13 +461,11 @@ prefill_tq_mfma_kernel(AttnArgs a, int T, int mirror) {
         {
             // thread -> rows k = 16r + tid / 16, r = 0..7, columns 8c .. 8c + 7 with c = tid % 16; of k only r is
             // not fixed per thread, and r moves the destination by whole steps t = r / 2 and halves 4 (r % 2)
-            const uint4* rsrc = reinterpret_cast<const uint4*>(a.rotation) + tid_wg;
             const int krow = tid_wg >> 4, c = tid_wg & 15;       // 512 threads: rows k = 32r + tid / 16, r = 0..3
-            char* dst0 = &rot_s[(c >> 1) * 4096 + ((krow >> 2) & 3) * 256 + (c & 1) * 128 + 2 * (krow & 3) + (W == 8 ? 8 * (krow >> 4) : 0)];
+            char* dst0 = &rot_s[(c >> 1) * kPtRotBlock + ((krow >> 2) & 3) * 256 + (c & 1) * 128 + 2 * (krow & 3) + (W == 8 ? 8 * (krow >> 4) : 0)];
 #pragma unroll
             for (int r = 0; r < 32 / W; r++) {
-                const uint4 rp = rsrc[r * (W * kWave)];
-                const uint32_t w[4] = {rp.x, rp.y, rp.z, rp.w};
+                const uint32_t w[4] = {rot_raw[r].x, rot_raw[r].y, rot_raw[r].z, rot_raw[r].w};
                 const int step = W == 4 ? (r >> 1) * 1024 + (r & 1) * 8 : r * 1024;
 #pragma unroll
                 for (int x = 0; x < 8; x++)
@@ -488,7 +509,7 @@ prefill_tq_mfma_kernel(AttnArgs a, int T, int mirror) {
             for (int nf = 0; nf < NF; nf++) y[nf] = float4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int t = 0; t < 4; t++) {
-                const half8_t ra = *reinterpret_cast<const half8_t*>(&rot_s[((db * 4 + t) * 64 + lane) * 16]);
+                const half8_t ra = *reinterpret_cast<const half8_t*>(&rot_s[db * kPtRotBlock + (t * 64 + lane) * 16]);
 #pragma unroll
                 for (int nf = 0; nf < NF; nf++) {
                     y[nf] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ra, oh[nf][t], y[nf], 0, 0, 0);
