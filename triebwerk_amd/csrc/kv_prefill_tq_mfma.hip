@@ -209,11 +209,15 @@ prefill_tq_mfma_kernel(AttnArgs a, int T, int mirror) {
         }
         if (tid < 2 * kWave && (tid & 32) == 0) n_s[vbuf][tid >> 6][tid & 31] = h2f_bits(st.nb);
     };
-    // The rotation, a piece per thread: rows k = 16r + tid / 16 (512 threads: 32r + tid / 16), columns 8c .. 8c + 7, c = tid % 16
-    auto load_rotation = [&](uint4 (&rp)[32 / W]) {
-        const uint4* rsrc = reinterpret_cast<const uint4*>(a.rotation) + tid_wg;
+    // the rotation, a piece per thread: rows k = 16r + tid / 16 (512 threads: 32r + tid / 16), columns 8c .. 8c + 7, c = tid % 16
+    struct RotPieces { uint4 p[32 / W]; };
+    auto load_rotation = [&]() -> RotPieces {
+        RotPieces rp;
+        int at = tid_wg;
+        asm volatile("" : "+v"(at));                       // asked for where it is written: not kept across passes
 #pragma unroll
-        for (int r = 0; r < 32 / W; r++) rp[r] = rsrc[r * (W * kWave)];
+        for (int r = 0; r < 32 / W; r++) rp.p[r] = reinterpret_cast<const uint4*>(a.rotation)[at + r * (W * kWave)];
+        return rp;
     };
 
     // mirror: a workgroup takes a token block and its mirror image from the other end, one after the other: with causal
@@ -240,8 +244,7 @@ prefill_tq_mfma_kernel(AttnArgs a, int T, int mirror) {
         half8_t qb[NQ][4], ql[NQ][4];
         Staged st;
         {
-            uint4 rp[32 / W];
-            load_rotation(rp);
+            const RotPieces rot = load_rotation();
             half8_t qv[NQ][4];                             // q[query ln][32t + 8kg .. +7]
 #pragma unroll
             for (int nq = 0; nq < NQ; nq++) {
@@ -257,7 +260,7 @@ prefill_tq_mfma_kernel(AttnArgs a, int T, int mirror) {
                 char* dst = &v_all[0][(16 * ((krow >> 2) & 1) + 4 * (krow >> 3) + (krow & 3)) * kPtKRow + 16 * c];
 #pragma unroll
                 for (int r = 0; r < 32 / W; r++)
-                    *reinterpret_cast<uint4*>(dst + (W == 4 ? 32 * (r >> 1) + 8 * (r & 1) : 32 * r) * kPtKRow) = rp[r];
+                    *reinterpret_cast<uint4*>(dst + (W == 4 ? 32 * (r >> 1) + 8 * (r & 1) : 32 * r) * kPtKRow) = rot.p[r];
             }
             lds_barrier();                                 // the table and R are there
             const char* rrow = &v_all[0][ln * kPtKRow + 16 * kg];
@@ -320,14 +323,14 @@ prefill_tq_mfma_kernel(AttnArgs a, int T, int mirror) {
 
         half8_t pa_prev[NQ], pl_prev[NQ];
         bool have_prev = false;
-        for (int it = 0; it < ntiles; it++) {
+        auto step = [&](int it) {
             const int buf = it & 1, nbuf = it % 3;
             const int tile = 32 * (KS * it + grp);
             const bool more = it + 1 < ntiles;
             // the wave's priority falls through the tile (scores 3, P.V 2, softmax 1, hand-over 0): of the two waves of a
             // SIMD the one earlier in its tile goes first; 1.5 % at 8192 tokens, 3 % at 4096
             __builtin_amdgcn_s_setprio(3);
-            if (more) load_tile(tile + 32 * KS, st);
+            if (more) load_tile(tile + 32 * KS, st);       // (requested two tiles ahead: no faster at any length)
 
             const bool active = tile <= q0 + 16 * NQ - 1 && q0 < T;      // the tile reaches this wave's queries (uniform over the wave)
             float4_t s[NQ][2];
@@ -408,10 +411,10 @@ prefill_tq_mfma_kernel(AttnArgs a, int T, int mirror) {
 
             __builtin_amdgcn_s_setprio(0);
             if (more) stash(buf ^ 1, (it + 1) % 3, st);
-            __syncthreads();
-        }
-        uint4 rot_raw[32 / W];
-        load_rotation(rot_raw);                            // for the epilogue, under the last tile's product
+            lds_barrier();
+        };
+        for (int it = 0; it < ntiles; it++) step(it);
+        const RotPieces rot_raw = load_rotation();         // for the epilogue, under the last tile's product
         if (have_prev) pv((ntiles - 1) % 3, pa_prev, pl_prev);
 
         // ---- epilogue: out[q][d] = sum_k R[k][d] o[q][k] / (sum + 1e-8) (kernels.cu:1946-1957) as
@@ -465,7 +468,7 @@ prefill_tq_mfma_kernel(AttnArgs a, int T, int mirror) {
             char* dst0 = &rot_s[(c >> 1) * kPtRotBlock + ((krow >> 2) & 3) * 256 + (c & 1) * 128 + 2 * (krow & 3) + (W == 8 ? 8 * (krow >> 4) : 0)];
 #pragma unroll
             for (int r = 0; r < 32 / W; r++) {
-                const uint32_t w[4] = {rot_raw[r].x, rot_raw[r].y, rot_raw[r].z, rot_raw[r].w};
+                const uint32_t w[4] = {rot_raw.p[r].x, rot_raw.p[r].y, rot_raw.p[r].z, rot_raw.p[r].w};
                 const int step = W == 4 ? (r >> 1) * 1024 + (r & 1) * 8 : r * 1024;
 #pragma unroll
                 for (int x = 0; x < 8; x++)
@@ -547,8 +550,8 @@ void launch_prefill_tq_mfma(const AttnArgs& a, hipStream_t s, int form) {
     const int R = a.num_heads / a.num_kv_heads;
     const int T = a.G;
     static constexpr PrefillForm kForms[] = {
-        {1, 4, 1, 1, 12.7, 0.785, 0.583, 3.0, 0.242}, {2, 8, 1, 2, 16.6, 0.917, 1.449, 8.8, 0.080}, {3, 8, 2, 2, 18.8, 1.702, 2.150, 6.8, 0.043},
-        {5, 8, 1, 1, 16.3, 0.946, 1.154, 5.5, 0.032}, {6, 8, 2, 1, 18.5, 1.657, 1.869, 7.9, 0.0}};
+        {1, 4, 1, 1, 5.83, 0.861, 0.590, 1.17, 0.157}, {2, 8, 1, 2, 7.43, 1.134, 1.437, 2.09, 0.116}, {3, 8, 2, 2, 10.2, 1.797, 2.274, 1.67, 0.043},
+        {5, 8, 1, 1, 8.43, 1.062, 1.277, 3.53, 0.0}, {6, 8, 2, 1, 10.9, 1.621, 2.143, 9.87, 0.003}};
     const PrefillChoice c = choose_prefill_form(kForms, 5, 0.97, T, R, a.num_kv_heads, form);
     const int mirror = c.mirror ? 1 : 0;
     const dim3 grid(mirror ? (c.blocks + 1) / 2 : c.blocks, a.num_kv_heads), block(c.waves * kWave);
