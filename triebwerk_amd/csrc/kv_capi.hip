@@ -239,18 +239,18 @@ static int shares_that_fit(int max_seq_len) {
     return n;
 }
 
-int tw_kv_decode_step_plan2(int G, int num_heads, int num_kv_heads, int bits, int max_seq_len, int ctx_min, int ctx_max,
-                            int can_share) {
-    if (G <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads != 0 || (bits != 2 && bits != 4)) return 0;
+static bool step_takes_one_launch(int G, int num_heads, int num_kv_heads, int bits, int max_seq_len, int ctx_min, int ctx_max,
+                                  bool can_share) {
+    if (G <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads != 0 || (bits != 2 && bits != 4)) return false;
     const int group = num_heads / num_kv_heads;
-    if (group != 1 && group != 2 && group != 4) return 0;
+    if (group != 1 && group != 2 && group != 4) return false;
     const bool allow_pairs = g_decode_fused.load() != 3;
     const int hkw = decode_fused_heads_per_workgroup(G, num_heads, num_kv_heads, bits, allow_pairs);
     const int split = 16 / hkw;                                   // parts of the context per head: waves / heads
     const bool known = ctx_max > 0;
     const int bound = known ? ctx_max : max_seq_len;
-    if (bound <= 256 * split) return 1;                           // at most 8 tiles of 32 tokens per wave
-    if (!known) return 0;                                         // lengths unknown: the balanced walk
+    if (bound <= 256 * split) return true;                        // at most 8 tiles of 32 tokens per wave
+    if (!known) return false;                                     // lengths unknown: the balanced walk
     const bool ragged = (long long)(ctx_max - ctx_min) * 8 > ctx_max;
     // The cheaper of the two by estimates fitted to measured launches (microseconds per layer; the
     // figures live in one table, plan_constants): one launch as decode_fused_shape counts it (with a sequence's context
@@ -258,12 +258,17 @@ int tw_kv_decode_step_plan2(int G, int num_heads, int num_kv_heads, int bits, in
     // launches as decode_three_estimate_us does.  Ragged batches take the balanced walk of the three launches, except
     // small ones whose longest sequence is shared by enough workgroups: that one decides how long the one launch takes,
     // the mean length the walk.
-    const int max_shares = can_share != 0 ? shares_that_fit(max_seq_len) : 1;
+    const int max_shares = can_share ? shares_that_fit(max_seq_len) : 1;
     const FusedShape shape = decode_fused_shape(G, num_heads, num_kv_heads, bits, allow_pairs, max_shares, ctx_max);
-    if (ragged && shape.shares == 1) return 0;
+    if (ragged && shape.shares == 1) return false;
     const double one = shape.us;
     const double three = decode_three_estimate_us(G, num_heads, num_kv_heads, bits, ragged ? 0.5 * (ctx_min + ctx_max) : ctx_max);
-    return one <= three ? 1 : 0;
+    return one <= three;
+}
+
+int tw_kv_decode_step_plan2(int G, int num_heads, int num_kv_heads, int bits, int max_seq_len, int ctx_min, int ctx_max,
+                            int can_share) {
+    return step_takes_one_launch(G, num_heads, num_kv_heads, bits, max_seq_len, ctx_min, ctx_max, can_share != 0) ? 1 : 0;
 }
 int tw_kv_decode_step_plan(int G, int num_heads, int num_kv_heads, int bits, int max_seq_len, int ctx_min, int ctx_max) {
     return tw_kv_decode_step_plan2(G, num_heads, num_kv_heads, bits, max_seq_len, ctx_min, ctx_max, 0);
@@ -676,19 +681,17 @@ static FusedArgs fused_args(const tw_half* k_buf, const tw_half* v_buf, int kv_d
 static bool try_decode_fused(const AttnArgs& a, const FusedArgs& f_in, int msl, hipStream_t s, const char* fn) {
     const int mode = g_decode_fused.load();
     FusedArgs f = f_in;
-    f.ctx_bound = t_ctx_max > 0 ? (t_ctx_max < msl ? t_ctx_max : msl) : msl;
     if (mode == 2 || g_variant.load() == 1) return false;
     if (!decode_fused_usable(a, f)) return false;
     // shares: the caller's tickets, and the attention scratch (G * num_heads * msl floats) for the shares' sums
     const bool can_share = t_tickets != nullptr && a.ws != nullptr && shares_that_fit(msl) >= 2 &&
                            (reinterpret_cast<uintptr_t>(a.ws) & 3u) == 0;
-    f.max_shares = 1;
-    if (can_share) { f.tickets = t_tickets; f.share_ws = a.ws; f.max_shares = shares_that_fit(msl); }
-    if (mode != 1 && mode != 3 &&
-        !tw_kv_decode_step_plan2(a.G, a.num_heads, a.num_kv_heads, a.bits, msl, t_ctx_min, t_ctx_max, can_share ? 1 : 0)) return false;
+    if (can_share) { f.tickets = t_tickets; f.share_ws = a.ws; }
+    const StepPlan plan = decode_step_plan(a.G, a.num_heads, a.num_kv_heads, a.bits, msl, t_ctx_min, t_ctx_max, can_share);
+    if (!plan.one) return false;
     attach_profiler(s);
     g_fused_launches.fetch_add(1);
-    launch_decode_fused(a, f, s, /*allow_pairs=*/mode != 3);
+    launch_decode_fused(a, f, s, /*allow_pairs=*/mode != 3, plan);
     t_scan_start = t_scan_stop = nullptr;
     check_launch(fn);
     return true;
@@ -1059,6 +1062,23 @@ void launch_turbo_gqa_prefill_attention(tw_half* out, const tw_half* q, const ui
 
 // ---------------------------------------------------------------- attention without any allocation
 }  // extern "C"
+
+namespace twkv {
+StepPlan decode_step_plan(int G, int num_heads, int num_kv_heads, int bits, int max_seq_len, int ctx_min, int ctx_max, bool can_share) {
+    const int mode = g_decode_fused.load();
+    StepPlan p{};
+    p.one = mode == 1 || mode == 3 ||
+            (mode == 0 && step_takes_one_launch(G, num_heads, num_kv_heads, bits, max_seq_len, ctx_min, ctx_max, can_share));
+    if (!p.one) return p;
+    const int bound = ctx_max > 0 ? std::min(ctx_max, max_seq_len) : max_seq_len;
+    const FusedShape shape = decode_fused_shape(G, num_heads, num_kv_heads, bits, mode != 3,
+                                                can_share ? shares_that_fit(max_seq_len) : 1, bound);
+    p.hkw = shape.hkw;
+    p.shares = shape.shares;
+    p.early = decode_fused_early(num_heads, num_kv_heads, bits, mode != 3, p.hkw, p.shares, bound);
+    return p;
+}
+}  // namespace twkv
 
 // The split workspace of launch_turbo_gqa_attention_batch as a device array of the library itself, for callers
 // that can neither allocate nor hand over scratch memory.  In host code the array's name only stands for the

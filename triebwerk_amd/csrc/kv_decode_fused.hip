@@ -995,21 +995,21 @@ bool decode_fused_usable(const AttnArgs& a, const FusedArgs& f) {
     return true;
 }
 
-void launch_decode_fused(const AttnArgs& a, const FusedArgs& f_in, hipStream_t s, bool allow_pairs) {
+bool decode_fused_early(int num_heads, int Hk, int bits, bool allow_pairs, int hkw, int shares, int ctx_bound) {
+    // when no wave gets more than 8 tiles of 32 tokens (two heads per wave: 16 / hkw parts per head)
+    return allow_pairs && pairs_fit(bits, num_heads / Hk, hkw) && shares == 1 && ctx_bound > 0 && ctx_bound <= 8 * 32 * (2 * kPairWaves / hkw);
+}
+
+void launch_decode_fused(const AttnArgs& a, const FusedArgs& f_in, hipStream_t s, bool allow_pairs, const StepPlan& plan) {
     FusedArgs f = f_in;
-    const FusedShape shape = decode_fused_shape(a.G, a.num_heads, a.num_kv_heads, a.bits, allow_pairs,
-                                                f.share_ws != nullptr && f.tickets != nullptr ? f.max_shares : 1,
-                                                f.ctx_bound > 0 ? (double)f.ctx_bound : 4096.0);
-    f.hkw = shape.hkw;
-    f.shares = shape.shares;
+    f.hkw = plan.hkw;
+    f.shares = plan.shares;
     f.q_scale = attention_mfma_q_scale(a.bits);
     const int R = a.num_heads / a.num_kv_heads;
     const bool pair = allow_pairs && decode_fused_pairs(a, f.hkw);
     const dim3 g3((unsigned)(a.G * (a.num_kv_heads / f.hkw) * f.shares)), b3((pair ? kPairWaves : kFusedWaves) * kWave);
     const bool prod = f.q_weight != nullptr || f.cos_table != nullptr;
-    // first tile in the middle of the prologue: when no wave gets more than 8 tiles of 32 tokens by the caller's bound
-    // of the context (two heads per wave: 16 / hkw parts per head)
-    const bool early = pair && f.shares == 1 && f.ctx_bound > 0 && f.ctx_bound <= 8 * 32 * (2 * kPairWaves / f.hkw);
+    const bool early = plan.early;
     note_scan_kernel(pair ? (f.shares > 1 ? "decode_fused_kernel, two KV heads per wave, context shared by workgroups"
                                           : "decode_fused_kernel, two KV heads per wave")
                           : (f.shares > 1 ? "decode_fused_kernel, one KV head per wave, context shared by workgroups"

@@ -81,7 +81,7 @@ struct tw_engine {
     hipGraphExec_t graph_exec = nullptr;
     const void* graph_key[4] = {};
     int graph_G = 0;
-    int graph_plan = 0;               // tw_kv_decode_step_plan's answer the captured launches were chosen under
+    twkv::StepPlan graph_plan{};      // what the captured launches were chosen as
     // generate_batch goes on without a graph when capture or instantiation fails (engine.cpp:2396-2410): so does
     // tw_engine_decode_step, until the buffers, the batch or the producers change
     bool graph_failed = false;
@@ -249,13 +249,13 @@ int zero_single(tw_engine* e) {
 // row left, and the append would land in the next sequence's rows (or past the array).
 bool cache_full(const tw_engine* e) { return e->pos_known && e->pos_max >= e->batch_msl; }
 
-// What tw_layer_attention_step will choose for the compressed cache from the host's view of the positions
-// (one launch per layer or three); the captured graph holds the launches of one such choice.
-int step_plan(const tw_engine* e) {
-    if (e->kv_bits == 0) return 0;
-    return tw_kv_decode_step_plan2(e->G, e->shape.num_heads, e->shape.num_kv_heads, e->kv_bits, e->batch_msl,
-                                   e->pos_known ? e->pos_min + 1 : 0, e->pos_known ? e->pos_max + 1 : 0,
-                                   e->d_tickets != nullptr);
+// What tw_layer_attention_step will choose for the compressed cache from the host's view of the positions (one launch
+// per layer, and its shape, or three); the captured graph holds the launches of one such choice.
+twkv::StepPlan step_plan(const tw_engine* e) {
+    if (e->kv_bits == 0) return twkv::StepPlan{};
+    return twkv::decode_step_plan(e->G, e->shape.num_heads, e->shape.num_kv_heads, e->kv_bits, e->batch_msl,
+                                  e->pos_known ? e->pos_min + 1 : 0, e->pos_known ? e->pos_max + 1 : 0,
+                                  e->d_tickets != nullptr);
 }
 
 // forward_layer_batch steps 4-5 (with producers: 3-5), engine.cpp:1972-2006.
@@ -705,10 +705,13 @@ int tw_engine_decode_step(tw_engine* e, const tw_half* q, const tw_half* k, cons
     // a capture that failed for these buffers is not tried again step after step (engine.cpp:2396-2410 tries once
     // per generate_batch and decodes eagerly when it fails)
     if (e->graph_failed && memcmp(key, e->graph_failed_key, sizeof(key)) == 0) return eager(2);
-    // The launches in a captured step were chosen from the context lengths at capture; when the lengths have
-    // grown (or spread) to where the other kernels are the better choice, the step is captured again.
-    const int plan = step_plan(e);
-    if (!e->graph_exec || e->graph_G != e->G || e->graph_plan != plan || memcmp(key, e->graph_key, sizeof(key)) != 0) {
+    // The launches in a captured step were chosen from the context lengths at capture, the number of workgroups that share
+    // a sequence among them.  When the lengths have grown (or spread) to where another form is the better choice, the step
+    // is captured again: at most ten times on the way from 1 to 16384 tokens, 60 us of the host's time each for 28 layers.
+    // (One sequence, 4 bit, 16 heads over 8 KV heads, at 16000 tokens: 18.5 us per layer in the form chosen there, 75.1 in
+    // the one a step captured at 512 tokens holds.)
+    const twkv::StepPlan plan = step_plan(e);
+    if (!e->graph_exec || e->graph_G != e->G || !(e->graph_plan == plan) || memcmp(key, e->graph_key, sizeof(key)) != 0) {
         e->drop_graph();
         // Capture records the launches without running them, so unlike the
         // reference (engine.cpp:2414-2444) nothing has to be re-prefilled.

@@ -210,13 +210,11 @@ struct FusedArgs {
     uint8_t* v_codes;
     half_t* k_norms;
     half_t* v_norms;
-    int ctx_bound;          // in: upper bound of positions + 1 that the host knows (0: none)
     int hkw;                // KV heads per workgroup (launch_decode_fused fills this in)
     float q_scale;          // likewise
     // A unit's context shared by several workgroups, for batches whose units alone leave compute units idle:
-    int shares;             // a power of two up to 64 (launch_decode_fused fills this in; > 1 only with the three below)
-    int max_shares;         // as many shares as share_ws has room for (1: none)
-    float* share_ws;        // G * num_heads * max_shares * (kHeadDim + 4) floats for the shares' unnormalised sums
+    int shares;             // a power of two up to 64 (launch_decode_fused fills this in; > 1 only with the two below)
+    float* share_ws;        // G * num_heads * shares * (kHeadDim + 4) floats for the shares' unnormalised sums
     unsigned* tickets;      // one word per (sequence, KV head): zero before the first launch, left zero by every launch
     // optional producers of q and k applied on the way in, as RotArgs has them (V rows stay as they are)
     const half_t* q_weight; // per-head RMSNorm weights (128); both or neither
@@ -255,8 +253,19 @@ struct FusedShape { int hkw, shares; double us; };
 FusedShape decode_fused_shape(int G, int num_heads, int num_kv_heads, int bits, bool allow_pairs, int max_shares, double ctx);
 // test hook (tw_kv_debug_set_fused_shape): force hkw and / or shares (0 = automatic)
 void decode_fused_force_shape(int hkw, int shares);
-// allow_pairs: the 4-bit kernel whose waves scan two KV heads each, where the shape admits it (false: one head per wave)
-void launch_decode_fused(const AttnArgs& a, const FusedArgs& f, hipStream_t s, bool allow_pairs);
+// whether the waves ask for their first tile in the prologue (allow_pairs as below; ctx_bound: no sequence is longer)
+bool decode_fused_early(int num_heads, int num_kv_heads, int bits, bool allow_pairs, int hkw, int shares, int ctx_bound);
+// How a compressed decode step runs: as three launches, or as one of this shape.  decode_step_plan (kv_capi.hip) is
+// what both the launch and the engine go by; a captured step holds the launches of exactly one such plan.
+struct StepPlan {
+    bool one;
+    int hkw, shares;
+    bool early;
+    bool operator==(const StepPlan& o) const { return one == o.one && hkw == o.hkw && shares == o.shares && early == o.early; }
+};
+StepPlan decode_step_plan(int G, int num_heads, int num_kv_heads, int bits, int max_seq_len, int ctx_min, int ctx_max, bool can_share);
+// allow_pairs: the kernel whose waves scan two KV heads each, where the shape admits it (false: one head per wave)
+void launch_decode_fused(const AttnArgs& a, const FusedArgs& f, hipStream_t s, bool allow_pairs, const StepPlan& plan);
 // causal prefill with blocks of query tokens per wave (kv_prefill_mfma.hip); same workspace and merge
 bool prefill_mfma_usable(const AttnArgs& a);
 void launch_prefill_mfma_scan(const AttnArgs& a, hipStream_t s);
