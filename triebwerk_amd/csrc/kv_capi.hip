@@ -240,35 +240,44 @@ static int shares_that_fit(int max_seq_len) {
 }
 
 static bool step_takes_one_launch(int G, int num_heads, int num_kv_heads, int bits, int max_seq_len, int ctx_min, int ctx_max,
-                                  bool can_share) {
+                                  double ctx_mean, bool can_share) {
     if (G <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads != 0 || (bits != 2 && bits != 4)) return false;
     const int group = num_heads / num_kv_heads;
     if (group != 1 && group != 2 && group != 4) return false;
     const bool allow_pairs = g_decode_fused.load() != 3;
-    const int hkw = decode_fused_heads_per_workgroup(G, num_heads, num_kv_heads, bits, allow_pairs);
-    const int split = 16 / hkw;                                   // parts of the context per head: waves / heads
     const bool known = ctx_max > 0;
     const int bound = known ? ctx_max : max_seq_len;
-    if (bound <= 256 * split) return true;                        // at most 8 tiles of 32 tokens per wave
-    if (!known) return false;                                     // lengths unknown: the balanced walk
-    const bool ragged = (long long)(ctx_max - ctx_min) * 8 > ctx_max;
-    // The cheaper of the two by estimates fitted to measured launches (microseconds per layer; the
-    // figures live in one table, plan_constants): one launch as decode_fused_shape counts it (with a sequence's context
-    // shared by workgroups where the caller can hand over tickets and the batch alone leaves compute units idle), three
-    // launches as decode_three_estimate_us does.  Ragged batches take the balanced walk of the three launches, except
-    // small ones whose longest sequence is shared by enough workgroups: that one decides how long the one launch takes,
-    // the mean length the walk.
-    const int max_shares = can_share ? shares_that_fit(max_seq_len) : 1;
-    const FusedShape shape = decode_fused_shape(G, num_heads, num_kv_heads, bits, allow_pairs, max_shares, ctx_max);
-    if (ragged && shape.shares == 1) return false;
-    const double one = shape.us;
-    const double three = decode_three_estimate_us(G, num_heads, num_kv_heads, bits, ragged ? 0.5 * (ctx_min + ctx_max) : ctx_max);
-    return one <= three;
+    const bool ragged = known && (long long)(ctx_max - ctx_min) * 8 > ctx_max;
+    if (!known || ragged) {
+        // at most 8 tiles of 32 tokens per wave: launch-bound whatever the lengths; a wave has 1 / (16 / heads) of the context
+        const int hkw = decode_fused_shape(G, num_heads, num_kv_heads, bits, allow_pairs, 1, bound).hkw;
+        if (bound <= 256 * (16 / hkw)) return true;
+        if (!known) return false;                                 // lengths unknown: the balanced walk
+    }
+    // The cheaper of the two by estimates fitted to measured launches (microseconds per layer; the figures live in one
+    // table, plan_constants): one launch as decode_fused_shape counts it (with a sequence's context shared by workgroups
+    // where the caller can hand over tickets and the batch alone leaves compute units idle), three launches as
+    // decode_three_estimate_us does.
+    const FusedShape shape = decode_fused_shape(G, num_heads, num_kv_heads, bits, allow_pairs,
+                                                can_share ? shares_that_fit(max_seq_len) : 1, ctx_max);
+    if (!ragged) return shape.us <= decode_three_estimate_us(G, num_heads, num_kv_heads, bits, ctx_max);
+    // Ragged batches take the balanced walk of the three launches, except small ones whose longest sequence is shared by
+    // workgroups: that one decides how long the one launch takes, and it streams the mean length.  The walk pays for the
+    // mean length too, and for the longest sequence's pieces: 4 bit, 16 heads over 8 KV heads, one sequence of 8192
+    // tokens and 15 of 200: 30.6 us in one launch, 40.6 in three (24 when all have 200); 32 sequences, one of 16001: 75 and 48.
+    // Over 1216 ragged batches (2 to 64 sequences, 1 to all but a quarter of them long) the choice is the faster form or within
+    // 3 % of it in 1180, and slower than the walk by more than that in 5.  A caller that says no mean gets the smallest one
+    // its bounds allow.
+    if (shape.shares == 1) return false;
+    if (ctx_mean <= 0.0) ctx_mean = ((double)ctx_min * (G - 1) + ctx_max) / G;
+    const PlanConstants& pc = plan_constants();
+    return decode_fused_estimate_us(G, num_heads, num_kv_heads, bits, allow_pairs, shape.hkw, shape.shares, ctx_max, ctx_mean / ctx_max) <=
+           pc.ragged_us + pc.ragged_token_us * ctx_max + pc.ragged_mean_share * decode_three_estimate_us(G, num_heads, num_kv_heads, bits, ctx_mean);
 }
 
 int tw_kv_decode_step_plan2(int G, int num_heads, int num_kv_heads, int bits, int max_seq_len, int ctx_min, int ctx_max,
                             int can_share) {
-    return step_takes_one_launch(G, num_heads, num_kv_heads, bits, max_seq_len, ctx_min, ctx_max, can_share != 0) ? 1 : 0;
+    return step_takes_one_launch(G, num_heads, num_kv_heads, bits, max_seq_len, ctx_min, ctx_max, 0.0, can_share != 0) ? 1 : 0;
 }
 int tw_kv_decode_step_plan(int G, int num_heads, int num_kv_heads, int bits, int max_seq_len, int ctx_min, int ctx_max) {
     return tw_kv_decode_step_plan2(G, num_heads, num_kv_heads, bits, max_seq_len, ctx_min, ctx_max, 0);
@@ -656,6 +665,7 @@ void launch_turbo_gqa_attention_batch(tw_half* out, const tw_half* q, const uint
 // (0, 0 = unknown), for the call being set up on this thread.
 static thread_local int t_ctx_min = 0;
 static thread_local int t_ctx_max = 0;
+static thread_local double t_ctx_mean = 0.0;   // and their mean (0: unknown)
 // Its tickets (tw_layer_step_args::tickets): with them the one-launch step may share a sequence's context between
 // workgroups; the shares' sums go to the attention scratch.
 static thread_local unsigned* t_tickets = nullptr;
@@ -687,7 +697,7 @@ static bool try_decode_fused(const AttnArgs& a, const FusedArgs& f_in, int msl, 
     const bool can_share = t_tickets != nullptr && a.ws != nullptr && shares_that_fit(msl) >= 2 &&
                            (reinterpret_cast<uintptr_t>(a.ws) & 3u) == 0;
     if (can_share) { f.tickets = t_tickets; f.share_ws = a.ws; }
-    const StepPlan plan = decode_step_plan(a.G, a.num_heads, a.num_kv_heads, a.bits, msl, t_ctx_min, t_ctx_max, can_share);
+    const StepPlan plan = decode_step_plan(a.G, a.num_heads, a.num_kv_heads, a.bits, msl, t_ctx_min, t_ctx_max, t_ctx_mean, can_share);
     if (!plan.one) return false;
     attach_profiler(s);
     g_fused_launches.fetch_add(1);
@@ -927,7 +937,10 @@ void launch_sigmoid_gate_batch(tw_half* data, const tw_half* gate, int dim, int 
     check_launch("launch_sigmoid_gate_batch");
 }
 
-void tw_layer_attention_step(const tw_layer_step_args* p, hipStream_t s) {
+void tw_layer_attention_step(const tw_layer_step_args* p, hipStream_t s) { layer_attention_step(p, 0.0, s); }
+}  // extern "C"
+
+void twkv::layer_attention_step(const tw_layer_step_args* p, double ctx_mean, hipStream_t s) {
     const char* fn = "tw_layer_attention_step";
     if (!p) { set_error(1, "%s: NULL arguments", fn); return; }
     if (p->kv_bits != 0 && !check_bits(fn, p->kv_bits)) return;
@@ -936,6 +949,7 @@ void tw_layer_attention_step(const tw_layer_step_args* p, hipStream_t s) {
     t_gate_stride = p->gate ? p->gate_stride : 0;
     t_ctx_min = p->ctx_max > 0 ? p->ctx_min : 0;
     t_ctx_max = p->ctx_max > 0 ? p->ctx_max : 0;
+    t_ctx_mean = p->ctx_max > 0 ? ctx_mean : 0.0;
     t_tickets = p->tickets;
     if (p->kv_bits == 0) {
         if (producers) {
@@ -962,8 +976,11 @@ void tw_layer_attention_step(const tw_layer_step_args* p, hipStream_t s) {
     t_gate = nullptr;
     t_gate_stride = 0;
     t_ctx_min = t_ctx_max = 0;
+    t_ctx_mean = 0.0;
     t_tickets = nullptr;
 }
+
+extern "C" {
 
 // Steps 3-5b of a layer over a prompt (prefill_chunked, engine.cpp:2097-2150): rows are the prompt's tokens,
 // the cache rows are sequence 0's.
@@ -1064,11 +1081,12 @@ void launch_turbo_gqa_prefill_attention(tw_half* out, const tw_half* q, const ui
 }  // extern "C"
 
 namespace twkv {
-StepPlan decode_step_plan(int G, int num_heads, int num_kv_heads, int bits, int max_seq_len, int ctx_min, int ctx_max, bool can_share) {
+StepPlan decode_step_plan(int G, int num_heads, int num_kv_heads, int bits, int max_seq_len, int ctx_min, int ctx_max, double ctx_mean,
+                          bool can_share) {
     const int mode = g_decode_fused.load();
     StepPlan p{};
     p.one = mode == 1 || mode == 3 ||
-            (mode == 0 && step_takes_one_launch(G, num_heads, num_kv_heads, bits, max_seq_len, ctx_min, ctx_max, can_share));
+            (mode == 0 && step_takes_one_launch(G, num_heads, num_kv_heads, bits, max_seq_len, ctx_min, ctx_max, ctx_mean, can_share));
     if (!p.one) return p;
     const int bound = ctx_max > 0 ? std::min(ctx_max, max_seq_len) : max_seq_len;
     const FusedShape shape = decode_fused_shape(G, num_heads, num_kv_heads, bits, mode != 3,

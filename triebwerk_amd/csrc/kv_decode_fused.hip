@@ -37,6 +37,7 @@
 // invalidation of the XCD's L2, cost 34 us per launch; with no fence at all, which is not correct, the launch took
 // 99 us against 97: the scan is not held up by the access pattern.)
 
+#include <algorithm>
 #include <atomic>
 #include <cmath>
 #include <cstring>
@@ -876,13 +877,20 @@ static bool pairs_fit(int bits, int R, int hkw) {
 }
 bool decode_fused_pairs(const AttnArgs& a, int hkw) { return pairs_fit(a.bits, a.num_heads / a.num_kv_heads, hkw); }
 
-// The measured figures behind the estimates below, fitted to 390 launches on MI355X (batches 1 to 256, contexts 300 to 16001, all
-// shapes of a launch, 1 to 64 shares): 4.6 % root mean square.  The shape with the smallest estimate is the fastest
-// measured one or within 3 % of it in 31 of 36 cases (the others within 7.5 %).
+// The measured figures behind the estimates below, fitted to 15400 launches on MI355X: batches 1 to 256, contexts 300 to 16000,
+// 1 to 16 KV heads, GQA groups of 1, 2 and 4, both widths, every shape of a launch with 1 to 64 shares and the three launches,
+// captured steps over as many layers as the last cache level does not hold (or a model's 28).  Single estimates are 7 to 9 %
+// off (root mean square); what counts is the choice: it is the fastest of the forms or within 3 % of it at 2354 of 2455
+// sizes, within 10 % at all but 8.  Fitted to 70 % of the sizes it does as well on the other 30 %.  (The table before had one rate
+// for the three launches' scan whatever the number of KV heads: with 2 of them the scan streams 3 TB/s and not 7, and
+// 192 sequences of 8192 tokens took 190 us in the form chosen, 80 in the best.)
 namespace {
 constexpr PlanConstants kPlanTable[] = {
-    {"gfx950", {10.8, 11.3}, {{{1.60, 1.93, 3.02}, {0.80, 1.25, 1.65}}, {{1.73, 2.11, 2.91}, {2.03, 1.58, 2.17}}},
-     {{7.4e6, 5.1e6}, {4.9e6, 3.4e6}}, {0.0, 2.9, 3.2, 3.4, 4.1, 4.9, 6.5}, {27.0, 25.0}, 2.5, {7.0e6, 5.4e6}},
+    {"gfx950", {7.45, 9.43}, {0.144, 0.125}, {8.37, 8.19},
+     {{{1.88, 2.05, 2.48}, {1.35, 1.48, 1.93}}, {{1.99, 2, 2.81}, {1.69, 1.77, 2.23}}},
+     {{{5.02e6, 7.61e6, 7.92e6, 7.69e6}, {3.62e6, 5.33e6, 5.91e6, 6.37e6}},
+      {{3.39e6, 7.65e6, 6.64e6, 7.18e6}, {1.83e6, 3.96e6, 5.99e6, 5.26e6}}}, {0, 3.34, 3.1, 3.28, 3.63, 4.02, 6.8},
+     {{19.7, 21.1, 24.9}, {19.1, 20, 22.6}}, {{6.67e6, 6.96e6, 6.32e6}, {5.91e6, 5.02e6, 4.94e6}}, {{1.16, 1.27, 0.588}, {1.12, 0.672, 1.14}}, {1.74, 1.51}, 0.000277, 16.2, 0.774e-3, 0.629},
 };
 }  // namespace
 const PlanConstants& plan_constants() {
@@ -902,74 +910,76 @@ const PlanConstants& plan_constants() {
     return *chosen;
 }
 
-// Microseconds one launch takes for G sequences of ctx tokens with hkw KV heads per workgroup: the workgroups run in
-// rounds of one per CU, and a round costs its fixed part and the cube-root sum of its waves' tiles, one after the other,
-// and of all its bytes at the rate the chip streams them in this pattern (waves with one head each: half lines).
-double decode_fused_estimate_us(int G, int num_heads, int Hk, int bits, bool allow_pairs, int hkw, double ctx) {
+// Microseconds one launch takes: the workgroups run in rounds of one per CU.  A round costs the cube-root sum of its waves'
+// tiles of the longest sequence, one after the other, and of its bytes at the rate the chip streams them in this pattern: a
+// workgroup with one KV head reads half lines, and unless the batch is a multiple of 8 the other half is fetched
+// again on another XCD.  A share is a sequence of its own of ctx / shares tokens, plus what the hand-over costs at the end.
+static int group_index(int R) { return R >= 4 ? 2 : R >= 2 ? 1 : 0; }
+static double bytes_per_token(int bits) { return bits == 4 ? 132.0 : 68.0; }       // and KV head: K and V codes and norms
+static double cube_sum(double x, double y) { return std::cbrt(x * x * x + y * y * y); }
+static int log2_of(int x) { int n = 0; while (x > 1) { x >>= 1; n++; } return n; }
+
+double decode_fused_estimate_us(int G, int num_heads, int Hk, int bits, bool allow_pairs, int hkw, int shares, double ctx, double fill) {
     const PlanConstants& pc = plan_constants();
     const double cus = compute_units();
     const int R = Hk > 0 ? num_heads / Hk : 1;
-    const int w = bits == 4 ? 0 : 1, r = R >= 4 ? 2 : R >= 2 ? 1 : 0;
-    const double bpt = bits == 4 ? 132.0 : 68.0;                  // bytes per token and KV head: K and V codes and norms
-    const double units = (double)G * (Hk / hkw);
-    const double rounds = std::ceil(units / cus), active = units < cus ? units : cus;
+    const int w = bits == 4 ? 0 : 1;
     const bool pair = allow_pairs && pairs_fit(bits, R, hkw);
+    const int p = pair ? 0 : 1;
     const int parts = (pair ? 2 * kPairWaves : kFusedWaves) / hkw;          // waves that share a head's tiles
-    const double tiles = std::ceil(std::ceil(ctx / 32.0) / parts) * pc.tile_us[pair ? 0 : 1][w][r];
-    const double bytes = active * hkw * bpt * ctx / pc.one_bw[pair ? 0 : 1][w];
-    return rounds * (pc.one_fixed_us[pair ? 0 : 1] + std::cbrt(tiles * tiles * tiles + bytes * bytes * bytes));
+    const double units = (double)G * (Hk / hkw) * shares, full = std::floor(units / cus), rest = units - full * cus;
+    const double tiles = std::ceil(std::ceil(ctx / shares / 32.0) / parts) * pc.tile_us[p][w][group_index(R)];
+    const double unit_bytes = hkw * bytes_per_token(bits) * ctx / shares * fill / pc.one_bw[G % 8 == 0 ? 0 : 1][w][log2_of(hkw)];
+    double us = pc.one_fixed_us[p] + pc.one_vector_us[p] * hkw * (2 + R) + pc.handover_us[log2_of(shares)];
+    us += full * cube_sum(tiles, cus * unit_bytes);
+    if (rest > 0.0) us += cube_sum(tiles, rest * unit_bytes);
+    return us + pc.one_round_us[p] * (full + (rest > 0.0 ? 0.0 : -1.0));
 }
 
-// Three launches (rotation, scan, merge) for the same step: their fixed cost and the scan at its rate.
+// Three launches (rotation, scan, merge) for the same step: what they cost before the scan and after it, the scan's bytes
+// at its rate or the tiles of one piece of a sequence, one after the other, and the pieces through the merge.
 double decode_three_estimate_us(int G, int num_heads, int Hk, int bits, double ctx) {
     const PlanConstants& pc = plan_constants();
-    const int w = bits == 4 ? 0 : 1;
-    const double bpt = bits == 4 ? 132.0 : 68.0;
-    return pc.three_fixed_us[w] + (num_heads >= 4 * Hk ? pc.three_gqa4_us : 0.0) + (double)G * Hk * bpt * ctx / pc.three_bw[w];
+    const int w = bits == 4 ? 0 : 1, r = group_index(num_heads / Hk);
+    const bool odd = (Hk & 1) != 0;
+    // as plan_splits and the scans' launches cut it: 512 (sequence, chunk) items, a group of waves each
+    int waves = odd ? std::min(Hk, 8) : std::min(Hk / 2, 4);
+    while (waves > 1 && (odd ? Hk : Hk / 2) % waves != 0) waves--;
+    const int groups = (odd ? 16 : 8) / waves, per_item = odd ? waves : 2 * waves;
+    const double base = (double)G * ((Hk + 7) / 8);
+    const double pieces = std::max(1.0, std::min({std::floor(512.0 / base), 64.0, std::ceil(ctx / 128.0)}));
+    const double rounds = std::ceil(G * pieces * (Hk / per_item) / ((double)compute_units() * groups));
+    const double tiles = std::ceil(ctx / pieces / 32.0) * rounds * (odd ? pc.three_tile_odd_us[w] : pc.three_tile_us[w][r]);
+    return pc.three_fixed_us[w][r] + cube_sum(tiles, (double)G * Hk * bytes_per_token(bits) * ctx / pc.three_bw[w][r]) +
+           pc.three_partial_us * G * num_heads * pieces;
 }
 
-// KV heads per workgroup (8, 4, 2 or 1): the choice with the smallest estimate at a context of 4096 tokens (the order
-// hardly depends on the context); among equals the larger number, whose workgroups read longer contiguous pieces of a
-// cache row.  (Batch 64 with 8 KV heads: 2, one round of 256 workgroups; batch 48: 2 again, 192 workgroups in one
-// round, where two rounds of 384 single-head workgroups took 119 us against 85; batch 96: 4.)
-int decode_fused_heads_per_workgroup(int G, int num_heads, int Hk, int bits, bool allow_pairs) {
-    int best = 1;
-    double best_us = 0.0;
-    for (int c = 1; c <= 8; c <<= 1) {
-        if (Hk % c != 0) continue;
-        const double us = decode_fused_estimate_us(G, num_heads, Hk, bits, allow_pairs, c, 4096.0);
-        if (c == 1 || us <= best_us) { best = c; best_us = us; }
-    }
-    return best;
-}
-
-// With shares: a launch of G * (Hk / hkw) * shares workgroups, each with 1 / shares of the context, plus what the
-// hand-over costs at the end (plan_constants).  Shares are only taken while all workgroups fit the compute units in
-// one round and a share still has a tile for every wave.
+// KV heads per workgroup (8, 4, 2 or 1) and shares with the smallest estimate; among equals without shares the larger number
+// of heads, whose workgroups read longer contiguous pieces of a cache row.  Shares are only taken while all workgroups
+// fit the compute units in one round and a share still has a tile for every wave.
 namespace {
 std::atomic<int> g_force_hkw{0}, g_force_shares{0};
 }  // namespace
 void decode_fused_force_shape(int hkw, int shares) { g_force_hkw.store(hkw); g_force_shares.store(shares); }
 
 FusedShape decode_fused_shape(int G, int num_heads, int Hk, int bits, bool allow_pairs, int max_shares, double ctx) {
-    const bool can_share = max_shares >= 2;
     const int R = Hk > 0 ? num_heads / Hk : 1;
     const double cus = compute_units();
-    FusedShape best{decode_fused_heads_per_workgroup(G, num_heads, Hk, bits, allow_pairs), 1, 0.0};
-    best.us = decode_fused_estimate_us(G, num_heads, Hk, bits, allow_pairs, best.hkw, ctx);
-    if (can_share) {
-        for (int c = 1; c <= 8; c <<= 1) {
-            if (Hk % c != 0) continue;
-            const bool pair = allow_pairs && pairs_fit(bits, R, c);
-            const int parts = (pair ? 2 * kPairWaves : kFusedWaves) / c;          // waves (parts of the context) per head
-            for (int sh = 2, lg = 1; sh <= kMaxShares && sh <= max_shares; sh <<= 1, lg++) {
-                if ((double)G * (Hk / c) * sh > cus) continue;
-                if (ctx < 32.0 * parts * sh) continue;
-                // every share is a launch of its own size: G * shares "sequences" of ctx / shares tokens
-                const double us = decode_fused_estimate_us(G * sh, num_heads, Hk, bits, allow_pairs, c, ctx / sh) +
-                                  plan_constants().handover_us[lg];
-                if (us < best.us) best = FusedShape{c, sh, us};
-            }
+    FusedShape best{1, 1, 0.0};
+    for (int c = 1; c <= 8; c <<= 1) {
+        if (Hk % c != 0) continue;
+        const double us = decode_fused_estimate_us(G, num_heads, Hk, bits, allow_pairs, c, 1, ctx, 1.0);
+        if (c == 1 || us <= best.us) best = FusedShape{c, 1, us};
+    }
+    for (int c = 1; c <= 8 && max_shares >= 2; c <<= 1) {
+        if (Hk % c != 0) continue;
+        const bool pair = allow_pairs && pairs_fit(bits, R, c);
+        const int parts = (pair ? 2 * kPairWaves : kFusedWaves) / c;          // waves (parts of the context) per head
+        for (int sh = 2; sh <= kMaxShares && sh <= max_shares; sh <<= 1) {
+            if ((double)G * (Hk / c) * sh > cus) continue;
+            if (ctx < 32.0 * parts * sh) continue;
+            const double us = decode_fused_estimate_us(G, num_heads, Hk, bits, allow_pairs, c, sh, ctx, 1.0);
+            if (us < best.us) best = FusedShape{c, sh, us};
         }
     }
     const int fh = g_force_hkw.load(), fs = g_force_shares.load();

@@ -107,6 +107,9 @@ struct tw_engine {
     // step); a caller that writes the device array itself makes it stale, which only costs kernel choice
     bool pos_known = false;
     int pos_min = 0, pos_max = 0;
+    long long pos_sum = 0;
+    double ctx_mean() const { return pos_known && G > 0 ? 1.0 + (double)pos_sum / G : 0.0; }
+    void one_token_on() { if (pos_known) { pos_min++; pos_max++; pos_sum += G; } }
     std::vector<char> h_finished;
     std::vector<std::vector<int>> outputs;
     std::vector<int> stop_ids;
@@ -254,7 +257,7 @@ bool cache_full(const tw_engine* e) { return e->pos_known && e->pos_max >= e->ba
 twkv::StepPlan step_plan(const tw_engine* e) {
     if (e->kv_bits == 0) return twkv::StepPlan{};
     return twkv::decode_step_plan(e->G, e->shape.num_heads, e->shape.num_kv_heads, e->kv_bits, e->batch_msl,
-                                  e->pos_known ? e->pos_min + 1 : 0, e->pos_known ? e->pos_max + 1 : 0,
+                                  e->pos_known ? e->pos_min + 1 : 0, e->pos_known ? e->pos_max + 1 : 0, e->ctx_mean(),
                                   e->d_tickets != nullptr);
 }
 
@@ -291,7 +294,7 @@ void layer_step(tw_engine* e, int layer, const tw_half* q, const tw_half* k, con
     // what the host knows of the context lengths (positions + 1, the appended token included)
     if (e->pos_known) { p.ctx_min = e->pos_min + 1; p.ctx_max = e->pos_max + 1; }
     p.tickets = e->d_tickets;
-    tw_layer_attention_step(&p, s);
+    twkv::layer_attention_step(&p, e->ctx_mean(), s);
 }
 
 void all_layers(tw_engine* e, const tw_half* q, const tw_half* k, const tw_half* v, tw_half* out,
@@ -397,6 +400,7 @@ int tw_engine_reset(tw_engine* e) {
     hipMemsetAsync(e->d_tickets, 0, (size_t)e->G * e->shape.num_kv_heads * sizeof(unsigned), s);
     e->pos_known = true;
     e->pos_min = e->pos_max = 0;
+    e->pos_sum = 0;
     return hipStreamSynchronize(s) == hipSuccess ? 0 : -1;
 }
 
@@ -417,7 +421,9 @@ int tw_engine_set_positions(tw_engine* e, const int* host_positions, int G) {
     e->pos_known = G == e->G && G > 0;
     if (e->pos_known) {
         e->pos_min = e->pos_max = host_positions[0];
+        e->pos_sum = host_positions[0];
         for (int g = 1; g < G; g++) {
+            e->pos_sum += host_positions[g];
             e->pos_min = host_positions[g] < e->pos_min ? host_positions[g] : e->pos_min;
             e->pos_max = host_positions[g] > e->pos_max ? host_positions[g] : e->pos_max;
         }
@@ -697,7 +703,7 @@ int tw_engine_decode_step(tw_engine* e, const tw_half* q, const tw_half* k, cons
     const void* key[4] = {q, k, v, out};
     auto eager = [&](int state) -> int {
         all_layers(e, q, k, v, out, s);
-        if (e->pos_known) { e->pos_min++; e->pos_max++; }
+        e->one_token_on();
         e->graph_state = state;
         return tw_kv_last_error();
     };
@@ -707,7 +713,7 @@ int tw_engine_decode_step(tw_engine* e, const tw_half* q, const tw_half* k, cons
     if (e->graph_failed && memcmp(key, e->graph_failed_key, sizeof(key)) == 0) return eager(2);
     // The launches in a captured step were chosen from the context lengths at capture, the number of workgroups that share
     // a sequence among them.  When the lengths have grown (or spread) to where another form is the better choice, the step
-    // is captured again: at most ten times on the way from 1 to 16384 tokens, 60 us of the host's time each for 28 layers.
+    // is captured again: up to 18 times on the way from 1 to 16384 tokens, 60 us of the host's time each for 28 layers.
     // (One sequence, 4 bit, 16 heads over 8 KV heads, at 16000 tokens: 18.5 us per layer in the form chosen there, 75.1 in
     // the one a step captured at 512 tokens holds.)
     const twkv::StepPlan plan = step_plan(e);
@@ -743,7 +749,7 @@ int tw_engine_decode_step(tw_engine* e, const tw_half* q, const tw_half* k, cons
         memcpy(e->graph_key, key, sizeof(key));
     }
     if (hipGraphLaunch(e->graph_exec, s) != hipSuccess) return -7;
-    if (e->pos_known) { e->pos_min++; e->pos_max++; }
+    e->one_token_on();
     e->graph_state = 1;
     return 0;
 }

@@ -8,6 +8,8 @@
 
 #include "kv_common.hpp"
 
+struct tw_layer_step_args;          // include/triebwerk_kv.h
+
 namespace twkv {
 
 // ---------------------------------------------------------------- timing the context-scanning kernel
@@ -231,21 +233,29 @@ struct FusedArgs {
 // use that number; tests/test_gpu_plan.py checks on the GPU at hand that the automatic choice is the faster form.
 struct PlanConstants {
     const char* device;         // substring of hipDeviceProp_t::gcnArchName
-    // one launch; first index: waves that scan two KV heads, one head
+    // one launch; first index of the pairs: waves that scan two KV heads, one head
     double one_fixed_us[2];     // prologue, first tile, epilogue, launch and drain
+    double one_vector_us[2];    // more for each vector of the new token that a workgroup has
+    double one_round_us[2];     // each further round of workgroups
     double tile_us[2][2][3];    // a wave's tile of 32 tokens, the waves of a compute unit side by side: [4 bit, 2 bit][GQA group 1, 2, 4]
-    double one_bw[2][2];        // bytes per us the whole chip streams: [4 bit, 2 bit]
+    double one_bw[2][2][4];     // bytes per us the whole chip streams: [batch a multiple of 8, any other][4 bit, 2 bit][1, 2, 4, 8 KV heads per workgroup]
     double handover_us[7];      // shares' sums through memory, by log2(shares)
-    double three_fixed_us[2];   // three launches: rotation, merge, launches and the scan's start and end
-    double three_gqa4_us;       // more with four query heads per KV head
-    double three_bw[2];         // bytes per us of the scan
+    // three launches (rotation, scan, merge): [4 bit, 2 bit][GQA group 1, 2, 4]
+    double three_fixed_us[2][3];   // the launches, the scan's start and end
+    double three_bw[2][3];         // bytes per us of the scan
+    double three_tile_us[2][3];    // a wave's tile of 32 tokens
+    double three_tile_odd_us[2];   // the same for an odd number of KV heads (one head per wave): [4 bit, 2 bit]
+    double three_partial_us;       // a piece of a (sequence, head) through memory and the merge
+    // the walk of a ragged batch: fixed, per token of its longest sequence, and this share of the estimate for the mean length
+    double ragged_us, ragged_token_us, ragged_mean_share;
 };
 const PlanConstants& plan_constants();
 bool decode_fused_usable(const AttnArgs& a, const FusedArgs& f);
-int decode_fused_heads_per_workgroup(int G, int num_heads, int num_kv_heads, int bits, bool allow_pairs);   // 8, 4, 2 or 1
-// estimated microseconds of one launch with hkw KV heads per workgroup, all sequences at ctx tokens
-double decode_fused_estimate_us(int G, int num_heads, int num_kv_heads, int bits, bool allow_pairs, int hkw, double ctx);
-// estimated microseconds of the same step as three launches (rotation, scan, merge)
+// estimated microseconds of one launch with hkw KV heads per workgroup and `shares` workgroups per sequence and head group,
+// the longest sequence at ctx tokens and the mean one at fill * ctx
+double decode_fused_estimate_us(int G, int num_heads, int num_kv_heads, int bits, bool allow_pairs, int hkw, int shares, double ctx,
+                                double fill);
+// estimated microseconds of the same step as three launches (rotation, scan, merge), all sequences at ctx tokens
 double decode_three_estimate_us(int G, int num_heads, int num_kv_heads, int bits, double ctx);
 // The launch's shape when a unit's context may be shared by up to max_shares workgroups (1: the caller has no tickets
 // or no room for the shares' sums): KV heads per workgroup, shares, and the estimate for sequences of ctx tokens.
@@ -263,7 +273,9 @@ struct StepPlan {
     bool early;
     bool operator==(const StepPlan& o) const { return one == o.one && hkw == o.hkw && shares == o.shares && early == o.early; }
 };
-StepPlan decode_step_plan(int G, int num_heads, int num_kv_heads, int bits, int max_seq_len, int ctx_min, int ctx_max, bool can_share);
+StepPlan decode_step_plan(int G, int num_heads, int num_kv_heads, int bits, int max_seq_len, int ctx_min, int ctx_max, double ctx_mean, bool can_share);
+// tw_layer_attention_step for a caller that knows the mean of positions + 1 as well (0: unknown)
+void layer_attention_step(const tw_layer_step_args* p, double ctx_mean, hipStream_t s);
 // allow_pairs: the kernel whose waves scan two KV heads each, where the shape admits it (false: one head per wave)
 void launch_decode_fused(const AttnArgs& a, const FusedArgs& f, hipStream_t s, bool allow_pairs, const StepPlan& plan);
 // causal prefill with blocks of query tokens per wave (kv_prefill_mfma.hip); same workspace and merge
