@@ -1,0 +1,59 @@
+"""The prompt kernels' automatic form against the forms themselves, timed as launches back to back in a graph: within 12 % of the
+fastest forced form from a few tokens to long prompts, with few and many KV heads (the fitted figures leave 2 of 371 sizes of the
+fp16 kernel outside 10 %; medians of seven replays)."""
+import statistics
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+D = 128
+
+
+@pytest.mark.parametrize("bits,H,Hk,T", [(0, 16, 8, 1), (0, 4, 1, 32), (0, 16, 8, 33), (0, 16, 8, 65), (0, 8, 8, 80), (0, 32, 8, 128),
+                                         (0, 16, 8, 300), (0, 32, 8, 1500), (0, 16, 16, 3000), (0, 16, 8, 8192), (4, 16, 8, 33),
+                                         (4, 16, 8, 200), (2, 16, 8, 1500), (4, 8, 2, 3000), (4, 16, 8, 4111)])
+def test_automatic_form_is_the_fastest(bits, H, Hk, T):
+    import torch
+    from triebwerk_amd import kvcache as kv
+    gt = torch.Generator(device="cuda"); gt.manual_seed(7)
+    q = torch.randn((T, H * D), generator=gt, device="cuda", dtype=torch.float16)
+    out = torch.zeros_like(q)
+    if bits:
+        ck, cv = (torch.randint(0, 256, (T, Hk * D * bits // 8), generator=gt, device="cuda", dtype=torch.uint8) for _ in range(2))
+        kn, vn = ((11.3 + 0.7 * torch.randn((T, Hk), generator=gt, device="cuda")).to(torch.float16) for _ in range(2))
+        rot = kv.make_rotation(D, 42).cuda()
+    else:
+        ck, cv = (torch.randn((T, Hk * D), generator=gt, device="cuda", dtype=torch.float16) for _ in range(2))
+    stream = torch.cuda.Stream()
+
+    def call():
+        if bits:
+            kv.launch_turbo_gqa_prefill_attention(out, q, ck, cv, kn, vn, rot, None, T, T, H, Hk, D, H * D, Hk * D, bits, stream=stream)
+        else:
+            kv.launch_gqa_prefill_attention(out, q, ck, cv, None, T, T, H, Hk, D, H * D, Hk * D, stream=stream)
+
+    n, graphs = 20, {}
+    try:
+        for form in (0, 1, 2, 3, 5, 6, 7, 8):
+            kv.set_prefill_form(form)
+            call()
+            stream.synchronize()
+            graphs[form] = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(graphs[form], stream=stream, capture_error_mode="relaxed"):
+                for _ in range(n):
+                    call()
+    finally:
+        kv.set_prefill_form(0)
+    e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    times = {f: [] for f in graphs}
+    with torch.cuda.stream(stream):
+        for _ in range(7):
+            for f, g in graphs.items():
+                e0.record(stream)
+                g.replay()
+                e1.record(stream)
+                stream.synchronize()
+                times[f].append(e0.elapsed_time(e1) / n * 1e3)
+    us = {f: statistics.median(t) for f, t in times.items()}
+    print(f"prefill choice bits={bits} H={H} Hk={Hk} T={T}: " + ", ".join(f"{f}: {t:.2f}" for f, t in us.items()), flush=True)
+    assert us[0] <= 1.12 * min(us.values()), us

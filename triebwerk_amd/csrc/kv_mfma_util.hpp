@@ -82,10 +82,13 @@ int compute_units();
 // chain (at the pace of a workgroup that has its compute unit for itself) and of the steps all workgroups make (at the pace of
 // a full compute unit): estimate = fixed + max(alone * longest, loaded * steps per unit) + per_wg * workgroups per unit
 //                                 + both * min(longest, steps per unit), in us.
-// The figures are fitted to launches of 31 to 8200 tokens with 8, 16 and 32 heads over 2 and 8 KV heads on MI355X (256 compute
-// units): within 15 % everywhere, and the form with the smallest estimate is the fastest measured one or within 3 %
-// of it in 41 of 42 cases (the other: 5 %).  The compressed kernel's figures are from 66 launches of 33 to 5500 tokens at 4 and 2
-// bit, 8, 16 and 32 heads over 8: within 14 %, and the choice the fastest one or within 3.3 % of it in all of them.
+// Measured on MI355X (256 compute units) as launches back to back in a graph, 2 to 32 heads over 1 to 16 KV heads.  fp16: fitted
+// to all forms at 371 sizes of 1 to 16384 tokens; the choice is the fastest form or within 3 % of it at 361, within 10 % at all
+// but 2 (18 %: 8500 tokens, 16 heads over 4).  (With figures fitted from 31 tokens up, launch gaps in them, prompts up to 80
+// tokens took the eight-wave forms: 16 heads over 8, 33 tokens 5.8 us against 4.7 in four waves; and 3000 tokens 66 us
+// against 53.)  The compressed kernel's figures are from 66 launches of 33 to 5500 tokens at 4 and 2 bit, 8, 16 and 32 heads
+// over 8; at 410 sizes of 1 to 8192 tokens and 1 to 16 KV heads the choice is the fastest form or within 3 % at 361, within
+// 7 % at all.
 struct PrefillForm { int id, waves, nq, groups; double fixed, alone, loaded, per_wg, both; };
 struct PrefillChoice { int id, waves, nq, groups; bool mirror; int blocks; };
 
