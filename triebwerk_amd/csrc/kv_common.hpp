@@ -136,4 +136,7 @@ __device__ __forceinline__ float wave_sum(float v) {
     return v;
 }
 
+// compute units of the current device (cached; kv_attention_mfma.hip)
+int compute_units();
+
 }  // namespace twkv

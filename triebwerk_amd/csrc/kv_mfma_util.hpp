@@ -73,9 +73,6 @@ constexpr int kStreamCodes = 2;
 // the norm rows (16 bytes per token for 8 heads) are shared by the workgroups of a sequence: kept in the caches
 constexpr int kStreamNorms = 0;
 
-// compute units of the current device (cached; kv_attention_mfma.hip)
-int compute_units();
-
 // The forms of the two flash prefill kernels, and the rule that picks one.  A workgroup of `waves` waves in `groups` groups takes
 // 16 * nq * (waves / groups) / R query tokens of one KV head; the groups take turns with the context's tiles.
 // With causal rows the last block's chain of tiles is twice the average, so what a launch takes is the larger of its longest

@@ -13,8 +13,8 @@
 // The sum of squares keeps the reference's reduction tree: a 32-lane shuffle-down tree per group of
 // 32 coordinates, then (s0 + s2) + (s1 + s3).
 //
-// Mapping: 16 lanes own a head vector, 16 bytes each (producer_rows_kernel).  Where a pointer or a stride does not admit
-// 16-byte accesses, one 64-lane wave owns it, lane l with coordinates l and l + 64 (producer_kernel).
+// Mapping: many vectors: 16 lanes own a head vector, 16 bytes each (producer_rows_kernel).  Few vectors, or where a pointer or
+// a stride does not admit 16-byte accesses: one 64-lane wave owns it, lane l with coordinates l and l + 64 (producer_kernel).
 
 #include "kv_common.hpp"
 #include "kv_kernels.hpp"
@@ -85,8 +85,9 @@ producer_kernel(ProducerArgs a) {
     dst[lane + 64] = (half_t)x1;
 }
 
-// The same, 16 lanes per vector: bound by memory.  RMSNorm of 4111 tokens of 16 + 8 heads: 11.1 us against
-// 24.6 of the kernel above, 1000 tokens 4.8 against 8.2; up to 256 tokens the same, a launch's own time.
+// The same, 16 lanes per vector: bound by memory.  RMSNorm of 1500 tokens of 16 + 8 heads (36000 vectors): 6.0 us
+// against 10.7 of the kernel above.  A few vectors are bound by one vector's chain of loads and arithmetic, which is shorter
+// with two coordinates to a lane than with eight: 24 to 1024 vectors 2.8 against 3.2.
 __global__ void __launch_bounds__(kProducerThreads)
 producer_rows_kernel(ProducerArgs a) {
     producer_rows(a, (long long)blockIdx.x * kProducerVecs, a.num_heads + a.num_kv_heads * (a.write_cache ? 2 : 1));
@@ -100,10 +101,17 @@ bool producer_rows_usable(const ProducerArgs& a) {
     return !a.write_cache || (ok(a.v) && ok(a.cache_k) && ok(a.cache_v) && (a.kv_dim & 7) == 0);
 }
 
+// Vectors from which on 16 lanes to a vector are the faster mapping, per compute unit.  RMSNorm: 3456 vectors 3.25 (a wave each)
+// against 3.29 us, 4608 3.52 against 3.33; rotation: 4608 3.41 against 3.44, 5376 3.66 against 3.48; both and the fp16
+// cache's rows in a decode step: 4608 18.3 against 18.9, 6144 19.4 against 19.7, 8192 21.6 against 21.1.
+static long long producer_rows_from(const ProducerArgs& a) {
+    return (long long)(a.norm && a.cos_table ? 24 : a.cos_table ? 20 : 16) * compute_units();
+}
+
 void launch_producer(const ProducerArgs& a, hipStream_t s) {
     const long long vecs = (long long)a.rows * (a.num_heads + a.num_kv_heads * (a.write_cache ? 2 : 1));
     if (vecs <= 0) return;
-    if (producer_rows_usable(a)) {
+    if (vecs > producer_rows_from(a) && producer_rows_usable(a)) {
         hipLaunchKernelGGL(producer_rows_kernel, dim3((unsigned)((vecs + kProducerVecs - 1) / kProducerVecs)), dim3(kProducerThreads), 0, s, a);
         return;
     }
