@@ -413,9 +413,11 @@ static void fill_quant_segments(RotArgs& r, uint8_t* c0, tw_half* n0, const tw_h
 }
 
 // Vectors from which on a launch takes them in tiles shared by a workgroup (append_tokens_kernel) instead of one tile and
-// 16 output coordinates per wave (rotate_kernel).  4 bit, 8 KV heads: 4 tokens 4.4 against 4.7 us, 190 4.6 against 5.8, 1000 9.3
-// against 13.6; 2 bit: 32 tokens 4.6 against 4.4, 64 the same, 190 4.7 against 5.5.
-static long long append_tokens_from(int bits) { return bits == 4 ? 64 : 1024; }
+// 16 output coordinates per wave (rotate_kernel).  8 KV heads, tiles against rotate_kernel as launches back to back in a graph.
+// 4 bit: 128 vectors 4.5 against 4.2 us, 512 4.5 against 4.3, 1024 4.6 against 4.5, 1536 4.6 against 4.6, 2304 4.6 against
+// 5.5, 8192 6.3 against 8.1.  2 bit, whose quantization is three comparisons: 1024 4.5 against 4.1, 2048 4.6 against 4.3, 2304 4.6
+// against 5.2.  (rotate_kernel's step past 2048 vectors is its waves' second round on the compute units.)
+static long long append_tokens_from(int bits) { return (bits == 4 ? 3 : 8) * (long long)compute_units() + 1; }
 
 static void fill_append_tokens(AppendTokensArgs& t, uint8_t* c0, tw_half* n0, const tw_half* s0, uint8_t* c1, tw_half* n1,
                                const tw_half* s1, int nstreams, const tw_half* rotation, const int* positions,
