@@ -198,24 +198,28 @@ void launch_increment(int* positions, int G, hipStream_t s) {
 // copy per (layer, array, destination); here one launch takes up to four arrays, every layer and every destination.
 // A launch costs 4-5 us before it moves anything and a prefix of 256 tokens has 270 KB per layer and destination at 4 bit, so
 // a launch per layer was mostly start and end: 16 prompts of 97 to 256 tokens, prefilled and handed to groups of 8 over 28
-// layers, took 14.13 ms with 448 launches of this kernel and 13.19 with 16.  blockIdx.y = group of destination slots, blockIdx.z = layer * narrays + array; the x blocks
-// stride over the array's bytes, and what a thread has read it stores to every destination of its group.
-constexpr int kBroadcastGroup = 8;
-template <typename W>
+// layers, took 14.13 ms with 448 launches of this kernel and 13.19 with 16.  blockIdx.y = group of destination slots,
+// blockIdx.z = layer * narrays + array; the x blocks stride over the array's bytes, and what a thread has read it stores to
+// every destination of its group.
+template <typename W, int GROUP>
 __global__ void __launch_bounds__(256)
 broadcast_rows_kernel(BroadcastArgs a, int ndst) {
     const int layer = blockIdx.z / a.narrays, which = blockIdx.z - layer * a.narrays;
     const size_t n = a.bytes[which] / sizeof(W);
     char* base = a.base[which] + (size_t)layer * a.layer_bytes;
     const W* from = reinterpret_cast<const W*>(base + (size_t)a.src * a.seq_bytes[which]);
-    const int d0 = blockIdx.y * kBroadcastGroup, d1 = min(d0 + kBroadcastGroup, ndst);
+    auto slot = [&](int d) -> W* {
+        int g = a.dst_begin + d;
+        if (a.src >= a.dst_begin && a.src < a.dst_end && g >= a.src) g++;   // destination slots skip the source
+        return reinterpret_cast<W*>(base + (size_t)g * a.seq_bytes[which]);
+    };
+    const int d0 = blockIdx.y * GROUP, d1 = min(d0 + GROUP, ndst);
+    W* first = slot(d0);
     for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (size_t)gridDim.x * 256) {
         const W w = from[i];
-        for (int d = d0; d < d1; d++) {
-            int g = a.dst_begin + d;
-            if (a.src >= a.dst_begin && a.src < a.dst_end && g >= a.src) g++;   // destination slots skip the source
-            reinterpret_cast<W*>(base + (size_t)g * a.seq_bytes[which])[i] = w;
-        }
+        first[i] = w;
+        if constexpr (GROUP > 1)
+            for (int d = d0 + 1; d < d1; d++) slot(d)[i] = w;
     }
 }
 
@@ -234,10 +238,18 @@ void launch_broadcast_rows(const BroadcastArgs& a, hipStream_t s) {
     size_t blocks = (most / width + 255) / 256;
     if (blocks > 64) blocks = 64;                          // a block copies up to 4 KB per pass
     if (blocks < 1) blocks = 1;
-    dim3 grid((unsigned)blocks, (unsigned)((ndst + kBroadcastGroup - 1) / kBroadcastGroup), (unsigned)(a.narrays * a.layers));
-    if (width == 16) hipLaunchKernelGGL(broadcast_rows_kernel<uint4>, grid, dim3(256), 0, s, a, ndst);
-    else if (width == 4) hipLaunchKernelGGL(broadcast_rows_kernel<uint32_t>, grid, dim3(256), 0, s, a, ndst);
-    else hipLaunchKernelGGL(broadcast_rows_kernel<uint16_t>, grid, dim3(256), 0, s, a, ndst);
+    // A row is read once for up to eight destinations where that leaves every compute unit 16 workgroups or more all the same;
+    // a smaller launch (one layer, few destinations) has a workgroup per destination, and with it the copies in flight that
+    // eight in one thread would make it wait for: 8192 tokens of one layer, 4 bit, to 7 destinations 12.1 us against 16.3, fp16 to 3
+    // of them 23.9 against 34.7.
+    const long long each = (long long)blocks * ndst * a.narrays * a.layers;
+    const int group = ndst > 1 && each > 16LL * compute_units() ? 8 : 1;
+    dim3 grid((unsigned)blocks, (unsigned)((ndst + group - 1) / group), (unsigned)(a.narrays * a.layers));
+#define TW_BROADCAST(WW) \
+    do { if (group == 8) hipLaunchKernelGGL((broadcast_rows_kernel<WW, 8>), grid, dim3(256), 0, s, a, ndst); \
+         else hipLaunchKernelGGL((broadcast_rows_kernel<WW, 1>), grid, dim3(256), 0, s, a, ndst); } while (0)
+    if (width == 16) TW_BROADCAST(uint4); else if (width == 4) TW_BROADCAST(uint32_t); else TW_BROADCAST(uint16_t);
+#undef TW_BROADCAST
 }
 
 }  // namespace twkv
