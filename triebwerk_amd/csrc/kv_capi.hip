@@ -368,8 +368,7 @@ int tw_kv_broadcast_rows(void* const* bases, const size_t* seq_bytes, const size
         b.bytes[b.narrays] = bytes[i];
         b.narrays++;
     }
-    launch_broadcast_rows(b, s);
-    check_launch("tw_kv_broadcast_rows");
+    (void)twkv::broadcast_rows("tw_kv_broadcast_rows", b, s);      // a failed launch is in the error state, as with the launchers
     return 0;
 }
 
@@ -1083,6 +1082,19 @@ void launch_turbo_gqa_prefill_attention(tw_half* out, const tw_half* q, const ui
 }  // extern "C"
 
 namespace twkv {
+int broadcast_rows(const char* fn, const BroadcastArgs& a, hipStream_t s) {
+    if (a.src < 0 || a.dst_begin < 0 || a.dst_end < a.dst_begin) {
+        set_error(1, "%s: bad arguments (source %d, destinations %d to %d)", fn, a.src, a.dst_begin, a.dst_end);
+        return -1;
+    }
+    const bool earlier = hipPeekAtLastError() != hipSuccess;       // of some other call on this thread: noted, but not this call's
+    launch_broadcast_rows(a, s);
+    const hipError_t e = hipGetLastError();
+    if (e == hipSuccess) return 0;
+    set_error((int)e, "%s: %s", fn, hipGetErrorString(e));
+    return earlier ? 0 : -2;
+}
+
 StepPlan decode_step_plan(int G, int num_heads, int num_kv_heads, int bits, int max_seq_len, int ctx_min, int ctx_max, double ctx_mean,
                           bool can_share) {
     const int mode = g_decode_fused.load();

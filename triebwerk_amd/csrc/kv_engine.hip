@@ -776,7 +776,6 @@ int tw_kv_set_trace_ranges(int on) {
 int tw_engine_broadcast_prefix(tw_engine* e, int src, int dst_begin, int dst_end, int T, hipStream_t s) {
     if (!e->arena || src < 0 || src >= e->G || dst_begin < 0 || dst_end > e->G || T < 0 || T > e->batch_msl)
         return -1;
-    if (dst_end < dst_begin) return -2;
     s = pick(e, s);
     e->note_step(s);
     // one launch: every layer, array and destination (carve() lays the layers out at equal distances)
@@ -793,8 +792,8 @@ int tw_engine_broadcast_prefix(tw_engine* e, int src, int dst_begin, int dst_end
         b.bytes[b.narrays] = (size_t)T * row_bytes;
         b.narrays++;
     }
-    if (T > 0) twkv::launch_broadcast_rows(b, s);
-    return hipGetLastError() == hipSuccess ? 0 : -2;
+    if (T == 0 && dst_end >= dst_begin) return 0;
+    return twkv::broadcast_rows("tw_engine_broadcast_prefix", b, s) == 0 ? 0 : -2;
 }
 
 }  // extern "C"

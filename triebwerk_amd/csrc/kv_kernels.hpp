@@ -64,6 +64,9 @@ struct BroadcastArgs {
     int narrays;
     int src, dst_begin, dst_end;
 };
+// checks the range, launches and notes what went wrong in the library's error state under fn's name (kv_capi.hip);
+// 0, -1 for a bad range, -2 for a launch that failed
+int broadcast_rows(const char* fn, const BroadcastArgs& a, hipStream_t s);
 void launch_broadcast_rows(const BroadcastArgs& a, hipStream_t s);
 
 // ---------------------------------------------------------------- producers of q and k (kv_producer.hip)

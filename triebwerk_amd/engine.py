@@ -164,6 +164,7 @@ class Engine:
     def broadcast_prefix(self, src: int, dst_begin: int, dst_end: int, T: int, stream=None) -> None:
         rc = self._lib.tw_engine_broadcast_prefix(self._h, src, dst_begin, dst_end, T, _stream(stream))
         if rc != 0:
+            _lib.check(self._lib)
             raise RuntimeError(f"broadcast_prefix failed ({rc})")
 
     def graph_state(self) -> int:
