@@ -50,3 +50,21 @@ def test_both_kernels(oracle, rotation_fixture, bits, Hk, streams, batch, past):
     for g, w in zip(got, want):
         for a, b in zip(g, w):
             same_bytes(a, b)
+
+
+@pytest.mark.parametrize("bits,T,Hk", [(4, 1366, 8), (2, 2303, 8), (4, 3500, 8), (4, 4097, 8), (2, 5001, 8)])
+def test_tiles_per_workgroup(oracle, rotation_fixture, bits, T, Hk):
+    """Sizes that give a workgroup 2, 3, 2, 3 and 4 tiles on 256 compute units, the last run ragged."""
+    from triebwerk_amd import kvcache as kv
+    r = gen.rng(7500 + T)
+    kv_dim, msl = Hk * D, T + 1
+    k, v = (gen.normal_f16(r, (T, kv_dim)) for _ in range(2))
+    pos = r.permutation(msl)[:T].astype(np.int32)
+    want = [(np.zeros((msl, kv_dim * bits // 8), np.uint8), np.zeros((msl, Hk), np.float16)) for _ in range(2)]
+    got = [tuple(dev(x) for x in w) for w in want]
+    for s, (c, n) in zip((k, v), want):
+        oracle.turbo_kv_quantize(c, n, s, rotation_fixture, pos, msl, T, Hk, D, kv_dim, bits)
+    kv.tw_turbo_kv_append_tokens(*got[0], *got[1], dev(k), dev(v), dev(rotation_fixture), dev(pos), msl, T, Hk, D, kv_dim, bits)
+    for g, w in zip(got, want):
+        for a, b in zip(g, w):
+            same_bytes(a, b)

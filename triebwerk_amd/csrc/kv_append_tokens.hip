@@ -206,11 +206,19 @@ void launch_append_tokens(const AppendTokensArgs& args, int bits, hipStream_t s)
     const bool prod = a.p.norm || a.p.cos_table;
     const int tiles = (a.p.rows * a.p.num_kv_heads * a.nstreams + kTileVecs - 1) / kTileVecs;
     if (tiles <= 0) return;
-    // One tile per workgroup while there are fewer than four workgroups per compute unit, then up to four: a workgroup's start
-    // (R, the first loads) is worth a tile, but a few workgroups more than four rounds' worth cost a whole round
-    // (2000 tiles, 4 bit: 17.0, 15.2, 16.4 us with 1, 2, 3 tiles each; 4111: 32.5, 29.7, 28.6, 31.3 with 1 to 4; 8192: 57, 49.5, 49.5,
-    // 47.4, and 47.6 with 8).
-    a.nper = std::max(1, std::min(4, (tiles + 1023) / 1365));
+    // Tiles per workgroup: a workgroup's start (R, the first loads) is worth a good part of a tile, but the compute units take the
+    // workgroups in turns, and a turn begun for a few of them costs all of it.  With n tiles each a launch takes start[n] and
+    // turn[n] for every turn of one workgroup per compute unit: within 7 % at 23 counts of 256 to 16384 tiles, and the n with
+    // the smallest sum is the fastest or within 1.4 % of it in all of them (4 bit, us with 1, 2, 3, 4: 1024 tiles 9.4, 9.3, 12.1,
+    // 10.6; 1536: 13.2, 12.0, 12.2, 15.5; 2300: 18.7, 18.2, 16.5, 20.4; 4096: 30.5, 27.1, 29.0, 26.0; 8192: 57.7, 50.1, 49.9, 47.8;
+    // 6 each: 52.8).
+    constexpr double kStart[] = {0.0, 3.3, 3.8, 4.4, 5.2}, kTurn[] = {0.0, 1.63, 2.8, 4.0, 5.2};
+    double least = 0.0;
+    for (int n = 1; n <= 4; n++) {
+        const int groups = (tiles + n - 1) / n, turns = (groups + compute_units() - 1) / compute_units();
+        const double us = kStart[n] + kTurn[n] * turns;
+        if (n == 1 || us < least) { least = us; a.nper = n; }
+    }
     a.kv_blocks = (tiles + a.nper - 1) / a.nper;
     a.q_blocks = prod ? (int)(((long long)a.p.rows * a.p.num_heads + kProducerVecs - 1) / kProducerVecs) : 0;
     // queries beside the tiles while everything runs at once; beyond that the low occupancy of this kernel costs them more than
