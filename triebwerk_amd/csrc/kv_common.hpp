@@ -18,20 +18,14 @@ typedef float float4_t __attribute__((ext_vector_type(4)));
 typedef float float16_t __attribute__((ext_vector_type(16)));
 
 // Lloyd-Max tables of the reference (kernels.cu:1426-1445).
-__device__ __constant__ const float kCentroids2[4] = {-0.13351f, -0.04003f, 0.04003f, 0.13351f};
-__device__ __constant__ const float kBounds2[3] = {-0.08677f, 0.0f, 0.08677f};
-__device__ __constant__ const float kCentroids4[16] = {
+__device__ __constant__ constexpr float kCentroids2[4] = {-0.13351f, -0.04003f, 0.04003f, 0.13351f};
+__device__ __constant__ constexpr float kCentroids4[16] = {
     -0.24155f, -0.18293f, -0.14304f, -0.11099f, -0.08330f, -0.05806f, -0.03432f, -0.01135f,
     0.01135f,  0.03432f,  0.05806f,  0.08330f,  0.11099f,  0.14304f,  0.18293f,  0.24155f};
-__device__ __constant__ const float kBounds4[15] = {
-    -0.21224f, -0.16299f, -0.12701f, -0.09715f, -0.07068f, -0.04619f, -0.02284f, 0.00000f,
-    0.02284f,  0.04619f,  0.07068f,  0.09715f,  0.12701f,  0.16299f,  0.21224f};
-
-// Host-side copies for building lookup tables.
-static const float kCentroids2Host[4] = {-0.13351f, -0.04003f, 0.04003f, 0.13351f};
-static const float kCentroids4Host[16] = {
-    -0.24155f, -0.18293f, -0.14304f, -0.11099f, -0.08330f, -0.05806f, -0.03432f, -0.01135f,
-    0.01135f,  0.03432f,  0.05806f,  0.08330f,  0.11099f,  0.14304f,  0.18293f,  0.24155f};
+// decision boundaries
+constexpr float kEdges2[3] = {-0.08677f, 0.00000f, 0.08677f};
+constexpr float kEdges4[15] = {-0.21224f, -0.16299f, -0.12701f, -0.09715f, -0.07068f, -0.04619f, -0.02284f, 0.00000f,
+                               0.02284f,  0.04619f,  0.07068f,  0.09715f,  0.12701f,  0.16299f,  0.21224f};
 
 // turbo_quantize of the reference (kernels.cu:1448-1473) with the boundaries as immediates.  The reference walks a
 // tree of strict `<` comparisons for 4 bits (a value on a boundary goes up, NaN -> 15) and counts `>=` for 2 bits
@@ -41,14 +35,12 @@ static const float kCentroids4Host[16] = {
 // around them (2 us per decode launch for the four values per lane of a rotation).
 __device__ __forceinline__ int turbo_quantize(float val, int bits) {
     if (bits == 4) {
-        constexpr float kB[15] = {-0.21224f, -0.16299f, -0.12701f, -0.09715f, -0.07068f, -0.04619f, -0.02284f, 0.00000f,
-                                  0.02284f,  0.04619f,  0.07068f,  0.09715f,  0.12701f,  0.16299f,  0.21224f};
         int idx = 0;
 #pragma unroll
-        for (int i = 0; i < 15; i++) idx += !(val < kB[i]) ? 1 : 0;
+        for (int i = 0; i < 15; i++) idx += !(val < kEdges4[i]) ? 1 : 0;
         return idx;
     }
-    return (int)(val >= -0.08677f) + (int)(val >= 0.0f) + (int)(val >= 0.08677f);
+    return (int)(val >= kEdges2[0]) + (int)(val >= kEdges2[1]) + (int)(val >= kEdges2[2]);
 }
 
 // Cache row of position p of sequence g: the reference's g*msl + p

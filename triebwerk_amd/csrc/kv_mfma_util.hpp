@@ -35,7 +35,7 @@ __device__ __forceinline__ float h2f_bits(uint32_t bits16) {
 // Centroid number c % 16 (4 bit) or c % 4 (2 bit) by selections between immediates: the values are in a register while the
 // first loads of a kernel are still under way, where a per-lane index into the constant array is one more load to wait for.
 template <int BITS>
-__device__ __forceinline__ float centroid_of(int c) {
+__host__ __device__ __forceinline__ constexpr float centroid_of(int c) {
     if constexpr (BITS == 4) {
         const int k = (c & 7) ^ ((c & 8) ? 0 : 7);                  // the tables are symmetric
         const float m01 = (k & 1) ? 0.03432f : 0.01135f, m23 = (k & 1) ? 0.08330f : 0.05806f;
@@ -47,6 +47,13 @@ __device__ __forceinline__ float centroid_of(int c) {
         return (c & 2) ? m : -m;
     }
 }
+
+constexpr bool centroids_agree() {
+    for (int c = 0; c < 16; c++)
+        if (centroid_of<4>(c) != kCentroids4[c] || centroid_of<2>(c) != kCentroids2[c & 3]) return false;
+    return true;
+}
+static_assert(centroids_agree(), "the selections give the tables' values");
 
 __device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
 

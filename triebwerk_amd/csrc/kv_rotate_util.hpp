@@ -78,13 +78,22 @@ __device__ __forceinline__ float rotation_tree_sum_sq(const float (&xv)[32]) {
     return (sgrp[0] + sgrp[2]) + (sgrp[1] + sgrp[3]);
 }
 
-// Decision boundaries of turbo_quantize (kernels.cu:1448-1473) and their buckets: boundary i lies in a bucket of its own, at
-// least 0.15 bucket widths from the bucket's edges, far more than bucket_of rounds.  A 4-bit code then comes from its
-// bucket -- at most one boundary lies in each -- instead of 15 comparisons.
-constexpr float kEdges4[15] = {-0.21224f, -0.16299f, -0.12701f, -0.09715f, -0.07068f, -0.04619f, -0.02284f, 0.00000f,
-                                0.02284f,  0.04619f,  0.07068f,  0.09715f,  0.12701f,  0.16299f,  0.21224f};
+// Buckets of the 4-bit decision boundaries: boundary i lies in a bucket of its own, at least 0.15 bucket widths from the
+// bucket's edges (checked below), far more than bucket_of rounds.  A 4-bit code then comes from its bucket -- at most one
+// boundary lies in each -- instead of 15 comparisons.
 constexpr int kBuckets = 32;
 constexpr float kBucketScale = 72.30f, kBucketShift = 16.50f;
+constexpr bool edges_have_buckets() {
+    int before = 0;                                // bucket 0 holds no boundary: -inf is code 0 by it
+    for (int i = 0; i < 15; i++) {
+        const double at = (double)kEdges4[i] * kBucketScale + kBucketShift;
+        const int b = (int)at;
+        if (b <= before || b >= kBuckets || at - b < 0.15 || b + 1 - at < 0.15) return false;
+        before = b;
+    }
+    return before == kBuckets - 1;                 // the last bucket holds one: +inf and NaN are code 15 by it
+}
+static_assert(edges_have_buckets(), "each boundary in a bucket of its own, the last one in the last bucket");
 // (the smaller bound comes last: a NaN ends up in the last bucket)
 __host__ __device__ __forceinline__ int bucket_of(float x) {
     return (int)fmaxf(fminf(__builtin_fmaf(x, kBucketScale, kBucketShift), (float)(kBuckets - 1)), 0.0f);
