@@ -87,7 +87,7 @@ constexpr int kStreamNorms = 0;
 // a full compute unit): estimate = fixed + max(alone * longest, loaded * steps per unit) + per_wg * workgroups per unit
 //                                 + both * min(longest, steps per unit), in us.
 // Measured on MI355X (256 compute units) as launches back to back in a graph, 2 to 32 heads over 1 to 16 KV heads.  fp16: fitted
-// to all forms at 371 sizes of 1 to 16384 tokens; the choice is the fastest form or within 3 % of it at 361, within 10 % at all
+// to all forms at 371 sizes of 1 to 16384 tokens; the choice is the fastest form or within 3 % of it at 362, within 10 % at all
 // but 2 (18 %: 8500 tokens, 16 heads over 4).  (With figures fitted from 31 tokens up, launch gaps in them, prompts up to 80
 // tokens took the eight-wave forms: 16 heads over 8, 33 tokens 5.8 us against 4.7 in four waves; and 3000 tokens 66 us
 // against 53.)  The compressed kernel's figures are from 66 launches of 33 to 5500 tokens at 4 and 2 bit, 8, 16 and 32 heads

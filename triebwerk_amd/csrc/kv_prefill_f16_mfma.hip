@@ -423,7 +423,7 @@ void launch_prefill_f16_mfma(const AttnArgs& a, hipStream_t s, int form) {
     const int T = a.G;
     // id: the number the test hook forces the form by
     static constexpr PrefillForm kForms[] = {
-        {1, 4, 1, 1, 3.83, 0.487, 0.321, 1.56, 0.0553}, {2, 8, 1, 2, 5.07, 0.617, 0.766, 2.21, 0.0}, {3, 8, 2, 2, 6.46, 0.903, 1.09, 2.05, 0.0},
+        {1, 4, 1, 1, 3.83, 0.487, 0.321, 1.56, 0.0553}, {2, 8, 1, 2, 5.32, 0.617, 0.766, 2.21, 0.0}, {3, 8, 2, 2, 6.46, 0.903, 1.09, 2.05, 0.0},
         {5, 8, 1, 1, 4.58, 0.613, 0.645, 0.0346, 0.0333}, {6, 8, 2, 1, 4.31, 0.884, 0.995, 0.509, 0.0}};
     const PrefillChoice c = choose_prefill_form(kForms, 5, 0.7, T, R, a.num_kv_heads, form);
     const dim3 grid(c.mirror ? (c.blocks + 1) / 2 : c.blocks, a.num_kv_heads), block(c.waves * kWave);
