@@ -239,8 +239,10 @@ static int shares_that_fit(int max_seq_len) {
     return n;
 }
 
+// (best: the one launch's shape at the length at hand, where that is needed for the answer; hkw 0: it was not)
 static bool step_takes_one_launch(int G, int num_heads, int num_kv_heads, int bits, int max_seq_len, int ctx_min, int ctx_max,
-                                  double ctx_mean, bool can_share) {
+                                  double ctx_mean, bool can_share, FusedShape& best) {
+    best = FusedShape{0, 0, 0.0};
     if (G <= 0 || num_kv_heads <= 0 || num_heads % num_kv_heads != 0 || (bits != 2 && bits != 4)) return false;
     const int group = num_heads / num_kv_heads;
     if (group != 1 && group != 2 && group != 4) return false;
@@ -259,7 +261,8 @@ static bool step_takes_one_launch(int G, int num_heads, int num_kv_heads, int bi
     // where the caller can hand over tickets and the batch alone leaves compute units idle), three launches as
     // decode_three_estimate_us does.
     const FusedShape shape = decode_fused_shape(G, num_heads, num_kv_heads, bits, allow_pairs,
-                                                can_share ? shares_that_fit(max_seq_len) : 1, ctx_max);
+                                                can_share ? shares_that_fit(max_seq_len) : 1, std::min(ctx_max, max_seq_len));
+    best = shape;
     if (!ragged) return shape.us <= decode_three_estimate_us(G, num_heads, num_kv_heads, bits, ctx_max);
     // Ragged batches take the balanced walk of the three launches, except small ones whose longest sequence is shared by
     // workgroups: that one decides how long the one launch takes, and it streams the mean length.  The walk pays for the
@@ -277,7 +280,8 @@ static bool step_takes_one_launch(int G, int num_heads, int num_kv_heads, int bi
 
 int tw_kv_decode_step_plan2(int G, int num_heads, int num_kv_heads, int bits, int max_seq_len, int ctx_min, int ctx_max,
                             int can_share) {
-    return step_takes_one_launch(G, num_heads, num_kv_heads, bits, max_seq_len, ctx_min, ctx_max, 0.0, can_share != 0) ? 1 : 0;
+    FusedShape shape;
+    return step_takes_one_launch(G, num_heads, num_kv_heads, bits, max_seq_len, ctx_min, ctx_max, 0.0, can_share != 0, shape) ? 1 : 0;
 }
 int tw_kv_decode_step_plan(int G, int num_heads, int num_kv_heads, int bits, int max_seq_len, int ctx_min, int ctx_max) {
     return tw_kv_decode_step_plan2(G, num_heads, num_kv_heads, bits, max_seq_len, ctx_min, ctx_max, 0);
@@ -1099,12 +1103,13 @@ StepPlan decode_step_plan(int G, int num_heads, int num_kv_heads, int bits, int 
                           bool can_share) {
     const int mode = g_decode_fused.load();
     StepPlan p{};
+    FusedShape shape{0, 0, 0.0};
     p.one = mode == 1 || mode == 3 ||
-            (mode == 0 && step_takes_one_launch(G, num_heads, num_kv_heads, bits, max_seq_len, ctx_min, ctx_max, ctx_mean, can_share));
+            (mode == 0 && step_takes_one_launch(G, num_heads, num_kv_heads, bits, max_seq_len, ctx_min, ctx_max, ctx_mean, can_share, shape));
     if (!p.one) return p;
     const int bound = ctx_max > 0 ? std::min(ctx_max, max_seq_len) : max_seq_len;
-    const FusedShape shape = decode_fused_shape(G, num_heads, num_kv_heads, bits, mode != 3,
-                                                can_share ? shares_that_fit(max_seq_len) : 1, bound);
+    if (shape.hkw == 0)
+        shape = decode_fused_shape(G, num_heads, num_kv_heads, bits, mode != 3, can_share ? shares_that_fit(max_seq_len) : 1, bound);
     p.hkw = shape.hkw;
     p.shares = shape.shares;
     p.early = decode_fused_early(num_heads, num_kv_heads, bits, mode != 3, p.hkw, p.shares, bound);
