@@ -190,19 +190,19 @@ const char* tw_kv_debug_last_scan_kernel(void);
 
 /* One launch or three for a layer's decode step over the compressed cache, as a pure function of what the host
  * knows (1 = one launch, 0 = three): G sequences,
- * cache width `bits`, max_seq_len, and the range of positions + 1 (ctx_max = 0: unknown).  One launch when every
- * wave gets at most 8 tiles of 32 tokens, or when the lengths are within 1/8 of each other and the one launch is the
- * cheaper of the two by estimates fitted to measured launches (one launch: rounds of one workgroup per CU, each the
- * time a workgroup needs for its heads of one sequence; three launches: their fixed cost plus the scan at its rate).
- * At 8 KV heads of 128 and a context of 8192 that is one launch for batches of about 40 to 64 sequences and again at
- * 128 (whole rounds of one workgroup per CU) at 4 bit, at batches 64 and 128 at 2 bit, and three for smaller ones,
- * which leave CUs idle, and for those in between; at 4096 tokens one launch up to batch 128 at both widths.
+ * cache width `bits`, max_seq_len, and the range of positions + 1 (ctx_max = 0: unknown).  Lengths unknown, or more than
+ * 1/8 apart: one launch when every wave gets at most 8 tiles of 32 tokens.  Else the cheaper of the two by estimates
+ * fitted to measured launches (one launch: rounds of one workgroup per CU, each the time a workgroup needs for its heads
+ * of one sequence; three launches: their fixed cost plus the scan at its rate).  At 8 KV heads, 16 query heads and a
+ * context of 8192 that is one launch for batches of 47 to 64 sequences and at 112, 120 and 128 (whole rounds of one
+ * workgroup per CU) at 4 bit, at 48, 56, 64 and from 109 to 128 at 2 bit, and three for smaller ones, which leave CUs
+ * idle, and for those in between; at 2048 tokens one launch up to batch 128 at both widths.
  * Alignment of the buffers, which the entry point also checks, is not part of it. */
 int tw_kv_decode_step_plan(int G, int num_heads, int num_kv_heads, int bits, int max_seq_len, int ctx_min, int ctx_max);
 /* The same for a caller that hands the step tickets (tw_layer_step_args::tickets; can_share != 0): the one launch may
  * then give a sequence's context to up to 64 workgroups where the batch alone leaves compute units idle, which
  * makes it the choice for small batches of long sequences too (1 sequence of 16000 tokens, 16 of 4096 or 8192), also
- * ragged ones. */
+ * ragged ones: there with the smallest mean length that the range allows; the engine, which knows the mean, plans with it. */
 int tw_kv_decode_step_plan2(int G, int num_heads, int num_kv_heads, int bits, int max_seq_len, int ctx_min, int ctx_max,
                             int can_share);
 /* Test hook: KV heads per workgroup (0 = automatic; 1, 2, 4, 8) and workgroups per sequence and head group (0 =
@@ -327,9 +327,10 @@ typedef struct tw_layer_step_args {
                                 * Only steers the choice between kernels (tw_kv_debug_set_decode_fused), never results. */
     unsigned* tickets;         /* NULL, or G*num_kv_heads device words that are ZERO before the first call and that
                                 * only these calls touch (every call leaves them zero): with them, the one-launch step
-                                * of a compressed layer may give a sequence's context to two, four or eight workgroups when
-                                * the batch alone leaves compute units idle (their sums meet in `scratch`).  Calls that
-                                * share tickets must not overlap.  Decode step only. */
+                                * of a compressed layer may give a sequence's context to a power of two up to 64 workgroups
+                                * when the batch alone leaves compute units idle (their sums meet in `scratch`: as many as
+                                * 132 floats each fit max_seq_len).  Calls that share tickets must not overlap.  Decode
+                                * step only. */
 } tw_layer_step_args;
 void tw_layer_attention_step(const tw_layer_step_args* args, hipStream_t s);
 

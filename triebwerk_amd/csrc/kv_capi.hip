@@ -675,15 +675,6 @@ static thread_local double t_ctx_mean = 0.0;   // and their mean (0: unknown)
 // workgroups; the shares' sums go to the attention scratch.
 static thread_local unsigned* t_tickets = nullptr;
 
-// The whole step in one launch (kv_decode_fused.hip)?  There one workgroup owns a sequence's heads from the first
-// token to the last: it saves two launches and the scan's ramp (~10 us of a layer) and loses to the three-kernel
-// path where that one's balanced walk or its row-wise loads matter.  Taken when
-//   - every wave gets at most 8 tiles (launch-bound whatever the spread of the lengths), or
-//   - the lengths are known to be within 1/8 of each other and the batch gives at least half the CUs a workgroup,
-//     up to the size where the three-kernel path's better streaming rate has made up for its start-up
-//     (measured on MI355X: 4 bit ~1M tokens per launch; 2 bit with 8 KV heads, where the three-kernel path
-//     loads whole rows cooperatively, ~256k).
-// false = not taken.
 static FusedArgs fused_args(const tw_half* k_buf, const tw_half* v_buf, int kv_dim, uint8_t* ck_q, uint8_t* cv_q,
                             tw_half* k_norms, tw_half* v_norms) {
     FusedArgs f;
@@ -693,6 +684,9 @@ static FusedArgs fused_args(const tw_half* k_buf, const tw_half* v_buf, int kv_d
     return f;
 }
 
+// The whole step in one launch (kv_decode_fused.hip)?  There workgroups own a sequence's heads from the rotations to the
+// output: it saves two launches and the scan's ramp (~10 us of a layer) and loses to the three launches where their balanced
+// walk or their row-wise loads matter.  decode_step_plan decides; alignment is checked here.  false = not taken.
 static bool try_decode_fused(const AttnArgs& a, const FusedArgs& f_in, int msl, hipStream_t s, const char* fn) {
     const int mode = g_decode_fused.load();
     FusedArgs f = f_in;

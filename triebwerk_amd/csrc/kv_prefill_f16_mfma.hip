@@ -270,7 +270,7 @@ prefill_f16_mfma_kernel(AttnArgs a, int T) {
             }
             if (STEADY || t + 2 < ntiles) read_k(t & 1, kf);                           // tile t + 2
             if (STEADY || t + 3 < ntiles) stash((t + 1) & 1, (t + 3) & 3, kr, vr);      // tile t + 3
-            if (STEADY || t + 4 < ntiles) load_tile(first_token(t + 4), kr, vr);              // STEADY: rows past the cache read as zeros
+            if (STEADY || t + 4 < ntiles) load_tile(first_token(t + 4), kr, vr);        // STEADY: past the end the last tile again, not used
             if (do_s) {
                 // maxima of tile t + 1 per query: this lane holds kv tokens tile1 + 16 sub + 4kg + i
 #pragma unroll

@@ -1,7 +1,7 @@
 // kv_producer_util.hpp -- per-head RMSNorm and rotary embedding of one head vector held by one wave
 // (lane l: coordinates l and l + 64), with the reference's roundings (qk_norm_batch_kernel, kernels.cu:880-923;
-// rope_batch_kernel, 927-961; rope_kernel, 193-235).  Shared by kv_producer.hip and kv_decode_fused.hip.  Second half:
-// the same with a vector on 16 lanes, for launches over many tokens (kv_producer.hip, kv_append_tokens.hip).
+// rope_batch_kernel, 927-961; rope_kernel, 193-235): kv_producer.hip with few vectors.  Second half:
+// the same with a vector on 16 lanes (kv_decode_fused.hip, kv_append_tokens.hip, kv_producer.hip with many vectors).
 //
 // Every product is rounded to fp32 before anything else happens to it, as in the reference's separate
 // kernels: no fused multiply-add where the source has none, and no multiply fused into the conversion to
