@@ -46,6 +46,7 @@ def test_automatic_choice_away_from_the_benchmark(bits, H, Hk, lens):
     k, v = (torch.randn((L, G, Hk * D), generator=gt, device="cuda", dtype=torch.float16) for _ in range(2))
     out = torch.zeros_like(q)
     stream = torch.cuda.Stream()
+    torch.cuda.synchronize()                    # the inputs were made on the default stream
     e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
     times = {0: [], 1: [], 2: []}
     try:

@@ -25,6 +25,7 @@ def test_automatic_form_is_the_fastest(bits, H, Hk, T):
     else:
         ck, cv = (torch.randn((T, Hk * D), generator=gt, device="cuda", dtype=torch.float16) for _ in range(2))
     stream = torch.cuda.Stream()
+    torch.cuda.synchronize()                    # the inputs were made on the default stream
 
     def call():
         if bits:
