@@ -258,9 +258,12 @@ attention_mfma_kernel(AttnArgs a, int total_items, int hgroups, int group_waves)
         const uint32_t hgrp = (uint32_t)(h >> 3) * 16u;          // 16-byte group of this head inside a row
         if (PAGED) {
             const long long rr = my_sub ? page_row(pages, 1) : page_row(pages, 0);
+            // (the rows that exist and no more: an unwritten slot's norm may be a NaN or an infinity, which a probability of
+            // zero does not take out; codes of any bits are finite values)
+            const bool exists = useful && tile + 16 * my_sub + ln < n;
             if (wide) {
                 uint32x4_t kq = {0, 0, 0, 0}, vq = {0, 0, 0, 0};
-                if (useful) {
+                if (exists) {
                     const char* kp = reinterpret_cast<const char*>(a.k_norms) + (rr + ln) * nrow + hgrp;
                     const char* vp = reinterpret_cast<const char*>(a.v_norms) + (rr + ln) * nrow + hgrp;
                     kq = *reinterpret_cast<const uint32x4_t*>(kp);
@@ -268,8 +271,11 @@ attention_mfma_kernel(AttnArgs a, int total_items, int hgroups, int group_waves)
                 }
                 return pick(kq) | (pick(vq) << 16);
             }
-            uint32_t kk = *reinterpret_cast<const uint16_t*>(knseq + (rr + ln) * nrow);
-            uint32_t vv = *reinterpret_cast<const uint16_t*>(vnseq + (rr + ln) * nrow);
+            uint32_t kk = 0, vv = 0;
+            if (exists) {
+                kk = *reinterpret_cast<const uint16_t*>(knseq + (rr + ln) * nrow);
+                vv = *reinterpret_cast<const uint16_t*>(vnseq + (rr + ln) * nrow);
+            }
             return kk | (vv << 16);
         }
         const long long row = seq_row0 + tile;

@@ -152,10 +152,14 @@ attention_pair_kernel(AttnArgs a, int total_items, int hgroups, int group_waves)
     // the pair's two fp16 norms of tokens tok0 and tok0 + 16, K and V
     auto issue_n = [&](PairTileRegs<BITS>& t, int tile, int pages, bool live = true) {
         if (PAGED) {
+            // (the rows that exist and no more: an unwritten slot's norm may be a NaN or an infinity, which a probability of
+            // zero does not take out; codes of any bits are finite values)
+            const int rows = live ? n - tile : 0;
 #pragma unroll
             for (int i = 0; i < 2; i++) {
-                __amdgpu_buffer_rsrc_t rk = make_rsrc(knpair + page_row(pages, i) * nrow, live ? kPageTokens * (int)nrow : 0);
-                __amdgpu_buffer_rsrc_t rv = make_rsrc(vnpair + page_row(pages, i) * nrow, live ? kPageTokens * (int)nrow : 0);
+                const int bytes = min(max(rows - kPageTokens * i, 0), kPageTokens) * (int)nrow;
+                __amdgpu_buffer_rsrc_t rk = make_rsrc(knpair + page_row(pages, i) * nrow, bytes);
+                __amdgpu_buffer_rsrc_t rv = make_rsrc(vnpair + page_row(pages, i) * nrow, bytes);
                 t.n[i][0] = __builtin_amdgcn_raw_buffer_load_b32(rk, (int)noff, 0, kStreamNorms);
                 t.n[i][1] = __builtin_amdgcn_raw_buffer_load_b32(rv, (int)noff, 0, kStreamNorms);
             }

@@ -515,10 +515,13 @@ decode_fused_kernel(AttnArgs a, FusedArgs f) {
         // the loop has no branch here)
         auto issue_n = [&](PairTileRegs<BITS>& t) {
             if constexpr (MODE == kPaged) {
+                // (the rows that exist and no more: an unwritten slot's norm may be a NaN or an infinity, which a probability of
+                // zero does not take out; codes of any bits are finite values)
 #pragma unroll
                 for (int i = 0; i < 2; i++) {
-                    __amdgpu_buffer_rsrc_t rk = make_rsrc(knpair + page_row(i) * nrow, page_bytes(nrow));
-                    __amdgpu_buffer_rsrc_t rv = make_rsrc(vnpair + page_row(i) * nrow, page_bytes(nrow));
+                    const int bytes = min(max(next_rows - kPageTokens * i, 0), kPageTokens) * (int)nrow;
+                    __amdgpu_buffer_rsrc_t rk = make_rsrc(knpair + page_row(i) * nrow, bytes);
+                    __amdgpu_buffer_rsrc_t rv = make_rsrc(vnpair + page_row(i) * nrow, bytes);
                     t.n[i][0] = __builtin_amdgcn_raw_buffer_load_b32(rk, (int)noff, 0, kStreamNorms);
                     t.n[i][1] = __builtin_amdgcn_raw_buffer_load_b32(rv, (int)noff, 0, kStreamNorms);
                 }
