@@ -2,9 +2,11 @@
 layer, whose kernels the other tests hold against the oracle: the caches bit for bit, the outputs within the parity
 tolerance (another order of additions and one fp16 rounding).  Contexts at the edges of a tile of 32 tokens and of the
 parts a sequence is cut into, ragged batches, every GQA group and number of heads per workgroup, the producers."""
+import numpy as np
 import pytest
 
-from test_gpu_parity import D, TOL, host, rel_err, rope_tables
+import gen
+from test_gpu_parity import D, TOL, dev, host, rel_err, rope_tables
 
 pytestmark = pytest.mark.gpu
 
@@ -142,3 +144,39 @@ def test_outputs_over_inputs_go_layer_by_layer():
         engines[1].layer_step(l, want[l], k[l], v[l], want[l + 1])
     torch.cuda.synchronize()
     assert torch.equal(chain, want) and chain[L].abs().sum() > 0
+
+
+@pytest.mark.parametrize("bits", [4, 2])
+def test_layers_without_room_for_partials_stay_in_fp32(oracle, bits):
+    """264 sequences of at most 256 rows: a layer by itself takes three launches there, which without room for partials are the
+    kernel that keeps p * norm in fp32, and V norms past 65504 / 2^5 give the oracle's output."""
+    import torch
+    from triebwerk_amd import Engine, kvcache
+    H, Hk, L, G, msl = 16, 8, 2, 264, 256
+    r = gen.rng(5600 + bits)
+    eng = Engine(max_seq_len=msl, kv_bits=bits)
+    eng.set_shape(L, H, Hk, D)
+    eng.alloc_batch(G, msl)
+    pos = np.full(G, msl - 1, np.int32)
+    eng.set_positions(pos)
+    rot = host(eng.rotation())
+    q = gen.normal_f16(r, (L, G, H * D)); k = gen.normal_f16(r, (L, G, Hk * D)); v = gen.normal_f16(r, (L, G, Hk * D))
+    caches = []
+    for l in range(L):
+        c = [r.integers(0, 256, (G, msl, Hk * D * bits // 8), dtype=np.uint8) for _ in range(2)]
+        c[0][:] = c[0][:, :1]
+        c.append(np.ascontiguousarray(np.broadcast_to((5 + 8 * (np.arange(msl) // 32)).astype(np.float16)[None, :, None], (G, msl, Hk))))
+        c.append((4000 + 300 * r.standard_normal((G, msl, Hk))).astype(np.float16))
+        for t, x in zip(eng.cache(l), c):
+            t.copy_(dev(x))
+        caches.append(c)
+    out = torch.zeros((L, G, H * D), dtype=torch.float16, device="cuda")
+    eng.decode_step(dev(q), dev(k), dev(v), out)
+    torch.cuda.synchronize()
+    for l, c in enumerate(caches):
+        oracle.turbo_kv_quantize_batch(c[0], c[2], k[l], rot, pos, msl, G, Hk, D, Hk * D, bits)
+        oracle.turbo_kv_quantize_batch(c[1], c[3], v[l], rot, pos, msl, G, Hk, D, Hk * D, bits)
+        want = np.zeros((G, H * D), np.float16)
+        oracle.turbo_gqa_attention_batch(want, q[l], *c, rot, pos, msl, G, H, Hk, D, H * D, Hk * D, bits)
+        assert rel_err(host(out[l]), want) <= TOL, f"layer {l}"
+    assert kvcache.last_scan_kernel() == "attention_valu_kernel"
