@@ -43,3 +43,35 @@ def test_replay_is_the_eager_step_at_every_length(bits, H, Hk, G):
         forms.add(kvcache.last_scan_kernel())
         assert torch.equal(replayed, out), f"context {ctx}: the replayed step is not the eager step's form"
     assert G > 4 or any("context shared" in f for f in forms), forms
+
+
+@pytest.mark.parametrize("bits,H,Hk,G,L", [(4, 16, 8, 1, 28), (2, 16, 8, 5, 28)])
+def test_every_layer_in_one_launch_is_captured_again_only_for_another_launch(bits, H, Hk, G, L):
+    """While every layer goes into the same one launch, what a layer by itself would take does not matter to the captured step."""
+    import torch
+    from triebwerk_amd import Engine, _lib, kvcache
+    lib = _lib.load()
+    msl = 4096
+    eng = Engine(max_seq_len=msl, kv_bits=bits)
+    eng.set_shape(L, H, Hk, D)
+    eng.alloc_batch(G, msl)
+    q = torch.randn((L, G, H * D), device="cuda").half()
+    k, v = (torch.randn((L, G, Hk * D), device="cuda").half() for _ in range(2))
+    out = torch.zeros_like(q)
+    torch.cuda.synchronize()
+    last, same = None, 0
+    for ctx in range(40, 4000, 33):
+        eng.set_positions([ctx - 1] * G)
+        eng.decode_step(q, k, v, out, use_graph=False)
+        name = kvcache.last_scan_kernel()
+        eng.set_positions([ctx - 1] * G)
+        recorded = lib.tw_kv_decode_fused_launches()
+        eng.decode_step(q, k, v, out, use_graph=True)
+        recorded = lib.tw_kv_decode_fused_launches() - recorded
+        assert eng.graph_state() == 1
+        if name == last and "decode_layers_kernel" in name:
+            same += 1
+            assert recorded == 0, f"context {ctx}: {name} captured again"
+        last = name
+    torch.cuda.synchronize()
+    assert same > 20

@@ -360,20 +360,31 @@ void layer_step(tw_engine* e, int layer, const tw_half* q, const tw_half* k, con
     twkv::layer_attention_step(&p, e->ctx_mean(), s);
 }
 
+// All of an engine's layers, from layer 0's: carve() lays them out at equal distances
+twkv::StepLayers step_layers(const tw_engine* e) {
+    size_t floats = 0;
+    return twkv::StepLayers{e->shape.num_layers, (long long)e->G * e->q_dim(), (long long)e->G * e->kv_dim(),
+                            e->shape.num_layers > 1 ? (char*)e->cache[1][0] - (char*)e->cache[0][0] : 0,
+                            e->kv_bits != 0 ? e->d_layers : nullptr, rows_ws(e, floats)};
+}
+
+// May they go together: independent of each other, in buffers that the kernels take?
+bool layers_together(tw_engine* e, const tw_half* q, const tw_half* k, const tw_half* v, tw_half* out) {
+    if (!layers_independent(e, q, k, v, out)) return false;
+    const tw_layer_step_args p = layer_args(e, 0, q, k, v, out);
+    return twkv::layers_attention_usable(&p, step_layers(e));
+}
+
 void all_layers(tw_engine* e, const twkv::StepPlan& plan, const tw_half* q, const tw_half* k, const tw_half* v, tw_half* out,
                 hipStream_t s) {
-    const size_t qs = (size_t)e->G * e->q_dim(), ks = (size_t)e->G * e->kv_dim();
-    bool done = false;
     if (plan.layers > 1) {
         const tw_layer_step_args p = layer_args(e, 0, q, k, v, out);
-        // carve() lays the layers out at equal distances
-        size_t floats = 0;
-        const twkv::StepLayers layers{plan.layers, (long long)qs, (long long)ks, (char*)e->cache[1][0] - (char*)e->cache[0][0],
-                                      e->kv_bits != 0 ? e->d_layers : nullptr, rows_ws(e, floats)};
-        done = twkv::layers_attention_step(&p, layers, plan, s);
+        twkv::layers_attention_step(&p, step_layers(e), plan, s);
+    } else {
+        const size_t qs = (size_t)e->G * e->q_dim(), ks = (size_t)e->G * e->kv_dim();
+        for (int l = 0; l < e->shape.num_layers; l++)
+            layer_step(e, l, q + l * qs, k + l * ks, v + l * ks, out + l * qs, s);
     }
-    for (int l = 0; l < e->shape.num_layers && !done; l++)
-        layer_step(e, l, q + l * qs, k + l * ks, v + l * ks, out + l * qs, s);
     launch_increment_positions(e->d_positions, e->G, s);  // engine.cpp:2394
 }
 
@@ -771,7 +782,7 @@ int tw_engine_decode_step(tw_engine* e, const tw_half* q, const tw_half* k, cons
     e->note_step(s);
     tw_kv_clear_error();
     const void* key[4] = {q, k, v, out};
-    const twkv::StepPlan plan = step_plan(e, layers_independent(e, q, k, v, out));
+    const twkv::StepPlan plan = step_plan(e, layers_together(e, q, k, v, out));
     auto eager = [&](int state) -> int {
         all_layers(e, plan, q, k, v, out, s);
         e->one_token_on();

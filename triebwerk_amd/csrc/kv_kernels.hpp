@@ -295,9 +295,10 @@ struct StepPlan {
     // instead, KV heads and waves per workgroup.  The fields above stay what a layer by itself would take.
     // (fp16 cache: in pieces of each sequence's context)
     int layers, layers_hkw, layers_waves, layers_pieces;
-    bool operator==(const StepPlan& o) const {
-        return one == o.one && hkw == o.hkw && shares == o.shares && early == o.early && layers == o.layers &&
-               layers_hkw == o.layers_hkw && layers_waves == o.layers_waves && layers_pieces == o.layers_pieces;
+    bool operator==(const StepPlan& o) const {                         // the same launches
+        if (layers != o.layers) return false;
+        if (layers > 1) return layers_hkw == o.layers_hkw && layers_waves == o.layers_waves && layers_pieces == o.layers_pieces;
+        return one == o.one && hkw == o.hkw && shares == o.shares && early == o.early;
     }
 };
 // layers: how many the caller can hand over at once (1: a layer by itself)
@@ -342,8 +343,9 @@ struct StepLayers {
 // fp16 cache: pieces every sequence's context is cut into when all layers go together, with ws_floats of workspace (0: not together)
 int rows_layers_most_pieces(int layers, int G, int num_heads, int num_kv_heads);     // the workspace is made for
 int rows_layers_pieces(int layers, int G, int num_heads, int num_kv_heads, double ctx_max, double ctx_mean, size_t ws_floats);
-// false = not taken, nothing launched
-bool layers_attention_step(const tw_layer_step_args* p, const StepLayers& layers, const StepPlan& plan, hipStream_t s);
+// Whether the buffers admit it (a plan with layers > 1 is for those that do)
+bool layers_attention_usable(const tw_layer_step_args* p, const StepLayers& layers);
+void layers_attention_step(const tw_layer_step_args* p, const StepLayers& layers, const StepPlan& plan, hipStream_t s);
 // allow_pairs: the kernel whose waves scan two KV heads each, where the shape admits it (false: one head per wave)
 void launch_decode_fused(const AttnArgs& a, const FusedArgs& f, hipStream_t s, bool allow_pairs, const StepPlan& plan);
 // the pair kernel (hkw KV heads a workgroup, no shares, no producers) for attention alone, or for the step over the paged cache
