@@ -175,7 +175,8 @@ void tw_kv_debug_set_prefill_form(int form);
 /* tw_turbo_append_attention_batch and the calls built on it can run a layer's decode step as ONE kernel (append,
  * query rotation, scan, merge, rotate-back; a workgroup owns a sequence's heads) instead of three.  0 (default):
  * what tw_kv_decode_step_plan says; 1: one kernel whenever the shape allows it (contiguous compressed cache, GQA
- * group 1, 2 or 4); 2: never; 3: as 1, with one KV head per wave also where the 4-bit kernel would give a wave two. */
+ * group 1, 2 or 4); 2: never; 3: as 1, with one KV head per wave also where the 4-bit kernel would give a wave two; 4: as 0.
+ * tw_engine_decode_step takes every layer by itself while this is not 0, the attention variant is not 0 or a split count is set. */
 void tw_kv_debug_set_decode_fused(int mode);
 /* Timing of the context-scanning attention kernel alone, with HIP events attached to that kernel's launches on
  * their stream.  Enable, run eager launches (not under stream capture; at most 4096 are kept), then read the

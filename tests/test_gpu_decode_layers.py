@@ -180,3 +180,29 @@ def test_layers_without_room_for_partials_stay_in_fp32(oracle, bits):
         oracle.turbo_gqa_attention_batch(want, q[l], *c, rot, pos, msl, G, H, Hk, D, H * D, Hk * D, bits)
         assert rel_err(host(out[l]), want) <= TOL, f"layer {l}"
     assert kvcache.last_scan_kernel() == "attention_valu_kernel"
+
+
+@pytest.mark.parametrize("bits", [4, 2, 0])
+@pytest.mark.parametrize("hook,value", [("set_decode_fused", 2), ("set_decode_fused", 4), ("set_attention_variant", 3), ("set_num_splits", 3)])
+def test_the_hooks_hold_in_an_engines_step(bits, hook, value):
+    """What a hook forces is a layer's kernels: with one set, the step is the layers one by one, bit for bit."""
+    import torch
+    from triebwerk_amd import kvcache
+    H, Hk, L, lens, msl = 16, 8, 4, [300, 77, 1200], 2048
+    G = len(lens)
+    engines, q, k, v = _pair(bits, H, Hk, L, G, msl, False)
+    outs = [torch.zeros_like(q) for _ in range(2)]
+    for e in engines:
+        e.set_positions([n - 1 for n in lens])
+    getattr(kvcache, hook)(value)
+    try:
+        engines[0].decode_step(q, k, v, outs[0], use_graph=True)
+        name = kvcache.last_scan_kernel()
+        for l in range(L):
+            engines[1].layer_step(l, q[l], k[l], v[l], outs[1][l])
+        torch.cuda.synchronize()
+        assert name == kvcache.last_scan_kernel()
+    finally:
+        getattr(kvcache, hook)(0)
+    assert torch.equal(*outs)
+    _same_caches(engines, L)

@@ -276,7 +276,8 @@ def set_prefill_form(form: int) -> None:
 
 def set_decode_fused(mode: int) -> None:
     """tw_kv_debug_set_decode_fused: 0 the library's own choice, 1 one launch whenever the shape allows it, 2 never,
-    3 as 1 but with one KV head per wave also where the 4-bit kernel would give a wave two."""
+    3 as 1 but with one KV head per wave also where the 4-bit kernel would give a wave two, 4 as 0.  Other than 0, an engine's
+    decode step takes every layer by itself."""
     _lib.load().tw_kv_debug_set_decode_fused(int(mode))
 
 
