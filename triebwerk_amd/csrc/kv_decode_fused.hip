@@ -1068,9 +1068,14 @@ bool decode_fused_early(int num_heads, int Hk, int bits, bool allow_pairs, int h
     return allow_pairs && pairs_fit(bits, num_heads / Hk, hkw) && shares == 1 && ctx_bound > 0 && ctx_bound <= 8 * 32 * (2 * kPairWaves / hkw);
 }
 
-// May the units of a sequence go to one XCD each (sequence g to XCD g % 8)?  Where that needs no more rounds of workgroups than any other order.
-static bool units_by_xcd(int G, int units) {
+// May the units of a sequence go to one XCD each (sequence g to XCD g % 8)?  Where that needs no more rounds of workgroups than any other
+// order, and does not leave two or more XCDs idle while the others stream shared contexts.  MI355X, us per layer, by XCD against
+// in any order: 8 over 8 heads, 4 bit, 5 x 16001 tokens 33.7 and 32.9, 6 x 8192 22.7 and 22.2, 2 x 2048 14.8 and 14.3; 7 x 4096 17.5 and
+// 18.1.  One workgroup a unit: 5 x 613 12.7 and 13.0.  16 over 8 heads: 11 x 4096 22.6 and 23.3.
+static bool units_by_xcd(int G, int units, int shares) {
     const int cus = compute_units(), per_xcd = std::max(1, cus / 8);
+    if (shares > 1 && G < 7) return false;
+    units *= shares;
     return (G & 7) == 0 || ((long long)(G + 7) / 8 * units + per_xcd - 1) / per_xcd <= ((long long)G * units + cus - 1) / cus;
 }
 
@@ -1081,7 +1086,7 @@ void launch_decode_fused(const AttnArgs& a, const FusedArgs& f_in, hipStream_t s
     f.q_scale = attention_mfma_q_scale(a.bits);
     const int R = a.num_heads / a.num_kv_heads;
     const bool pair = allow_pairs && decode_fused_pairs(a, f.hkw);
-    f.by_xcd = units_by_xcd(a.G, a.num_kv_heads / f.hkw * f.shares) ? 1 : 0;
+    f.by_xcd = units_by_xcd(a.G, a.num_kv_heads / f.hkw, f.shares) ? 1 : 0;
     const dim3 g3((unsigned)((f.by_xcd ? (a.G + 7) / 8 * 8 : a.G) * (a.num_kv_heads / f.hkw) * f.shares)), b3((pair ? kPairWaves : kFusedWaves) * kWave);
     const bool prod = f.q_weight != nullptr || f.cos_table != nullptr;
     const bool early = plan.early;
@@ -1130,7 +1135,7 @@ void launch_decode_fused_mode(const AttnArgs& a, const FusedArgs& f_in, hipStrea
     f.shares = 1;
     f.q_scale = attention_mfma_q_scale(a.bits);
     const int R = a.num_heads / a.num_kv_heads;
-    f.by_xcd = units_by_xcd(a.G, a.num_kv_heads / hkw) ? 1 : 0;
+    f.by_xcd = units_by_xcd(a.G, a.num_kv_heads / hkw, 1) ? 1 : 0;
     const dim3 g3((unsigned)((f.by_xcd ? (a.G + 7) / 8 * 8 : a.G) * (a.num_kv_heads / hkw))), b3(kPairWaves * kWave);
     note_scan_kernel(a.block_table ? "decode_fused_kernel, two KV heads per wave, paged" : "decode_fused_kernel, two KV heads per wave, attention alone");
 #define TW_MODE(RR, BB) do { if (a.block_table) launch_scan_kernel(decode_fused_kernel<RR, BB, false, true, false, false, kPaged>, g3, b3, s, a, f); \
