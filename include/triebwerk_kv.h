@@ -445,7 +445,11 @@ int tw_engine_set_shape(tw_engine* e, const tw_model_shape* shape);
  * held when that is big enough -- so the steps below always work on exactly G rows (the reference keeps a
  * larger batch and its strides, engine.cpp:1339). */
 int tw_engine_alloc_batch(tw_engine* e, int G, int max_seq_len);
-/* set_arena, engine.cpp:1609-1620: carve out of caller-owned device memory. */
+/* set_arena, engine.cpp:1609-1620: carve out of caller-owned device memory.  Beside the arena, caller-owned or not, and not
+ * counted by arena_bytes_needed, alloc_batch allocates what steps of every layer in one launch need (tw_engine_decode_step; engines of
+ * one layer: nothing): 64 KB for a compressed cache; for an fp16 cache with KV heads in eights at most 4.3 MB, with an even number of
+ * query heads to a KV head 8.7 MB, with a multiple of four 17.3 MB.  Without that memory the steps run all the same: compressed
+ * layer by layer, fp16 with the attention scratch for it.  Freed with the batch (set_arena, set_shape, sleep, destroy). */
 int tw_engine_set_arena(tw_engine* e, void* device_ptr, size_t bytes);
 size_t tw_engine_arena_bytes_needed(const tw_engine* e, int G, int max_seq_len);
 

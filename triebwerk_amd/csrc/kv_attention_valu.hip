@@ -890,19 +890,21 @@ void launch_attention_rows_layers(const AttnArgs& a, const LayerStrides& layers,
 #undef TW_ROWS_D
 }
 
+constexpr int kMostPieces = 32;                              // (at most kMergeSlots)
+// What the workspace is made for: as many as leave 1024 workgroups in all.
 int rows_layers_most_pieces(int layers, int G, int num_heads, int Hk) {
     if (Hk <= 0 || Hk % kRowHeads != 0) return 0;
     AttnArgs a{};
     a.num_heads = num_heads; a.num_kv_heads = Hk;
-    return (int)std::min<long long>(kMergeSlots, 1024 / std::max<long long>(1, (long long)layers * G * attention_rows_groups(a)));
+    return (int)std::min<long long>(kMostPieces, 1024 / std::max<long long>(1, (long long)layers * G * attention_rows_groups(a)));
 }
 
 // Pieces of a sequence's context, one workgroup each: the number with the smallest estimate.  A round of workgroups (two to a compute unit,
 // one with four query heads to a KV head) takes its start and end and the cube-root sum of its waves' tokens, one after the other, and
 // of its bytes at the rate the chip streams; a compute unit with two workgroups beside some with one holds the round up as if a third
 // of those had two as well.  More than one piece: the merge, a launch with the pieces' loads one after the other in every block.
-// Fitted on MI355X to all numbers of pieces from 1 to 64 (as the workspace allows) of 203 steps, 2 to 36 layers, 1 to 192 sequences
-// of 64 to 16000 tokens, even and ragged: the choice is the fastest or within 3 % at 86 %, within 10 % at 97 %.
+// Fitted on MI355X to all numbers of pieces from 1 to 64 (as the workspace allowed) of 203 steps, 2 to 36 layers, 1 to 192 sequences
+// of 64 to 16000 tokens, even and ragged: the choice, of up to kMostPieces, is the fastest or within 3 % at 86 %, within 10 % at 97 %.
 int rows_layers_pieces(int layers, int G, int num_heads, int Hk, double ctx_max, double ctx_mean, size_t ws_floats) {
     if (Hk <= 0 || Hk % kRowHeads != 0) return 0;
     const int group = num_heads / Hk;
@@ -912,7 +914,7 @@ int rows_layers_pieces(int layers, int G, int num_heads, int Hk, double ctx_max,
     const double token_us = group % 4 == 0 ? 0.743 : group % 2 == 0 ? 0.612 : 0.45, start_us = 6.15, rate = 7.16e6;
     int best = 1;
     double best_us = 0.0;
-    for (int pieces = 1; pieces <= 32; pieces++) {
+    for (int pieces = 1; pieces <= kMostPieces; pieces++) {
         if (pieces > 1 && ((size_t)layers * G * num_heads * pieces * kPartialFloats > ws_floats || ctx_max < kRowUnit * (double)pieces)) break;
         const double units = (double)layers * G * attention_rows_groups(a) * pieces, full = std::floor(units / slots);
         const double tokens = std::ceil(ctx_mean / pieces / kRowUnit), bytes = tokens * kRowUnit * kRowHeads * kHeadDim * 4;

@@ -190,8 +190,9 @@ const Rotation& rotation() {
     return r;
 }
 
-// Bytes beside the arena for steps that take all layers at once: compressed, the rotation in operand order; fp16, the partial results
-// of up to 1024 workgroups of sequences cut into pieces (16 query heads and 8 KV heads: 8.7 MB; larger batches are not cut).
+// Bytes beside the arena for steps that take all layers at once: compressed, the rotation in operand order (64 KB); fp16, the partial
+// results of up to 1024 workgroups of sequences cut into pieces (16 query heads and 8 KV heads: up to 8.7 MB).  Where the batch's
+// attention scratch is larger, that is the workspace (rows_ws).
 size_t layers_need(const tw_engine* e) {
     const tw_model_shape& m = e->shape;
     if (m.num_layers < 2) return 0;
