@@ -50,21 +50,11 @@ __device__ __forceinline__ int lane_dim(int c, int e) {
     return 32 * c + e;                                     // one contiguous piece of codes
 }
 
-// Load and dequantize the lane's values (16 of an fp16 row, 32 of a compressed one) of one cache row (one KV head).
-// fresh: fp16 only, the head's 128 halves come from there instead (the row of the token being appended), or NULL.
+// Load and dequantize the lane's 32 values of one compressed cache row (one KV head).
 template <int MODE>
 __device__ __forceinline__ void load_vals(const void* __restrict__ base, long long row, int num_kv_heads,
-                                          int h, int c, const float* __restrict__ cent_s, float* vals,
-                                          const half_t* fresh = nullptr) {
-    if (MODE == 0) {
-        const half_t* p = reinterpret_cast<const half_t*>(base) + (row * num_kv_heads + h) * kHeadDim;
-#pragma unroll
-        for (int j = 0; j < 2; j++) {
-            half8_t h8 = *reinterpret_cast<const half8_t*>((fresh ? fresh : p) + 64 * j + 8 * c);
-#pragma unroll
-            for (int i = 0; i < 8; i++) vals[8 * j + i] = (float)h8[i];
-        }
-    } else if (MODE == 4) {
+                                          int h, int c, const float* __restrict__ cent_s, float* vals) {
+    if (MODE == 4) {
         const uint8_t* p = reinterpret_cast<const uint8_t*>(base) + (row * num_kv_heads + h) * 64 + 16 * c;
         uint4 w4 = *reinterpret_cast<const uint4*>(p);
         uint32_t w[4] = {w4.x, w4.y, w4.z, w4.w};
@@ -318,22 +308,17 @@ attention_valu_kernel(AttnArgs a) {
         finish(acc, m, l);
         return;
     } else {
-    // Query, rotated for the compressed cache: q_rot = R q (kernels.cu:1671-1681).
+    // ---- compressed cache: the query rotated, q_rot = R q (kernels.cu:1671-1681)
     for (int idx = tid; idx < RT * kHeadDim; idx += kAttnThreads) {
         int r = idx / kHeadDim, d = idx % kHeadDim;
         const half_t* qh = a.q + (long long)g * a.q_stride + (long long)(head0 + r) * kHeadDim;
-        float val;
-        if (MODE == 0) {
-            val = (float)qh[d];
-        } else {
-            const half8_t* rot8 = reinterpret_cast<const half8_t*>(a.rotation + d * kHeadDim);
-            const half8_t* q8 = reinterpret_cast<const half8_t*>(qh);
-            val = 0.0f;
-            for (int k8 = 0; k8 < kHeadDim / 8; k8++) {
-                half8_t rr = rot8[k8], qq = q8[k8];
+        const half8_t* rot8 = reinterpret_cast<const half8_t*>(a.rotation + d * kHeadDim);
+        const half8_t* q8 = reinterpret_cast<const half8_t*>(qh);
+        float val = 0.0f;
+        for (int k8 = 0; k8 < kHeadDim / 8; k8++) {
+            half8_t rr = rot8[k8], qq = q8[k8];
 #pragma unroll
-                for (int i = 0; i < 8; i++) val = __builtin_fmaf((float)rr[i], (float)qq[i], val);
-            }
+            for (int i = 0; i < 8; i++) val = __builtin_fmaf((float)rr[i], (float)qq[i], val);
         }
         q_s[r][d] = val;
     }
@@ -359,11 +344,7 @@ attention_valu_kernel(AttnArgs a) {
         const bool valid = t < t1;
         const int tc = valid ? t : (t1 - 1);    // clamp: keep the shuffles among a token's lanes convergent
         const long long row = cache_row(a.block_table, a.bt_stride, a.seq_stride_rows, g, tc);
-        float kn = 1.0f, vn = 1.0f;
-        if (MODE != 0) {
-            kn = (float)a.k_norms[row * a.num_kv_heads + h];
-            vn = (float)a.v_norms[row * a.num_kv_heads + h];
-        }
+        const float kn = (float)a.k_norms[row * a.num_kv_heads + h], vn = (float)a.v_norms[row * a.num_kv_heads + h];
         float vals[E];
         load_vals<MODE>(a.k, row, a.num_kv_heads, h, c, cent_s, vals);
         float s[RT];
