@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 
 import gen
-from test_gpu_parity import D, TOL, dev, host, rel_err, rope_tables
+from test_gpu_parity import D, TOL, assert_bytes_equal, dev, host, rel_err, rope_tables
 
 pytestmark = pytest.mark.gpu
 
@@ -205,4 +205,83 @@ def test_the_hooks_hold_in_an_engines_step(bits, hook, value):
     finally:
         getattr(kvcache, hook)(0)
     assert torch.equal(*outs)
+    _same_caches(engines, L)
+
+
+@pytest.mark.parametrize("norm,biased,rope_dim", [(True, False, 0), (True, True, 0), (False, False, 128), (False, False, 16),
+                                                  (True, True, 64), (True, False, 48)])
+@pytest.mark.parametrize("bits", [4, 2, 0])
+def test_producers_of_every_layer_in_one_launch(oracle, bits, norm, biased, rope_dim):
+    """RMSNorm or RoPE alone, biased weights, a rotary part of the head, per-layer weights: against the oracle, from empty caches on."""
+    import torch
+    from triebwerk_amd import Engine, kvcache
+    L, H, Hk, G, msl, steps = 3, 16, 8, 5, 48, 3
+    q_dim, kv_dim = H * D, Hk * D
+    r = gen.rng(5800 + bits + rope_dim + 2 * norm + biased)
+    eng = Engine(max_seq_len=msl, kv_bits=bits)
+    eng.set_shape(L, H, Hk, D)
+    eng.alloc_batch(G, msl)
+    pos = np.array([0, 3, 30, 31, 41], np.int32)
+    eng.set_positions(pos)
+    rot = host(eng.rotation()) if bits else None
+    w = [((0.0 if biased else 1.0) + 0.2 * r.standard_normal((L, D))).astype(np.float16) for _ in range(2)]
+    tables = rope_tables(msl, rope_dim) if rope_dim else ()
+    d_w, d_tables = [dev(x) for x in w] if norm else [None] * 2, [dev(t) for t in tables] if rope_dim else [None] * 2
+    eng.set_producers(1, *d_w, 1e-6, biased, *d_tables, rope_dim)
+    width = kv_dim * bits // 8 if bits else kv_dim
+    caches = [[np.zeros((G, msl, width), np.uint8 if bits else np.float16) for _ in range(2)] +
+              ([np.zeros((G, msl, Hk), np.float16) for _ in range(2)] if bits else []) for _ in range(L)]
+    out = torch.zeros((L, G, q_dim), dtype=torch.float16, device="cuda")
+    for step in range(steps):
+        q = gen.normal_f16(r, (L, G, q_dim)); k = gen.normal_f16(r, (L, G, kv_dim)); v = gen.normal_f16(r, (L, G, kv_dim))
+        eng.decode_step(dev(q), dev(k), dev(v), out)
+        torch.cuda.synchronize()
+        assert "decode_layers_kernel" in kvcache.last_scan_kernel() or kvcache.last_scan_kernel() == "attention_rows_kernel, every layer"
+        got = host(out)
+        for l, c in enumerate(caches):
+            want, ql, kl = np.zeros((G, q_dim), np.float16), q[l].copy(), k[l].copy()
+            if norm: oracle.qk_norm_batch(ql, kl, w[0][l], w[1][l], H, Hk, D, G, 1e-6, q_dim, kv_dim, biased)
+            if rope_dim: oracle.rope_batch(ql, kl, *tables, pos, msl, G, H, Hk, D, q_dim, kv_dim, rope_dim)
+            if bits == 0:
+                oracle.kv_cache_write_batch(*c, kl, v[l], pos, msl, G, kv_dim)
+                oracle.gqa_attention_batch(want, ql, *c, pos, msl, G, H, Hk, D, q_dim, kv_dim)
+            else:
+                oracle.turbo_kv_quantize_batch(c[0], c[2], kl, rot, pos, msl, G, Hk, D, kv_dim, bits)
+                oracle.turbo_kv_quantize_batch(c[1], c[3], v[l], rot, pos, msl, G, Hk, D, kv_dim, bits)
+                oracle.turbo_gqa_attention_batch(want, ql, *c, rot, pos, msl, G, H, Hk, D, q_dim, kv_dim, bits)
+            assert rel_err(got[l], want) <= TOL, f"step {step} layer {l}"
+        pos += 1
+    for l, c in enumerate(caches):
+        for got, want, what in zip(eng.cache(l), c, ("K", "V", "K norms", "V norms")):
+            assert_bytes_equal(host(got), want, f"layer {l} {what}")
+
+
+@pytest.mark.parametrize("bits", [4, 2, 0])
+@pytest.mark.parametrize("why", ["producers in launches of their own", "unaligned k"])
+def test_what_one_launch_does_not_take_goes_layer_by_layer(bits, why):
+    import torch
+    from triebwerk_amd import kvcache
+    H, Hk, L, lens, msl = 16, 8, 4, [70, 64, 7], 96
+    G = len(lens)
+    engines, q, k, v = _pair(bits, H, Hk, L, G, msl, False)
+    outs = [torch.zeros_like(q) for _ in range(2)]
+    if why == "unaligned k":
+        flat = torch.zeros(k.numel() + 8, dtype=torch.float16, device="cuda")
+        flat[2:2 + k.numel()].copy_(k.view(-1))
+        k = flat[2:2 + k.numel()].view(k.shape)
+    else:
+        w = [torch.full((L, D), 1.25, dtype=torch.float16, device="cuda") for _ in range(2)]
+        for e in engines:
+            e.set_producers(2, *w)
+    ins = [(q.clone(), k if why == "unaligned k" else k.clone()) for _ in range(2)]       # (the producers work in place)
+    for e in engines:
+        e.set_positions([n - 1 for n in lens])
+    torch.cuda.synchronize()
+    engines[0].decode_step(*ins[0], v, outs[0])
+    name = kvcache.last_scan_kernel()
+    assert "decode_layers_kernel" not in name and "every layer" not in name, name
+    for l in range(L):
+        engines[1].layer_step(l, ins[1][0][l], ins[1][1][l], v[l], outs[1][l])
+    torch.cuda.synchronize()
+    assert torch.equal(*outs) and outs[0].abs().sum() > 0
     _same_caches(engines, L)
