@@ -44,6 +44,15 @@ def rotation_fixture():
     return raw.reshape(128, 128)
 
 
+@pytest.fixture
+def layers_apart():
+    """An engine's decode step takes every layer by itself, in the form that it would take without the hook."""
+    from triebwerk_amd import kvcache
+    kvcache.set_decode_fused(4)
+    yield
+    kvcache.set_decode_fused(0)
+
+
 def pytest_terminal_summary(terminalreporter, exitstatus, config):
     """How much of the attention tolerance the GPU parity tests used: one line (shown with -q too) and the table of
     every test's largest relative error as a JSON file in the run's output folder."""

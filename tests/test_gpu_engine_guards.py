@@ -101,12 +101,12 @@ def test_engine_refuses_a_step_on_a_full_cache(kv_bits, use_graph):
                 assert_bytes_equal(host(t), before[l][i], f"layer {l} array {i}")
 
 
-def test_engine_captured_step_follows_the_plan(oracle):
+def test_engine_captured_step_follows_the_plan(oracle, layers_apart):
     """A step captured at short contexts holds the one-launch kernel; when the contexts the host knows of move
     to where the three-kernel path is the choice (and back), the step is captured again with that choice, and
-    the results stay the oracle's."""
+    the results stay the oracle's.  Every layer by itself."""
     import torch
-    from triebwerk_amd import Engine, _lib
+    from triebwerk_amd import Engine, _lib, kvcache
     lib = _lib.load()
     r = gen.rng(8803)
     # (the engine hands the step its tickets, so small batches of long sequences stay on the one launch with their
@@ -135,6 +135,8 @@ def test_engine_captured_step_follows_the_plan(oracle):
             n0 = lib.tw_kv_decode_fused_launches()
             eng.decode_step(d_q, d_k, d_v, d_out, use_graph=True)
             fused_recorded.append(lib.tw_kv_decode_fused_launches() - n0)
+            name = kvcache.last_scan_kernel()
+            assert ("attention_pair_kernel" if start == 4200 else "decode_fused_kernel") in name, name
             got = host(d_out)
             for l in range(L):
                 want = _oracle_step(oracle, caches[l], q[l], k[l], v[l], rot, pos, msl, G, H, Hk, bits)

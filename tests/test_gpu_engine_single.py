@@ -248,13 +248,13 @@ def test_decode_goes_on_without_a_graph_when_capture_fails(oracle, capfd, kv_bit
             assert_bytes_equal(host(c[i])[:, :5], oc[l][i][:, :5], f"layer {l} array {i}")
 
 
-def test_graph_replay_equals_the_eager_step_across_a_plan_flip_at_full_size():
+def test_graph_replay_equals_the_eager_step_across_a_plan_flip_at_full_size(layers_apart):
     """28 layers, 16 heads over 8 KV heads, 2 bit, 80 sequences around the context where tw_kv_decode_step_plan2 changes
     its answer for a caller with tickets: an engine that replays a captured step and one that runs every step eagerly
     take the same plan at every step (both go by the positions the host knows), so their outputs and caches are equal
-    bit for bit before, at and after the change, and the change happens inside the run."""
+    bit for bit before, at and after the change, and the change happens inside the run.  Every layer by itself."""
     import torch
-    from triebwerk_amd import Engine, _lib
+    from triebwerk_amd import Engine, _lib, kvcache
     lib = _lib.load()
     L, H, Hk, G, bits = 28, 16, 8, 80, 2
     kv_dim, q_dim = Hk * D, H * D
@@ -291,6 +291,8 @@ def test_graph_replay_equals_the_eager_step_across_a_plan_flip_at_full_size():
         n0 = lib.tw_kv_decode_fused_launches()
         engines[1].decode_step(q, k, v, outs[1], use_graph=False)
         one_launch_steps.append(lib.tw_kv_decode_fused_launches() - n0 == L)
+        name = kvcache.last_scan_kernel()
+        assert ("decode_fused_kernel" if one_launch_steps[-1] else "attention_pair_kernel") in name, name
         engines[0].decode_step(q, k, v, outs[0], use_graph=True)
         assert engines[0].graph_state() == 1
         torch.cuda.synchronize()

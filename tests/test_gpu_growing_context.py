@@ -9,7 +9,7 @@ D = 128
 
 
 @pytest.mark.parametrize("bits,H,Hk,G", [(4, 16, 8, 1), (4, 16, 8, 4), (2, 32, 8, 2), (4, 16, 8, 24)])
-def test_replay_is_the_eager_step_at_every_length(bits, H, Hk, G):
+def test_replay_is_the_eager_step_at_every_length(layers_apart, bits, H, Hk, G):
     import torch
     from triebwerk_amd import Engine, _lib, kvcache
     lib = _lib.load()
@@ -42,6 +42,7 @@ def test_replay_is_the_eager_step_at_every_length(bits, H, Hk, G):
         torch.cuda.synchronize()
         forms.add(kvcache.last_scan_kernel())
         assert torch.equal(replayed, out), f"context {ctx}: the replayed step is not the eager step's form"
+    assert len(forms) > 1 and not any("decode_layers_kernel" in f for f in forms), forms
     assert G > 4 or any("context shared" in f for f in forms), forms
 
 
