@@ -969,8 +969,11 @@ const PlanConstants& plan_constants() {
 
 // Microseconds one launch takes: the workgroups run in rounds of one per CU.  A round costs the cube-root sum of its waves'
 // tiles of the longest sequence, one after the other, and of its bytes at the rate the chip streams them in this pattern: a
-// workgroup with one KV head reads half lines, and unless the batch is a multiple of 8 the other half is fetched
+// workgroup with one KV head reads half lines, and unless the batch is a multiple of 8 the other half may be fetched
 // again on another XCD.  A share is a sequence of its own of ctx / shares tokens, plus what the hand-over costs at the end.
+// (The rates of other batches were fitted before units_by_xcd placed them.  With it, over 700 steps of 2 to 63 sequences, 64 to
+// 16000 tokens, six shapes of heads: the choice is the fastest or within 3 % of it at 95 % of the batches of 8 or more that are no
+// multiple of 8, at 94 % of the smaller ones and at 96 % of the multiples, 0.5 % from the fastest in the geometric mean of each.)
 static int group_index(int R) { return R >= 4 ? 2 : R >= 2 ? 1 : 0; }
 static double bytes_per_token(int bits) { return bits == 4 ? 132.0 : 68.0; }       // and KV head: K and V codes and norms
 static double cube_sum(double x, double y) { return std::cbrt(x * x * x + y * y * y); }
