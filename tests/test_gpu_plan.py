@@ -68,9 +68,14 @@ def test_automatic_choice_is_the_faster_form(G, ctx, bits, H):
     assert auto <= 1.05 * min(one, three), (auto, one, three)
 
 
+def _ragged(G, lo, hi):
+    return random.Random(G).sample(range(lo, hi + 1), G)
+
+
 @pytest.mark.parametrize("bits,H,Hk,L,lens", [
     (4, 16, 8, 28, [613] * 4), (4, 16, 8, 12, [8192] * 64), (2, 32, 8, 12, [4097] * 16), (4, 16, 8, 2, [16000]), (2, 16, 8, 3, [8192] * 3),
-    (4, 8, 2, 28, [300, 4000] * 8), (4, 8, 8, 28, [7000] + [100] * 10), (0, 16, 8, 28, [133]), (0, 16, 8, 2, [7000]), (0, 16, 8, 4, [8192] * 12)])
+    (4, 8, 2, 28, [300, 4000] * 8), (4, 8, 8, 28, [7000] + [100] * 10), (0, 16, 8, 28, [133]), (0, 16, 8, 2, [7000]), (0, 16, 8, 4, [8192] * 12),
+    (0, 16, 8, 2, _ragged(83, 877, 8777)), (0, 8, 8, 4, _ragged(116, 538, 5383)), (0, 32, 8, 4, [7880] + [788] * 43)])
 def test_every_layer_in_one_launch_is_no_slower(bits, H, Hk, L, lens):
     import torch
     from triebwerk_amd import Engine, kvcache

@@ -411,8 +411,8 @@ __device__ __forceinline__ float sum_8_lanes(float v) {
 
 // LAYERS: the items of every layer of a step, one workgroup each, in even chunks: the launches' starts, ends and merges are paid once
 // a step, and most batches need no cutting, hence no merge.  us a step, layer by layer -> at once (16 heads over 8 KV heads, 28
-// layers): 1 x 133 tokens 327 -> 20; 4 x 1117 497 -> 91; 35 x 2285 1799 -> 1372 (6.7 TB/s); 8 layers of 64 x 8192 10440 -> 10089 (6.8).
-// Over 300 random steps 2.4 times faster in the geometric mean, none below 0.977 (those: KV heads not in eights, unchanged).
+// layers): 1 x 133 tokens 231 -> 20; 4 x 1117 339 -> 96; 35 x 2285 1745 -> 1420 (6.5 TB/s); 8 layers of 64 x 8192 2696 -> 2616 (6.6).
+// Over 418 random steps 2.7 times faster in the geometric mean; ragged batches that are slower so go layer by layer (rows_layers_pieces).
 template <int RT, bool APPEND, bool DESC, bool LAYERS = false>
 __global__ void __launch_bounds__(kRowThreads) __attribute__((amdgpu_waves_per_eu(RT == 4 ? 2 : 4, RT == 4 ? 2 : 4)))
 attention_rows_kernel(AttnArgs a, int total_items, int hgroups, std::conditional_t<LAYERS, LayerStrides, int> strides) {
@@ -886,7 +886,16 @@ int rows_layers_most_pieces(int layers, int G, int num_heads, int Hk) {
 // of those had two as well.  More than one piece: the merge, a launch with the pieces' loads one after the other in every block.
 // Fitted on MI355X to all numbers of pieces from 1 to 64 (as the workspace allowed) of 203 steps, 2 to 36 layers, 1 to 192 sequences
 // of 64 to 16000 tokens, even and ragged: the choice, of up to kMostPieces, is the fastest or within 3 % at 86 %, within 10 % at 97 %.
-int rows_layers_pieces(int layers, int G, int num_heads, int Hk, double ctx_max, double ctx_mean, size_t ws_floats) {
+//
+// 0: layer by layer, whose balanced walk does not wait for a ragged batch's long sequences.  At once these are started in the middle of the
+// launch and end after the others, and the estimate above knows means only: it is raised by what the longest piece takes beyond the mean one,
+// by how uneven the lengths are and by the bytes of a layer's longest sequence beyond the mean.  Layer by layer a launch streams the mean
+// at its rate and waits for a piece of the longest; batches that attention_rows_kernel does not take by themselves (plan_splits) run their
+// sequences side by side.  us a step, at once -> layer by layer: 2 layers of 83 sequences of 877 to 8777 tokens 620 -> 485; 4 layers, 32 heads
+// over 8, one of 7880 and 43 of 788 224 -> 190; 8 layers of one of 7629 and 79 of 762 847 -> 457.  Over 1363 ragged steps (2 to 36 layers, 1
+// to 192 sequences, uniform to one long among short) at once was slower by more than 2 % in 117, the worst 1.85; with this rule in 32, the
+// worst 1.31, and 19 are slower than at once, the worst 1.36.
+int rows_layers_pieces(int layers, int G, int num_heads, int Hk, int max_seq_len, double ctx_max, double ctx_mean, size_t ws_floats) {
     if (Hk <= 0 || Hk % kRowHeads != 0) return 0;
     const int group = num_heads / Hk;
     AttnArgs a{};
@@ -894,7 +903,7 @@ int rows_layers_pieces(int layers, int G, int num_heads, int Hk, double ctx_max,
     const double cus = compute_units(), slots = group % 4 == 0 ? cus : 2 * cus;
     const double token_us = group % 4 == 0 ? 0.743 : group % 2 == 0 ? 0.612 : 0.45, start_us = 6.15, rate = 7.16e6;
     int best = 1;
-    double best_us = 0.0;
+    double best_us = 0.0, uneven_us = 0.0;
     for (int pieces = 1; pieces <= kMostPieces; pieces++) {
         if (pieces > 1 && ((size_t)layers * G * num_heads * pieces * kPartialFloats > ws_floats || ctx_max < kRowUnit * (double)pieces)) break;
         const double units = (double)layers * G * attention_rows_groups(a) * pieces, full = std::floor(units / slots);
@@ -905,12 +914,23 @@ int rows_layers_pieces(int layers, int G, int num_heads, int Hk, double ctx_max,
             return start_us + std::cbrt(by_tokens * by_tokens * by_tokens + by_bytes * by_bytes * by_bytes);
         };
         const double rest = units - full * slots;
-        double us = std::max(full * round_us(slots) + (rest > 0.0 ? round_us(rest) : 0.0),
-                             start_us + std::ceil(ctx_max / pieces / kRowUnit) * token_us);
-        if (pieces > 1) us += 2.57 + 0.174 * pieces + 0.73e-4 * layers * G * num_heads * pieces;
-        if (pieces == 1 || us < best_us) { best = pieces; best_us = us; }
+        const double rounds = full * round_us(slots) + (rest > 0.0 ? round_us(rest) : 0.0), longest = std::ceil(ctx_max / pieces / kRowUnit);
+        const double merge = pieces > 1 ? 2.57 + 0.174 * pieces + 0.73e-4 * layers * G * num_heads * pieces : 0.0;
+        const double us = std::max(rounds, start_us + longest * token_us) + merge;
+        if (pieces == 1 || us < best_us) {
+            best = pieces;
+            best_us = us;
+            uneven_us = std::max(us, (rounds + merge) * (1.0 + 0.28 * (1.0 - ctx_mean / ctx_max)) + 0.75 * (longest - tokens) * token_us +
+                                          layers * (ctx_max - ctx_mean) * Hk * kHeadDim * 4 / 5.9e6);
+        }
     }
-    return best;
+    if (ctx_max <= 1.125 * ctx_mean) return best;
+    const double pairs = (double)G * attention_rows_groups(a), mean_bytes = (double)G * Hk * ctx_mean * kHeadDim * 4;
+    const double chunks = std::ceil(max_seq_len / 64.0), pieces = std::max(1.0, std::min({64.0, chunks, std::floor(2.0 * cus / pairs)}));
+    const double layer_us = pairs >= 16.0 || pairs * std::min(64.0, chunks) >= 256.0
+                                ? 21.0 + mean_bytes / (group % 4 == 0 ? 6.2e6 : group % 2 == 0 ? 7.8e6 : 9.1e6) + 0.096 * std::ceil(ctx_max / pieces / kRowUnit)
+                                : 8.4 + mean_bytes / 5.9e6 + 0.0043 * ctx_max;
+    return layer_us * layers < 0.97 * uneven_us ? 0 : best;
 }
 
 void launch_attention_valu(const AttnArgs& a, hipStream_t s) {

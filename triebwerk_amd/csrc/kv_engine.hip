@@ -311,7 +311,7 @@ twkv::StepPlan step_plan(const tw_engine* e, bool together) {
         size_t floats = 0;
         (void)rows_ws(e, floats);
         const double longest = e->pos_known ? e->pos_max + 1 : e->batch_msl;
-        if (together) p.layers_pieces = twkv::rows_layers_pieces(e->shape.num_layers, e->G, e->shape.num_heads, e->shape.num_kv_heads, longest,
+        if (together) p.layers_pieces = twkv::rows_layers_pieces(e->shape.num_layers, e->G, e->shape.num_heads, e->shape.num_kv_heads, e->batch_msl, longest,
                                                                  e->pos_known ? e->ctx_mean() : longest, floats);
         p.layers = p.layers_pieces > 0 ? e->shape.num_layers : 0;
         return p;

@@ -342,7 +342,7 @@ struct StepLayers {
 };
 // fp16 cache: pieces every sequence's context is cut into when all layers go together, with ws_floats of workspace (0: not together)
 int rows_layers_most_pieces(int layers, int G, int num_heads, int num_kv_heads);     // the workspace is made for
-int rows_layers_pieces(int layers, int G, int num_heads, int num_kv_heads, double ctx_max, double ctx_mean, size_t ws_floats);
+int rows_layers_pieces(int layers, int G, int num_heads, int num_kv_heads, int max_seq_len, double ctx_max, double ctx_mean, size_t ws_floats);
 // Whether the buffers admit it (a plan with layers > 1 is for those that do)
 bool layers_attention_usable(const tw_layer_step_args* p, const StepLayers& layers);
 void layers_attention_step(const tw_layer_step_args* p, const StepLayers& layers, const StepPlan& plan, hipStream_t s);
