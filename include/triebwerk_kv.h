@@ -383,9 +383,11 @@ void tw_paged_turbo_gqa_attention_batch(tw_half* out, const tw_half* q, const ui
 
 /* One decode step of one layer over the paged compressed cache in a single call: append K and V at positions[g]
  * (into the page block_table names), then attention over 0..positions[g] -- tw_turbo_append_attention_batch with
- * the paged contract above.  The appended rows and the query are rotated in one launch, so the call is three
- * launches where tw_paged_turbo_kv_append_batch + tw_paged_turbo_gqa_attention_batch are four; same cache bytes,
- * same outputs.  ws and max_context as for tw_paged_turbo_gqa_attention_batch. */
+ * the paged contract above.  One launch where max_context is short enough for that to be faster (GQA group 1, 2 or 4, KV heads in
+ * pairs, ws handed over, out not over k_buf or v_buf); else the appended rows and the query are rotated in one launch, which makes
+ * three where tw_paged_turbo_kv_append_batch + tw_paged_turbo_gqa_attention_batch are four.  Same cache bytes; the three launches give
+ * the same outputs as the two calls, the one launch adds up in another order.  ws and max_context as for
+ * tw_paged_turbo_gqa_attention_batch.  Slots past positions[g] need not have been written. */
 void tw_paged_turbo_append_attention_batch(tw_half* out, const tw_half* q, const tw_half* k_buf, const tw_half* v_buf,
                                            uint8_t* ck_q, uint8_t* cv_q, tw_half* k_norms, tw_half* v_norms,
                                            const tw_half* rotation, float* ws, const int* positions,
@@ -495,9 +497,10 @@ int tw_engine_prompt_layer(tw_engine* e, int layer, int seq, const tw_half* q, c
                            tw_half* out, const int* token_positions, int T, hipStream_t s);
 
 /* All layers, then positions += 1.  q/out: (L, G, q_dim); k/v: (L, G, kv_dim).
- * Every layer's inputs are at hand, so the layers are taken as independent of each other, and all of them go
- * into one launch where that is faster (fp16 cache: KV heads in eights) -- unless `out` lies over q, k or v (fp16 with producers: q, which they transform in place,
- * over k or v), or the producers run as launches of their own (mode 2): then layer by layer, in order.
+ * Every layer's inputs are needed before the call, so the layers are taken as independent of each other (a model whose layer l + 1 reads
+ * layer l's output calls tw_engine_layer_step), and all of them go into one launch where that is faster (fp16 cache: KV heads in eights)
+ * -- unless `out` lies over q, k or v (fp16 with producers: q, which they transform in place, over k or v), or the producers run as
+ * launches of their own (mode 2): then layer by layer, in order.
  * With use_graph != 0 the step is captured once into a hipGraph and replayed
  * (engine.cpp:2369-2412, 2480); the capture is dropped when the arena, G or
  * the buffers change, and made again when the context lengths the host knows of have moved to where the other
