@@ -1,6 +1,6 @@
 """Small fp16 batches (attention_valu_kernel and attention_merge_kernel): the appended token at the first, a middle and the last place
 of a step of 32 tokens and alone in its chunk, one token in all, query heads in tiles of 1, 2 and 4, up to 64 partials (one group
-of threads merges up to 8 of them, four merge more), a query buffer that is not 16-byte aligned, gates.  Against the oracle."""
+of threads merges up to 8 of them, four merge more of up to 1024 heads), a query buffer that is not 16-byte aligned, gates.  Against the oracle."""
 import numpy as np
 import pytest
 
@@ -14,6 +14,7 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("H,Hk,lens,msl,splits", [
     (16, 8, [1, 2, 32, 33], 256, 0), (16, 8, [1], 64, 0), (8, 8, [64, 65, 31], 1200, 8), (16, 8, [129, 257], 2048, 9),
     (32, 8, [300, 1], 4096, 30), (16, 8, [1025], 8704, 64), (4, 1, [97, 161, 3], 1500, 0), (6, 2, [200], 1500, 10), (16, 4, [2049], 4096, 0),
+    (16, 8, [700] + [40] * 63, 1408, 9), (16, 8, [700] + [40] * 64, 1408, 9), (32, 8, [300, 17] * 20, 2176, 16),
 ])
 def test_append_and_attention(oracle, H, Hk, lens, msl, splits, aligned):
     import torch

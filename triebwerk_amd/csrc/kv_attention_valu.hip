@@ -945,7 +945,11 @@ void launch_attention_valu(const AttnArgs& a, hipStream_t s) {
 void launch_attention_merge(const AttnArgs& a, hipStream_t s, const LayerStrides& layers) {
     if (a.G <= 0 || (a.nsplit <= 1 && !a.force_merge)) return;
     const dim3 grid(a.num_heads, a.G, layers.layers);
-    if ((a.slots_from_ws ? std::max(a.max_slots, a.nsplit) : a.nsplit) > 8)
+    // Four groups where there are many partials and the blocks, four to a compute unit, make one round: with more the chip has enough to do
+    // without them, and they cost a second round.  us of the merge, one group and four: 148 x 16 heads, 9 slots 5.4 and 8.9; 100 x 32 6.0
+    // and 12.5; whole calls, four against one: 0.95 at 256 to 512 blocks, 0.98 to 1024, 1.02 at 1280 to 1536, 1.08 from 3072.
+    const long long blocks = (long long)a.num_heads * a.G * layers.layers;
+    if ((a.slots_from_ws ? std::max(a.max_slots, a.nsplit) : a.nsplit) > 8 && blocks <= 4 * compute_units())
         hipLaunchKernelGGL(attention_merge_kernel<kMergeManyGroups>, grid, dim3(kMergeManyGroups * kHeadDim), 0, s, a, layers.q);
     else
         hipLaunchKernelGGL(attention_merge_kernel<1>, grid, dim3(kHeadDim), 0, s, a, layers.q);
