@@ -52,10 +52,10 @@ BYTES_HEAD = {0: 256, 4: 66, 2: 34}  # per (token, kv head): fp16 row | codes + 
 # Keyed by (workload, kv_bits, kernel that ran).  Counters are not read in this run: the figures belong to
 # the kernel sources whose digest is recorded with them (`python bench.py --csrc-digest` prints the current
 # one) and are only reported while the sources are still those; otherwise `traffic` is null.
-MEASURED_TRAFFIC_CSRC_DIGEST = "3036fe479556683e"
-MEASURED_TRAFFIC_BYTES = {("target", 4, "one-launch"): 555.1e6, ("target", 4, "scan"): 560.8e6,
-                          ("target", 2, "one-launch"): 286.8e6, ("target", 2, "scan"): 292.3e6,
-                          ("target", 0, "scan"): 2154.8e6}
+MEASURED_TRAFFIC_CSRC_DIGEST = "61b1f4a90e3ef6ba"
+MEASURED_TRAFFIC_BYTES = {("target", 4, "every layer"): 15535.0e6, ("target", 4, "one-launch"): 555.1e6, ("target", 4, "scan"): 560.8e6,
+                          ("target", 2, "every layer"): 8017.9e6, ("target", 2, "one-launch"): 286.7e6, ("target", 2, "scan"): 292.3e6,
+                          ("target", 0, "every layer"): 60191.6e6, ("target", 0, "scan"): 2154.8e6}
 TRAFFIC_SOURCE = "profiles/scan_target_hbm_traffic_pmc.txt"
 
 
@@ -70,11 +70,11 @@ def csrc_digest() -> str:
     return h.hexdigest()[:16]
 
 
-def measured_traffic(workload: str, kv_bits: int, one_launch: bool):
-    """(bytes or None, where the figure comes from)."""
+def measured_traffic(workload: str, kv_bits: int, form: str):
+    """(bytes of the launch or None, where the figure comes from).  form: "every layer" of a step, "one-launch" for a layer, or "scan"."""
     if csrc_digest() != MEASURED_TRAFFIC_CSRC_DIGEST:
         return None, f"none: kernel sources changed since {TRAFFIC_SOURCE} was measured"
-    val = MEASURED_TRAFFIC_BYTES.get((workload, kv_bits, "one-launch" if one_launch else "scan"))
+    val = MEASURED_TRAFFIC_BYTES.get((workload, kv_bits, form))
     return val, (f"{TRAFFIC_SOURCE} (rocprofv3 --pmc, not read in this run; kernel sources {MEASURED_TRAFFIC_CSRC_DIGEST})"
                  if val is not None else "none: not measured for this workload")
 
@@ -372,7 +372,7 @@ def paged_bench(args):
                    "launches_per_layer": 4 if args.launchers == "reference" else 3,
                    "step": ("paged append K,V + paged decode attention for every layer (two calls, four launches), positions += 1"
                             if args.launchers == "reference" else
-                            "tw_paged_turbo_append_attention_batch for every layer (three launches), positions += 1")},
+                            "tw_paged_turbo_append_attention_batch for every layer, positions += 1")},
         "step_algorithmic_GB": step_bytes * 1e-9, "step_achieved_GBps": step_gbs,
         "step_frac_of_hbm_peak": step_gbs / HBM_PEAK_GBS,
         "roofline": {"bound": "hbm", "kernel": "paged decode attention (context scan), one launch per layer",
@@ -391,8 +391,8 @@ def main():
     ap.add_argument("--kv-bits", type=int, default=None, choices=[0, 2, 4])
     ap.add_argument("--variant", type=int, default=0, help="0 auto, 1 vector-ALU kernel, 2 MFMA kernel")
     ap.add_argument("--nsplit", type=int, default=0)
-    ap.add_argument("--one-launch", type=int, default=None, choices=[0, 1, 2, 3],
-                    help="decode step of a compressed layer as one kernel: 0 by max_seq_len, 1 whenever possible, 2 never "
+    ap.add_argument("--one-launch", type=int, default=None, choices=[0, 1, 2, 3, 4],
+                    help="decode step of a compressed layer as one kernel: 0 by max_seq_len, 1 whenever possible, 2 never, 4 as 0 with every layer by itself "
                          "(default: what the engine picks from the spread of the context lengths)")
     ap.add_argument("--fused-shape", default=None, metavar="HKW,SHARES",
                     help="force the one-launch step's KV heads per workgroup and workgroups per (sequence, head group); "
@@ -782,11 +782,11 @@ def decode_bench(args, kv_bits, with_probe):
             reps += 1
             if reps == 6:
                 break
-        read_same = same / max(reps, 1)
+        read_same = same / reps if reps else None        # (a launch of more bytes than the probe has)
         del probe
 
-    traffic, traffic_source = (measured_traffic(args.workload, kv_bits, one_launch)
-                               if not w["overridden"] and args.producers == "none" and args.launchers == "engine"
+    traffic, traffic_source = (measured_traffic(args.workload, kv_bits, "every layer" if whole_step else "one-launch" if one_launch else "scan")
+                               if not w["overridden"] and args.producers == "none" and args.launchers in ("engine", "layer")
                                else (None, "none: not measured for this variation of the workload"))
     result = {
         "metric": "decode-attn tokens/s",
