@@ -47,13 +47,19 @@ decode_layers_kernel(LayersArgs a) {
     static_assert(NQ <= kUnitVecs && 2 * HKW <= kUnitVecs && kPairs * kParts == NW && kBlocks * NW == 8, "the unit fits its waves and LDS region");
     __shared__ __attribute__((aligned(16))) uint32_t tab_s[kTableWords];
     __shared__ __attribute__((aligned(16))) half_t p_s[NW][16][32];
-    // in turn: the new token's vectors (16 at a time), the rotated queries, the parts' sums, the outputs
+    // in turn: the new token's vectors, the rotated queries, the parts' sums, the outputs
     __shared__ __attribute__((aligned(16))) float x_s[kRows][kUnitRowFloats];
     __shared__ __attribute__((aligned(8))) float2 bucket_s[kBuckets];
+    __shared__ float inv_s[kUnitVecs];                           // 1 / |vector| of the K and V vectors
+    static_assert(NV * 16 * sizeof(uint4) <= sizeof(x_s), "the unit's vectors as halves");
 
     const int tid = threadIdx.x;
     const int wave = uniform(tid / kWave), lane = tid % kWave;
     const int ln = lane & 15, kg = lane >> 4;
+    // the arguments in one trip: fetched where they are first used, the start is five of them one after the other
+    asm volatile("" :: "s"(a.q), "s"(a.k), "s"(a.v), "s"(a.positions), "s"(a.rot_ops), "s"(a.q_layer), "s"(a.kv_layer), "s"(a.cache_layer),
+                 "s"(a.rotation), "s"(PROD ? a.q_weight : nullptr), "s"(PROD ? a.k_weight : nullptr), "s"(PROD ? a.cos_table : nullptr),
+                 "s"(PROD ? a.sin_table : nullptr), "s"(PROD ? a.rope_dim : 0), "s"(a.layers), "s"(a.G), "s"(a.num_kv_heads), "s"(a.q_stride), "s"(a.kv_stride), "s"(a.seq_stride_rows));
     const int Hk = a.num_kv_heads;
 
     // ---- the unit: (layer, sequence) pairs in one row, eight of them side by side on the XCDs (workgroups are dealt to
@@ -63,51 +69,70 @@ decode_layers_kernel(LayersArgs a) {
     if (at >= a.layers * a.G) return;
     const int hg = j8 % nhg, layer = at / a.G, g = at - layer * a.G;
     const half_t* q = a.q + layer * a.q_layer + (long long)g * a.q_stride + (long long)hg * NQ * kHeadDim;
-    const half_t* kv_src[2] = {a.k + layer * a.kv_layer + (long long)g * a.kv_stride + (long long)hg * HKW * kHeadDim,
-                               a.v + layer * a.kv_layer + (long long)g * a.kv_stride + (long long)hg * HKW * kHeadDim};
+    const long long kv_at = layer * a.kv_layer + (long long)g * a.kv_stride + (long long)hg * HKW * kHeadDim;
+    const half_t *k_src = a.k + kv_at, *v_src = a.v + kv_at;
     const long long cache_at = layer * a.cache_layer;
     const long long row0 = (long long)g * a.seq_stride_rows;
 
     // ---- requests that do not depend on the position
-    uint4 stage[kPasses], prod_w[kPasses];
+    const int pos_request = a.positions[g];
+    uint4 stage[kPasses], prod_w[kPasses] = {};
+    const half_t* q_weight = PROD && a.q_weight ? a.q_weight + layer * kHeadDim : a.rotation;
+    const half_t* k_weight = PROD && a.q_weight ? a.k_weight + layer * kHeadDim : a.rotation;
     const int piece = tid & 15;
     auto vec_kind = [&](int vc) -> int { return vc < HKW ? 0 : vc < 2 * HKW ? 1 : 2; };
 #pragma unroll
     for (int p = 0; p < kPasses; p++) {
-        const int vc = kUnitVecs * p + (tid >> 4);
-        stage[p] = prod_w[p] = uint4{0u, 0u, 0u, 0u};
-        if (vc < NV && tid < kUnitVecs * 16) {
-            const int kind = vec_kind(vc);
-            const half_t* src = kind == 2 ? q + (vc - 2 * HKW) * kHeadDim : kv_src[kind] + (vc - kind * HKW) * kHeadDim;
-            stage[p] = reinterpret_cast<const uint4*>(src)[piece];
-            if (PROD && a.q_weight && kind != 1)
-                prod_w[p] = reinterpret_cast<const uint4*>((kind == 0 ? a.k_weight : a.q_weight) + layer * kHeadDim)[piece];
-        }
+        // (threads without a vector repeat one, and producers that are not there read the rotation: a load in a branch is waited for at
+        // the branch's end, and these waits one after the other were 4 us of a unit's start)
+        const int vc = min(kUnitVecs * p + ((tid >> 4) & (kUnitVecs - 1)), NV - 1), kind = vec_kind(vc);
+        const half_t* src = kind == 2 ? q + (vc - 2 * HKW) * kHeadDim : (kind == 0 ? k_src : v_src) + (vc - kind * HKW) * kHeadDim;
+        stage[p] = reinterpret_cast<const uint4*>(src)[piece];
+        if (PROD) prod_w[p] = reinterpret_cast<const uint4*>((kind == 0 ? k_weight : q_weight))[piece];
     }
-    // A operands of the rotation, dblk = wave and wave + NW: R[16 dblk + ln][4s + kg] for K and V, whose codes want the fp32 chain, and
-    // R[16 dblk + ln][32 t + 8 kg ..] for the queries
-    uint4 rraw[kBlocks][4], rq[kBlocks][4];
+    // A operands of the rotation, dblk = wave and wave + NW: R[16 dblk + ln][4s + kg], s = 8j .. 8j + 7
+    uint4 rraw[kBlocks][4];
 #pragma unroll
-    for (int i = 0; i < kBlocks; i++) {
+    for (int i = 0; i < kBlocks; i++)
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            rraw[i][j] = a.rot_ops[((wave + NW * i) * 4 + j) * kWave + lane];
-            rq[i][j] = reinterpret_cast<const uint4*>(a.rotation)[(16 * (wave + NW * i) + ln) * 16 + 4 * j + kg];
-        }
-    }
+        for (int j = 0; j < 4; j++) rraw[i][j] = a.rot_ops[((wave + NW * i) * 4 + j) * kWave + lane];
 
-    const int pos = uniform(a.positions[g]);
-    const int n = pos + 1;
-    uint4 prod_c[kPasses], prod_s[kPasses];
+    // ---- table and bucket table while the loads are under way
+    {   // as kv_decode_fused.hip: a thread's entries share their low four bits, a wave's their upper four
+        constexpr int kStep = NW * kWave * 4, kRounds = kTableWords / kStep;
+        const float cent_lane = kAlpha * centroid_of<BITS>(lane);
+        const int e0 = tid >> 4, hi0 = uniform(tid >> 8);
+        auto cent_of = [&](int c) -> float {                // c uniform over the wave
+            return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, cent_lane), c));
+        };
+        if constexpr (BITS == 4) {
+            const half_t lo = (half_t)__shfl(cent_lane, e0 & 15, 64);
 #pragma unroll
-    for (int p = 0; p < kPasses; p++) {
-        prod_c[p] = prod_s[p] = uint4{0u, 0u, 0u, 0u};
-        const int vc = kUnitVecs * p + (tid >> 4);
-        if (PROD && a.cos_table && tid < kUnitVecs * 16 && vc < NV && vec_kind(vc) != 1) {
-            const long long t = (long long)pos * (a.rope_dim >> 4) + rope_piece16(piece, a.rope_dim);
-            prod_c[p] = reinterpret_cast<const uint4*>(a.cos_table)[t];
-            prod_s[p] = reinterpret_cast<const uint4*>(a.sin_table)[t];
+            for (int k = 0; k < kRounds; k++) {
+                half2_t p = {lo, (half_t)cent_of(hi0 + (NW / 4) * k)};
+                const uint32_t w = *reinterpret_cast<uint32_t*>(&p);
+                *reinterpret_cast<uint4*>(&tab_s[tid * 4 + k * kStep]) = uint4{w, w, w, w};
+            }
+        } else {
+            const half_t c0 = (half_t)__shfl(cent_lane, e0 & 3, 64), c1 = (half_t)__shfl(cent_lane, (e0 >> 2) & 3, 64);
+#pragma unroll
+            for (int k = 0; k < kRounds; k++) {
+                const int hi = hi0 + (NW / 4) * k;          // e >> 4
+                half2_t p0 = {c0, c1}, p1 = {(half_t)cent_of(hi & 3), (half_t)cent_of(hi >> 2)};
+                const uint32_t w0 = *reinterpret_cast<uint32_t*>(&p0), w1 = *reinterpret_cast<uint32_t*>(&p1);
+                *reinterpret_cast<uint4*>(&tab_s[tid * 4 + k * kStep]) = uint4{w0, w1, w0, w1};
+            }
         }
+    }
+    if (BITS == 4 && wave == NW - 1 && lane < kBuckets) bucket_s[lane] = bucket_entry(lane);
+
+    const int pos = uniform(pos_request);
+    const int n = pos + 1;
+    uint4 prod_c = {0u, 0u, 0u, 0u}, prod_s = {0u, 0u, 0u, 0u};              // the same for every vector a thread carries
+    if (PROD) {
+        const long long at = a.cos_table ? (long long)pos * (a.rope_dim >> 4) + rope_piece16(piece, a.rope_dim) : 0;
+        prod_c = reinterpret_cast<const uint4*>(a.cos_table ? a.cos_table : a.rotation)[at];
+        prod_s = reinterpret_cast<const uint4*>(a.cos_table ? a.sin_table : a.rotation)[at];
     }
 
     // ---- the wave's tiles: part p of a pair takes tiles p, p + kParts, ...
@@ -160,39 +185,11 @@ decode_layers_kernel(LayersArgs a) {
         t.n[1][1] = __builtin_amdgcn_raw_buffer_load_b32(rv, (int)(noff + 16u * nrow), 0, kStreamNorms);
     };
 
-    // ---- table and bucket table while the loads are under way
-    {   // as kv_decode_fused.hip: a thread's entries share their low four bits, a wave's their upper four
-        constexpr int kStep = NW * kWave * 4, kRounds = kTableWords / kStep;
-        const float cent_lane = kAlpha * centroid_of<BITS>(lane);
-        const int e0 = tid >> 4, hi0 = uniform(tid >> 8);
-        auto cent_of = [&](int c) -> float {                // c uniform over the wave
-            return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, cent_lane), c));
-        };
-        if constexpr (BITS == 4) {
-            const half_t lo = (half_t)__shfl(cent_lane, e0 & 15, 64);
-#pragma unroll
-            for (int k = 0; k < kRounds; k++) {
-                half2_t p = {lo, (half_t)cent_of(hi0 + (NW / 4) * k)};
-                const uint32_t w = *reinterpret_cast<uint32_t*>(&p);
-                *reinterpret_cast<uint4*>(&tab_s[tid * 4 + k * kStep]) = uint4{w, w, w, w};
-            }
-        } else {
-            const half_t c0 = (half_t)__shfl(cent_lane, e0 & 3, 64), c1 = (half_t)__shfl(cent_lane, (e0 >> 2) & 3, 64);
-#pragma unroll
-            for (int k = 0; k < kRounds; k++) {
-                const int hi = hi0 + (NW / 4) * k;          // e >> 4
-                half2_t p0 = {c0, c1}, p1 = {(half_t)cent_of(hi & 3), (half_t)cent_of(hi >> 2)};
-                const uint32_t w0 = *reinterpret_cast<uint32_t*>(&p0), w1 = *reinterpret_cast<uint32_t*>(&p1);
-                *reinterpret_cast<uint4*>(&tab_s[tid * 4 + k * kStep]) = uint4{w0, w1, w0, w1};
-            }
-        }
-    }
-    if (BITS == 4 && wave == NW - 1 && lane < kBuckets) bucket_s[lane] = bucket_entry(lane);
-
-    // ---- the new token's vectors into LDS, 16 lanes to one: K and V as fp32 unit vectors regrouped for the matrix cores (coordinate
-    // 4s + kk at kk * 32 + s), the queries as the halves they are, where the probabilities will be (16-byte piece c of row v at c ^ v)
+    // ---- the new token's vectors into LDS, 16 lanes to one, as the halves they are, regrouped for the matrix cores: coordinate 4s + kk of
+    // vector v in 16-byte piece 4kk + s / 8 of its row, which lies at that piece ^ 5v (no bank twice, written or read)
     PairTileRegs<BITS> t;
-    uint4 (*q_s)[16] = reinterpret_cast<uint4 (*)[16]>(&p_s[0][0][0]);
+    uint4 (*x_h)[16] = reinterpret_cast<uint4 (*)[16]>(&x_s[0][0]);
+    auto piece_of = [&](int v, int p) -> int { return (p ^ (5 * v)) & 15; };
 #pragma unroll
     for (int p = 0; p < kPasses; p++) {
         const int vc = kUnitVecs * p + (tid >> 4), kind = vec_kind(vc);
@@ -201,19 +198,20 @@ decode_layers_kernel(LayersArgs a) {
             unpack_halves(stage[p], x);
             if (PROD && kind != 1) {
                 if (a.q_weight) norm_head16(x, prod_w[p], a.eps, a.biased);
-                if (a.cos_table) rope_head16(x, prod_c[p], prod_s[p], piece, a.rope_dim, 0);
+                if (a.cos_table) rope_head16(x, prod_c, prod_s, piece, a.rope_dim, 0);
             }
-            if (kind == 2) {
-                q_s[vc - 2 * HKW][piece ^ (vc - 2 * HKW)] = PROD ? pack_halves(x) : stage[p];
-            } else {
+            const uint4 w = PROD ? pack_halves(x) : stage[p];          // coordinates 8 piece .. 8 piece + 7
+            const uint32_t by_kk[4] = {(w.x & 0xffffu) | (w.z << 16), (w.x >> 16) | (w.z & 0xffff0000u),
+                                       (w.y & 0xffffu) | (w.w << 16), (w.y >> 16) | (w.w & 0xffff0000u)};
+#pragma unroll
+            for (int kk = 0; kk < 4; kk++)
+                reinterpret_cast<uint32_t*>(&x_h[vc][piece_of(vc, 4 * kk + (piece >> 2))])[piece & 3] = by_kk[kk];
+            if (kind != 2) {
 #pragma unroll
                 for (int e = 0; e < 8; e++) sq[e] = x[e] * x[e];       // exact: fp16 values
                 const float norm = sqrtf(head_tree_sum16(sq) + 1e-12f);
-                const float inv = 1.0f / norm;
-                float* dst = &x_s[vc][2 * piece];
-#pragma unroll
-                for (int e = 0; e < 4; e++) *reinterpret_cast<float2*>(dst + 32 * e) = float2{x[e] * inv, x[e + 4] * inv};
                 if (piece == 0) {
+                    inv_s[vc] = 1.0f / norm;
                     half_t* norms = reinterpret_cast<half_t*>(reinterpret_cast<char*>(kind == 0 ? a.k_norms : a.v_norms) + cache_at);
                     norms[(row0 + pos) * Hk + hg * HKW + vc - kind * HKW] = (half_t)norm;
                 }
@@ -224,31 +222,54 @@ decode_layers_kernel(LayersArgs a) {
     // the first tile, when all of its rows are older than the token this launch appends (whose own row is only there after the
     // barrier that ends the rotations)
     const bool first_early = ntiles > 0 && 32 * part + 32 <= pos;
-    if (first_early) { set_next(0); issue_k(t); issue_n(t); issue_v(t); }
-    {   // K and V: the fp32 chain of kv_rotate.hip (same code bits), the wave's blocks side by side
-        float4_t acc[kBlocks];
+    set_next(0);
+    if (!first_early) next_rows = 0;         // (asked for without a branch: behind one, the rotation's operands would be waited for with the tile)
+    issue_k(t); issue_n(t); issue_v(t);
+    // ---- rotation of all of them on fp16 matrix instructions: fp16 values times an fp16 matrix, every product exact in the fp32
+    // accumulator, 4 matrix instructions a block and 16 vectors
+    float4_t y[kPasses][kBlocks];
+#pragma unroll
+    for (int p = 0; p < kPasses; p++) {
+        const int v = kUnitVecs * p + ln < NV ? kUnitVecs * p + ln : 0;
+#pragma unroll
+        for (int i = 0; i < kBlocks; i++) y[p][i] = float4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            union { uint4 u; half8_t h; } xv, rv;
+            xv.u = x_h[v][piece_of(v, 4 * kg + j)];
+#pragma unroll
+            for (int i = 0; i < kBlocks; i++) {
+                rv.u = rraw[i][j];
+                y[p][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(rv.h, xv.h, y[p][i], 0, 0, 0);
+            }
+        }
+    }
+    {   // Codes of K and V.  They are those of the fp32 chain of kv_rotate.hip, which is 32 matrix instructions of twice the length a
+        // block; the sums above differ from it by less than kCodeDoubt (kv_rotate_util.hpp), so they decide every coordinate that is
+        // further from a boundary, and a block with one that is not (one in 6 with 16 vectors, one in 23 with 4) runs the chain.
         const int v = ln, vk = vec_kind(v);                // this lane's vector
         const bool live = v < 2 * HKW;
-        const float* urow = &x_s[live ? v : 0][32 * kg];
-#pragma unroll
-        for (int i = 0; i < kBlocks; i++) acc[i] = float4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int s8 = 0; s8 < 4; s8++) {
-            float rv[kBlocks][8];
-#pragma unroll
-            for (int i = 0; i < kBlocks; i++) unpack_halves(rraw[i][s8], rv[i]);
-            const float4 u0 = *reinterpret_cast<const float4*>(urow + 8 * s8), u1 = *reinterpret_cast<const float4*>(urow + 8 * s8 + 4);
-            const float uv[8] = {u0.x, u0.y, u0.z, u0.w, u1.x, u1.y, u1.z, u1.w};
-#pragma unroll
-            for (int e = 0; e < 8; e++)
-#pragma unroll
-                for (int i = 0; i < kBlocks; i++) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(rv[i][e], uv[e], acc[i], 0, 0, 0);
-        }
+        const float inv = inv_s[live ? v : 0];
 #pragma unroll
         for (int i = 0; i < kBlocks; i++) {                  // lane: coordinates 16 dblk + 4 kg .. + 3 of vector v
             uint32_t packed = 0;
+            bool doubt = false;
 #pragma unroll
-            for (int r = 0; r < 4; r++) packed |= bucket_quantize<BITS>(bucket_s, acc[i][r]) << (r * BITS);
+            for (int r = 0; r < 4; r++) packed |= bucket_quantize_sure<BITS>(bucket_s, y[0][i][r] * inv, kCodeDoubt, doubt) << (r * BITS);
+            if (__any(live && doubt)) {
+                float4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int s8 = 0; s8 < 4; s8++) {
+                    float rv[8], uv[8];
+                    unpack_halves(rraw[i][s8], rv);
+                    unpack_halves(x_h[live ? v : 0][piece_of(live ? v : 0, 4 * kg + s8)], uv);
+#pragma unroll
+                    for (int e = 0; e < 8; e++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(rv[e], uv[e] * inv, acc, 0, 0, 0);
+                }
+                packed = 0;
+#pragma unroll
+                for (int r = 0; r < 4; r++) packed |= bucket_quantize<BITS>(bucket_s, acc[r]) << (r * BITS);
+            }
             if (live) {
                 uint8_t* dst = (vk == 0 ? a.k_codes : a.v_codes) + cache_at + ((row0 + pos) * Hk + hg * HKW + v - vk * HKW) * kHeadBytes +
                                (4 * (wave + NW * i) + kg) * (BITS / 2);
@@ -257,30 +278,16 @@ decode_layers_kernel(LayersArgs a) {
             }
         }
     }
-    // the queries: fp16 values times an fp16 matrix, every product exact in the fp32 accumulator (4 matrix instructions a block where
-    // the chain above takes 32 of twice the length)
-    float4_t qacc[kBlocks];
-    {
-        const int v = ln < NQ ? ln : 0;
-#pragma unroll
-        for (int i = 0; i < kBlocks; i++) qacc[i] = float4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            union { uint4 u; half8_t h; } qv, rv;
-            qv.u = q_s[v][(4 * j + kg) ^ v];
-#pragma unroll
-            for (int i = 0; i < kBlocks; i++) {
-                rv.u = rq[i][j];
-                qacc[i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(rv.h, qv.h, qacc[i], 0, 0, 0);
-            }
-        }
-    }
     lds_barrier();                                           // the vectors have been read
-    if (ln < NQ) {                                           // the rotated queries, scaled
 #pragma unroll
-        for (int i = 0; i < kBlocks; i++)
-            *reinterpret_cast<float4*>(&x_s[ln][16 * (wave + NW * i) + 4 * kg]) =
-                float4{qacc[i][0] * a.q_scale, qacc[i][1] * a.q_scale, qacc[i][2] * a.q_scale, qacc[i][3] * a.q_scale};
+    for (int p = 0; p < kPasses; p++) {                      // the rotated queries, scaled
+        const int v = kUnitVecs * p + ln - 2 * HKW;
+        if (v >= 0 && v < NQ) {
+#pragma unroll
+            for (int i = 0; i < kBlocks; i++)
+                *reinterpret_cast<float4*>(&x_s[v][16 * (wave + NW * i) + 4 * kg]) =
+                    float4{y[p][i][0] * a.q_scale, y[p][i][1] * a.q_scale, y[p][i][2] * a.q_scale, y[p][i][3] * a.q_scale};
+        }
     }
     *reinterpret_cast<uint4*>(&p_s[wave][0][0] + 8 * lane) = uint4{0u, 0u, 0u, 0u};       // the wave's probabilities start at zero
     __syncthreads();                                         // table, queries and the new row are in place
@@ -295,6 +302,10 @@ decode_layers_kernel(LayersArgs a) {
     S.reset();
     S.load_query(L, [&](int i) -> const float* { return &x_s[hk_local * R + i][0]; });
     lds_barrier();                                           // the queries have been read
+    // The step's last act, positions + 1 (engine.cpp:2394): every wave of this unit has used its sequence's position by now, and the unit
+    // that draws a sequence's last ticket is behind all others in that, so it writes the next one.
+    unsigned ticket = 0;
+    if (tid == 0) ticket = __hip_atomic_fetch_add(a.tickets + g, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     for (int it = 0; it < ntiles; it++) {
         const int tile = next_tile;
         set_next(it + 1);
@@ -383,6 +394,10 @@ decode_layers_kernel(LayersArgs a) {
             const int vec = 4 * kg + r;
             if (vec < NQ) out[(long long)vec * kHeadDim + 16 * (wave + NW * i) + ln] = (half_t)acc[r];
         }
+    }
+    if (tid == 0 && ticket == (unsigned)(a.layers * nhg) - 1u) {
+        a.positions[g] = n;
+        a.tickets[g] = 0u;                                   // for the next launch
     }
 }
 

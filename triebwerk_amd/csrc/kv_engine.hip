@@ -381,6 +381,7 @@ void all_layers(tw_engine* e, const twkv::StepPlan& plan, const tw_half* q, cons
     if (plan.layers > 1) {
         const tw_layer_step_args p = layer_args(e, 0, q, k, v, out);
         twkv::layers_attention_step(&p, step_layers(e), plan, s);
+        if (e->kv_bits != 0) return;                         // the launch has advanced the positions
     } else {
         const size_t qs = (size_t)e->G * e->q_dim(), ks = (size_t)e->G * e->kv_dim();
         for (int l = 0; l < e->shape.num_layers; l++)

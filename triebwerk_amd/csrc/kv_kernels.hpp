@@ -316,7 +316,8 @@ struct LayersArgs {
     half_t *k_norms, *v_norms;
     const half_t* rotation;     // (128, 128)
     const uint4* rot_ops;       // order_rotation's 64 KB
-    const int* positions;
+    int* positions;             // one token on when the launch is done
+    unsigned* tickets;          // G words, zero before the launch and left zero
     int layers, G, num_kv_heads;
     int q_stride, kv_stride;
     long long q_layer, kv_layer, cache_layer;

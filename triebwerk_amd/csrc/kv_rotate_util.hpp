@@ -120,4 +120,25 @@ __device__ __forceinline__ uint32_t bucket_quantize(const float2* buckets, float
     }
 }
 
+// How far the rotation of a unit vector by v_mfma_f32_16x16x32_f16 -- raw fp16 coordinates, the sum scaled by 1 / |x| afterwards -- can be
+// from the fp32 chain whose codes the reference's are, for rows of R of norm 1.  The chain's 128 fused multiply-adds lose 2^-24 of a
+// partial sum each, at most |R row| |u| = 1 (Cauchy-Schwarz), and the unit coordinates 2^-24 each: together at most 129 * 2^-24 = 7.7e-6.
+// The four matrix instructions: at most 2.8e-7 of |x| from the exact sum over 2.4 million vectors (normal, outliers, one
+// large coordinate, multiples of R's rows, denormals, magnitudes over 2^24), taken as 1.2e-6.
+constexpr float kCodeDoubt = 9e-6f;
+// bucket_quantize, with doubt set where val is not further than eps from a boundary (or no number): there val + an error of eps may have
+// another code.  A boundary is further than that from its bucket's edges.
+static_assert(0.15 / kBucketScale > 100.0 * kCodeDoubt, "a value near a boundary is in its bucket");
+template <int BITS>
+__device__ __forceinline__ uint32_t bucket_quantize_sure(const float2* buckets, float val, float eps, bool& doubt) {
+    if constexpr (BITS == 4) {
+        const float2 e = buckets[bucket_of(val)];
+        doubt = doubt || !(fabsf(val - e.x) > eps);
+        return __builtin_bit_cast(uint32_t, e.y) + (!(val < e.x) ? 1u : 0u);
+    } else {
+        doubt = doubt || !(fminf(fabsf(val), fabsf(fabsf(val) - kEdges2[2])) > eps);
+        return (uint32_t)turbo_quantize(val, 2);
+    }
+}
+
 }  // namespace twkv
