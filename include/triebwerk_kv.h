@@ -502,7 +502,8 @@ int tw_engine_prompt_layer(tw_engine* e, int layer, int seq, const tw_half* q, c
  * -- unless `out` lies over q, k or v (fp16 with producers: q, which they transform in place, over k or v), or the producers run as
  * launches of their own (mode 2): then layer by layer, in order.
  * With use_graph != 0 the step is captured once into a hipGraph and replayed
- * (engine.cpp:2369-2412, 2480); the capture is dropped when the arena, G or
+ * (engine.cpp:2369-2412, 2480; all layers together are one to four launches, which are issued again without the graph around
+ * them: that is the faster replay); the capture is dropped when the arena, G or
  * the buffers change, and made again when the context lengths the host knows of have moved to where the other
  * choice of kernels (tw_kv_decode_step_plan) applies.  -8: a sequence has no row left (see
  * tw_engine_set_positions). */

@@ -61,7 +61,6 @@ constexpr int kFusedMaxQ = 32;                 // query heads of a unit: HKW * R
 constexpr int kRowFloats = kHeadDim + 4;       // LDS row of a vector: conflict-free 16-byte accesses
 constexpr int kMaxShares = 64;                 // workgroups that may share one sequence's context
 enum { kStep = 0, kAttend = 1, kPaged = 2 };
-constexpr int kDeviceScope = 16;               // the sc1 bit of a raw buffer access: device scope
 
 }  // namespace
 
@@ -86,7 +85,7 @@ template <int R, int BITS, bool PROD, bool PAIR, bool EARLY, bool SHARES = false
 __global__ void __launch_bounds__((PAIR ? kPairWaves : kFusedWaves) * kWave)
 decode_fused_kernel(AttnArgs a, FusedArgs f) {
     static_assert(MODE == kStep || (PAIR && !SHARES && !EARLY && (MODE == kPaged || !PROD)), "modes of the pair kernel");
-    constexpr bool kAppends = MODE != kAttend;
+    constexpr bool kAppends = MODE != kAttend, kEarly = EARLY || SHARES || MODE != kStep;
     constexpr int NW = PAIR ? kPairWaves : kFusedWaves;        // waves of the workgroup
     constexpr int KW = BITS, VW = BITS;
     constexpr uint32_t kHeadBytes = BITS * 16;
@@ -99,41 +98,45 @@ decode_fused_kernel(AttnArgs a, FusedArgs f) {
     constexpr int kRotBytes = 8 * kOperandTileDwords * 4;
     constexpr int kMaxVecs = PAIR ? 4 * NW : 8 * (2 + R);      // vectors of a unit: a thread group of 16 each
     static_assert(kMaxVecs <= 4 * NW, "a vector per 16 threads");
-    constexpr int kPrologueBytes = kRotBytes + kMaxVecs * kRowFloats * 4;
+    constexpr int kPrologueBytes = kRotBytes + kMaxVecs * kHeadDim * 2;
     __shared__ __attribute__((aligned(16))) char scan_s[kPBytes + kPartBytes > kPrologueBytes ? kPBytes + kPartBytes : kPrologueBytes];
     half_t (*p_s)[16][32] = reinterpret_cast<half_t (*)[16][32]>(scan_s);
     float (*part_s)[R][kRowFloats] = reinterpret_cast<float (*)[R][kRowFloats]>(scan_s + kPBytes);
     uint32_t* rot_s = reinterpret_cast<uint32_t*>(scan_s);
-    float (*u_s)[kRowFloats] = reinterpret_cast<float (*)[kRowFloats]>(scan_s + kRotBytes);
-    __shared__ __attribute__((aligned(16))) float qrot_s[kFusedMaxQ][kHeadDim];
+    uint4 (*x_s)[16] = reinterpret_cast<uint4 (*)[16]>(scan_s + kRotBytes);
+    auto piece_of = [](int v, int p) -> int { return (p ^ (5 * v)) & 15; };
+    __shared__ float inv_s[16];                                // 1 / |vector| of the K and V vectors
+    // the rotated queries: floats, or (PAIR, at most 16 of them) operands of the score MFMAs
+    __shared__ __attribute__((aligned(16))) char q_buf[PAIR ? 2 * 16 * 256 : kFusedMaxQ * kHeadDim * 4];
+    float (*qrot_s)[kHeadDim] = reinterpret_cast<float (*)[kHeadDim]>(q_buf);
+    uint4* qop_s = reinterpret_cast<uint4*>(q_buf);
     __shared__ __attribute__((aligned(16))) float o_s[kFusedMaxQ][kRowFloats];
     __shared__ __attribute__((aligned(8))) float2 bucket_s[kBuckets];
 
     const int tid = threadIdx.x;
     const int wave = uniform(tid / kWave), lane = tid % kWave;
     const int ln = lane & 15, kg = lane >> 4;          // names of the scan; the rotations call them i16, kk
+    // the arguments in one trip: fetched where they are first used, the start is several of them one after the other
+    asm volatile("" :: "s"(a.q), "s"(f.k_src), "s"(f.v_src), "s"(a.rotation), "s"(a.positions), "s"(a.num_kv_heads), "s"(f.hkw), "s"(f.nhg), "s"(f.shares),
+                 "s"(f.by_xcd), "s"(a.G), "s"(a.q_stride), "s"(f.kv_stride), "s"(a.seq_stride_rows), "s"(PROD ? f.q_weight : nullptr),
+                 "s"(PROD ? f.k_weight : nullptr), "s"(PROD ? f.cos_table : nullptr), "s"(PROD ? f.sin_table : nullptr), "s"(PROD ? f.rope_dim : 0));
     const int Hk = a.num_kv_heads;
-    const int HKW = f.hkw;
-    const int nhg = Hk / HKW;
-    const int SPLIT = kParts / HKW;                    // parts of the context per head
+    const int HKW = f.hkw, hkw_log2 = __builtin_ctz(HKW);      // (powers of two: a division is fifty instructions here)
+    const int nhg = f.nhg;                             // Hk / HKW
+    const int SPLIT = kParts >> hkw_log2;              // parts of the context per head
 
     // ---- unit of this workgroup.  Workgroups are dealt to the 8 XCDs in turn; the units of one sequence
     // go to one XCD so that the norm rows they all read (16 bytes per token for 8 heads) come out of one L2.
     int g, hg, share = 0;
-    const int nshares = SHARES ? f.shares : 1;
+    const int nshares = SHARES ? f.shares : 1, share_log2 = SHARES ? __builtin_ctz(f.shares) : 0;
     {
-        int b = (int)blockIdx.x;
+        int b = (int)blockIdx.x >> (f.by_xcd ? 3 : 0);
+        if (SHARES) { share = b & (nshares - 1); b >>= share_log2; }      // the shares of a unit on one XCD as well
+        if ((nhg & (nhg - 1)) == 0) { g = b >> __builtin_ctz(nhg); hg = b & (nhg - 1); }
+        else { g = b / nhg; hg = b - g * nhg; }
         if (f.by_xcd) {
-            const int xcd = b & 7;
-            int j = b >> 3;
-            if (SHARES) { share = j % nshares; j /= nshares; }      // the shares of a unit on one XCD as well
-            g = (j / nhg) * 8 + xcd;
-            hg = j % nhg;
+            g = g * 8 + ((int)blockIdx.x & 7);
             if (g >= a.G) return;                                   // (the grid covers whole eights of sequences)
-        } else {
-            if (SHARES) { share = b % nshares; b /= nshares; }
-            g = b / nhg;
-            hg = b % nhg;
         }
     }
     const bool appends = kAppends && (!SHARES || share == nshares - 1);   // the share that holds the sequence's last tile
@@ -156,45 +159,77 @@ decode_fused_kernel(AttnArgs a, FusedArgs f) {
         kind = 2; head = hg * HKW * R + (vc - first_q);
         return a.q + (long long)g * a.q_stride + (long long)head * kHeadDim;
     };
+    // (Threads without a vector repeat one, waves without rows of R repeat some, and producers that are not there read the rotation: a load
+    // in a branch is waited for, with all before it, at the branch's end.)
     const int my_vec = tid >> 4, my_piece = tid & 15;  // what this thread carries of the unit's vectors
     const bool carries = my_vec < nvec;
     int my_kind, my_head;
-    const half_t* my_src = unit_vector(carries ? my_vec : 0, my_kind, my_head);
-    uint4 stage = {0u, 0u, 0u, 0u}, prod_w = {0u, 0u, 0u, 0u};
+    const half_t* my_src = unit_vector(min(my_vec, nvec - 1), my_kind, my_head);
+    const int pos_request = a.positions[g];
+    const uint4 stage = reinterpret_cast<const uint4*>(my_src)[my_piece];
+    uint4 prod_w = {0u, 0u, 0u, 0u};
     const bool normed = PROD && f.q_weight != nullptr, roped = PROD && f.cos_table != nullptr;
-    if (carries) {
-        stage = reinterpret_cast<const uint4*>(my_src)[my_piece];
-        if (normed && my_kind != 1) prod_w = reinterpret_cast<const uint4*>(my_kind == 0 ? f.k_weight : f.q_weight)[my_piece];
-    }
+    if (PROD) prod_w = reinterpret_cast<const uint4*>(normed ? (my_kind == 0 ? f.k_weight : f.q_weight) : a.rotation)[my_piece];
     // R: wave w < 8 fetches rows 16w .. 16w + 15 (4 KB in a row, 4 fully used pieces per lane) and stages them
     // as an operand tile; the rotating waves read their operand from there
-    uint4 rraw[4] = {};
-    if (wave < 8) {
+    uint4 rraw[4];
 #pragma unroll
-        for (int j = 0; j < 4; j++)
-            rraw[j] = reinterpret_cast<const uint4*>(a.rotation + wave * 16 * kHeadDim)[j * kWave + lane];
+    for (int j = 0; j < 4; j++) rraw[j] = reinterpret_cast<const uint4*>(a.rotation + (wave & 7) * 16 * kHeadDim)[j * kWave + lane];
+
+    // ---- the centroid table while the loads are under way: entry e fills 256 bytes with replicas.  A thread writes
+    // entries e0 + 4 NW k, k = 0, 1, ...: the low four bits of e are the thread's own in every round (their
+    // centroids come out of a register by wave shuffle, once: lane c holds centroid c; indexing the constant array
+    // with a per-lane index is a dependent memory load per look-up, several microseconds for this loop), the
+    // upper four are the same for the whole wave (v_readlane).
+    {
+        const float cent_lane = kAlpha * centroid_of<BITS>(lane);
+        constexpr int kStep = NW * kWave * 4, kRounds = kTableWords / kStep;
+        static_assert(kRounds * kStep == kTableWords && kStep % 1024 == 0, "a round advances e by a multiple of 16");
+        const int e0 = tid >> 4, hi0 = uniform(tid >> 8);
+        auto cent_of = [&](int c) -> float {                // c uniform over the wave
+            return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, cent_lane), c));
+        };
+        if constexpr (BITS == 4) {
+            const half_t lo = (half_t)__shfl(cent_lane, e0 & 15, 64);
+#pragma unroll
+            for (int k = 0; k < kRounds; k++) {
+                half2_t p = {lo, (half_t)cent_of(hi0 + (NW / 4) * k)};
+                const uint32_t w = *reinterpret_cast<uint32_t*>(&p);
+                *reinterpret_cast<uint4*>(&tab_s[tid * 4 + k * kStep]) = uint4{w, w, w, w};
+            }
+        } else {
+            // a byte's four codes in the order 0, 2, 1, 3 (one head per wave: what its lane-pair exchange wants) or
+            // in their own order (two heads per wave)
+            const half_t c0 = (half_t)__shfl(cent_lane, e0 & 3, 64), c1 = (half_t)__shfl(cent_lane, (e0 >> 2) & 3, 64);
+#pragma unroll
+            for (int k = 0; k < kRounds; k++) {
+                const int hi = hi0 + (NW / 4) * k;          // e >> 4
+                const half_t c2 = (half_t)cent_of(hi & 3), c3 = (half_t)cent_of(hi >> 2);
+                half2_t p0 = {c0, PAIR ? c1 : c2};
+                half2_t p1 = {PAIR ? c2 : c1, c3};
+                const uint32_t w0 = *reinterpret_cast<uint32_t*>(&p0), w1 = *reinterpret_cast<uint32_t*>(&p1);
+                *reinterpret_cast<uint4*>(&tab_s[tid * 4 + k * kStep]) = uint4{w0, w1, w0, w1};
+            }
+        }
     }
+    if (BITS == 4 && wave == NW - 1 && lane < kBuckets) bucket_s[lane] = bucket_entry(lane);
 
-    // scaled centroid number lane % 16 (4 bit) or lane % 4 (2 bit), for the table build
-    const float cent_lane = kAlpha * centroid_of<BITS>(lane);
-
-    const int pos = uniform(a.positions[g]);
+    const int pos = uniform(pos_request);
     const int n = pos + 1;
     const int* bt = MODE == kPaged ? a.block_table + (long long)g * a.bt_stride : nullptr;
+    // producers: the pieces of the table rows of this sequence's position that go with this thread's coordinates
+    uint4 prod_c = {0u, 0u, 0u, 0u}, prod_s = {0u, 0u, 0u, 0u};
+    if (PROD) {
+        const long long at = roped ? (long long)pos * (f.rope_dim >> 4) + rope_piece16(my_piece, f.rope_dim) : 0;
+        prod_c = reinterpret_cast<const uint4*>(roped ? f.cos_table : a.rotation)[at];
+        prod_s = reinterpret_cast<const uint4*>(roped ? f.sin_table : a.rotation)[at];
+    }
     // the new token's cache row
     const long long new_row = MODE == kPaged ? (long long)uniform(bt[pos / kPageTokens]) * kPageTokens + pos % kPageTokens
                                              : (long long)g * a.seq_stride_rows + pos;
     // PAIR: wave = part * (HKW / 2) + pair; hk_local is the first head of the pair
-    const int hk_local = PAIR ? 2 * (wave % (HKW >> 1)) : wave % HKW, part = PAIR ? wave / (HKW >> 1) : wave / HKW;
+    const int hk_local = PAIR ? 2 * (wave & ((HKW >> 1) - 1)) : wave & (HKW - 1), part = PAIR ? 2 * wave >> hkw_log2 : wave >> hkw_log2;
     const int h = hg * HKW + hk_local;                 // (first) KV head of this wave
-
-    // producers: the pieces of the table rows of this sequence's position that go with this thread's coordinates
-    uint4 prod_c = {0u, 0u, 0u, 0u}, prod_s = {0u, 0u, 0u, 0u};
-    if (roped && carries && my_kind != 1) {
-        const long long at = (long long)pos * (f.rope_dim >> 4) + rope_piece16(my_piece, f.rope_dim);
-        prod_c = reinterpret_cast<const uint4*>(f.cos_table)[at];
-        prod_s = reinterpret_cast<const uint4*>(f.sin_table)[at];
-    }
 
     // ---- tiles of 32 tokens this wave scans.  They are dealt round by round: in round r part p takes tile
     // r * SPLIT + p, so that at any moment the workgroup -- and with it the other workgroups of the sequence,
@@ -203,14 +238,15 @@ decode_fused_kernel(AttnArgs a, FusedArgs f) {
     // the tiles); what is left goes round the lower waves' parts.
     const int ntile_seq = (n + 31) >> 5;
     // SHARES: this workgroup's run of the sequence's tiles (even runs, the last one ends with the sequence)
-    const int tile_lo = SHARES ? (int)((long long)share * ntile_seq / nshares) : 0;
-    const int ntile = SHARES ? (int)((long long)(share + 1) * ntile_seq / nshares) - tile_lo : ntile_seq;
+    const int tile_lo = SHARES ? (int)((unsigned)(share * ntile_seq) >> share_log2) : 0;
+    const int ntile = SHARES ? (int)((unsigned)((share + 1) * ntile_seq) >> share_log2) - tile_lo : ntile_seq;
     const int halfparts = SPLIT >> 1;                      // SPLIT is 2, 4, 8 or 16
     const int lower = min(ntile, (int)((ntile * (PAIR ? kPairTileShare : kFusedShare) + 63u) / 64u));
-    const int rounds = (ntile - lower) / halfparts;
+    const int split_log2 = 31 - __builtin_clz(SPLIT), half_log2 = split_log2 - 1;
+    const int rounds = (ntile - lower) >> half_log2;
     const int tail0 = rounds * SPLIT;                      // tail tiles tail0 + part + j * halfparts, lower parts only
     const int left = ntile - tail0 - part;
-    const int ntiles = rounds + ((part < halfparts && left > 0) ? (left + halfparts - 1) / halfparts : 0);
+    const int ntiles = rounds + ((part < halfparts && left > 0) ? (left + halfparts - 1) >> half_log2 : 0);
     auto tile_at = [&](int i) -> int {                     // first token of this wave's i-th tile
         return 32 * (tile_lo + (i < rounds ? i * SPLIT + part : tail0 + part + (i - rounds) * halfparts));
     };
@@ -324,47 +360,11 @@ decode_fused_kernel(AttnArgs a, FusedArgs f) {
     auto rotate_unit = [&](auto early) {
         const int i16 = ln, kk = kg;
         const int dblk = rot_dblk;
-        // the centroid table while the loads are under way: entry e fills 256 bytes with replicas.  A thread writes
-        // entries e0 + 4 NW k, k = 0, 1, ...: the low four bits of e are the thread's own in every round (their
-        // centroids come out of a register by wave shuffle, once: lane c holds centroid c; indexing the constant array
-        // with a per-lane index is a dependent memory load per look-up, several microseconds for this loop), the
-        // upper four are the same for the whole wave (v_readlane).
-        constexpr int kStep = NW * kWave * 4, kRounds = kTableWords / kStep;
-        static_assert(kRounds * kStep == kTableWords && kStep % 1024 == 0, "a round advances e by a multiple of 16");
-        const int e0 = tid >> 4, hi0 = uniform(tid >> 8);
-        auto cent_of = [&](int c) -> float {                // c uniform over the wave
-            return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, cent_lane), c));
-        };
-        if constexpr (BITS == 4) {
-            const half_t lo = (half_t)__shfl(cent_lane, e0 & 15, 64);
-#pragma unroll
-            for (int k = 0; k < kRounds; k++) {
-                half2_t p = {lo, (half_t)cent_of(hi0 + (NW / 4) * k)};
-                const uint32_t w = *reinterpret_cast<uint32_t*>(&p);
-                *reinterpret_cast<uint4*>(&tab_s[tid * 4 + k * kStep]) = uint4{w, w, w, w};
-            }
-        } else {
-            // a byte's four codes in the order 0, 2, 1, 3 (one head per wave: what its lane-pair exchange wants) or
-            // in their own order (two heads per wave)
-            const half_t c0 = (half_t)__shfl(cent_lane, e0 & 3, 64), c1 = (half_t)__shfl(cent_lane, (e0 >> 2) & 3, 64);
-#pragma unroll
-            for (int k = 0; k < kRounds; k++) {
-                const int hi = hi0 + (NW / 4) * k;          // e >> 4
-                const half_t c2 = (half_t)cent_of(hi & 3), c3 = (half_t)cent_of(hi >> 2);
-                half2_t p0 = {c0, PAIR ? c1 : c2};
-                half2_t p1 = {PAIR ? c2 : c1, c3};
-                const uint32_t w0 = *reinterpret_cast<uint32_t*>(&p0), w1 = *reinterpret_cast<uint32_t*>(&p1);
-                *reinterpret_cast<uint4*>(&tab_s[tid * 4 + k * kStep]) = uint4{w0, w1, w0, w1};
-            }
-        }
-
-        if (BITS == 4 && wave == NW - 1 && lane < kBuckets) bucket_s[lane] = bucket_entry(lane);
         if (wave < 8) stage_operand_tile(rot_s + wave * kOperandTileDwords, rraw, lane);
         // This thread's piece of its vector: the optional producers (K and queries; each step rounded to fp16 as the
-        // reference's in-place kernels leave it), the norm in the reference's order, and K and V as unit vectors, once for
-        // all waves, into LDS as fp32 regrouped for the matrix cores (coordinate 4s + kk at kk * 32 + s).  (Each rotating wave
-        // doing norm and regrouping for itself, and a wave per vector for the producers: rotations 2.3 us of a launch and
-        // producers 3.5.)
+        // reference's in-place kernels leave it), the norm in the reference's order, and the halves into LDS, once for
+        // all waves, regrouped for the matrix cores: coordinate 4s + kk of vector v in 16-byte piece 4kk + s / 8 of its row, which lies at
+        // that piece ^ 5v (no bank twice, written or read).
         if (carries) {                                     // the same for the 16 lanes of a vector
             float x[8], t[8];
             unpack_halves(stage, x);
@@ -372,52 +372,82 @@ decode_fused_kernel(AttnArgs a, FusedArgs f) {
                 if (normed) norm_head16(x, prod_w, f.eps, f.biased);
                 if (roped) rope_head16(x, prod_c, prod_s, my_piece, f.rope_dim, 0);
             }
+            const uint4 w = PROD ? pack_halves(x) : stage;
+            const uint32_t by_kk[4] = {(w.x & 0xffffu) | (w.z << 16), (w.x >> 16) | (w.z & 0xffff0000u),
+                                       (w.y & 0xffffu) | (w.w << 16), (w.y >> 16) | (w.w & 0xffff0000u)};
 #pragma unroll
-            for (int e = 0; e < 8; e++) t[e] = x[e] * x[e];            // exact: fp16 values
-            const float norm = sqrtf(head_tree_sum16(t) + 1e-12f);
-            const float inv = my_kind == 2 ? 1.0f : 1.0f / norm;
-            float* dst = &u_s[my_vec][2 * my_piece];
+            for (int k4 = 0; k4 < 4; k4++)
+                reinterpret_cast<uint32_t*>(&x_s[my_vec][piece_of(my_vec, 4 * k4 + (my_piece >> 2))])[my_piece & 3] = by_kk[k4];
+            if (kAppends && my_kind != 2) {
 #pragma unroll
-            for (int e = 0; e < 4; e++) *reinterpret_cast<float2*>(dst + 32 * e) = float2{x[e] * inv, x[e + 4] * inv};
-            if (my_kind != 2 && my_piece == 0 && appends)
-                (my_kind == 0 ? f.k_norms : f.v_norms)[new_row * Hk + my_head] = (half_t)norm;
+                for (int e = 0; e < 8; e++) t[e] = x[e] * x[e];            // exact: fp16 values
+                const float norm = sqrtf(head_tree_sum16(t) + 1e-12f);
+                if (my_piece == 0) {
+                    inv_s[my_vec] = 1.0f / norm;
+                    if (appends) (my_kind == 0 ? f.k_norms : f.v_norms)[new_row * Hk + my_head] = (half_t)norm;
+                }
+            }
         }
         lds_barrier();
         early();
-        float rv[32];                                      // R[16 * rot_dblk + ln][4s + kg]
-        if (rotating) read_operand_tile(rot_s + rot_dblk * kOperandTileDwords, lane, rv);
+        uint4 rv[4];                                       // R[16 * rot_dblk + ln][4s + kg], s = 8j .. 8j + 7
+        float doubt_eps = 0.0f;
+        if (rotating) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) rv[j] = *reinterpret_cast<const uint4*>(rot_s + rot_dblk * kOperandTileDwords + operand_tile_dword(lane, 4 * j));
+            if (appends) doubt_eps = operand_rows_doubt(rv);
+        }
         for (int vt = wave >> 3; rotating && vt * 16 < nvec; vt += kRotGroups) {  // uniform over the wave
             const int vi = vt * 16 + i16;
             const int vc = vi < nvec ? vi : nvec - 1;              // clamp reads, mask stores
             int kind, head;
             (void)unit_vector(vc, kind, head);
             const bool is_query = kind == 2;
-            // B operand: coordinate 4s + kk of vector vc
+            // fp16 values times an fp16 matrix: every product exact, the sums in fp32
             float4_t acc = {0.f, 0.f, 0.f, 0.f};
-            const float* urow = &u_s[vc][32 * kk];
 #pragma unroll
-            for (int t = 0; t < 8; t++) {
-                const float4 u = *reinterpret_cast<const float4*>(urow + 4 * t);
-                const float uv[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-                for (int j = 0; j < 4; j++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(rv[4 * t + j], uv[j], acc, 0, 0, 0);
+            for (int j = 0; j < 4; j++) {
+                union { uint4 u; half8_t h; } xv, rm;
+                xv.u = x_s[vc][piece_of(vc, 4 * kk + j)];
+                rm.u = rv[j];
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(rm.h, xv.h, acc, 0, 0, 0);
             }
             if (is_query && vi < nvec) {
                 float4 o = {acc[0] * f.q_scale, acc[1] * f.q_scale, acc[2] * f.q_scale, acc[3] * f.q_scale};
-                *reinterpret_cast<float4*>(&qrot_s[vc - first_q][dblk * 16 + 4 * kk]) = o;
+                if (PAIR) store_query_operand(qop_s, vc - first_q, dblk, kk, acc, f.q_scale);
+                else *reinterpret_cast<float4*>(&qrot_s[vc - first_q][dblk * 16 + 4 * kk]) = o;
             }
             if (appends && vt * 16 < first_q) {                    // lane: coordinates 16 dblk + 4kk .. + 3
+                // codes: those of the fp32 chain, by the sums above unless one of the block's is too near to a boundary
+                // for them (kv_rotate_util.hpp; one block in 6 with 16 vectors, one in 23 with 4)
+                const bool live = vi < nvec && !is_query;
+                const float inv = live ? inv_s[vc] : 0.0f;
                 uint32_t packed = 0;
+                bool doubt = false;
 #pragma unroll
-                for (int r = 0; r < 4; r++) packed |= bucket_quantize<BITS>(bucket_s, acc[r]) << (r * BITS);
-                if (vi < nvec && !is_query) {
+                for (int r = 0; r < 4; r++) packed |= bucket_quantize_sure<BITS>(bucket_s, acc[r] * inv, doubt_eps, doubt) << (r * BITS);
+                if (__any(live && doubt)) {
+                    acc = float4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        float rf[8], uf[8];
+                        unpack_halves(rv[j], rf);
+                        unpack_halves(x_s[vc][piece_of(vc, 4 * kk + j)], uf);
+#pragma unroll
+                        for (int e = 0; e < 8; e++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(rf[e], uf[e] * inv, acc, 0, 0, 0);
+                    }
+                    packed = 0;
+#pragma unroll
+                    for (int r = 0; r < 4; r++) packed |= bucket_quantize<BITS>(bucket_s, acc[r]) << (r * BITS);
+                }
+                if (live) {
                     uint8_t* dst = (kind == 0 ? f.k_codes : f.v_codes) + (new_row * Hk + head) * kHeadBytes + (4 * dblk + kk) * (BITS / 2);
                     if (BITS == 4) *reinterpret_cast<uint16_t*>(dst) = (uint16_t)packed;
                     else *dst = (uint8_t)packed;
                 }
             }
         }
-        if (kAppends) __syncthreads();        // table, q_rot and the new cache row are in place; R has been read
+        if (appends) __syncthreads();         // table, q_rot and the new cache row are in place; R has been read
         else lds_barrier();                   // (no new row: the first tile stays in flight)
         // the wave's slice of the probabilities starts at zero (no other wave touches it)
         *reinterpret_cast<uint4*>(&p_s[wave][0][0] + 8 * lane) = uint4{0u, 0u, 0u, 0u};
@@ -465,7 +495,7 @@ decode_fused_kernel(AttnArgs a, FusedArgs f) {
             next_tile = tile_at(i);
             next_rows = i < ntiles ? max(min(n - next_tile, 32), 0) : 0;
             if (MODE == kPaged) {
-                pages = i == 0 ? fetch_pages(0) : pages_after;
+                pages = pages_after;
                 pages_after = fetch_pages(i + 1);
             }
         };
@@ -543,7 +573,7 @@ decode_fused_kernel(AttnArgs a, FusedArgs f) {
         // with one head per wave; the scores of tile i + 1 placed beside the P.V of tile i for the scheduler to
         // interleave, 3 % slower.)
         PairTileRegs<BITS> t;
-        // EARLY: a wave asks for its first tile in the middle of the prologue, behind the prologue's own loads
+        // (EARLY) a wave asks for its first tile in the middle of the prologue, behind the prologue's own loads
         // and ahead of the rotations, when all of its rows are older than the token this launch appends (the launch's
         // own row only exists after the barrier that ends the rotations).  Rollouts of a few hundred tokens gain
         // 4.5 % (128 sequences at 257..768 tokens: 21.6 against 22.6 us per launch); with 8 tiles per wave it makes no
@@ -553,19 +583,21 @@ decode_fused_kernel(AttnArgs a, FusedArgs f) {
         // 22.9 against 21.2 us per launch on the rollout, 24.7 against 23.5 at 64 x 1024 tokens, 8 % and 5 % slower; with
         // four query heads per KV head it does not fit the registers.  A wave's tile time at these sizes is the tile's
         // own chain of look-ups and matrix instructions, not the wait for its loads.)
-        const bool first_early = MODE == kAttend ? ntiles > 0 : EARLY && ntiles > 0 && tile_at(0) + 32 <= pos;      // uniform over the wave
+        const bool first_early = kEarly && ntiles > 0 && (MODE == kAttend || tile_at(0) + 32 <= pos);      // uniform over the wave
+        pages_after = MODE == kPaged ? fetch_pages(0) : 0;
         rotate_unit([&]() {
-            if (first_early) { set_next(0); issue_k(t); issue_n(t); issue_v(t); }
-        });
-        if (!first_early) {
             set_next(0);
-            issue_k(t);
-            issue_n(t);
-            issue_v(t);
-        }
-        load_rb();              // behind the first tile's loads; the registers are there, and the epilogue need not wait
+            if (kEarly) {                    // (asked for without a branch: behind one, the next wait of the prologue takes the tile with it)
+                const int rows = next_rows;
+                if (!first_early) next_rows = 0;
+                issue_k(t); issue_n(t); issue_v(t);
+                next_rows = rows;
+            }
+        });
+        if (!first_early) { issue_k(t); issue_n(t); issue_v(t); }
+        if (!SHARES) load_rb(); // behind the first tile's loads; the registers are there, and the epilogue need not wait
         if (ntiles > 0) {
-            S.load_query(L, [&](int i) -> const float* { return &qrot_s[hk_local * R + i][0]; });
+            S.load_query_operands(L, [&](int i, int part2, int p) { return &qop_s[query_piece(2 * (hk_local * R + i) + part2, p)]; });
             for (int it = 0; it < ntiles; it++) {
                 const int tile = next_tile;
                 set_next(it + 1);
@@ -756,7 +788,7 @@ decode_fused_kernel(AttnArgs a, FusedArgs f) {
             }
         }
 
-    load_rb();
+    if (!SHARES) load_rb();
     #pragma unroll
         for (int r = 0; r < R; r++) {
             l_run[r] = wave_sum(l_run[r]);
@@ -784,16 +816,30 @@ decode_fused_kernel(AttnArgs a, FusedArgs f) {
         float4 av = {0.f, 0.f, 0.f, 0.f};
         if (vec < nv) {
             const int hk_l = vec / R, r = vec - hk_l * R;
-            for (int p = 0; p < SPLIT; p++) mg = fmaxf(mg, part_s[p * HKW + hk_l][r][kHeadDim]);
-            for (int p = 0; p < SPLIT; p++) {
-                const float* pr = &part_s[p * HKW + hk_l][r][0];
-                const float fs = __builtin_amdgcn_exp2f(pr[kHeadDim] - mg);
-                const float4 c = *reinterpret_cast<const float4*>(pr + k4);
-                lsum = __builtin_fmaf(pr[kHeadDim + 1], fs, lsum);
-                av.x = __builtin_fmaf(c.x, fs, av.x);
-                av.y = __builtin_fmaf(c.y, fs, av.y);
-                av.z = __builtin_fmaf(c.z, fs, av.z);
-                av.w = __builtin_fmaf(c.w, fs, av.w);
+            // (four parts' reads at a time: one after the other each is a trip through LDS)
+            for (int p0 = 0; p0 < SPLIT; p0 += 4) {
+                float2 ml[4];
+                float4 c[4];
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const float* pr = &part_s[min(p0 + j, SPLIT - 1) * HKW + hk_l][r][0];
+                    ml[j] = *reinterpret_cast<const float2*>(pr + kHeadDim);
+                    c[j] = *reinterpret_cast<const float4*>(pr + k4);
+                }
+                const float m0 = mg;
+#pragma unroll
+                for (int j = 0; j < 4; j++) mg = fmaxf(mg, ml[j].x);
+                const float f0 = __builtin_amdgcn_exp2f(m0 - mg);
+                lsum *= f0; av.x *= f0; av.y *= f0; av.z *= f0; av.w *= f0;
+#pragma unroll
+                for (int j = 0; j < 4; j++) {
+                    const float fs = p0 + j < SPLIT ? __builtin_amdgcn_exp2f(ml[j].x - mg) : 0.0f;
+                    lsum = __builtin_fmaf(ml[j].y, fs, lsum);
+                    av.x = __builtin_fmaf(c[j].x, fs, av.x);
+                    av.y = __builtin_fmaf(c[j].y, fs, av.y);
+                    av.z = __builtin_fmaf(c[j].z, fs, av.z);
+                    av.w = __builtin_fmaf(c[j].w, fs, av.w);
+                }
             }
         }
         if constexpr (SHARES) {
@@ -820,14 +866,16 @@ decode_fused_kernel(AttnArgs a, FusedArgs f) {
             }
             __syncthreads();
             if (!last_s) return;                    // uniform over the workgroup: the last share finishes the unit
+            load_rb();                              // (by every share beside its scan, these 32 loads a wave hold the second tile up)
             if (tid == 0) __hip_atomic_store(f.tickets + unit, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // for the next launch
             // The slots of 32 threads that the unit's vectors leave free take a part of the shares each (slot = (part, vector),
             // shares part, part + nsub, ...), eight shares' loads in flight at a time -- one share after the other costs
             // a trip to memory each -- and the parts meet in LDS, where the waves' partial sums were.  All orders
             // are fixed by the shape alone.
             constexpr int kSlots = NW * kWave / 32;
-            const int nsub = min(kSlots, kParts * R) / nv;                 // nv is a power of two, at most both
-            const int mv = vec & (nv - 1), msub = vec / nv;
+            const int nv_log2 = 31 - __builtin_clz(nv);                    // nv is a power of two, at most both
+            const int nsub = min(kSlots, kParts * R) >> nv_log2;
+            const int mv = vec & (nv - 1), msub = vec >> nv_log2;
             float (*sum_s)[kRowFloats] = &part_s[0][0];
             if (msub < nsub) {
                 float m = kNegBig, l = 0.0f;
@@ -1085,6 +1133,7 @@ static bool units_by_xcd(int G, int units, int shares) {
 void launch_decode_fused(const AttnArgs& a, const FusedArgs& f_in, hipStream_t s, bool allow_pairs, const StepPlan& plan) {
     FusedArgs f = f_in;
     f.hkw = plan.hkw;
+    f.nhg = a.num_kv_heads / f.hkw;
     f.shares = plan.shares;
     f.q_scale = attention_mfma_q_scale(a.bits);
     const int R = a.num_heads / a.num_kv_heads;
@@ -1135,6 +1184,7 @@ int decode_fused_mode_shape(int G, int num_heads, int Hk, int bits, int ctx_boun
 void launch_decode_fused_mode(const AttnArgs& a, const FusedArgs& f_in, hipStream_t s, int hkw) {
     FusedArgs f = f_in;
     f.hkw = hkw;
+    f.nhg = a.num_kv_heads / hkw;
     f.shares = 1;
     f.q_scale = attention_mfma_q_scale(a.bits);
     const int R = a.num_heads / a.num_kv_heads;

@@ -51,7 +51,8 @@ decode_layers_kernel(LayersArgs a) {
     __shared__ __attribute__((aligned(16))) float x_s[kRows][kUnitRowFloats];
     __shared__ __attribute__((aligned(8))) float2 bucket_s[kBuckets];
     __shared__ float inv_s[kUnitVecs];                           // 1 / |vector| of the K and V vectors
-    static_assert(NV * 16 * sizeof(uint4) <= sizeof(x_s), "the unit's vectors as halves");
+    uint4* qop_s = reinterpret_cast<uint4*>(&x_s[0][0]);
+    static_assert(NV * 16 * sizeof(uint4) <= sizeof(x_s) && 2 * NQ * 16 * sizeof(uint4) <= sizeof(x_s), "the unit's vectors, and its queries, as halves");
 
     const int tid = threadIdx.x;
     const int wave = uniform(tid / kWave), lane = tid % kWave;
@@ -59,15 +60,16 @@ decode_layers_kernel(LayersArgs a) {
     // the arguments in one trip: fetched where they are first used, the start is five of them one after the other
     asm volatile("" :: "s"(a.q), "s"(a.k), "s"(a.v), "s"(a.positions), "s"(a.rot_ops), "s"(a.q_layer), "s"(a.kv_layer), "s"(a.cache_layer),
                  "s"(a.rotation), "s"(PROD ? a.q_weight : nullptr), "s"(PROD ? a.k_weight : nullptr), "s"(PROD ? a.cos_table : nullptr),
-                 "s"(PROD ? a.sin_table : nullptr), "s"(PROD ? a.rope_dim : 0), "s"(a.layers), "s"(a.G), "s"(a.num_kv_heads), "s"(a.q_stride), "s"(a.kv_stride), "s"(a.seq_stride_rows));
+                 "s"(PROD ? a.sin_table : nullptr), "s"(PROD ? a.rope_dim : 0), "s"(a.layers), "s"(a.G), "s"(a.nhg), "s"(a.g_magic), "s"(a.num_kv_heads), "s"(a.q_stride), "s"(a.kv_stride), "s"(a.seq_stride_rows));
     const int Hk = a.num_kv_heads;
 
     // ---- the unit: (layer, sequence) pairs in one row, eight of them side by side on the XCDs (workgroups are dealt to
     // those in turn), the units of a pair one after the other on its XCD: they share cache lines of codes and norms
-    const int nhg = Hk / HKW;
-    const int j8 = (int)blockIdx.x >> 3, at = (j8 / nhg) * 8 + ((int)blockIdx.x & 7);
+    const int nhg = a.nhg;
+    const int j8 = (int)blockIdx.x >> 3, group = (nhg & (nhg - 1)) == 0 ? j8 >> __builtin_ctz(nhg) : j8 / nhg;
+    const int at = group * 8 + ((int)blockIdx.x & 7);
     if (at >= a.layers * a.G) return;
-    const int hg = j8 % nhg, layer = at / a.G, g = at - layer * a.G;
+    const int hg = j8 - group * nhg, layer = a.g_magic ? (int)__umulhi((unsigned)at, a.g_magic) : at / a.G, g = at - layer * a.G;
     const half_t* q = a.q + layer * a.q_layer + (long long)g * a.q_stride + (long long)hg * NQ * kHeadDim;
     const long long kv_at = layer * a.kv_layer + (long long)g * a.kv_stride + (long long)hg * HKW * kHeadDim;
     const half_t *k_src = a.k + kv_at, *v_src = a.v + kv_at;
@@ -284,9 +286,7 @@ decode_layers_kernel(LayersArgs a) {
         const int v = kUnitVecs * p + ln - 2 * HKW;
         if (v >= 0 && v < NQ) {
 #pragma unroll
-            for (int i = 0; i < kBlocks; i++)
-                *reinterpret_cast<float4*>(&x_s[v][16 * (wave + NW * i) + 4 * kg]) =
-                    float4{y[p][i][0] * a.q_scale, y[p][i][1] * a.q_scale, y[p][i][2] * a.q_scale, y[p][i][3] * a.q_scale};
+            for (int i = 0; i < kBlocks; i++) store_query_operand(qop_s, v, wave + NW * i, kg, y[p][i], a.q_scale);
         }
     }
     *reinterpret_cast<uint4*>(&p_s[wave][0][0] + 8 * lane) = uint4{0u, 0u, 0u, 0u};       // the wave's probabilities start at zero
@@ -300,70 +300,59 @@ decode_layers_kernel(LayersArgs a) {
         for (int j = 0; j < 4; j++) rb[i][j] = a.rot_ops[2048 + ((wave + NW * i) * 4 + j) * kWave + lane];
     PairState<R> S;
     S.reset();
-    S.load_query(L, [&](int i) -> const float* { return &x_s[hk_local * R + i][0]; });
+    S.load_query_operands(L, [&](int i, int part2, int p) { return &qop_s[query_piece(2 * (hk_local * R + i) + part2, p)]; });
     lds_barrier();                                           // the queries have been read
     // The step's last act, positions + 1 (engine.cpp:2394): every wave of this unit has used its sequence's position by now, and the unit
     // that draws a sequence's last ticket is behind all others in that, so it writes the next one.
-    unsigned ticket = 0;
-    if (tid == 0) ticket = __hip_atomic_fetch_add(a.tickets + g, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // (Every thread asks, all but the first out of range: drawn in a branch, the ticket is waited for at the branch's end.)
+    const unsigned ticket = (unsigned)__builtin_amdgcn_raw_ptr_buffer_atomic_add_i32(
+        1, make_rsrc(reinterpret_cast<const char*>(a.tickets + g), 4), tid == 0 ? 0 : 1 << 30, 0, kDeviceScope);
     for (int it = 0; it < ntiles; it++) {
         const int tile = next_tile;
         set_next(it + 1);
         pair_scan_tile<R>(L, S, t, tile, n, [&]() { issue_k(t); }, [&]() { issue_n(t); }, [&]() { issue_v(t); });
     }
 
-    // ---- the parts meet in LDS, the upper half's sums handed to the lower half until one is left
-    float ov[R][16];
-    pair_scan_finish<R>(L, S, 1.0f / kAlpha, [&](int, int r, const float (&o)[16]) {
+    // ---- the parts meet in LDS: every wave leaves its sums, then 32 threads to an output merge them (in halves, the upper handed to the lower
+    // until one is left, with two barriers each: 0.5 us of a unit's end)
+    constexpr bool kInPlace = NW * 2 * R <= kRows;            // else where the table was, once every wave is through with it
+    float (*sum_s)[kUnitRowFloats] = kInPlace ? x_s : reinterpret_cast<float (*)[kUnitRowFloats]>(tab_s);
+    if (kParts > 1 && !kInPlace) lds_barrier();
+    pair_scan_finish<R>(L, S, 1.0f / kAlpha, [&](int, int r, const float (&o)[16]) {     // dims 16 (pn % 8) .. of head hd
+        float* row = kParts > 1 ? sum_s[(part * kPairs + pair) * 2 * R + L.hd * R + r] : x_s[pair * 2 * R + L.hd * R + r];
+        const float inv = kParts > 1 ? 1.0f : 1.0f / (S.l_run[r] + 1e-8f);               // kernels.cu:1746
 #pragma unroll
-        for (int j = 0; j < 16; j++) ov[r][j] = o[j];
+        for (int j4 = 0; j4 < 4; j4++)
+            *reinterpret_cast<float4*>(row + 16 * (L.pn & 7) + 4 * j4) = float4{o[4 * j4] * inv, o[4 * j4 + 1] * inv, o[4 * j4 + 2] * inv, o[4 * j4 + 3] * inv};
+        if (kParts > 1 && (L.pn & 7) == 0) *reinterpret_cast<float2*>(row + kHeadDim) = float2{S.m_run[r], S.l_run[r]};
     });
-    const bool owner = L.pkg == L.hd;                        // the 16 lanes that hold the sums (head L.hd, dims 16 (pn % 8) ..)
-    const int d16 = 16 * (L.pn & 7);
-    auto row_of = [&](int pt, int r) -> float* { return &x_s[(pt * kPairs + pair) * 2 * R + L.hd * R + r][0]; };
-#pragma unroll
-    for (int half = kParts / 2; half >= 1; half >>= 1) {
-        if (part >= half && part < 2 * half && owner) {
-#pragma unroll
-            for (int r = 0; r < R; r++) {
-                float* row = row_of(part - half, r);
-#pragma unroll
-                for (int j4 = 0; j4 < 4; j4++) *reinterpret_cast<float4*>(row + d16 + 4 * j4) = float4{ov[r][4 * j4], ov[r][4 * j4 + 1], ov[r][4 * j4 + 2], ov[r][4 * j4 + 3]};
-                if ((L.pn & 7) == 0) { row[kHeadDim] = S.m_run[r]; row[kHeadDim + 1] = S.l_run[r]; }
-            }
-        }
-        lds_barrier();
-        if (part < half && owner) {
-#pragma unroll
-            for (int r = 0; r < R; r++) {
-                const float* row = row_of(part, r);
-                const float m2 = row[kHeadDim], l2r = row[kHeadDim + 1];
-                const float mg = fmaxf(S.m_run[r], m2);
-                const float f1 = __builtin_amdgcn_exp2f(S.m_run[r] - mg), f2 = __builtin_amdgcn_exp2f(m2 - mg);
-                S.m_run[r] = mg;
-                S.l_run[r] = S.l_run[r] * f1 + l2r * f2;
-#pragma unroll
-                for (int j4 = 0; j4 < 4; j4++) {
-                    const float4 c = *reinterpret_cast<const float4*>(row + d16 + 4 * j4);
-                    const float cv[4] = {c.x, c.y, c.z, c.w};
-#pragma unroll
-                    for (int e = 0; e < 4; e++) ov[r][4 * j4 + e] = __builtin_fmaf(cv[e], f2, ov[r][4 * j4 + e] * f1);
-                }
-            }
-        }
-        lds_barrier();
-    }
-    if (part == 0 && owner) {
-#pragma unroll
-        for (int r = 0; r < R; r++) {
-            float* row = row_of(0, r);                       // = the output's vector: heads of pair, then query heads
-            const float inv = 1.0f / (S.l_run[r] + 1e-8f);   // kernels.cu:1746
-#pragma unroll
-            for (int j4 = 0; j4 < 4; j4++)
-                *reinterpret_cast<float4*>(row + d16 + 4 * j4) = float4{ov[r][4 * j4] * inv, ov[r][4 * j4 + 1] * inv, ov[r][4 * j4 + 2] * inv, ov[r][4 * j4 + 3] * inv};
-        }
-    }
     lds_barrier();
+    if constexpr (kParts > 1) {
+        for (int v = tid >> 5; v < NQ; v += NW * kWave / 32) {                           // output: heads of the pairs, then query heads
+            const int k4 = (tid & 31) * 4;
+            float2 ml[kParts];
+            float4 c[kParts];
+            float m = kNegBig, l = 0.0f;
+#pragma unroll
+            for (int p = 0; p < kParts; p++) {
+                const float* row = sum_s[p * kPairs * 2 * R + v];
+                ml[p] = *reinterpret_cast<const float2*>(row + kHeadDim);
+                c[p] = *reinterpret_cast<const float4*>(row + k4);
+                m = fmaxf(m, ml[p].x);
+            }
+            float4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int p = 0; p < kParts; p++) {
+                const float fs = __builtin_amdgcn_exp2f(ml[p].x - m);
+                l = __builtin_fmaf(ml[p].y, fs, l);
+                o.x = __builtin_fmaf(c[p].x, fs, o.x); o.y = __builtin_fmaf(c[p].y, fs, o.y);
+                o.z = __builtin_fmaf(c[p].z, fs, o.z); o.w = __builtin_fmaf(c[p].w, fs, o.w);
+            }
+            const float inv = 1.0f / (l + 1e-8f);            // kernels.cu:1746
+            *reinterpret_cast<float4*>(&x_s[v][k4]) = float4{o.x * inv, o.y * inv, o.z * inv, o.w * inv};
+        }
+        lds_barrier();
+    }
 
     // ---- rotate back (as kv_decode_fused.hip): o as fp16 value + remainder, R exact in fp16
     half_t* out = a.out + layer * a.q_layer + (long long)g * a.q_stride + (long long)hg * NQ * kHeadDim;
@@ -453,7 +442,11 @@ LayersShape decode_layers_shape(int layers, int G, int num_heads, int Hk, int bi
     return best;
 }
 
-void launch_decode_layers(const LayersArgs& a, int num_heads, int bits, int hkw, int waves, hipStream_t s) {
+void launch_decode_layers(const LayersArgs& args, int num_heads, int bits, int hkw, int waves, hipStream_t s) {
+    LayersArgs a = args;
+    a.nhg = a.num_kv_heads / hkw;
+    const uint64_t G = (uint64_t)a.G, two32 = 1ull << 32;
+    a.g_magic = G > 1 && ((uint64_t)a.layers * G + 8) * G < two32 ? (uint32_t)((two32 + G - 1) / G) : 0u;
     const int R = num_heads / a.num_kv_heads;
     const long long pairs = ((long long)a.layers * a.G + 7) / 8 * 8;
     const dim3 g3((unsigned)(pairs * (a.num_kv_heads / hkw))), b3(waves * kWave);

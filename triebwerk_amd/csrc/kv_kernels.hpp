@@ -223,7 +223,7 @@ struct FusedArgs {
     uint8_t* v_codes;
     half_t* k_norms;
     half_t* v_norms;
-    int hkw;                // KV heads per workgroup (launch_decode_fused fills this in)
+    int hkw, nhg;           // KV heads per workgroup, workgroups for all of them (launch_decode_fused fills these in)
     int by_xcd;             // sequence g's workgroups on XCD g % 8 (likewise)
     float q_scale;          // likewise
     // A unit's context shared by several workgroups, for batches whose units alone leave compute units idle:
@@ -319,6 +319,8 @@ struct LayersArgs {
     int* positions;             // one token on when the launch is done
     unsigned* tickets;          // G words, zero before the launch and left zero
     int layers, G, num_kv_heads;
+    int nhg;                    // num_kv_heads / the launch's heads per workgroup
+    uint32_t g_magic;           // ceil(2^32 / G) where (layers * G + 8) * G < 2^32: a division by multiplication; 0 elsewhere
     int q_stride, kv_stride;
     long long q_layer, kv_layer, cache_layer;
     long long seq_stride_rows;
@@ -346,7 +348,8 @@ int rows_layers_most_pieces(int layers, int G, int num_heads, int num_kv_heads);
 int rows_layers_pieces(int layers, int G, int num_heads, int num_kv_heads, int max_seq_len, double ctx_max, double ctx_mean, size_t ws_floats);
 // Whether the buffers admit it (a plan with layers > 1 is for those that do)
 bool layers_attention_usable(const tw_layer_step_args* p, const StepLayers& layers);
-void layers_attention_step(const tw_layer_step_args* p, const StepLayers& layers, const StepPlan& plan, hipStream_t s);
+// (recorded: the launches of a captured step, issued again)
+void layers_attention_step(const tw_layer_step_args* p, const StepLayers& layers, const StepPlan& plan, hipStream_t s, bool recorded);
 // allow_pairs: the kernel whose waves scan two KV heads each, where the shape admits it (false: one head per wave)
 void launch_decode_fused(const AttnArgs& a, const FusedArgs& f, hipStream_t s, bool allow_pairs, const StepPlan& plan);
 // the pair kernel (hkw KV heads a workgroup, no shares, no producers) for attention alone, or for the step over the paged cache

@@ -77,6 +77,7 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const char* base, in
 // Only for lines that one load instruction of one wave covers in full: a line touched by two instructions (two
 // waves, or two half-line loads of one wave) is fetched twice, and the launch gets slower than without the hint.
 constexpr int kStreamCodes = 2;
+constexpr int kDeviceScope = 16;               // the sc1 bit of a raw buffer access: device scope
 // the norm rows (16 bytes per token for 8 heads) are shared by the workgroups of a sequence: kept in the caches
 constexpr int kStreamNorms = 0;
 

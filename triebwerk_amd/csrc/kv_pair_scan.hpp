@@ -38,6 +38,8 @@
 // instruction per look-up), so that a look-up yields four consecutive contraction slots.
 #pragma once
 
+#include <type_traits>
+
 #include "kv_common.hpp"
 #include "kv_mfma_util.hpp"
 
@@ -77,16 +79,21 @@ struct PairLane {
     __device__ __forceinline__ uint2 lut64(uint32_t addr) const { return *reinterpret_cast<const uint2*>(tab + addr); }
     // reductions over the lanes of this lane's head (lane groups of both parities included: those that own nothing
     // contribute the neutral element)
-    __device__ __forceinline__ float head_max(float v) const {
-        v = fmaxf(v, __shfl_xor(v, 1, 64)); v = fmaxf(v, __shfl_xor(v, 2, 64)); v = fmaxf(v, __shfl_xor(v, 4, 64));
-        v = fmaxf(v, __shfl_xor(v, 16, 64)); v = fmaxf(v, __shfl_xor(v, 32, 64));
-        return v;
+    // The partners lanes 1, 2, 4 (mirrored in the eight: they hold the quads' results), 16 and 32 apart, all on the vector ALU: five
+    // cross-lane reads through LDS one after the other are half a microsecond of a scan's first tile.
+    template <class Op>
+    static __device__ __forceinline__ float over_head(float v, Op op) {
+        auto dpp = [](float x, auto ctrl) { return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, x), decltype(ctrl)::value, 0xf, 0xf, true)); };
+        v = op(v, dpp(v, std::integral_constant<int, 0xB1>{}));      // quad_perm 1, 0, 3, 2
+        v = op(v, dpp(v, std::integral_constant<int, 0x4E>{}));      // quad_perm 2, 3, 0, 1
+        v = op(v, dpp(v, std::integral_constant<int, 0x141>{}));     // row_half_mirror
+        uint32x2_t w = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        v = op(__uint_as_float(w[0]), __uint_as_float(w[1]));
+        w = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+        return op(__uint_as_float(w[0]), __uint_as_float(w[1]));
     }
-    __device__ __forceinline__ float head_sum(float v) const {
-        v += __shfl_xor(v, 1, 64); v += __shfl_xor(v, 2, 64); v += __shfl_xor(v, 4, 64);
-        v += __shfl_xor(v, 16, 64); v += __shfl_xor(v, 32, 64);
-        return v;
-    }
+    __device__ __forceinline__ float head_max(float v) const { return over_head(v, [](float x, float y) { return fmaxf(x, y); }); }
+    __device__ __forceinline__ float head_sum(float v) const { return over_head(v, [](float x, float y) { return x + y; }); }
 };
 
 // The registers of one tile in flight.
@@ -100,6 +107,23 @@ struct PairTileRegs {
     uint32_t n[2][2];       // [token tok0 | tok0 + 16][K | V]: the pair's two fp16 norms
 };
 
+// Rotated queries as operands in LDS: rows of 16 pieces of 16 bytes, row 2 q + part of query head q, piece p of a row at p ^ 5 row (the
+// rows a wave reads are neighbours: no bank twice).
+__device__ __forceinline__ int query_piece(int row, int p) { return row * 16 + ((p ^ (5 * row)) & 15); }
+// coordinates 16 dblk + 4 kg .. + 3 of query head q
+__device__ __forceinline__ void store_query_operand(uint4* ops, int q, int dblk, int kg, const float4_t& y, float scale) {
+    half4_t hi, lo;
+#pragma unroll
+    for (int r = 0; r < 4; r++) {
+        const float x = y[r] * scale;
+        hi[r] = (half_t)x;
+        lo[r] = (half_t)(x - (float)hi[r]);
+    }
+    const int p = 2 * dblk + (kg >> 1);
+    reinterpret_cast<half4_t*>(&ops[query_piece(2 * q, p)])[kg & 1] = hi;
+    reinterpret_cast<half4_t*>(&ops[query_piece(2 * q + 1, p)])[kg & 1] = lo;
+}
+
 template <int R>
 struct PairState {
     float4_t o[16];         // accumulator of P.V MFMA j
@@ -111,6 +135,15 @@ struct PairState {
         for (int j = 0; j < 16; j++) o[j] = float4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int r = 0; r < R; r++) { m_run[r] = kNegBig; l_run[r] = 0.0f; }
+    }
+    // The same from operands: piece(i, part, p) -> 16-byte piece p of the 128 halves of query head i, part 0 their fp16 values and 1 what
+    // rounding left over.  (160 instructions less per wave than making them here from floats; the operand rows m with
+    // m % 4 >= R repeat a head, their scores are not read.)
+    template <class Lane, class PieceOf>
+    __device__ __forceinline__ void load_query_operands(const Lane& L, PieceOf piece_of) {
+        const int m = L.pn & 7, head = (m >> 2) * R + ((m & 3) < R ? (m & 3) : R - 1);
+#pragma unroll
+        for (int j = 0; j < 4; j++) aq[j] = __builtin_bit_cast(half8_t, *piece_of(head, L.pn >> 3, 4 * L.pkg + j));
     }
     // q_rot of the pair's query heads: row(i) -> the 128 floats of query head i (i = hd * R + r, 0 <= i < 2 R)
     template <class Lane, class RowOf>

@@ -129,6 +129,34 @@ constexpr float kCodeDoubt = 9e-6f;
 // bucket_quantize, with doubt set where val is not further than eps from a boundary (or no number): there val + an error of eps may have
 // another code.  A boundary is further than that from its bucket's edges.
 static_assert(0.15 / kBucketScale > 100.0 * kCodeDoubt, "a value near a boundary is in its bucket");
+// The same for the 16 rows of any R whose halves the lanes of a wave hold as operands (16 lanes a row quarter): as large as the longest
+// of them (a R that is no number leaves no value sure).
+__device__ __forceinline__ float operand_rows_doubt(const uint4 (&rows)[4]) {
+    float n2 = 0.0f;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const uint32_t w[4] = {rows[j].x, rows[j].y, rows[j].z, rows[j].w};
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const half2_t h = __builtin_bit_cast(half2_t, w[i]);
+            n2 = __builtin_amdgcn_fdot2(h, h, n2, false);
+        }
+    }
+    typedef unsigned swapped_t __attribute__((ext_vector_type(2)));
+    swapped_t w = __builtin_amdgcn_permlane16_swap(__float_as_uint(n2), __float_as_uint(n2), false, false);
+    n2 = __uint_as_float(w[0]) + __uint_as_float(w[1]);
+    w = __builtin_amdgcn_permlane32_swap(__float_as_uint(n2), __float_as_uint(n2), false, false);
+    n2 = __uint_as_float(w[0]) + __uint_as_float(w[1]);
+    auto larger = [](float x, int moved) {                 // (a NaN stays)
+        const float y = __builtin_bit_cast(float, moved);
+        return x > y || x != x ? x : y;
+    };
+    n2 = larger(n2, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, n2), 0xB1, 0xf, 0xf, true));      // 1, 2, then 4 and 8 rows apart
+    n2 = larger(n2, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, n2), 0x4E, 0xf, 0xf, true));
+    n2 = larger(n2, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, n2), 0x141, 0xf, 0xf, true));
+    n2 = larger(n2, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, n2), 0x140, 0xf, 0xf, true));
+    return 1.001f * kCodeDoubt * sqrtf(n2);
+}
 template <int BITS>
 __device__ __forceinline__ uint32_t bucket_quantize_sure(const float2* buckets, float val, float eps, bool& doubt) {
     if constexpr (BITS == 4) {
