@@ -15,6 +15,7 @@
 // 8192 tokens, 8 KV heads, 4 bit: 47.4 us against rotate_kernel's 79.7 (2 bit 47.4 against 70.6); 4111 tokens 28.6 against 43.
 
 #include <algorithm>
+#include <type_traits>
 
 #include "kv_common.hpp"
 #include "kv_kernels.hpp"
@@ -27,10 +28,8 @@ namespace twkv {
 namespace {
 
 constexpr int kTileVecs = 16;
-constexpr int kUnitRow = kHeadDim + 4;         // floats per unit vector in LDS: 16 lanes' 16-byte reads touch every bank once
 constexpr int kAppendWaves = 4;
-static_assert(kAppendWaves * kWave == kProducerThreads && 2 * kTileVecs * kUnitRow >= kAppendWaves * kOperandTileDwords,
-              "the space of the unit vectors first holds a wave's 16 rows of R each");
+static_assert(kAppendWaves * kWave == kProducerThreads, "the workgroups of the queries");
 
 }  // namespace
 
@@ -39,7 +38,10 @@ __global__ void __launch_bounds__(kAppendWaves* kWave, 3)
 append_tokens_kernel(AppendTokensArgs a) {
     constexpr int kHeadBytes = kHeadDim * BITS / 8;
     constexpr int kCodeRow = kHeadBytes + 4;           // bytes per vector of codes in LDS
-    __shared__ __attribute__((aligned(16))) float u_s[2][kTileVecs][kUnitRow];
+    // two tiles of vectors as halves; first a wave's 16 rows of R each
+    __shared__ __attribute__((aligned(16))) uint4 x_s[kAppendWaves * kOperandTileDwords / 4];
+    static_assert(sizeof(x_s) >= 2 * kTileVecs * kHeadDim * 2, "two tiles");
+    __shared__ float inv_s[2][kTileVecs];
     __shared__ __attribute__((aligned(8))) float2 bucket_s[kBuckets];
     __shared__ __attribute__((aligned(16))) char code_s[2][kTileVecs][kCodeRow];
 
@@ -54,6 +56,8 @@ append_tokens_kernel(AppendTokensArgs a) {
             return;
         }
     }
+    asm volatile("" :: "s"(a.p.k), "s"(a.p.v), "s"(a.p.positions), "s"(a.rotation), "s"(a.p.kv_stride), "s"(a.nper), "s"(a.nstreams), "s"(a.p.rows),
+                 "s"(a.p.num_kv_heads), "s"(PROD ? a.p.k_weight : nullptr), "s"(PROD ? a.p.cos_table : nullptr), "s"(PROD ? a.p.sin_table : nullptr));
     const int tid = threadIdx.x;
     const int wave = uniform(tid / kWave), lane = tid % kWave;
     const int i16 = lane & 15, kk = lane >> 4;
@@ -81,10 +85,10 @@ append_tokens_kernel(AppendTokensArgs a) {
         Request q{};
         const half_t* src = (x.h >= Hk ? a.p.v - (long long)Hk * kHeadDim : a.p.k) + (long long)row_of(x) * a.p.kv_stride + x.h * kHeadDim;
         q.x = reinterpret_cast<const uint4*>(src)[c];
-        if (roped && x.h < Hk) {
-            const long long at = (long long)pos * (a.p.rope_dim >> 4) + rope_piece16(c, a.p.rope_dim);
-            q.cp = reinterpret_cast<const uint4*>(a.p.cos_table)[at];
-            q.sp = reinterpret_cast<const uint4*>(a.p.sin_table)[at];
+        if (PROD) {            // (no table: the rotation is read.  A load in a branch is waited for, with all before it, at the branch's end.)
+            const long long at = roped ? (long long)pos * (a.p.rope_dim >> 4) + rope_piece16(c, a.p.rope_dim) : 0;
+            q.cp = reinterpret_cast<const uint4*>(roped ? a.p.cos_table : a.rotation)[at];
+            q.sp = reinterpret_cast<const uint4*>(roped ? a.p.sin_table : a.rotation)[at];
         }
         return q;
     };
@@ -95,7 +99,6 @@ append_tokens_kernel(AppendTokensArgs a) {
     x0.h = (int)((unsigned)x0.v - (unsigned)x0.row * per_row);
     Vec x1 = advance(x0), x2 = advance(x1);
     int pos0 = request_pos(x0), pos1 = request_pos(x1), pos2 = request_pos(x2);
-    if (BITS == 4 && tid < kBuckets) bucket_s[tid] = bucket_entry(tid);
     uint4 rraw[2][4];
 #pragma unroll
     for (int d = 0; d < 2; d++)
@@ -103,20 +106,30 @@ append_tokens_kernel(AppendTokensArgs a) {
         for (int j = 0; j < 4; j++)
             rraw[d][j] = reinterpret_cast<const uint4*>(a.rotation + (wave + 4 * d) * 16 * kHeadDim)[j * kWave + lane];
     uint4 kw{};
-    if (normed) kw = reinterpret_cast<const uint4*>(a.p.k_weight)[c];
+    if (PROD) kw = reinterpret_cast<const uint4*>(normed ? a.p.k_weight : a.rotation)[c];
     Request cur = request(x0, pos0);
-    float rv[2][32];                                   // R[16 * (wave + 4 d) + i16][4s + kk]
+    Request next = request(x1, pos1);
+    if (BITS == 4 && tid < kBuckets) bucket_s[tid] = bucket_entry(tid);
+    uint4 rv[2][4];                                    // R[16 * (wave + 4 d) + i16][4s + kk], s = 8j .. 8j + 7
+    float row_norm[2];
     {
-        uint32_t* mine = reinterpret_cast<uint32_t*>(&u_s[0][0][0]) + wave * kOperandTileDwords;
+        uint32_t* mine = reinterpret_cast<uint32_t*>(x_s) + wave * kOperandTileDwords;      // this wave's own: no barrier in between
 #pragma unroll
         for (int d = 0; d < 2; d++) {
             stage_operand_tile(mine, rraw[d], lane);
-            lds_barrier();
-            read_operand_tile(mine, lane, rv[d]);
-            lds_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront", "local");
+            __builtin_amdgcn_wave_barrier();
+#pragma unroll
+            for (int j = 0; j < 4; j++) rv[d][j] = *reinterpret_cast<const uint4*>(mine + operand_tile_dword(lane, 4 * j));
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
+            __builtin_amdgcn_wave_barrier();
+            row_norm[d] = a.row_norm == 0.0f && !a.chains ? operand_rows_norm(rv[d]) : a.row_norm;
         }
     }
+    lds_barrier();                                     // every wave has its rows of R
 
+    // coordinate 4s + kk of vector v in 16-byte piece 4kk + s / 8 of its row, which lies at that piece ^ 5v (no bank twice, written or read)
+    auto vec_piece = [](int buf, int v, int p) -> int { return (buf * kTileVecs + v) * 16 + ((p ^ (5 * v)) & 15); };
     // transform, measure and regroup the vector piece of tile i
     auto fill = [&](int buf, const Vec& r, int pos, const Request& q) {
         float x[8], t[8];
@@ -127,16 +140,21 @@ append_tokens_kernel(AppendTokensArgs a) {
             if (roped) rope_head16(x, q.cp, q.sp, c, a.p.rope_dim, 0);
             if (live) reinterpret_cast<uint4*>(a.p.k + (long long)r.row * a.p.kv_stride + r.h * kHeadDim)[c] = pack_halves(x);
         }
+        const uint4 w = PROD ? pack_halves(x) : q.x;
+        const uint32_t by_kk[4] = {(w.x & 0xffffu) | (w.z << 16), (w.x >> 16) | (w.z & 0xffff0000u),
+                                   (w.y & 0xffffu) | (w.w << 16), (w.y >> 16) | (w.w & 0xffff0000u)};
+#pragma unroll
+        for (int k4 = 0; k4 < 4; k4++)
+            reinterpret_cast<uint32_t*>(&x_s[vec_piece(buf, vl, 4 * k4 + (c >> 2))])[c & 3] = by_kk[k4];
 #pragma unroll
         for (int e = 0; e < 8; e++) t[e] = x[e] * x[e];                // exact: fp16 values
         const float norm = sqrtf(head_tree_sum16(t) + 1e-12f);
-        const float inv = 1.0f / norm;
-        float* dst = &u_s[buf][vl][2 * c];
-#pragma unroll
-        for (int e = 0; e < 4; e++) *reinterpret_cast<float2*>(dst + 32 * e) = float2{x[e] * inv, x[e + 4] * inv};
-        if (live && c == 0) {
-            const long long crow = (long long)r.row * a.seq_stride_rows + pos;
-            (is_v ? a.norms[1] : a.norms[0])[crow * Hk + (is_v ? r.h - Hk : r.h)] = (half_t)norm;
+        if (c == 0) {
+            inv_s[buf][vl] = 1.0f / norm;
+            if (live) {
+                const long long crow = (long long)r.row * a.seq_stride_rows + pos;
+                (is_v ? a.norms[1] : a.norms[0])[crow * Hk + (is_v ? r.h - Hk : r.h)] = (half_t)norm;
+            }
         }
     };
     auto store_codes = [&](int buf, const Vec& r, int pos) {
@@ -148,9 +166,7 @@ append_tokens_kernel(AppendTokensArgs a) {
         if (BITS == 4) *reinterpret_cast<uint32_t*>(dst) = *reinterpret_cast<const uint32_t*>(src);
         else *reinterpret_cast<uint16_t*>(dst) = *reinterpret_cast<const uint16_t*>(src);
     };
-    auto quantize = [&](float val) -> uint32_t { return bucket_quantize<BITS>(bucket_s, val); };
 
-    Request next = request(x1, pos1);
     fill(0, x0, pos0, cur);
     Vec xs = x0, xf = x0;                              // whose codes are stored next; whose piece was filled in last
     int ps = pos0, pf = pos0;
@@ -168,22 +184,64 @@ append_tokens_kernel(AppendTokensArgs a) {
             pos2 = request_pos(x2);
             fill((i + 1) & 1, xf, pf, now);
         }
-        float4_t acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-        const float* urow = &u_s[i & 1][i16][32 * kk];
+        uint4 xv[4];
 #pragma unroll
-        for (int t = 0; t < 8; t++) {
-            const float4 u = *reinterpret_cast<const float4*>(urow + 4 * t);
-            const float uv[4] = {u.x, u.y, u.z, u.w};
+        for (int j = 0; j < 4; j++) xv[j] = x_s[vec_piece(i & 1, i16, 4 * kk + j)];
+        const float inv = inv_s[i & 1][i16];
+        uint32_t codes[2] = {0u, 0u};
+        // the fp32 chain of blocks D0 .. D1, side by side
+        auto chains = [&](auto first, auto last) {
+            constexpr int D0 = decltype(first)::value, D1 = decltype(last)::value;
+            float4_t acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                float rf[2][8], uf[8];
+#pragma unroll
+                for (int d = D0; d <= D1; d++) {
+                    uint4 rr = rv[d][j];
+                    asm volatile("" : "+v"(rr.x), "+v"(rr.y), "+v"(rr.z), "+v"(rr.w));       // not expanded ahead of the loop: 64 registers
+                    unpack_halves(rr, rf[d]);
+                }
+                unpack_halves(xv[j], uf);
+#pragma unroll
+                for (int e = 0; e < 8; e++)
+#pragma unroll
+                    for (int d = D0; d <= D1; d++) acc[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(rf[d][e], uf[e] * inv, acc[d], 0, 0, 0);
+            }
+#pragma unroll
+            for (int d = D0; d <= D1; d++) {
+                codes[d] = 0;
+#pragma unroll
+                for (int r = 0; r < 4; r++) codes[d] |= bucket_quantize<BITS>(bucket_s, acc[d][r]) << (r * BITS);
+            }
+        };
+        constexpr std::integral_constant<int, 0> d0{};
+        constexpr std::integral_constant<int, 1> d1{};
+        if (a.chains) {
+            chains(d0, d1);
+        } else {
+            // Sums of the fp16 values times the fp16 matrix: every product exact, 8 matrix instructions where the chains take 64 of twice
+            // the length.  The codes are those of the chain, by the sums unless one of a block's 256 is too near to a boundary
+            // for them (kv_rotate_util.hpp; one block in 17).
+            float4_t acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}}, sums[2][4];
 #pragma unroll
             for (int j = 0; j < 4; j++)
 #pragma unroll
-                for (int d = 0; d < 2; d++) acc[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(rv[d][4 * t + j], uv[j], acc[d], 0, 0, 0);
+                for (int d = 0; d < 2; d++) {
+                    acc[d] = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(half8_t, rv[d][j]), __builtin_bit_cast(half8_t, xv[j]), acc[d], 0, 0, 0);
+                    sums[d][j] = acc[d];
+                }
+            bool doubt[2] = {false, false};
+#pragma unroll
+            for (int d = 0; d < 2; d++)                // lane: coordinates 16 (wave + 4d) + 4kk .. + 3 of vector i16
+#pragma unroll
+                for (int r = 0; r < 4; r++) codes[d] |= bucket_quantize_sure<BITS>(bucket_s, sums[d], r, inv, row_norm[d], doubt[d]) << (r * BITS);
+            if (__any(doubt[0])) chains(d0, d0);
+            if (__any(doubt[1])) chains(d1, d1);
         }
 #pragma unroll
-        for (int d = 0; d < 2; d++) {                  // lane: coordinates 16 (wave + 4d) + 4kk .. + 3 of vector i16
-            uint32_t packed = 0;
-#pragma unroll
-            for (int r = 0; r < 4; r++) packed |= quantize(acc[d][r]) << (r * BITS);
+        for (int d = 0; d < 2; d++) {
+            const uint32_t packed = codes[d];
             char* dst = &code_s[i & 1][i16][((wave + 4 * d) * 4 + kk) * (BITS / 2)];
             if (BITS == 4) *reinterpret_cast<uint16_t*>(dst) = (uint16_t)packed;
             else *reinterpret_cast<uint8_t*>(dst) = (uint8_t)packed;
@@ -220,6 +278,10 @@ void launch_append_tokens(const AppendTokensArgs& args, int bits, hipStream_t s)
         if (n == 1 || us < least) { least = us; a.nper = n; }
     }
     a.kv_blocks = (tiles + a.nper - 1) / a.nper;
+    // A launch whose workgroups run all at once, a tile each, lasts as long as the one that runs the chain besides the sums: there all of
+    // them run it at once (256 tokens over 8 KV heads, 4 bit: 5.2 us with the sums, 4.4 without; beside producers, which take longer, the
+    // sums are faster: 200 tokens 8.1 against 8.8).
+    a.chains = !prod && a.kv_blocks <= compute_units() && a.nper == 1 ? 1 : 0;
     a.q_blocks = prod ? (int)(((long long)a.p.rows * a.p.num_heads + kProducerVecs - 1) / kProducerVecs) : 0;
     // queries beside the tiles while everything runs at once; beyond that the low occupancy of this kernel costs them more than
     // a launch of their own

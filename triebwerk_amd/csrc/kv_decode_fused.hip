@@ -119,7 +119,7 @@ decode_fused_kernel(AttnArgs a, FusedArgs f) {
     // the arguments in one trip: fetched where they are first used, the start is several of them one after the other
     asm volatile("" :: "s"(a.q), "s"(f.k_src), "s"(f.v_src), "s"(a.rotation), "s"(a.positions), "s"(a.num_kv_heads), "s"(f.hkw), "s"(f.nhg), "s"(f.shares),
                  "s"(f.by_xcd), "s"(a.G), "s"(a.q_stride), "s"(f.kv_stride), "s"(a.seq_stride_rows), "s"(PROD ? f.q_weight : nullptr),
-                 "s"(PROD ? f.k_weight : nullptr), "s"(PROD ? f.cos_table : nullptr), "s"(PROD ? f.sin_table : nullptr), "s"(PROD ? f.rope_dim : 0));
+                 "s"(PROD ? f.k_weight : nullptr), "s"(PROD ? f.cos_table : nullptr), "s"(PROD ? f.sin_table : nullptr), "s"(PROD ? f.rope_dim : 0), "s"(f.row_norm));
     const int Hk = a.num_kv_heads;
     const int HKW = f.hkw, hkw_log2 = __builtin_ctz(HKW);      // (powers of two: a division is fifty instructions here)
     const int nhg = f.nhg;                             // Hk / HKW
@@ -391,11 +391,11 @@ decode_fused_kernel(AttnArgs a, FusedArgs f) {
         lds_barrier();
         early();
         uint4 rv[4];                                       // R[16 * rot_dblk + ln][4s + kg], s = 8j .. 8j + 7
-        float doubt_eps = 0.0f;
+        float row_norm = f.row_norm;
         if (rotating) {
 #pragma unroll
             for (int j = 0; j < 4; j++) rv[j] = *reinterpret_cast<const uint4*>(rot_s + rot_dblk * kOperandTileDwords + operand_tile_dword(lane, 4 * j));
-            if (appends) doubt_eps = operand_rows_doubt(rv);
+            if (appends && row_norm == 0.0f) row_norm = operand_rows_norm(rv);
         }
         for (int vt = wave >> 3; rotating && vt * 16 < nvec; vt += kRotGroups) {  // uniform over the wave
             const int vi = vt * 16 + i16;
@@ -404,13 +404,14 @@ decode_fused_kernel(AttnArgs a, FusedArgs f) {
             (void)unit_vector(vc, kind, head);
             const bool is_query = kind == 2;
             // fp16 values times an fp16 matrix: every product exact, the sums in fp32
-            float4_t acc = {0.f, 0.f, 0.f, 0.f};
+            float4_t acc = {0.f, 0.f, 0.f, 0.f}, sums[4];
 #pragma unroll
             for (int j = 0; j < 4; j++) {
                 union { uint4 u; half8_t h; } xv, rm;
                 xv.u = x_s[vc][piece_of(vc, 4 * kk + j)];
                 rm.u = rv[j];
                 acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(rm.h, xv.h, acc, 0, 0, 0);
+                sums[j] = acc;
             }
             if (is_query && vi < nvec) {
                 float4 o = {acc[0] * f.q_scale, acc[1] * f.q_scale, acc[2] * f.q_scale, acc[3] * f.q_scale};
@@ -419,13 +420,13 @@ decode_fused_kernel(AttnArgs a, FusedArgs f) {
             }
             if (appends && vt * 16 < first_q) {                    // lane: coordinates 16 dblk + 4kk .. + 3
                 // codes: those of the fp32 chain, by the sums above unless one of the block's is too near to a boundary
-                // for them (kv_rotate_util.hpp; one block in 6 with 16 vectors, one in 23 with 4)
+                // for them (kv_rotate_util.hpp; one block in 17 with 16 vectors, one in 66 with 4)
                 const bool live = vi < nvec && !is_query;
                 const float inv = live ? inv_s[vc] : 0.0f;
                 uint32_t packed = 0;
                 bool doubt = false;
 #pragma unroll
-                for (int r = 0; r < 4; r++) packed |= bucket_quantize_sure<BITS>(bucket_s, acc[r] * inv, doubt_eps, doubt) << (r * BITS);
+                for (int r = 0; r < 4; r++) packed |= bucket_quantize_sure<BITS>(bucket_s, sums, r, inv, row_norm, doubt) << (r * BITS);
                 if (__any(live && doubt)) {
                     acc = float4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll

@@ -229,7 +229,7 @@ decode_layers_kernel(LayersArgs a) {
     issue_k(t); issue_n(t); issue_v(t);
     // ---- rotation of all of them on fp16 matrix instructions: fp16 values times an fp16 matrix, every product exact in the fp32
     // accumulator, 4 matrix instructions a block and 16 vectors
-    float4_t y[kPasses][kBlocks];
+    float4_t y[kPasses][kBlocks], sums[kBlocks][4];         // sums: after each operand of the first 16 vectors
 #pragma unroll
     for (int p = 0; p < kPasses; p++) {
         const int v = kUnitVecs * p + ln < NV ? kUnitVecs * p + ln : 0;
@@ -243,12 +243,13 @@ decode_layers_kernel(LayersArgs a) {
             for (int i = 0; i < kBlocks; i++) {
                 rv.u = rraw[i][j];
                 y[p][i] = __builtin_amdgcn_mfma_f32_16x16x32_f16(rv.h, xv.h, y[p][i], 0, 0, 0);
+                if (p == 0) sums[i][j] = y[p][i];
             }
         }
     }
     {   // Codes of K and V.  They are those of the fp32 chain of kv_rotate.hip, which is 32 matrix instructions of twice the length a
-        // block; the sums above differ from it by less than kCodeDoubt (kv_rotate_util.hpp), so they decide every coordinate that is
-        // further from a boundary, and a block with one that is not (one in 6 with 16 vectors, one in 23 with 4) runs the chain.
+        // block; the sums above decide every coordinate that is further from a boundary than the two can be apart (kv_rotate_util.hpp), and
+        // a block with one that is not (one in 17 with 16 vectors, one in 66 with 4) runs the chain.
         const int v = ln, vk = vec_kind(v);                // this lane's vector
         const bool live = v < 2 * HKW;
         const float inv = inv_s[live ? v : 0];
@@ -257,7 +258,7 @@ decode_layers_kernel(LayersArgs a) {
             uint32_t packed = 0;
             bool doubt = false;
 #pragma unroll
-            for (int r = 0; r < 4; r++) packed |= bucket_quantize_sure<BITS>(bucket_s, y[0][i][r] * inv, kCodeDoubt, doubt) << (r * BITS);
+            for (int r = 0; r < 4; r++) packed |= bucket_quantize_sure<BITS>(bucket_s, sums[i], r, inv, kUnitRows, doubt) << (r * BITS);
             if (__any(live && doubt)) {
                 float4_t acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll

@@ -358,6 +358,7 @@ void layer_step(tw_engine* e, int layer, const tw_half* q, const tw_half* k, con
                                            m.num_heads, m.num_kv_heads, m.head_dim, e->q_dim(), e->kv_dim(),
                                            e->rope_dim, s);
     }
+    const twkv::KnownRotation known;
     twkv::layer_attention_step(&p, e->ctx_mean(), s);
 }
 
@@ -618,6 +619,7 @@ int tw_engine_single_step(tw_engine* e, int layer, const tw_half* q, const tw_ha
     p.rotation = e->single_rotation; p.scratch = e->single_scores;
     p.ctx_min = p.ctx_max = e->single_pos + 1;
     p.tickets = e->single_tickets;          // one sequence leaves most compute units idle: its context may be shared
+    const twkv::KnownRotation known;
     tw_layer_attention_step(&p, s);
     return tw_kv_last_error();
 }
@@ -771,6 +773,7 @@ int tw_engine_prompt_layer(tw_engine* e, int layer, int seq, const tw_half* q, c
     // the batch's attention scratch holds G * num_heads * max_seq_len floats (engine.cpp:1371); the prefill
     // launchers count on T floats per (token, head) and do without a workspace when there is none
     p.scratch = ((size_t)T * T <= (size_t)e->G * msl) ? e->attn_scores : nullptr;
+    const twkv::KnownRotation known;
     tw_layer_prompt_step(&p, s);
     return tw_kv_last_error();
 }

@@ -113,9 +113,16 @@ struct AppendTokensArgs {
     half_t* norms[2];
     const half_t* rotation;
     long long seq_stride_rows;   // row r goes to cache row r * seq_stride_rows + positions[r]
-    int nper, kv_blocks, q_blocks;   // launch_append_tokens fills these in
+    float row_norm;              // as FusedArgs has it
+    int nper, kv_blocks, q_blocks, chains;   // launch_append_tokens fills these in
 };
 bool append_tokens_usable(const AppendTokensArgs& a);
+// While one of these lives the calls of this thread have the engine's rotation, whose rows are of norm 1: the kernels need not measure them
+// (FusedArgs::row_norm).
+struct KnownRotation {
+    KnownRotation();
+    ~KnownRotation();
+};
 void launch_append_tokens(const AppendTokensArgs& a, int bits, hipStream_t s);
 // data[r][i] = half(data[r][i] / (1 + exp(-gate[r][i]))), rows of `dim` halves with their own strides
 void launch_sigmoid_gate(half_t* data, long long data_stride, const half_t* gate, long long gate_stride, int dim,
@@ -226,6 +233,7 @@ struct FusedArgs {
     int hkw, nhg;           // KV heads per workgroup, workgroups for all of them (launch_decode_fused fills these in)
     int by_xcd;             // sequence g's workgroups on XCD g % 8 (likewise)
     float q_scale;          // likewise
+    float row_norm;         // an upper bound on the norms of R's rows; 0: the kernel finds one
     // A unit's context shared by several workgroups, for batches whose units alone leave compute units idle:
     int shares;             // a power of two up to 64 (launch_decode_fused fills this in; > 1 only with the two below)
     float* share_ws;        // G * num_heads * shares * (kHeadDim + 4) floats for the shares' unnormalised sums

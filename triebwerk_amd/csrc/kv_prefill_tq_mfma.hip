@@ -59,6 +59,7 @@ prefill_tq_mfma_kernel(AttnArgs a, int T, int mirror) {
     __shared__ __attribute__((aligned(16))) float n_all[KS][3][2][32];    // [group][buffer][k | v][token]
     __shared__ __attribute__((aligned(16))) uint32_t tab_s[256 * kPtReplicas * kEntryDwords];
 
+    asm volatile("" :: "s"(a.q), "s"(a.k), "s"(a.v), "s"(a.k_norms), "s"(a.v_norms), "s"(a.rotation), "s"(a.q_stride), "s"(a.num_kv_heads), "s"(T), "s"(mirror));
     const int tid_wg = threadIdx.x;
     const int wave_wg = uniform(tid_wg / kWave), lane = tid_wg % kWave;
     const int grp = KS == 1 ? 0 : wave_wg / GW, wave = KS == 1 ? wave_wg : wave_wg % GW;
@@ -89,23 +90,34 @@ prefill_tq_mfma_kernel(AttnArgs a, int T, int mirror) {
     constexpr float kRaise = 5.0f;
 
     // ---- table: byte -> its codes' centroids (low field first) as fp16(alpha c), kPtReplicas copies
-    // A thread stores 16 bytes at a time; the centroids come out of a register by wave shuffle (lane c holds centroid c):
-    // an index into the constant array that differs between lanes is a load per look-up, one waiting for the other.
+    // A thread stores 16 bytes at a time; its entries share their low four bits and a wave's their upper four, so one centroid comes out of
+    // a register by wave shuffle and the others by v_readlane (lane c holds centroid c).  An index into the constant array that differs
+    // between lanes is a load per look-up, one waiting for the other; a shuffle per entry, a trip through LDS each, was 1 us of a launch.
     auto build_table = [&]() {
+        constexpr int kStep = W * kWave * 4, kRounds = 256 * kPtReplicas * kEntryDwords / kStep;
+        static_assert(kPtReplicas * kEntryDwords == 16 && kRounds * kStep == 4096 && kStep % 256 == 0, "a round advances the entry by a multiple of 16");
         const float cent_lane = kAlpha * centroid_of<BITS>(lane);
-        auto cent = [&](int c) -> half_t { return (half_t)__shfl(cent_lane, c, 64); };
+        const int e0 = tid_wg >> 2, hi0 = uniform(tid_wg >> 6);        // entry = e0 + W * 16 k: upper bits hi0 + W k
+        auto cent_of = [&](int c) -> half_t {                 // c uniform over the wave
+            return (half_t)__builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, cent_lane), c));
+        };
+        if constexpr (BITS == 4) {
+            const half_t lo = (half_t)__shfl(cent_lane, e0 & 15, 64);
 #pragma unroll
-        for (int i = tid_wg * 4; i < 256 * kPtReplicas * kEntryDwords; i += W * kWave * 4) {
-            const int e = i / (kPtReplicas * kEntryDwords);
-            if constexpr (BITS == 4) {
-                half2_t p = {cent(e & 15), cent(e >> 4)};
+            for (int k = 0; k < kRounds; k++) {
+                half2_t p = {lo, cent_of(hi0 + W * k)};
                 const uint32_t w = *reinterpret_cast<uint32_t*>(&p);
-                *reinterpret_cast<uint4*>(&tab_s[i]) = uint4{w, w, w, w};
-            } else {
-                half2_t p0 = {cent(e & 3), cent((e >> 2) & 3)};
-                half2_t p1 = {cent((e >> 4) & 3), cent((e >> 6) & 3)};
-                const uint32_t w0 = *reinterpret_cast<uint32_t*>(&p0), w1 = *reinterpret_cast<uint32_t*>(&p1);
-                *reinterpret_cast<uint4*>(&tab_s[i]) = uint4{w0, w1, w0, w1};
+                *reinterpret_cast<uint4*>(&tab_s[tid_wg * 4 + k * kStep]) = uint4{w, w, w, w};
+            }
+        } else {
+            half2_t p0 = {(half_t)__shfl(cent_lane, e0 & 3, 64), (half_t)__shfl(cent_lane, (e0 >> 2) & 3, 64)};
+            const uint32_t w0 = *reinterpret_cast<uint32_t*>(&p0);
+#pragma unroll
+            for (int k = 0; k < kRounds; k++) {
+                const int hi = hi0 + W * k;
+                half2_t p1 = {cent_of(hi & 3), cent_of(hi >> 2)};
+                const uint32_t w1 = *reinterpret_cast<uint32_t*>(&p1);
+                *reinterpret_cast<uint4*>(&tab_s[tid_wg * 4 + k * kStep]) = uint4{w0, w1, w0, w1};
             }
         }
     };
@@ -244,7 +256,9 @@ prefill_tq_mfma_kernel(AttnArgs a, int T, int mirror) {
         half8_t qb[NQ][4], ql[NQ][4];
         Staged st;
         {
-            const RotPieces rot = load_rotation();
+            uint32x4_t rot[32 / W];
+#pragma unroll
+            for (int r = 0; r < 32 / W; r++) rot[r] = reinterpret_cast<const uint32x4_t*>(a.rotation)[tid_wg + r * (W * kWave)];
             half8_t qv[NQ][4];                             // q[query ln][32t + 8kg .. +7]
 #pragma unroll
             for (int nq = 0; nq < NQ; nq++) {
@@ -253,6 +267,7 @@ prefill_tq_mfma_kernel(AttnArgs a, int T, int mirror) {
                 for (int t = 0; t < 4; t++) qv[nq][t] = *reinterpret_cast<const half8_t*>(qsrc + 32 * t);
             }
             load_tile(32 * grp, st);
+            __builtin_amdgcn_sched_barrier(0);             // (everything is asked for here, not behind the table)
             if (pass == 0) build_table();
             else lds_barrier();                            // the previous pass's epilogue reads the rotation in the same place
             {
@@ -260,7 +275,7 @@ prefill_tq_mfma_kernel(AttnArgs a, int T, int mirror) {
                 char* dst = &v_all[0][(16 * ((krow >> 2) & 1) + 4 * (krow >> 3) + (krow & 3)) * kPtKRow + 16 * c];
 #pragma unroll
                 for (int r = 0; r < 32 / W; r++)
-                    *reinterpret_cast<uint4*>(dst + (W == 4 ? 32 * (r >> 1) + 8 * (r & 1) : 32 * r) * kPtKRow) = rot.p[r];
+                    *reinterpret_cast<uint32x4_t*>(dst + (W == 4 ? 32 * (r >> 1) + 8 * (r & 1) : 32 * r) * kPtKRow) = rot[r];
             }
             lds_barrier();                                 // the table and R are there
             const char* rrow = &v_all[0][ln * kPtKRow + 16 * kg];

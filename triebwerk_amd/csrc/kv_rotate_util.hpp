@@ -120,18 +120,37 @@ __device__ __forceinline__ uint32_t bucket_quantize(const float2* buckets, float
     }
 }
 
-// How far the rotation of a unit vector by v_mfma_f32_16x16x32_f16 -- raw fp16 coordinates, the sum scaled by 1 / |x| afterwards -- can be
-// from the fp32 chain whose codes the reference's are, for rows of R of norm 1.  The chain's 128 fused multiply-adds lose 2^-24 of a
-// partial sum each, at most |R row| |u| = 1 (Cauchy-Schwarz), and the unit coordinates 2^-24 each: together at most 129 * 2^-24 = 7.7e-6.
-// The four matrix instructions: at most 2.8e-7 of |x| from the exact sum over 2.4 million vectors (normal, outliers, one
-// large coordinate, multiples of R's rows, denormals, magnitudes over 2^24), taken as 1.2e-6.
-constexpr float kCodeDoubt = 9e-6f;
-// bucket_quantize, with doubt set where val is not further than eps from a boundary (or no number): there val + an error of eps may have
-// another code.  A boundary is further than that from its bucket's edges.
-static_assert(0.15 / kBucketScale > 100.0 * kCodeDoubt, "a value near a boundary is in its bucket");
-// The same for the 16 rows of any R whose halves the lanes of a wave hold as operands (16 lanes a row quarter): as large as the longest
-// of them (a R that is no number leaves no value sure).
-__device__ __forceinline__ float operand_rows_doubt(const uint4 (&rows)[4]) {
+// K and V codes from v_mfma_f32_16x16x32_f16 -- raw fp16 coordinates, the sum scaled by 1 / |x| afterwards -- where they are sure to be those
+// of the fp32 chain, whose codes the reference's are.  How far can the two be apart, for a row of R of norm |R|?
+// The chain's fused multiply-adds lose at most 2^-24 of a partial sum s_k each, and the unit coordinates 2^-24 of |R| in all.  The
+// matrix instructions leave the sums S_1 .. S_4 over the first 32, 64, 96 and 128 coordinates (operand j holds coordinates 32j .. 32j + 31); a
+// partial sum in between is at most (|S_j| + |S_j+1| + t_j) / 2, t_j the sum of the block's |products|, and the four t_j are at most
+// 2 |R| together (Cauchy-Schwarz).  So the sum of all |s_k| is at most 32 (|S_1| + |S_2| + |S_3|) + 16 |S_4| + 32 |R|.
+// The matrix instructions themselves: at most 2.8e-7 of |R| |x| from the exact sum over 2.4 million vectors (normal, outliers,
+// one large coordinate, multiples of R's rows, denormals, magnitudes over 2^24), taken as 8e-7.
+constexpr float kUlp = 5.9604645e-8f;                          // 2^-24
+constexpr float kSureBase = 34.0f * kUlp + 8e-7f;              // times |R|
+// Code of y = S[3][r] * inv; doubt is set where it is not further than that from a boundary (or no number).
+static_assert(0.15 / kBucketScale > 100.0 * 170.0 * kUlp, "a value near a boundary is in its bucket, which no boundary lies near to the edge of");
+template <int BITS>
+__device__ __forceinline__ uint32_t bucket_quantize_sure(const float2* buckets, const float4_t (&S)[4], int r, float inv, float row_norm, bool& doubt) {
+    const float val = S[3][r] * inv;
+    const float sums = __builtin_fmaf(2.0f, fabsf(S[0][r]) + fabsf(S[1][r]) + fabsf(S[2][r]), fabsf(S[3][r]));
+    const float eps = __builtin_fmaf(sums, inv * (16.0f * kUlp), row_norm * kSureBase);
+    if constexpr (BITS == 4) {
+        const float2 e = buckets[bucket_of(val)];
+        doubt = doubt || !(fabsf(val - e.x) > eps);
+        return __builtin_bit_cast(uint32_t, e.y) + (!(val < e.x) ? 1u : 0u);
+    } else {
+        doubt = doubt || !(fminf(fabsf(val), fabsf(fabsf(val) - kEdges2[2])) > eps);
+        return (uint32_t)turbo_quantize(val, 2);
+    }
+}
+// What the engine's own rotation (rows of norm 1 within 1e-4) is given as; for any other R the kernels take the norm from its rows.
+constexpr float kUnitRows = 1.001f;
+// The norm of the longest of the 16 rows of R whose halves the lanes of a wave hold as operands (16 lanes a row quarter); a row that is no
+// number leaves none sure.
+__device__ __forceinline__ float operand_rows_norm(const uint4 (&rows)[4]) {
     float n2 = 0.0f;
 #pragma unroll
     for (int j = 0; j < 4; j++) {
@@ -155,18 +174,7 @@ __device__ __forceinline__ float operand_rows_doubt(const uint4 (&rows)[4]) {
     n2 = larger(n2, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, n2), 0x4E, 0xf, 0xf, true));
     n2 = larger(n2, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, n2), 0x141, 0xf, 0xf, true));
     n2 = larger(n2, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, n2), 0x140, 0xf, 0xf, true));
-    return 1.001f * kCodeDoubt * sqrtf(n2);
-}
-template <int BITS>
-__device__ __forceinline__ uint32_t bucket_quantize_sure(const float2* buckets, float val, float eps, bool& doubt) {
-    if constexpr (BITS == 4) {
-        const float2 e = buckets[bucket_of(val)];
-        doubt = doubt || !(fabsf(val - e.x) > eps);
-        return __builtin_bit_cast(uint32_t, e.y) + (!(val < e.x) ? 1u : 0u);
-    } else {
-        doubt = doubt || !(fminf(fabsf(val), fabsf(fabsf(val) - kEdges2[2])) > eps);
-        return (uint32_t)turbo_quantize(val, 2);
-    }
+    return 1.001f * __builtin_amdgcn_sqrtf(n2);
 }
 
 }  // namespace twkv
