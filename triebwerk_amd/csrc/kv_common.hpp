@@ -117,6 +117,20 @@ __device__ __forceinline__ void lds_barrier() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
+// max and sum over the four lanes 16 and 32 apart, on the vector ALU (a shuffle is a trip through LDS)
+typedef unsigned lane_pair_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ float quarter_max(float v) {
+    lane_pair_t w = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = fmaxf(__uint_as_float(w[0]), __uint_as_float(w[1]));
+    w = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(w[0]), __uint_as_float(w[1]));
+}
+__device__ __forceinline__ float quarter_sum(float v) {
+    lane_pair_t w = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(w[0]) + __uint_as_float(w[1]);
+    w = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(w[0]) + __uint_as_float(w[1]);
+}
 __device__ __forceinline__ float wave_max(float v) {
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));

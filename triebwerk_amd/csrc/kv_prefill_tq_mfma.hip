@@ -27,8 +27,7 @@ constexpr int kPtKRow = 2 * kHeadDim + 32;   // bytes per expanded K row in LDS 
 constexpr int kPtVRow = 2 * 32 + 32;         // bytes per V^T row (32 token slots) in LDS (96: full rate, 80: 54 %)
 constexpr int kPtVTile = kHeadDim * kPtVRow; // bytes of a V^T tile
 constexpr int kPtVBytes = 3 * kPtVTile;      // 3 tiles, and room for the 128 x 128 fp16 rotation
-constexpr int kPtRotBlock = 4 * kWave * 16 + 16;   // bytes per 16 output dims of the rotation in the epilogue: 16 more than the entries, so that its 2-byte writes meet no bank twice
-static_assert(kPtVBytes >= kHeadDim * kPtKRow && kPtVBytes >= 8 * kPtRotBlock, "the rotation fits in both layouts");
+static_assert(kPtVBytes >= kHeadDim * kPtKRow, "the rotation fits in the V tiles' space");
 
 // a masked score: below the initial maximum by more than the exponent's range, also when a group's first tile is all masked
 constexpr float kMasked = -3.0e38f;
@@ -222,13 +221,13 @@ prefill_tq_mfma_kernel(AttnArgs a, int T, int mirror) {
         if (tid < 2 * kWave && (tid & 32) == 0) n_s[vbuf][tid >> 6][tid & 31] = h2f_bits(st.nb);
     };
     // the rotation, a piece per thread: rows k = 16r + tid / 16 (512 threads: 32r + tid / 16), columns 8c .. 8c + 7, c = tid % 16
-    struct RotPieces { uint4 p[32 / W]; };
+    struct RotPieces { uint32x4_t p[32 / W]; };
     auto load_rotation = [&]() -> RotPieces {
         RotPieces rp;
         int at = tid_wg;
         asm volatile("" : "+v"(at));                       // asked for where it is written: not kept across passes
 #pragma unroll
-        for (int r = 0; r < 32 / W; r++) rp.p[r] = reinterpret_cast<const uint4*>(a.rotation)[at + r * (W * kWave)];
+        for (int r = 0; r < 32 / W; r++) rp.p[r] = reinterpret_cast<const uint32x4_t*>(a.rotation)[at + r * (W * kWave)];
         return rp;
     };
 
@@ -400,8 +399,7 @@ prefill_tq_mfma_kernel(AttnArgs a, int T, int mirror) {
 #pragma unroll
                     for (int i = 1; i < 8; i++) mx = fmaxf(mx, x[i]);
                     if (__any(mx > m_run[nq] + kRaise)) {  // rare after the first tiles
-                        mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-                        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));    // the query's maximum over the tile
+                        mx = quarter_max(mx);              // the query's maximum over the tile
                         const float m_new = fmaxf(m_run[nq], mx);
                         const float alpha = __builtin_amdgcn_exp2f(m_run[nq] - m_new);
                         m_run[nq] = m_new;
@@ -433,14 +431,15 @@ prefill_tq_mfma_kernel(AttnArgs a, int T, int mirror) {
         if (have_prev) pv((ntiles - 1) % 3, pa_prev, pl_prev);
 
         // ---- epilogue: out[q][d] = sum_k R[k][d] o[q][k] / (sum + 1e-8) (kernels.cu:1946-1957) as
-        // out^T = R^T . O^T.  The rotation goes into the V buffers in operand order: 16-byte entry
-        // t * 64 + lane of block db holds R[k][16 db + ln] for the 8 k that lane (ln, kg) carries in step t,
-        // k = 32t + 16 (e / 4) + 4kg + e % 4 -- the dims its accumulators o[.][2t + e / 4][e % 4] belong to.
+        // out^T = R^T . O^T.  The rotation goes into the V buffers as it lies in memory, row by row, and lane (ln, kg) reads R[k][16 db + ln]
+        // for the 8 k it carries in step t, k = 32t + 16 (e / 4) + 4kg + e % 4 -- the dims its accumulators o[.][2t + e / 4][e % 4]
+        // belong to -- by two transposing reads: the 16 lanes of a quarter point at 4 rows of 16 halves, 4 lanes to a row, and
+        // lane ln gets column ln of the four.  (Regrouped on the way in, 64 two-byte writes a thread, it cost 0.5 us of a launch.)
         __syncthreads();                                   // every wave is done with the tiles
         // two groups: their sums change hands through the V tiles -- with two query blocks group s finishes block s, with one
         // query block both groups merge the whole of it and each rotates half of the dims -- and the rotation takes the K tiles
         char* rot_s = KS == 2 ? &k_all[0][0][0] : &v_all[0][0];
-        static_assert(KS == 1 || (sizeof(k_all) >= 8 * kPtRotBlock && (int)sizeof(v_all) >= W * kWave * (8 * 16 + 8)), "both fit");
+        static_assert(KS == 1 || (sizeof(k_all) >= kHeadDim * kPtKRow && (int)sizeof(v_all) >= W * kWave * (8 * 16 + 8)), "both fit");
         float4_t* ex = reinterpret_cast<float4_t*>(&v_all[0][0]);                                  // [wave of the workgroup][8][lane]
         float2* exml = reinterpret_cast<float2*>(&v_all[0][0] + W * 8 * kWave * 16);               // [wave][lane]: maximum, sum
         constexpr int NF = KS == 2 ? 1 : NQ;               // query blocks this wave finishes
@@ -449,10 +448,7 @@ prefill_tq_mfma_kernel(AttnArgs a, int T, int mirror) {
         float lsum[NQ];
 #pragma unroll
         for (int nq = 0; nq < NQ; nq++) {
-            float l = l_run[nq];
-            l += __shfl_xor(l, 16, 64);
-            l += __shfl_xor(l, 32, 64);
-            lsum[nq] = l;
+            lsum[nq] = quarter_sum(l_run[nq]);
         }
         float4_t of[NF][8];
         float lf[NF], m_own = 0.0f;
@@ -477,18 +473,10 @@ prefill_tq_mfma_kernel(AttnArgs a, int T, int mirror) {
             }
         }
         {
-            // thread -> rows k = 16r + tid / 16, r = 0..7, columns 8c .. 8c + 7 with c = tid % 16; of k only r is
-            // not fixed per thread, and r moves the destination by whole steps t = r / 2 and halves 4 (r % 2)
-            const int krow = tid_wg >> 4, c = tid_wg & 15;       // 512 threads: rows k = 32r + tid / 16, r = 0..3
-            char* dst0 = &rot_s[(c >> 1) * kPtRotBlock + ((krow >> 2) & 3) * 256 + (c & 1) * 128 + 2 * (krow & 3) + (W == 8 ? 8 * (krow >> 4) : 0)];
+            // thread -> rows k = 16r + tid / 16 (512 threads: 32r + tid / 16), columns 8c .. 8c + 7, c = tid % 16
+            char* dst = rot_s + (tid_wg >> 4) * kPtKRow + 16 * (tid_wg & 15);
 #pragma unroll
-            for (int r = 0; r < 32 / W; r++) {
-                const uint32_t w[4] = {rot_raw.p[r].x, rot_raw.p[r].y, rot_raw.p[r].z, rot_raw.p[r].w};
-                const int step = W == 4 ? (r >> 1) * 1024 + (r & 1) * 8 : r * 1024;
-#pragma unroll
-                for (int x = 0; x < 8; x++)
-                    *reinterpret_cast<uint16_t*>(dst0 + step + x * 16) = (uint16_t)(w[x >> 1] >> (16 * (x & 1)));
-            }
+            for (int r = 0; r < 32 / W; r++) *reinterpret_cast<uint32x4_t*>(dst + r * (W * kWave / 16) * kPtKRow) = rot_raw.p[r];
         }
         __syncthreads();
         if constexpr (KS == 2) {                           // a lane's accumulators all belong to query ln, its maximum and sum too
@@ -527,7 +515,13 @@ prefill_tq_mfma_kernel(AttnArgs a, int T, int mirror) {
             for (int nf = 0; nf < NF; nf++) y[nf] = float4_t{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int t = 0; t < 4; t++) {
-                const half8_t ra = *reinterpret_cast<const half8_t*>(&rot_s[db * kPtRotBlock + (t * 64 + lane) * 16]);
+                typedef __fp16 __attribute__((ext_vector_type(4))) fp16x4_t;
+                typedef __attribute__((address_space(3))) fp16x4_t* lds_fp16x4_t;
+                const char* at = rot_s + (32 * t + 4 * kg + (ln >> 2)) * kPtKRow + 32 * db + 8 * (ln & 3);
+                union { fp16x4_t q[2]; half8_t h; } rt;
+                rt.q[0] = __builtin_amdgcn_ds_read_tr16_b64_v4f16((lds_fp16x4_t)at);
+                rt.q[1] = __builtin_amdgcn_ds_read_tr16_b64_v4f16((lds_fp16x4_t)(at + 16 * kPtKRow));
+                const half8_t ra = rt.h;
 #pragma unroll
                 for (int nf = 0; nf < NF; nf++) {
                     y[nf] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ra, oh[nf][t], y[nf], 0, 0, 0);
