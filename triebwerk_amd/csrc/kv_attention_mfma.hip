@@ -656,12 +656,12 @@ bool prepare_attention_mfma(AttnArgs& a, hipStream_t s, bool rotate_query) {
         RotArgs r;
         memset(&r, 0, sizeof(r));
         r.nseg = 1;
-        r.seg_src[0] = a.q;
-        r.seg_stride[0] = a.q_stride;
-        r.seg_heads[0] = a.num_heads;
-        r.seg_nvec[0] = a.G * a.num_heads;
-        r.seg_units[0] = (r.seg_nvec[0] + 15) / 16 * 8;
-        r.seg_kind[0] = 1;
+        r.seg[0].src = a.q;
+        r.seg[0].stride = a.q_stride;
+        r.seg[0].heads = a.num_heads;
+        r.seg[0].nvec = a.G * a.num_heads;
+        r.seg[0].units = (r.seg[0].nvec + 15) / 16 * 8;
+        r.seg[0].kind = 1;
         r.rotation = a.rotation;
         r.qrot = a.qrot;
         r.qrot_stride = a.ws_stride;

@@ -130,16 +130,21 @@ void launch_sigmoid_gate(half_t* data, long long data_stride, const half_t* gate
 
 // ---------------------------------------------------------------- rotation on the matrix cores
 struct RotArgs {
-    int nseg;                    // up to 3 segments: K rows, V rows (quantize), Q rows (rotate only)
-    const half_t* seg_src[3];    // fp16 source, row r at src + r * stride
-    long long seg_stride[3];     // halves per source row
-    int seg_heads[3];            // head vectors per source row
-    int seg_nvec[3];             // rows * heads
-    int seg_units[3];            // work units = ceil(tiles / nper) * 8 (launch_rotate fills this in)
+    // up to 3 segments: K rows, V rows (quantize), Q rows (rotate only); each 64 bytes, one scalar load of a kernel
+    struct alignas(64) Segment {
+        const half_t* src;       // fp16 source, row r at src + r * stride
+        long long stride;        // halves per source row
+        uint8_t* codes;
+        half_t* norms;
+        const half_t* weight;    // optional producers applied to the vectors before anything else (kv_producer.hip has the rules): RMSNorm weight (128), NULL = none
+        int heads;               // head vectors per source row
+        int nvec;                // rows * heads
+        int kind;                // 0 = quantize into the cache, 1 = query rotation
+        int rope;                // rotate with the tables below at positions[row]
+        int units;               // work units = ceil(tiles / nper) * 8 (launch_rotate fills this in)
+    } seg[3];
+    int nseg;
     int nper;                    // tiles of 16 vectors a wave walks (launch_rotate fills this in)
-    int seg_kind[3];             // 0 = quantize into the cache, 1 = query rotation
-    uint8_t* seg_codes[3];
-    half_t* seg_norms[3];
     const half_t* rotation;
     const int* positions;
     const int* block_table;
@@ -150,9 +155,7 @@ struct RotArgs {
     float* qrot;                 // query output: vector v at qrot + v * qrot_stride (fp32)
     long long qrot_stride;
     float q_scale;
-    // optional producers applied to a segment's vectors before anything else (kv_producer.hip has the rules)
-    const half_t* seg_weight[3]; // per-head RMSNorm weight (128), NULL = none
-    int seg_rope[3];             // rotate with the tables below at positions[row]
+    // producers of the segments that have them
     float eps;
     int biased;
     const half_t* cos_table;     // (positions, rope_dim / 2)

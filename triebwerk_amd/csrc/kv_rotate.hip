@@ -36,6 +36,7 @@
 
 #include "kv_common.hpp"
 #include "kv_kernels.hpp"
+#include "kv_mfma_util.hpp"
 #include "kv_rotate_util.hpp"
 
 namespace twkv {
@@ -65,25 +66,37 @@ template <int BITS, bool PROD>
 __global__ void __launch_bounds__(kWave)
 rotate_kernel(RotArgs a) {
     __shared__ __attribute__((aligned(16))) uint32_t x_s[kOperandTileDwords];
+    __shared__ __attribute__((aligned(8))) float2 bucket_s[kBuckets];
     const int lane = threadIdx.x;
     const int i16 = lane & 15, kk = lane >> 4;
 
     // ---- which unit: (segment, group of a.nper vector tiles, block of 16 output coordinates)
+    asm volatile("" :: "s"(a.seg[0].units), "s"(a.seg[1].units), "s"(a.nseg), "s"(a.nper), "s"(a.rotation), "s"(a.positions), "s"(a.block_table),
+                 "s"(a.seq_stride_rows), "s"(a.token_list));
     int unit = blockIdx.x;
-    int seg = 0;
-    while (seg < a.nseg - 1 && unit >= a.seg_units[seg]) { unit -= a.seg_units[seg]; seg++; }
+    const int after0 = unit - a.seg[0].units, after1 = after0 - a.seg[1].units;
+    const int seg = a.nseg > 1 && after0 >= 0 ? (a.nseg > 2 && after1 >= 0 ? 2 : 1) : 0;
+    unit = seg == 0 ? unit : seg == 1 ? after0 : after1;
+    const RotArgs::Segment& sg = a.seg[seg];
+    asm volatile("" :: "s"(sg.src), "s"(sg.stride), "s"(sg.heads), "s"(sg.nvec), "s"(sg.kind), "s"(sg.units));
     // Units of a segment in blocks of 64 = 8 tile groups x 8 coordinate blocks, the coordinate blocks of one
     // tile group 8 workgroups apart (same XCD; every segment starts at a multiple of 8); what is left over at the
     // end of the segment is numbered plainly.
     int dblk = unit & 7, vgroup = unit >> 3;
-    if (unit < (a.seg_units[seg] >> 6) << 6) {
+    if (unit < (sg.units >> 6) << 6) {
         vgroup = (unit >> 6) * 8 + (unit & 7);
         dblk = (unit >> 3) & 7;
     }
-    const int nvec = a.seg_nvec[seg];
-    const int heads = a.seg_heads[seg];                  // head vectors per source row
-    const bool is_query = a.seg_kind[seg] != 0;
-    const bool roped = PROD && a.seg_rope[seg] != 0;
+    const int nvec = sg.nvec;
+    const int heads = sg.heads;               // head vectors per source row
+    const bool is_query = sg.kind != 0;
+    const bool roped = PROD && sg.rope != 0;
+    const half_t* weight = PROD ? sg.weight : nullptr;
+    uint8_t* codes = sg.codes;
+    half_t* norms = sg.norms;
+    const bool heads_pow2 = (heads & (heads - 1)) == 0;  // (else a division: twenty instructions)
+    const int heads_log2 = __builtin_ctz(heads);
+    auto row_of = [&](int v) -> int { return heads_pow2 ? v >> heads_log2 : v / heads; };
 
     // ---- A operand, once per wave: R rows d0 .. d0 + 15 (4 KB in a row); requested now, staged after the
     // first tile of vectors has been requested too
@@ -93,13 +106,13 @@ rotate_kernel(RotArgs a) {
         raw[j] = reinterpret_cast<const uint4*>(a.rotation + dblk * 16 * kHeadDim)[j * kWave + lane];
 
     // 16-byte piece j * 64 + lane of a tile of vectors: piece lane % 16 of vector 4j + lane / 16
-    const half_t* src = a.seg_src[seg];
-    const long long stride = a.seg_stride[seg];
+    const half_t* src = sg.src;
+    const long long stride = sg.stride;
     auto request_tile = [&](int vtile, uint4 (&dst)[4]) {
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             const int vi = min(vtile * 16 + 4 * j + (lane >> 4), nvec - 1);
-            const int ri = vi / heads, hi = vi - ri * heads;
+            const int ri = row_of(vi), hi = vi - ri * heads;
             dst[j] = reinterpret_cast<const uint4*>(src + (long long)ri * stride + (long long)hi * kHeadDim)[lane & 15];
         }
     };
@@ -107,6 +120,15 @@ rotate_kernel(RotArgs a) {
     if (vtile0 * 16 >= nvec) return;
     uint4 xraw[4];
     request_tile(vtile0, xraw);
+    // The position of a vector's row: needed for the cache row and for the rotary table row.  Asked for without a branch (at whose end it
+    // would be waited for, with all requests before it): where neither is wanted a word of R is read.
+    const bool want_pos = !is_query || roped;
+    auto request_pos = [&](int vtile) -> int {
+        const int row = row_of(min(vtile * 16 + i16, nvec - 1));
+        return (want_pos ? a.positions : reinterpret_cast<const int*>(a.rotation))[want_pos ? row : 0];
+    };
+    int next_pos = request_pos(vtile0);
+    if (BITS == 4 && lane < kBuckets) bucket_s[lane] = bucket_entry(lane);
 
     float rv[32];
     stage_operand_tile(x_s, raw, lane);
@@ -120,20 +142,19 @@ rotate_kernel(RotArgs a) {
     if (vtile * 16 >= nvec) break;
     const int v = vtile * 16 + i16;
     const int vc = v < nvec ? v : nvec - 1;              // clamp loads, mask stores
-    const int row = vc / heads, head = vc - row * heads;
+    const int row = row_of(vc), head = vc - row * heads;
 
-    // position of this vector's row: needed for the cache row and for the rotary table row, so it is asked for
-    // early; everything that depends on it is requested before the operands are used
-    const int pos_row = (!is_query || roped) ? a.positions[row] : 0;
-    long long crow = 0;
-    if (!is_query) {
-        if (a.token_list) crow = pos_row;                                // sequence 0, kernels.cu:1499, 1553
-        else crow = cache_row(a.block_table, a.bt_stride, a.seq_stride_rows, row, pos_row);
-    }
+    // everything that depends on the position is requested before the operands are used
+    const int pos_row = next_pos;
+    const bool paged = !is_query && !a.token_list && a.block_table != nullptr;
+    const int page = (paged ? a.block_table : reinterpret_cast<const int*>(a.rotation))[paged ? (long long)row * a.bt_stride + pos_row / kPageTokens : 0];
     // ---- B operand: the tile's vectors through LDS
     lds_barrier();                                        // the reads of the previous tile (or of R) are done
     stage_operand_tile(x_s, xraw, lane);
-    if (it + 1 < a.nper) request_tile(vtile + 1, xraw);   // clamped to the last vector: never out of bounds
+    if (it + 1 < a.nper) {                                // clamped to the last vector: never out of bounds
+        request_tile(vtile + 1, xraw);
+        next_pos = request_pos(vtile + 1);
+    }
     lds_barrier();
     float xv[32];
     read_operand_tile(x_s, lane, xv);
@@ -152,10 +173,10 @@ rotate_kernel(RotArgs a) {
 
     // ---- optional producers: per-head RMSNorm (kernels.cu:880-923), then rotary embedding (927-961),
     // each rounded to fp16 as the in-place kernels of the reference leave it
-    if (PROD && a.seg_weight[seg]) {
+    if (PROD && weight) {
 #pragma clang fp contract(off)      // (x * rms) * w: two fp32 roundings, then the one to fp16
         const float rms = 1.0f / sqrtf(rotation_tree_sum_sq(xv) / (float)kHeadDim + a.eps);
-        const uint4* wsrc = reinterpret_cast<const uint4*>(a.seg_weight[seg]);
+        const uint4* wsrc = reinterpret_cast<const uint4*>(weight);
 #pragma unroll
         for (int q = 0; q < 16; q++) {
             const uint4 wp = wsrc[q];
@@ -197,25 +218,18 @@ rotate_kernel(RotArgs a) {
         continue;
     }
 
-    // ---- quantize the lane's 4 consecutive coordinates d0 + 4kk .. +3 and pack (low field first)
+    // ---- quantize the lane's 4 consecutive coordinates d0 + 4kk .. +3, pack (low field first) and store them
     uint32_t packed = 0;
 #pragma unroll
-    for (int r = 0; r < 4; r++) packed |= (uint32_t)turbo_quantize(acc[r], BITS) << (r * BITS);
-    // gather the four lanes of a vector (kk = 0..3) into the kk == 0 lane
-    constexpr int PB = 4 * BITS;                                  // bits per lane
-    uint32_t p1 = (uint32_t)__shfl((int)packed, i16 + 16, 64);
-    uint32_t p2 = (uint32_t)__shfl((int)packed, i16 + 32, 64);
-    uint32_t p3 = (uint32_t)__shfl((int)packed, i16 + 48, 64);
-    if (kk == 0 && v < nvec) {
+    for (int r = 0; r < 4; r++) packed |= bucket_quantize<BITS>(bucket_s, acc[r]) << (r * BITS);
+    if (v < nvec) {
+        const long long crow = a.token_list ? pos_row                                   // sequence 0, kernels.cu:1499, 1553
+                               : paged ? (long long)page * kPageTokens + pos_row % kPageTokens : (long long)row * a.seq_stride_rows + pos_row;
         constexpr int BPH = kHeadDim * BITS / 8;                  // bytes per head: 64 or 32
-        uint8_t* dst = a.seg_codes[seg] + (crow * a.num_kv_heads + head) * BPH + dblk * (2 * BITS);
-        if (BITS == 4) {
-            uint2 o = {packed | (p1 << PB), p2 | (p3 << PB)};
-            *reinterpret_cast<uint2*>(dst) = o;                   // 16 codes = 8 bytes
-        } else {
-            *reinterpret_cast<uint32_t*>(dst) = packed | (p1 << PB) | (p2 << (2 * PB)) | (p3 << (3 * PB));
-        }
-        if (dblk == 0) a.seg_norms[seg][crow * a.num_kv_heads + head] = (half_t)sqrtf(n2 + 1e-12f);
+        uint8_t* dst = codes + (crow * a.num_kv_heads + head) * BPH + dblk * (2 * BITS) + kk * (BITS / 2);
+        if (BITS == 4) *reinterpret_cast<uint16_t*>(dst) = (uint16_t)packed;
+        else *dst = (uint8_t)packed;
+        if (dblk == 0 && kk == 0) norms[crow * a.num_kv_heads + head] = (half_t)sqrtf(n2 + 1e-12f);
     }
     }   // tiles of this wave
 }
@@ -225,7 +239,7 @@ void launch_rotate(const RotArgs& args, int bits, hipStream_t s) {
     // tiles of 16 vectors per wave: one while the launch is small, more once there are far more tiles than
     // the GPU holds waves
     long long tiles = 0;
-    for (int i = 0; i < a.nseg; i++) tiles += (a.seg_nvec[i] + 15) / 16;
+    for (int i = 0; i < a.nseg; i++) tiles += (a.seg[i].nvec + 15) / 16;
     constexpr long long kWantUnits = 16384;               // 64 single-wave workgroups per CU
     int nper = (int)((tiles * 8 + kWantUnits - 1) / kWantUnits);
     if (nper < 1) nper = 1;
@@ -233,13 +247,13 @@ void launch_rotate(const RotArgs& args, int bits, hipStream_t s) {
     a.nper = nper;
     int units = 0;
     for (int i = 0; i < a.nseg; i++) {
-        const int t = (a.seg_nvec[i] + 15) / 16;
-        a.seg_units[i] = (t + nper - 1) / nper * 8;
-        units += a.seg_units[i];
+        const int t = (a.seg[i].nvec + 15) / 16;
+        a.seg[i].units = (t + nper - 1) / nper * 8;
+        units += a.seg[i].units;
     }
     if (units <= 0) return;
     bool prod = false;
-    for (int i = 0; i < a.nseg; i++) prod = prod || a.seg_weight[i] != nullptr || a.seg_rope[i] != 0;
+    for (int i = 0; i < a.nseg; i++) prod = prod || a.seg[i].weight != nullptr || a.seg[i].rope != 0;
     if (bits == 4) {
         if (prod) hipLaunchKernelGGL((rotate_kernel<4, true>), dim3(units), dim3(kWave), 0, s, a);
         else hipLaunchKernelGGL((rotate_kernel<4, false>), dim3(units), dim3(kWave), 0, s, a);
@@ -254,49 +268,55 @@ void launch_rotate(const RotArgs& args, int bits, hipStream_t s) {
 // f_c = exp(m_c - max_c m_c): the log-sum-exp merge of the split partials, the
 // normalisation of kernels.cu:1746 and the rotate-back of kernels.cu:1769-1775.
 // A workgroup of 8 waves takes 16 (sequence, head) vectors: all threads merge into LDS,
-// then wave w produces output coordinates [16w, 16w+16) with 32 fp32 MFMAs
-// (v_mfma_f32_16x16x4_f32; A = merged vectors from LDS, B = a column block of R).
+// then wave w produces output coordinates [16w, 16w+16) with 8 fp16 MFMAs (A = merged vectors from LDS, B = a column block of R).
+// R lies in LDS as in memory and a wave's columns of it come out by transposing reads (four rows of 16 halves, four lanes to a row, lane ln
+// gets column ln); the merged vectors enter as fp16 value and remainder, every product exact in the fp32 accumulator.
 constexpr int kMergeVecs = 16;
-constexpr int kMergeStride = kHeadDim + 4;     // floats per LDS row: conflict-free 16-byte reads
+constexpr int kMergeRow = 2 * kHeadDim + 16;   // bytes per LDS row of merged halves: no bank twice in 16-byte reads
+constexpr int kMergeRot = 2 * kHeadDim + 32;   // and of R
 
 __global__ void __launch_bounds__(8 * kWave)
 merge_rotate_kernel(AttnArgs a, int nper) {
-    __shared__ __attribute__((aligned(16))) float o_s[kMergeVecs][kMergeStride];
+    __shared__ __attribute__((aligned(16))) char o_s[2][kMergeVecs * kMergeRow];
+    __shared__ __attribute__((aligned(16))) char r_s[kHeadDim * kMergeRot];
+    asm volatile("" :: "s"(a.rotation), "s"(a.positions), "s"(a.ws), "s"(a.ws_stride), "s"(a.num_heads), "s"(a.G), "s"(a.nsplit), "s"(a.max_slots),
+                 "s"(a.pos_mode), "s"(a.pos_scalar), "s"(a.slots_from_ws), "s"(a.m_log2), "s"(nper), "s"(a.out), "s"(a.q_stride));
     const int tid = threadIdx.x;
     const int wave = tid / kWave, lane = tid % kWave;
     const int i16 = lane & 15, kk = lane >> 4;
     const int total = a.G * a.num_heads;
-
-    // B operand first (its loads overlap the merge): R[32kk + s][16*wave + i16], s = 0..31
-    uint16_t rb[32];
-    {
-        const uint16_t* rp = reinterpret_cast<const uint16_t*>(a.rotation) + (32 * kk) * kHeadDim + 16 * wave + i16;
+    uint32x4_t rot[4];
 #pragma unroll
-        for (int s = 0; s < 32; s++) rb[s] = rp[s * kHeadDim];
-    }
+    for (int r = 0; r < 4; r++) rot[r] = reinterpret_cast<const uint32x4_t*>(a.rotation)[tid + 512 * r];
+    const int room = max(a.max_slots, a.nsplit);
+    const bool heads_pow2 = (a.num_heads & (a.num_heads - 1)) == 0;
+    const int heads_log2 = __builtin_ctz(a.num_heads);
+    auto row_of = [&](int v) -> int { return heads_pow2 ? v >> heads_log2 : v / a.num_heads; };
 
     // A workgroup keeps its block of R and walks nper tiles of 16 vectors (1 in a decode step, more for a prompt).
     for (int it = 0; it < nper; it++) {
     const int v0 = (blockIdx.x * nper + it) * kMergeVecs;
     if (v0 >= total) break;
-    if (it > 0) __syncthreads();                      // the previous tile's vectors have been read
+    if (it > 0) lds_barrier();                        // the previous tile's vectors have been read
 
     // ---- merge: thread -> (vector tid/32, coordinates 4*(tid%32) .. +3)
     {
         const int vl = tid >> 5, k4 = (tid & 31) * 4;
         const int vv = min(v0 + vl, total - 1);
-        const int g = vv / a.num_heads;
-        int n;
-        if (a.pos_mode == kPosArray) n = a.positions[g] + 1;
-        else if (a.pos_mode == kPosScalar) n = a.pos_scalar + 1;
-        else n = g + 1;
+        const int g = row_of(vv);
+        // (both loads without a branch, at whose end they would be waited for: a word of R where there is no array of positions)
+        const bool array = a.pos_mode == kPosArray;
+        const int pos_read = (array ? a.positions : reinterpret_cast<const int*>(a.rotation))[array ? g : 0];
         const float* part = a.ws + (long long)vv * a.ws_stride;
-        const int nseg = a.slots_from_ws ? reinterpret_cast<const int*>(part)[kHeadDim + 2] : 0;
+        const int nseg_read = reinterpret_cast<const int*>(part)[kHeadDim + 2];
         // Slots in blocks with every load of a block issued before the first use, so a block costs one memory
         // latency rather than one per slot; the running maximum is carried across blocks as in an online softmax.
         float mg = -1e30f, lsum = 0.0f;
         float4 av = {0.f, 0.f, 0.f, 0.f};
-        const int nslots = nseg > 0 ? nseg : a.nsplit;
+        int n = 0, nslots = room;
+        // (a sequence of at least nsplit tiles has a token in every slot; only shorter ones are asked slot by slot, a division each)
+        bool some_empty = false, any_empty = false;
+        const float to_log2 = a.m_log2 ? 1.0f : kLog2e;
         auto merge_block = [&](int c0, auto width) {
             constexpr int W = decltype(width)::value;
             float mc[W], lc[W];
@@ -304,26 +324,40 @@ merge_rotate_kernel(AttnArgs a, int nper) {
 #pragma unroll
             for (int j = 0; j < W; j++) {
                 const int c = c0 + j;
-                // else: no workgroup wrote this slot.  With a fixed split (a decode step) the address does not wait
-                // for that answer, which needs the position, a load of its own: every slot the workspace has room
-                // for may be read, and what it holds is dropped below.
-                const bool live = c < nslots && (nseg > 0 || chunk_nonempty(n, c, a.nsplit));
-                const bool fetch = a.slots_from_ws ? live : c < a.max_slots;
-                const float* pc = part + (long long)(fetch ? c : 0) * kPartialFloats;
-                mc[j] = pc[kHeadDim];
-                lc[j] = pc[kHeadDim + 1];
+                // (perhaps no workgroup wrote this slot.)  The address does not wait for that answer, which needs the position or the
+                // workspace's own count, a load in front of these: every slot the workspace has room for may be read, and what it
+                // holds is dropped below.
+                const float* pc = part + (long long)(c < room ? c : 0) * kPartialFloats;
+                const float2 ml = *reinterpret_cast<const float2*>(pc + kHeadDim);
+                mc[j] = ml.x;
+                lc[j] = ml.y;
                 pc4[j] = *reinterpret_cast<const float4*>(pc + k4);
-                if (!live) { mc[j] = -1e30f; lc[j] = 0.0f; pc4[j] = float4{0.f, 0.f, 0.f, 0.f}; }
             }
+            if (c0 == 0) {
+                n = (array ? pos_read : a.pos_mode == kPosScalar ? a.pos_scalar : g) + 1;
+                const int nseg = a.slots_from_ws ? nseg_read : 0;
+                nslots = nseg > 0 ? nseg : a.nsplit;
+                some_empty = nseg == 0 && ((unsigned)(n + 31) >> 5) < (unsigned)a.nsplit;
+                any_empty = __any(some_empty);
+            }
+            unsigned live = nslots >= c0 + W ? (1u << W) - 1u : nslots > c0 ? (1u << (nslots - c0)) - 1u : 0u;
+            if (any_empty) {
+#pragma unroll 1
+                for (int j = 0; j < W; j++)
+                    if (some_empty && c0 + j < nslots && !chunk_nonempty(n, c0 + j, a.nsplit)) live &= ~(1u << j);
+            }
+#pragma unroll
+            for (int j = 0; j < W; j++)
+                if (!(live >> j & 1u)) { mc[j] = -1e30f; lc[j] = 0.0f; pc4[j] = float4{0.f, 0.f, 0.f, 0.f}; }
             float mb = mg;
 #pragma unroll
             for (int j = 0; j < W; j++) mb = fmaxf(mb, mc[j]);
-            const float fo = a.m_log2 ? __builtin_amdgcn_exp2f(mg - mb) : __expf(mg - mb);
+            const float fo = __builtin_amdgcn_exp2f((mg - mb) * to_log2);
             lsum *= fo; av.x *= fo; av.y *= fo; av.z *= fo; av.w *= fo;
             mg = mb;
 #pragma unroll
             for (int j = 0; j < W; j++) {
-                float f = a.m_log2 ? __builtin_amdgcn_exp2f(mc[j] - mg) : __expf(mc[j] - mg);
+                float f = __builtin_amdgcn_exp2f((mc[j] - mg) * to_log2);
                 lsum = __builtin_fmaf(lc[j], f, lsum);
                 av.x = __builtin_fmaf(pc4[j].x, f, av.x);
                 av.y = __builtin_fmaf(pc4[j].y, f, av.y);
@@ -331,38 +365,51 @@ merge_rotate_kernel(AttnArgs a, int nper) {
                 av.w = __builtin_fmaf(pc4[j].w, f, av.w);
             }
         };
-        // blocks of 8; a count of 1 or 2 (a prompt: the workspace says how many) is not padded to 8 loads
-        if (nslots <= 2) {
+        // blocks of 8 (the first one before anything is known of the count); room for 1 or 2 (a prompt) is not padded to 8 loads
+        if (room <= 2) {
             merge_block(0, std::integral_constant<int, 2>{});
         } else {
-            for (int c0 = 0; c0 < nslots; c0 += 8) merge_block(c0, std::integral_constant<int, 8>{});
+            merge_block(0, std::integral_constant<int, 8>{});
+            for (int c0 = 8; c0 < nslots; c0 += 8) merge_block(c0, std::integral_constant<int, 8>{});
         }
         const float inv = 1.0f / (lsum + 1e-8f);
-        float4 o4 = {av.x * inv, av.y * inv, av.z * inv, av.w * inv};
-        *reinterpret_cast<float4*>(&o_s[vl][k4]) = o4;
-    }
-    __syncthreads();
-
-    // ---- out[vector][d] = sum_k o[vector][k] R[k][d]; lane group kk owns k in [32kk, 32kk+32)
-    float4_t acc = {0.f, 0.f, 0.f, 0.f};
-    const float* orow = &o_s[i16][32 * kk];
+        const float o4[4] = {av.x * inv, av.y * inv, av.z * inv, av.w * inv};
+        half4_t hi, lo;
 #pragma unroll
-    for (int s4 = 0; s4 < 8; s4++) {
-        float4 o4 = *reinterpret_cast<const float4*>(orow + 4 * s4);
-        const float ov[4] = {o4.x, o4.y, o4.z, o4.w};
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            union { uint16_t u; half_t h; } cv;
-            cv.u = rb[4 * s4 + j];
-            acc = __builtin_amdgcn_mfma_f32_16x16x4f32(ov[j], (float)cv.h, acc, 0, 0, 0);
+        for (int i = 0; i < 4; i++) {
+            hi[i] = (half_t)o4[i];
+            lo[i] = (half_t)(o4[i] - (float)hi[i]);
         }
+        *reinterpret_cast<half4_t*>(&o_s[0][vl * kMergeRow + 2 * k4]) = hi;
+        *reinterpret_cast<half4_t*>(&o_s[1][vl * kMergeRow + 2 * k4]) = lo;
+    }
+    if (it == 0) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) *reinterpret_cast<uint32x4_t*>(&r_s[((tid >> 4) + 32 * r) * kMergeRot + 16 * (tid & 15)]) = rot[r];
+    }
+    lds_barrier();
+
+    // ---- out[vector][d] = sum_k o[vector][k] R[k][d]; lane group kk owns k = 32 t + 8 kk ..
+    float4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int t = 0; t < 4; t++) {
+        const half8_t hi = *reinterpret_cast<const half8_t*>(&o_s[0][i16 * kMergeRow + 64 * t + 16 * kk]);
+        const half8_t lo = *reinterpret_cast<const half8_t*>(&o_s[1][i16 * kMergeRow + 64 * t + 16 * kk]);
+        typedef __fp16 __attribute__((ext_vector_type(4))) fp16x4_t;
+        typedef __attribute__((address_space(3))) fp16x4_t* lds_fp16x4_t;
+        const char* at = &r_s[(32 * t + 8 * kk + (i16 >> 2)) * kMergeRot + 32 * wave + 8 * (i16 & 3)];
+        union { fp16x4_t q[2]; half8_t h; } rt;
+        rt.q[0] = __builtin_amdgcn_ds_read_tr16_b64_v4f16((lds_fp16x4_t)at);
+        rt.q[1] = __builtin_amdgcn_ds_read_tr16_b64_v4f16((lds_fp16x4_t)(at + 4 * kMergeRot));
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi, rt.h, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(lo, rt.h, acc, 0, 0, 0);
     }
     // lane holds out[vector 4kk + r][d = 16*wave + i16]
 #pragma unroll
     for (int r = 0; r < 4; r++) {
         const int vv = v0 + 4 * kk + r;
         if (vv < total) {
-            const int g = vv / a.num_heads, head = vv - g * a.num_heads;
+            const int g = row_of(vv), head = vv - g * a.num_heads;
             const long long col = (long long)head * kHeadDim + 16 * wave + i16;
             half_t h = (half_t)acc[r];
             if (a.gate) h = gated(h, a.gate[(long long)g * a.gate_stride + col]);

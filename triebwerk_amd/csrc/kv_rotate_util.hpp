@@ -72,8 +72,11 @@ __device__ __forceinline__ float rotation_tree_sum_sq(const float (&xv)[32]) {
         float a0 = t[0] + t[4], a1 = t[1] + t[5], a2 = t[2] + t[6], a3 = t[3] + t[7];
         float b0 = a0 + a2, b1 = a1 + a3;
         float c = b0 + b1;                                   // c_kk of the tree
-        float d = c + __shfl_xor(c, 32, 64);                 // offset 2: c0+c2 | c1+c3
-        sgrp[w] = d + __shfl_xor(d, 16, 64);                 // offset 1: d0+d1
+        // offset 2: c0+c2 | c1+c3, offset 1: d0+d1, on the vector ALU (a shuffle is a trip through LDS)
+        lane_pair_t p = __builtin_amdgcn_permlane32_swap(__float_as_uint(c), __float_as_uint(c), false, false);
+        const float d = __uint_as_float(p[0]) + __uint_as_float(p[1]);
+        p = __builtin_amdgcn_permlane16_swap(__float_as_uint(d), __float_as_uint(d), false, false);
+        sgrp[w] = __uint_as_float(p[0]) + __uint_as_float(p[1]);
     }
     return (sgrp[0] + sgrp[2]) + (sgrp[1] + sgrp[3]);
 }
