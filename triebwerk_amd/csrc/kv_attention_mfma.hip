@@ -636,6 +636,10 @@ bool takes_prefill_tq(const AttnArgs& a) {
 }
 }  // namespace
 
+bool attention_takes_operands(const AttnArgs& a) {                   // KV heads in pairs: two heads per wave
+    return !takes_prefill_tq(a) && !prefill_mfma_usable(a) && attention_variant() != 3 && attention_pair_usable(a);
+}
+
 // Shape check; with rotate_query also q_rot = R q (kernels.cu:1671-1681) into the workspace.
 bool prepare_attention_mfma(AttnArgs& a, hipStream_t s, bool rotate_query) {
     const int R = a.num_heads / a.num_kv_heads;
@@ -666,6 +670,7 @@ bool prepare_attention_mfma(AttnArgs& a, hipStream_t s, bool rotate_query) {
         r.qrot = a.qrot;
         r.qrot_stride = a.ws_stride;
         r.q_scale = attention_mfma_q_scale(a.bits);
+        r.q_operands = attention_takes_operands(a) ? 1 : 0;
         launch_rotate(r, a.bits, s);
     }
     return true;
@@ -682,7 +687,7 @@ bool launch_attention_mfma_scan(const AttnArgs& a, hipStream_t s) {
         launch_prefill_mfma_scan(a, s);
         return false;
     }
-    if (attention_variant() != 3 && attention_pair_usable(a)) {      // KV heads in pairs: two heads per wave
+    if (attention_takes_operands(a)) {
         launch_attention_pair_scan(a, s);
         return false;
     }

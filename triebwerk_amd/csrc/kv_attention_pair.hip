@@ -30,6 +30,9 @@ attention_pair_kernel(AttnArgs a, int total_items, int hgroups, int group_waves)
     __shared__ int pre_s[kMaxBalanceSeqs + 1];
     __shared__ int bal_s[2];
 
+    asm volatile("" :: "s"(a.k), "s"(a.v), "s"(a.k_norms), "s"(a.v_norms), "s"(a.positions), "s"(a.ws), "s"(a.qrot), "s"(a.ws_stride), "s"(a.G),
+                 "s"(a.num_heads), "s"(a.num_kv_heads), "s"(a.nsplit), "s"(a.max_slots), "s"(a.balance), "s"(a.seq_stride_rows), "s"(a.pos_mode),
+                 "s"(a.pos_scalar), "s"(total_items), "s"(hgroups), "s"(group_waves), "s"(a.block_table), "s"(a.bt_stride));
     const int tid = threadIdx.x;
     const int nthreads = blockDim.x;
     const int wave = uniform(tid / kWave), lane = tid % kWave;
@@ -204,21 +207,13 @@ attention_pair_kernel(AttnArgs a, int total_items, int hgroups, int group_waves)
             const int tl = gg < a.G ? (seq_pos(a, gg) + 1 + 31) >> 5 : 0;
             if (gg < a.G) { tmin = min(tmin, tl); tmax = max(tmax, tl); }
             if (wave == 0) {
-                int inc = tl;
-#pragma unroll
-                for (int off = 1; off < kWave; off <<= 1) {
-                    int up = __shfl_up(inc, off, 64);
-                    if (lane >= off) inc += up;
-                }
+                const int inc = wave_prefix_sum(tl);
                 if (gg < a.G) pre_s[gg + 1] = carry + inc;
-                carry += __shfl(inc, kWave - 1, 64);
+                carry += __builtin_amdgcn_readlane(inc, kWave - 1);
             }
         }
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) {
-            tmin = min(tmin, __shfl_xor(tmin, off, 64));
-            tmax = max(tmax, __shfl_xor(tmax, off, 64));
-        }
+        tmin = wave_over(tmin, [](int x, int y) { return min(x, y); });
+        tmax = wave_over(tmax, [](int x, int y) { return max(x, y); });
         balanced = uniform((tmax - tmin) * 8 > tmax ? 1 : 0) != 0;   // even chunks serve (nearly) equal lengths better
         if (wave == 0 && lane == 0) {
             pre_s[0] = 0;
@@ -232,16 +227,19 @@ attention_pair_kernel(AttnArgs a, int total_items, int hgroups, int group_waves)
     const int item_step = (int)gridDim.x * ngroups;
     int item = (int)blockIdx.x * ngroups + grp;
     bool ready = false;          // the item is decoded, holds tokens, and its first loads are issued
+    PairState<R> S;
+    auto load_query = [&]() {
+        S.load_query_operands(L, [&](int i, int part, int p) {
+            return reinterpret_cast<const uint4*>(a.qrot + ((long long)g * a.num_heads + (long long)h * R + i) * a.ws_stride) + 16 * part + p;
+        });
+    };
     if (!balanced && item < total_items && decode(item)) {
+        load_query();
         issue_first();
         ready = true;
     }
-    // ---- dequantization table, once per workgroup
-    build_centroid_table<BITS, true>(tab_s, kAlpha, tid, nthreads);
-    for (int i = tid; i < kPairScanWaves * 16 * 32 / 2; i += nthreads) reinterpret_cast<uint32_t*>(p_s)[i] = 0u;
-    __syncthreads();             // the only workgroup-wide barrier; every wave reaches it
-
-    if (balanced) {
+    if (balanced) {              // (the same for every wave of the workgroup: all looked at the same lengths)
+        lds_barrier();           // wave 0's prefix of tiles is there
         bal_quota = bal_s[0];
         bal_gb = (int)blockIdx.x * ngroups + grp;
         const long long start = (long long)bal_gb * bal_quota;
@@ -253,26 +251,35 @@ attention_pair_kernel(AttnArgs a, int total_items, int hgroups, int group_waves)
             if (pre_s[mid] <= bal_cur) lo = mid; else hi = mid;
         }
         bal_g = lo;
+        if (next_piece()) {
+            load_query();
+            issue_first();
+            ready = true;
+        }
     }
+    // ---- dequantization table, once per workgroup
+    build_centroid_table<BITS, true>(tab_s, kAlpha, tid, nthreads);
+    for (int i = tid; i < kPairScanWaves * 16 * 32 / 2; i += nthreads) reinterpret_cast<uint32_t*>(p_s)[i] = 0u;
+    lds_barrier();               // the last workgroup-wide barrier; every wave reaches it, its first loads in flight
 
-    PairState<R> S;
     for (;;) {
         if (balanced) {
-            if (!next_piece()) break;
-            issue_first();
+            if (!ready) {
+                if (!next_piece()) break;
+                load_query();
+                issue_first();
+            }
         } else {
             if (item >= total_items) break;
             if (!ready) {
                 if (!decode(item)) { item += item_step; continue; }   // uniform over the wave
+                load_query();
                 issue_first();
             }
-            ready = false;
             item += item_step;
         }
+        ready = false;
         S.reset();
-        S.load_query(L, [&](int i) -> const float* {
-            return a.qrot + ((long long)g * a.num_heads + (long long)h * R + i) * a.ws_stride;
-        });
 
         for (int tile = t0; tile < t1; tile += 32) {
             const bool more = tile + 32 < t1;

@@ -131,6 +131,27 @@ __device__ __forceinline__ float quarter_sum(float v) {
     w = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
     return __uint_as_float(w[0]) + __uint_as_float(w[1]);
 }
+// op over all lanes, in every lane; and the sum over this lane and those below it: DPP and lane swaps, no trip through LDS
+template <class Op>
+__device__ __forceinline__ int wave_over(int v, Op op) {
+    v = op(v, __builtin_amdgcn_mov_dpp(v, 0xB1, 0xf, 0xf, true));        // 1, 2 apart
+    v = op(v, __builtin_amdgcn_mov_dpp(v, 0x4E, 0xf, 0xf, true));
+    v = op(v, __builtin_amdgcn_mov_dpp(v, 0x141, 0xf, 0xf, true));       // the other quad, mirrored, then the other eight
+    v = op(v, __builtin_amdgcn_mov_dpp(v, 0x140, 0xf, 0xf, true));
+    lane_pair_t w = __builtin_amdgcn_permlane16_swap((unsigned)v, (unsigned)v, false, false);
+    v = op((int)w[0], (int)w[1]);
+    w = __builtin_amdgcn_permlane32_swap((unsigned)v, (unsigned)v, false, false);
+    return op((int)w[0], (int)w[1]);
+}
+__device__ __forceinline__ int wave_prefix_sum(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);      // row_shr 1, 2, 4, 8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);      // lane 15 to the next row, lane 31 to the upper half
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
+    return v;
+}
 __device__ __forceinline__ float wave_max(float v) {
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));

@@ -153,6 +153,7 @@ struct RotArgs {
     int token_list;              // 1: source row r goes to cache row positions[r] of sequence 0
     int num_kv_heads;
     float* qrot;                 // query output: vector v at qrot + v * qrot_stride (fp32)
+    int q_operands;              // instead of the floats 128 halves of fp16 values and 128 of what rounding left over (attention_takes_operands)
     long long qrot_stride;
     float q_scale;
     // producers of the segments that have them
@@ -384,6 +385,8 @@ int prefill_form();
 // 4-bit decode scan whose waves take two KV heads each and read whole cache lines (kv_attention_pair.hip); same
 // workspace, partials and merge as attention_mfma_kernel
 bool attention_pair_usable(const AttnArgs& a);
+// will launch_attention_mfma_scan run it: then the rotated queries are left as operands
+bool attention_takes_operands(const AttnArgs& a);
 void launch_attention_pair_scan(const AttnArgs& a, hipStream_t s);
 // test hook (tw_kv_debug_set_attention_variant): 0 automatic, 1 vector-ALU kernels, 2 MFMA kernels, 3 MFMA kernels
 // with one KV head per wave also where the 4-bit scan would give a wave two

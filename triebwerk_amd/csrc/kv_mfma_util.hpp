@@ -130,27 +130,34 @@ inline PrefillChoice choose_prefill_form(const PrefillForm* forms, int nforms, d
 
 // The dequantization table of the MFMA scans, built by the nthreads threads of a workgroup: entry e (a cache byte)
 // fills 256 bytes with replicas of its centroids as fp16 -- 4 bit: 64 replicas of (low code, high code); 2 bit: 32
-// replicas of the byte's four codes, in their own order (NATURAL) or as 0, 2, 1, 3.  The centroids come out of a
-// register by wave shuffle (lane c holds centroid c, scaled): indexing the constant arrays with a per-lane index is a
-// dependent memory load per look-up, microseconds for this loop.  Lower lanes run at least as many rounds as higher
-// ones, so the lanes the shuffles read (0..15) are active whenever any lane is.
+// replicas of the byte's four codes, in their own order (NATURAL) or as 0, 2, 1, 3.  nthreads: whole waves.  The four entries a
+// wave fills in a round share their upper four bits and start at a multiple of four: the upper centroids come out of a register by
+// v_readlane (lane c holds centroid c, scaled), the lower ones out of four shuffles made once.  (Indexing the constant arrays with
+// a per-lane index is a dependent memory load per look-up, a shuffle per entry and round a trip through LDS each.)
 template <int BITS, bool NATURAL>
 __device__ __forceinline__ void build_centroid_table(uint32_t* tab_s, float alpha, int tid, int nthreads) {
-    const int lane = tid & 63;
+    const int lane = tid & 63, wave = uniform(tid >> 6), nwaves = nthreads >> 6;
     const float cent_lane = alpha * centroid_of<BITS>(lane);
-    auto cent = [&](int c) -> half_t { return (half_t)__shfl(cent_lane, c, 64); };
-    for (int i = tid * 4; i < kTableWords; i += nthreads * 4) {
-        const int e = i >> 6;
-        if constexpr (BITS == 4) {
-            half2_t p = {cent(e & 15), cent(e >> 4)};
+    auto cent_of = [&](int c) -> half_t {                    // c uniform over the wave
+        return (half_t)__builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, cent_lane), c));
+    };
+    if constexpr (BITS == 4) {
+        half_t lo[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) lo[j] = (half_t)__shfl(cent_lane, 4 * j + (lane >> 4), 64);
+        for (int e = 4 * wave; e < 256; e += 4 * nwaves) {   // this thread: entry e + lane / 16, 16 bytes of it
+            const int j = (e >> 2) & 3;
+            half2_t p = {j == 0 ? lo[0] : j == 1 ? lo[1] : j == 2 ? lo[2] : lo[3], cent_of(e >> 4)};
             const uint32_t w = *reinterpret_cast<uint32_t*>(&p);
-            *reinterpret_cast<uint4*>(&tab_s[i]) = uint4{w, w, w, w};
-        } else {
-            constexpr int f1 = NATURAL ? 2 : 4, f2 = NATURAL ? 4 : 2;
-            half2_t p0 = {cent(e & 3), cent((e >> f1) & 3)};
-            half2_t p1 = {cent((e >> f2) & 3), cent((e >> 6) & 3)};
+            *reinterpret_cast<uint4*>(&tab_s[e * 64 + lane * 4]) = uint4{w, w, w, w};
+        }
+    } else {
+        const half_t c0 = (half_t)__shfl(cent_lane, lane >> 4, 64);
+        for (int e = 4 * wave; e < 256; e += 4 * nwaves) {
+            const half_t c1 = cent_of((e >> 2) & 3), c2 = cent_of((e >> 4) & 3), c3 = cent_of(e >> 6);
+            half2_t p0 = {c0, NATURAL ? c1 : c2}, p1 = {NATURAL ? c2 : c1, c3};
             const uint32_t w0 = *reinterpret_cast<uint32_t*>(&p0), w1 = *reinterpret_cast<uint32_t*>(&p1);
-            *reinterpret_cast<uint4*>(&tab_s[i]) = uint4{w0, w1, w0, w1};
+            *reinterpret_cast<uint4*>(&tab_s[e * 64 + lane * 4]) = uint4{w0, w1, w0, w1};
         }
     }
 }

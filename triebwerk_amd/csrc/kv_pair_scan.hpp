@@ -136,35 +136,14 @@ struct PairState {
 #pragma unroll
         for (int r = 0; r < R; r++) { m_run[r] = kNegBig; l_run[r] = 0.0f; }
     }
-    // The same from operands: piece(i, part, p) -> 16-byte piece p of the 128 halves of query head i, part 0 their fp16 values and 1 what
-    // rounding left over.  (160 instructions less per wave than making them here from floats; the operand rows m with
+    // q_rot of the pair's query heads (i = hd * R + r, 0 <= i < 2 R) from operands: piece(i, part, p) -> 16-byte piece p of the 128 halves of query head i, part 0 their fp16 values and 1 what
+    // rounding left over.  (160 instructions less per wave than making them here from floats.  The operand rows m with
     // m % 4 >= R repeat a head, their scores are not read.)
     template <class Lane, class PieceOf>
     __device__ __forceinline__ void load_query_operands(const Lane& L, PieceOf piece_of) {
         const int m = L.pn & 7, head = (m >> 2) * R + ((m & 3) < R ? (m & 3) : R - 1);
 #pragma unroll
         for (int j = 0; j < 4; j++) aq[j] = __builtin_bit_cast(half8_t, *piece_of(head, L.pn >> 3, 4 * L.pkg + j));
-    }
-    // q_rot of the pair's query heads: row(i) -> the 128 floats of query head i (i = hd * R + r, 0 <= i < 2 R)
-    template <class Lane, class RowOf>
-    __device__ __forceinline__ void load_query(const Lane& L, RowOf row_of) {
-        const int m = L.pn & 7;                                // operand row m (and m + 8): head m / 4, query head m % 4
-        const bool lo_part = (L.pn & 8) != 0;
-        const bool live = (m & 3) < R;
-        const float* qr = row_of(live ? (m >> 2) * R + (m & 3) : 0) + 32 * L.pkg;
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            float4 v0 = *reinterpret_cast<const float4*>(qr + 8 * j);
-            float4 v1 = *reinterpret_cast<const float4*>(qr + 8 * j + 4);
-            float v[8] = {v0.x, v0.y, v0.z, v0.w, v1.x, v1.y, v1.z, v1.w};
-#pragma unroll
-            for (int i = 0; i < 8; i++) {
-                float x = live ? v[i] : 0.0f;
-                half_t hi = (half_t)x;
-                half_t lo = (half_t)(x - (float)hi);
-                aq[j][i] = lo_part ? lo : hi;
-            }
-        }
     }
 };
 

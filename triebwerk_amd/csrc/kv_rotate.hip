@@ -211,9 +211,21 @@ rotate_kernel(RotArgs a) {
 
     if (is_query) {
         if (v < nvec) {
-            float* dst = a.qrot + (long long)v * a.qrot_stride + dblk * 16 + 4 * kk;
-            float4 o = {acc[0] * a.q_scale, acc[1] * a.q_scale, acc[2] * a.q_scale, acc[3] * a.q_scale};
-            *reinterpret_cast<float4*>(dst) = o;
+            float* dst = a.qrot + (long long)v * a.qrot_stride;
+            const float o[4] = {acc[0] * a.q_scale, acc[1] * a.q_scale, acc[2] * a.q_scale, acc[3] * a.q_scale};
+            if (a.q_operands) {
+                half4_t hi, lo;
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    hi[r] = (half_t)o[r];
+                    lo[r] = (half_t)(o[r] - (float)hi[r]);
+                }
+                half4_t* ops = reinterpret_cast<half4_t*>(dst) + dblk * 4 + kk;
+                ops[0] = hi;
+                ops[kHeadDim / 4] = lo;
+            } else {
+                *reinterpret_cast<float4*>(dst + dblk * 16 + 4 * kk) = float4{o[0], o[1], o[2], o[3]};
+            }
         }
         continue;
     }
