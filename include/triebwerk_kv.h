@@ -333,7 +333,8 @@ typedef struct tw_layer_step_args {
                                 * only these calls touch (every call leaves them zero): with them, the one-launch step
                                 * of a compressed layer may give a sequence's context to a power of two up to 64 workgroups
                                 * when the batch alone leaves compute units idle (their sums meet in `scratch`: as many as
-                                * 132 floats each fit max_seq_len).  Calls that share tickets must not overlap.  Decode
+                                * 132 floats each fit max_seq_len), and the chunks of an fp16 layer's contexts merge in its
+                                * launch.  Calls that share tickets must not overlap.  Decode
                                 * step only. */
 } tw_layer_step_args;
 void tw_layer_attention_step(const tw_layer_step_args* args, hipStream_t s);

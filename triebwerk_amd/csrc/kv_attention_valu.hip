@@ -93,12 +93,28 @@ __device__ __forceinline__ void store_head(const AttnArgs& a, int g, int head, i
     a.out[(long long)g * a.q_stride + (long long)head * kHeadDim + d] = h;
 }
 
+// sum over the eight lanes of a token's head (the lanes 8i .. 8i+7 of a wave), in every one of them: lane ^ 1, lane ^ 2
+// and the mirror image within the eight, as DPP operands of the additions
+__device__ __forceinline__ float sum_8_lanes(float v) {
+    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0xB1, 0xf, 0xf, true));
+    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x4E, 0xf, 0xf, true));
+    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x141, 0xf, 0xf, true));
+    return v;
+}
+
 // APPEND (fp16 cache, batch decode): the token at positions[g] is not in the cache yet; its rows are a.k_new and
 // a.v_new, read from there by whichever lane meets that token and stored into the cache by the workgroup whose
 // chunk holds it (the one of the KV head's first query-head tile).
-template <int MODE, int RT, bool APPEND>
+// SHARED (fp16 cache, one query-head tile per KV head): the chunks of a sequence are merged by whichever of their workgroups draws the
+// last ticket, as decode_fused_kernel's shares are (device-scope stores of the sums, acknowledged before the ticket; no fence), instead of
+// by a launch of its own.
+template <int MODE, int RT, bool APPEND, bool SHARED = false>
 __global__ void __launch_bounds__(kAttnThreads)
 attention_valu_kernel(AttnArgs a) {
+    static_assert(!SHARED || MODE == 0, "the fp16 step");
+    asm volatile("" :: "s"(a.q), "s"(a.k), "s"(a.v), "s"(a.positions), "s"(a.num_heads), "s"(a.num_kv_heads), "s"(a.nsplit), "s"(a.seq_stride_rows),
+                 "s"(a.q_stride), "s"(a.pos_mode), "s"(a.block_table), "s"(APPEND ? a.k_new : nullptr), "s"(APPEND ? a.v_new : nullptr),
+                 "s"(APPEND ? a.kv_new_stride : 0));
     __shared__ float q_s[RT][kHeadDim];
     __shared__ float red_s[kAttnWaves][RT][kHeadDim];
     __shared__ float ml_s[kAttnWaves][RT][2];
@@ -121,7 +137,7 @@ attention_valu_kernel(AttnArgs a) {
     const int n = seq_pos(a, g) + 1;
     int t0, t1;
     chunk_range(n, chunk, a.nsplit, t0, t1);
-    if (t0 >= t1) return;                       // uniform for the workgroup
+    if (!SHARED && t0 >= t1) return;            // uniform for the workgroup (SHARED: an empty chunk draws its ticket)
 
     // fp16 rows of a contiguous cache come in through buffer loads with the non-temporal hint (the eight lanes of a
     // token take one whole 128-byte line per instruction; written as an ordinary load beside the load of the appended
@@ -141,13 +157,6 @@ attention_valu_kernel(AttnArgs a) {
     if (APPEND) {
         k_fresh = a.k_new + (long long)g * a.kv_new_stride + (long long)h * kHeadDim;
         v_fresh = a.v_new + (long long)g * a.kv_new_stride + (long long)h * kHeadDim;
-        if (t0 <= n - 1 && n - 1 < t1 && blockIdx.y % subs == 0 && tid < 32) {      // 16 pieces of 16 bytes each for K and V
-            const long long row = cache_row(a.block_table, a.bt_stride, a.seq_stride_rows, g, n - 1);
-            const half_t* src = (tid < 16 ? k_fresh : v_fresh) + 8 * (tid & 15);
-            half_t* cache = reinterpret_cast<half_t*>(const_cast<void*>(tid < 16 ? a.k : a.v));
-            half_t* dst = cache + (row * a.num_kv_heads + h) * kHeadDim + 8 * (tid & 15);
-            *reinterpret_cast<uint4*>(dst) = *reinterpret_cast<const uint4*>(src);
-        }
     }
 
     // ---- the workgroup's sums
@@ -172,14 +181,39 @@ attention_valu_kernel(AttnArgs a) {
 #pragma unroll
         for (int e = 0; e < E; e++) acc[r][e] *= f;
         // sum over the token streams of the wave (lanes with equal c)
+        if constexpr (LPT == 8) {
+            // halved at each step: the lanes' upper half sums values e + 8, their odd rows e + 4; then the two streams of a row, 8 lanes
+            // apart (28 vector instructions for the head; 48 cross-lane reads through LDS before)
+            float v[8], w[4];
 #pragma unroll
-        for (int off = LPT; off < 64; off <<= 1) {
-            l[r] += __shfl_xor(l[r], off, 64);
+            for (int e = 0; e < 8; e++) {
+                const lane_pair_t p = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc[r][e]), __float_as_uint(acc[r][(e + 8) % E]), false, false);
+                v[e] = __uint_as_float(p[0]) + __uint_as_float(p[1]);
+            }
 #pragma unroll
-            for (int e = 0; e < E; e++) acc[r][e] += __shfl_xor(acc[r][e], off, 64);
+            for (int e = 0; e < 4; e++) {
+                const lane_pair_t p = __builtin_amdgcn_permlane16_swap(__float_as_uint(v[e]), __float_as_uint(v[e + 4]), false, false);
+                w[e] = __uint_as_float(p[0]) + __uint_as_float(p[1]);
+            }
+            const int e0 = 8 * (lane >> 5) + 4 * ((lane >> 4) & 1);
+#pragma unroll
+            for (int e = 0; e < 4; e++) {
+                w[e] += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, w[e]), 0x128, 0xf, 0xf, true));
+                if ((lane & 8) == 0) red_s[wave][r][lane_dim<MODE>(c, e0 + e)] = w[e];
+            }
+            l[r] += __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, l[r]), 0x128, 0xf, 0xf, true));
+            l[r] = quarter_sum(l[r]);
+            if (lane == 0) ml_s[wave][r][1] = l[r];
+        } else {
+#pragma unroll
+            for (int off = LPT; off < 64; off <<= 1) {
+                l[r] += __shfl_xor(l[r], off, 64);
+#pragma unroll
+                for (int e = 0; e < E; e++) acc[r][e] += __shfl_xor(acc[r][e], off, 64);
+            }
         }
     }
-    if (qd == 0) {
+    if (LPT != 8 && qd == 0) {
 #pragma unroll
         for (int r = 0; r < RT; r++) {
 #pragma unroll
@@ -201,16 +235,68 @@ attention_valu_kernel(AttnArgs a) {
         if (a.nsplit > 1) {
             float* part = a.ws + ((long long)g * a.num_heads + head0 + r) * a.ws_stride +
                           (long long)chunk * kPartialFloats;
-            part[d] = av;
-            if (d == 0) {
-                part[kHeadDim] = mg;
-                part[kHeadDim + 1] = lv;
+            if constexpr (SHARED) {
+                __hip_atomic_store(part + d, av, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (d < 2) __hip_atomic_store(part + kHeadDim + d, d == 0 ? mg : lv, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            } else {
+                part[d] = av;
+                if (d == 0) {
+                    part[kHeadDim] = mg;
+                    part[kHeadDim + 1] = lv;
+                }
             }
         } else {
             q_s[r][d] = av * (1.0f / (lv + 1e-8f));   // kernels.cu:1746
         }
     }
-    if (a.nsplit > 1) return;
+    };
+    // ---- SHARED: the last of the sequence's chunks merges them; false for the others
+    auto merge_shared = [&]() -> bool {
+        __shared__ unsigned last_s;
+        unsigned* ticket = a.tickets + (long long)g * a.num_kv_heads + h;
+        __builtin_amdgcn_s_waitcnt(0);          // every store of this wave has been acknowledged
+        __syncthreads();
+        if (tid == 0) last_s = __hip_atomic_fetch_add(ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)a.nsplit - 1u ? 1u : 0u;
+        __syncthreads();
+        if (!last_s) return false;              // uniform over the workgroup
+        if (tid == 0) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);     // for the next launch
+        const bool all_live = ((unsigned)(n + 31) >> 5) >= (unsigned)a.nsplit;
+        for (int idx = tid; idx < RT * kHeadDim; idx += kAttnThreads) {
+            const int r = idx / kHeadDim, d = idx % kHeadDim;
+            const float* part = a.ws + ((long long)g * a.num_heads + head0 + r) * a.ws_stride;
+            float mg = kNegBig, lsum = 0.0f, av = 0.0f;
+            for (int c0 = 0; c0 < a.nsplit; c0 += 8) {       // eight chunks' loads in flight at a time, in a fixed order
+                float mc[8], lc[8], vc[8];
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+                    const float* pc = part + (long long)min(c0 + j, a.nsplit - 1) * kPartialFloats;
+                    mc[j] = __hip_atomic_load(pc + kHeadDim, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    lc[j] = __hip_atomic_load(pc + kHeadDim + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                    vc[j] = __hip_atomic_load(pc + d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                }
+                float mb = mg;
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+                    const int cc = c0 + j;
+                    const bool live = cc < a.nsplit && (all_live || chunk_nonempty(n, cc, a.nsplit));     // no workgroup wrote the others
+                    if (!live) { mc[j] = kNegBig; lc[j] = 0.0f; vc[j] = 0.0f; }
+                    mb = fmaxf(mb, mc[j]);
+                }
+                const float fo = __expf(mg - mb);
+                lsum *= fo; av *= fo;
+                mg = mb;
+#pragma unroll
+                for (int j = 0; j < 8; j++) {
+                    const float f = __expf(mc[j] - mg);
+                    lsum = __builtin_fmaf(lc[j], f, lsum);
+                    av = __builtin_fmaf(vc[j], f, av);
+                }
+            }
+            q_s[r][d] = av * (1.0f / (lsum + 1e-8f));        // kernels.cu:1746
+        }
+        return true;
+    };
+    auto store_heads = [&]() {
     __syncthreads();
     for (int idx = tid; idx < RT * kHeadDim; idx += kAttnThreads) {
         int r = idx / kHeadDim, d = idx % kHeadDim;
@@ -226,7 +312,7 @@ attention_valu_kernel(AttnArgs a) {
         const int t_end = APPEND ? min(t1, n - 1) : t1;
         const bool has_fresh = APPEND && t0 <= n - 1 && n - 1 < t1;
         Row kf, vf;
-        if (has_fresh) {
+        if (APPEND) {                            // (every chunk asks: a load in a branch is waited for at the branch's end)
 #pragma unroll
             for (int j = 0; j < 2; j++) {
                 kf.u[j] = *reinterpret_cast<const uint32x4_t*>(k_fresh + 64 * j + 8 * c);
@@ -260,13 +346,8 @@ attention_valu_kernel(AttnArgs a) {
             l[r] = 0.0f;
             const half_t* qh = a.q + (long long)g * a.q_stride + (long long)(head0 + r) * kHeadDim;
             Row qr;
-            if ((reinterpret_cast<uintptr_t>(qh) & 15u) == 0) {      // uniform
 #pragma unroll
-                for (int j = 0; j < 2; j++) qr.u[j] = *reinterpret_cast<const uint32x4_t*>(qh + 64 * j + 8 * c);
-            } else {
-#pragma unroll
-                for (int e = 0; e < E; e++) qr.h[e / 8][e % 8] = qh[lane_dim<MODE>(c, e)];
-            }
+            for (int j = 0; j < 2; j++) __builtin_memcpy(&qr.u[j], qh + 64 * j + 8 * c, 16);       // (q rows of any alignment)
 #pragma unroll
             for (int e = 0; e < E; e++) { qreg[r][e] = (float)qr.h[e / 8][e % 8]; acc[r][e] = 0.0f; }
         }
@@ -278,8 +359,7 @@ attention_valu_kernel(AttnArgs a) {
                 float dot = 0.0f;
 #pragma unroll
                 for (int e = 0; e < E; e++) dot = __builtin_fmaf(qreg[r][e], (float)kt.h[e / 8][e % 8], dot);
-#pragma unroll
-                for (int off = 1; off < LPT; off <<= 1) dot += __shfl_xor(dot, off, 64);
+                dot = sum_8_lanes(dot);
                 s[r] = dot * scale;
             }
             if (!valid) return;
@@ -305,7 +385,21 @@ attention_valu_kernel(AttnArgs a) {
             kr = kn; vr = vn;
         }
         if (has_fresh && wave == 0) token(kf, vf, qd == 0);
-        finish(acc, m, l);
+        if (has_fresh && blockIdx.y % subs == 0 && tid < 8) {        // lane c of the first token holds pieces c and 8 + c of both rows
+            const long long row = cache_row(a.block_table, a.bt_stride, a.seq_stride_rows, g, n - 1);
+            const long long at = (row * a.num_kv_heads + h) * kHeadDim + 8 * c;
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                *reinterpret_cast<uint32x4_t*>(reinterpret_cast<half_t*>(const_cast<void*>(a.k)) + at + 64 * j) = kf.u[j];
+                *reinterpret_cast<uint32x4_t*>(reinterpret_cast<half_t*>(const_cast<void*>(a.v)) + at + 64 * j) = vf.u[j];
+            }
+        }
+        if (!SHARED || t0 < t1) finish(acc, m, l);
+        if constexpr (SHARED) {
+            if (merge_shared()) store_heads();
+        } else {
+            if (a.nsplit <= 1) store_heads();
+        }
         return;
     } else {
     // ---- compressed cache: the query rotated, q_rot = R q (kernels.cu:1671-1681)
@@ -378,6 +472,7 @@ attention_valu_kernel(AttnArgs a) {
     }
 
     finish(acc, m, l);
+    if (a.nsplit <= 1) store_heads();
     }
 }
 
@@ -399,15 +494,6 @@ constexpr int kRowThreads = kRowWaves * kWave;
 constexpr int kRowHeads = 8;               // KV heads per workgroup = lanes / 8
 constexpr int kRowUnit = 8;                // tokens: one per wave
 union Half8Bits { uint32x4_t u; half8_t h; half2_t p[4]; };
-
-// sum over the eight lanes of a token's head (the lanes 8i .. 8i+7 of a wave), in every one of them: lane ^ 1, lane ^ 2
-// and the mirror image within the eight, as DPP operands of the additions
-__device__ __forceinline__ float sum_8_lanes(float v) {
-    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0xB1, 0xf, 0xf, true));
-    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x4E, 0xf, 0xf, true));
-    v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x141, 0xf, 0xf, true));
-    return v;
-}
 
 // LAYERS: the items of every layer of a step, one workgroup each, in even chunks: the launches' starts, ends and merges are paid once
 // a step, and most batches need no cutting, hence no merge.  us a step, layer by layer -> at once (16 heads over 8 KV heads, 28
@@ -786,12 +872,26 @@ attention_merge_kernel(AttnArgs a, long long out_layer) {
     if (grp == 0) store_head(a, g, head, d, o_s[0]);
 }
 
+// Whether attention_valu_kernel's chunks meet by tickets and need no merge launch
+bool attention_valu_merges(const AttnArgs& a) {
+    const int group = a.num_heads / a.num_kv_heads;
+    return a.bits == 0 && !a.even_chunks && a.tickets && a.nsplit > 1 && a.pos_mode == kPosArray && (group == 1 || group == 2 || group == 4);
+}
+
 template <int MODE>
 static void launch_valu_mode(const AttnArgs& a, hipStream_t s) {
     const int group = a.num_heads / a.num_kv_heads;
     const int rt = (group % 4 == 0) ? 4 : (group % 2 == 0) ? 2 : 1;
     dim3 grid(a.nsplit, a.num_kv_heads * (group / rt), a.G);
     dim3 block(kAttnThreads);
+    if (MODE == 0 && attention_valu_merges(a)) {
+#define TW_SHARED(AP_) do { if (rt == 4) launch_scan_kernel(attention_valu_kernel<0, 4, AP_, true>, grid, block, s, a); \
+                            else if (rt == 2) launch_scan_kernel(attention_valu_kernel<0, 2, AP_, true>, grid, block, s, a); \
+                            else launch_scan_kernel(attention_valu_kernel<0, 1, AP_, true>, grid, block, s, a); } while (0)
+        if (a.k_new) TW_SHARED(true); else TW_SHARED(false);
+#undef TW_SHARED
+        return;
+    }
     if (MODE == 0 && a.k_new) {
         if (rt == 4) launch_scan_kernel(attention_valu_kernel<0, 4, true>, grid, block, s, a);
         else if (rt == 2) launch_scan_kernel(attention_valu_kernel<0, 2, true>, grid, block, s, a);

@@ -153,14 +153,10 @@ __device__ __forceinline__ int wave_prefix_sum(int v) {
     return v;
 }
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v = fmaxf(v, __shfl_xor(v, off, 64));
-    return v;
+    return __int_as_float(wave_over(__float_as_int(v), [](int x, int y) { return __float_as_int(fmaxf(__int_as_float(x), __int_as_float(y))); }));
 }
 __device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-    return v;
+    return __int_as_float(wave_over(__float_as_int(v), [](int x, int y) { return __float_as_int(__int_as_float(x) + __int_as_float(y)); }));
 }
 
 // compute units of the current device (cached; kv_attention_mfma.hip)

@@ -194,6 +194,7 @@ struct AttnArgs {
     int m_log2;             // partial maxima are in base-2 units
     int balance;            // MFMA scan: may cut the batch by tiles instead of by sequence (ragged lengths)
     int max_slots;          // partials the workspace holds per (sequence, head): >= nsplit
+    unsigned* tickets;      // fp16 step: G * num_kv_heads words, zero before and after a launch, or NULL
     int slots_from_ws;      // merge: the spare word of partial 0 holds the number of partials (0: even chunks)
     int even_chunks;        // the chunks are the fp16 whole-row scan's (even_chunk_range), not chunk_range's
     // optional output gate (gated attention, kernels.cu:2987-2995): out = half(float(half(out)) * sigmoid(gate))
@@ -210,6 +211,7 @@ struct AttnArgs {
 constexpr int kPartialFloats = kHeadDim + 4;  // acc[128], running max, running sum, 2 pad (16-byte rows)
 
 void launch_attention_valu(const AttnArgs& a, hipStream_t s);
+bool attention_valu_merges(const AttnArgs& a);     // its chunks merge themselves (AttnArgs::tickets): no launch_attention_merge
 // fp16 cache: will launch_attention_valu run the kernel whose waves read whole rows (eight KV heads)?  Its workgroups
 // have eight waves that share one chunk, so the split planner gives it more and smaller chunks.
 bool attention_rows_usable(const AttnArgs& a);
