@@ -260,40 +260,61 @@ attention_valu_kernel(AttnArgs a) {
         __syncthreads();
         if (!last_s) return false;              // uniform over the workgroup
         if (tid == 0) __hip_atomic_store(ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);     // for the next launch
+        // Wave r weighs the chunks of query head r, a lane each (at most 64), while the threads' own sums are on the way, eight or sixteen
+        // at a time.  (With the weights eight chunks after eight, 53 chunks of one sequence cost 3 us more.)
+        __shared__ float w_s[RT][kWave];
+        __shared__ float lsum_s[RT];
         const bool all_live = ((unsigned)(n + 31) >> 5) >= (unsigned)a.nsplit;
-        for (int idx = tid; idx < RT * kHeadDim; idx += kAttnThreads) {
-            const int r = idx / kHeadDim, d = idx % kHeadDim;
-            const float* part = a.ws + ((long long)g * a.num_heads + head0 + r) * a.ws_stride;
-            float mg = kNegBig, lsum = 0.0f, av = 0.0f;
-            for (int c0 = 0; c0 < a.nsplit; c0 += 8) {       // eight chunks' loads in flight at a time, in a fixed order
-                float mc[8], lc[8], vc[8];
+        const float* mine = a.ws + ((long long)g * a.num_heads + head0 + min(wave, RT - 1)) * a.ws_stride;
+        const float* at = mine + (long long)min(lane, a.nsplit - 1) * kPartialFloats + kHeadDim;
+        const float m_raw = __hip_atomic_load(at, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const float l_raw = __hip_atomic_load(at + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        auto merge = [&](auto width) {
+            constexpr int W = decltype(width)::value;
+            constexpr int kOwn = (RT * kHeadDim + kAttnThreads - 1) / kAttnThreads;       // outputs of a thread
+            float vc[kOwn][W], av[kOwn];
+            auto load = [&](int c0) {
 #pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    const float* pc = part + (long long)min(c0 + j, a.nsplit - 1) * kPartialFloats;
-                    mc[j] = __hip_atomic_load(pc + kHeadDim, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    lc[j] = __hip_atomic_load(pc + kHeadDim + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    vc[j] = __hip_atomic_load(pc + d, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                for (int o = 0; o < kOwn; o++) {
+                    const int idx = min(tid + o * kAttnThreads, RT * kHeadDim - 1);
+                    const float* part = a.ws + ((long long)g * a.num_heads + head0 + idx / kHeadDim) * a.ws_stride + idx % kHeadDim;
+#pragma unroll
+                    for (int j = 0; j < W; j++)
+                        vc[o][j] = __hip_atomic_load(part + (long long)min(c0 + j, a.nsplit - 1) * kPartialFloats, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
                 }
-                float mb = mg;
+            };
+            load(0);
+            if (wave < RT) {
+                const bool live = lane < a.nsplit && (all_live || chunk_nonempty(n, lane, a.nsplit));      // no workgroup wrote the others
+                const float mg = wave_max(live ? m_raw : kNegBig);
+                const float w = live ? __expf(m_raw - mg) : 0.0f;
+                w_s[wave][lane] = w;
+                const float ls = wave_sum(live ? l_raw * w : 0.0f);
+                if (lane == 0) lsum_s[wave] = ls;
+            }
+            __syncthreads();
 #pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    const int cc = c0 + j;
-                    const bool live = cc < a.nsplit && (all_live || chunk_nonempty(n, cc, a.nsplit));     // no workgroup wrote the others
-                    if (!live) { mc[j] = kNegBig; lc[j] = 0.0f; vc[j] = 0.0f; }
-                    mb = fmaxf(mb, mc[j]);
-                }
-                const float fo = __expf(mg - mb);
-                lsum *= fo; av *= fo;
-                mg = mb;
+            for (int o = 0; o < kOwn; o++) av[o] = 0.0f;
+            for (int c0 = 0; c0 < a.nsplit; c0 += W) {
+                if (c0 > 0) load(c0);
 #pragma unroll
-                for (int j = 0; j < 8; j++) {
-                    const float f = __expf(mc[j] - mg);
-                    lsum = __builtin_fmaf(lc[j], f, lsum);
-                    av = __builtin_fmaf(vc[j], f, av);
+                for (int o = 0; o < kOwn; o++) {
+                    const int r = min(tid + o * kAttnThreads, RT * kHeadDim - 1) / kHeadDim;
+#pragma unroll
+                    for (int j = 0; j < W; j++) {
+                        const float w = c0 + j < a.nsplit ? w_s[r][min(c0 + j, kWave - 1)] : 0.0f;
+                        av[o] = w != 0.0f ? __builtin_fmaf(vc[o][j], w, av[o]) : av[o];
+                    }
                 }
             }
-            q_s[r][d] = av * (1.0f / (lsum + 1e-8f));        // kernels.cu:1746
-        }
+#pragma unroll
+            for (int o = 0; o < kOwn; o++) {
+                const int idx = tid + o * kAttnThreads;
+                if (idx < RT * kHeadDim) q_s[idx / kHeadDim][idx % kHeadDim] = av[o] * (1.0f / (lsum_s[idx / kHeadDim] + 1e-8f));       // kernels.cu:1746
+            }
+        };
+        if (a.nsplit <= 8) merge(std::integral_constant<int, 8>{});
+        else merge(std::integral_constant<int, 16>{});
         return true;
     };
     auto store_heads = [&]() {
@@ -875,7 +896,7 @@ attention_merge_kernel(AttnArgs a, long long out_layer) {
 // Whether attention_valu_kernel's chunks meet by tickets and need no merge launch
 bool attention_valu_merges(const AttnArgs& a) {
     const int group = a.num_heads / a.num_kv_heads;
-    return a.bits == 0 && !a.even_chunks && a.tickets && a.nsplit > 1 && a.pos_mode == kPosArray && (group == 1 || group == 2 || group == 4);
+    return a.bits == 0 && !a.even_chunks && a.tickets && a.nsplit > 1 && a.nsplit <= kWave && a.pos_mode == kPosArray && (group == 1 || group == 2 || group == 4);
 }
 
 template <int MODE>
