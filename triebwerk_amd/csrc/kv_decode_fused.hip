@@ -982,22 +982,32 @@ static bool pairs_fit(int bits, int R, int hkw) {
 }
 bool decode_fused_pairs(const AttnArgs& a, int hkw) { return pairs_fit(a.bits, a.num_heads / a.num_kv_heads, hkw); }
 
-// The measured figures behind the estimates below, fitted to 15400 launches on MI355X: batches 1 to 256, contexts 300 to 16000,
-// 1 to 16 KV heads, GQA groups of 1, 2 and 4, both widths, every shape of a launch with 1 to 64 shares and the three launches,
-// captured steps over as many layers as the last cache level does not hold (or a model's 28).  Single estimates are 7 to 9 %
-// off (root mean square); what counts is the choice: it is the fastest of the forms or within 3 % of it at 2354 of 2455
-// sizes, within 10 % at all but 8.  Fitted to 70 % of the sizes it does as well on the other 30 %.  (The table before had one rate
-// for the three launches' scan whatever the number of KV heads: with 2 of them the scan streams 3 TB/s and not 7, and
-// 192 sequences of 8192 tokens took 190 us in the form chosen, 80 in the best.)
+// The measured figures behind the estimates below, fitted on MI355X.  One launch or three: 1330 steps of 1 to 256 sequences, 64 to
+// 16000 tokens, 1 to 16 KV heads, GQA groups of 1, 2 and 4, both widths, each in every shape of a launch with 1 to 32 shares and in
+// three launches, over as many layers as the last cache level does not hold (12 at most).  Single estimates are 6 % off (root mean
+// square); what counts is the choice: it is the fastest of the forms or within 3 % of it at 91 % of the sizes and within 10 % at
+// 99 %; fitted to 70 % of them, at 88 and 98 % of the other 30 %.  (Before the launches' starts and ends were made shorter, with the
+// figures of then and a tile for every wave of a share: 71 % and 93 %.)  A rate above what the memory gives is one the last
+// cache level helped with.  Every layer in one
+// launch: 11100 steps of 4 to 36 layers in each of the four shapes, choice within 3 % of the fastest at 91 %, 10 % at 98 %
+// of the sizes that were not fitted to (85 and 95 % before).  64 shares and ragged batches keep figures from earlier fits.
 namespace {
 constexpr PlanConstants kPlanTable[] = {
-    {"gfx950", {7.45, 9.43}, {0.144, 0.125}, {8.37, 8.19},
-     {{{1.88, 2.05, 2.48}, {1.35, 1.48, 1.93}}, {{1.99, 2, 2.81}, {1.69, 1.77, 2.23}}},
-     {{{5.02e6, 7.61e6, 7.92e6, 7.69e6}, {3.62e6, 5.33e6, 5.91e6, 6.37e6}},
-      {{3.39e6, 7.65e6, 6.64e6, 7.18e6}, {1.83e6, 3.96e6, 5.99e6, 5.26e6}}}, {0, 3.34, 3.1, 3.28, 3.63, 4.02, 6.8},
-     {{19.7, 21.1, 24.9}, {19.1, 20, 22.6}}, {{6.67e6, 6.96e6, 6.32e6}, {5.91e6, 5.02e6, 4.94e6}}, {{1.16, 1.27, 0.588}, {1.12, 0.672, 1.14}}, {1.74, 1.51}, 0.000277, 16.2, 0.774e-3, 0.629,
-     6.68, {11.38, 9.34}, 0.0225, {{1.38, 1.44, 1.96}, {0.967, 0.986, 1.40}}, 0.713, {{6.34e6, 6.97e6, 7.01e6}, {4.44e6, 4.74e6, 5.04e6}}, 0.268},
+    {"gfx950", {3.79, 4.8}, {0.231, 0.125}, {7.12, 5.02},
+     {{{2.63, 2, 2.66}, {1.38, 1.69, 1.63}}, {{2.51, 2.26, 3.47}, {1.81, 2.3, 4.19}}},
+     {{{3.18e6, 6.29e6, 7.87e6, 9e6}, {2.62e6, 4.13e6, 5.51e6, 8.74e6}},
+      {{2.78e6, 5.32e6, 8.6e6, 9e6}, {1.33e6, 3.41e6, 5.28e6, 8.97e6}}}, {0, 3.75, 3.95, 2.32, 2.14, 2.1, 4.7},
+     {{17.1, 17, 26}, {19.7, 16.7, 22.7}}, {{6.33e6, 7.06e6, 6.96e6}, {6.54e6, 4.88e6, 4.86e6}}, {{2.64, 1.69, 2.17}, {1.34, 1.41, 1.22}}, {2.56, 2.18}, 0.0004, 16.2, 0.774e-3, 0.629,
+     2.5, {8.81, 7.67}, 0.01, {{1.39, 1.42, 1.29}, {1.08, 1.1, 1.09}}, 0.80, {{7.91e6, 8.52e6, 8.41e6}, {7.93e6, 8.41e6, 9.97e6}}, 0.112},
 };
+// Where scratch has no room for partials: fitted when both forms took longer, kept because the line that they draw decides
+// which steps stay in fp32.
+constexpr PlanConstants kWithoutRoom = {
+    "", {7.45, 9.43}, {0.144, 0.125}, {8.37, 8.19},
+    {{{1.88, 2.05, 2.48}, {1.35, 1.48, 1.93}}, {{1.99, 2, 2.81}, {1.69, 1.77, 2.23}}},
+    {{{5.02e6, 7.61e6, 7.92e6, 7.69e6}, {3.62e6, 5.33e6, 5.91e6, 6.37e6}}, {{3.39e6, 7.65e6, 6.64e6, 7.18e6}, {1.83e6, 3.96e6, 5.99e6, 5.26e6}}},
+    {}, {{19.7, 21.1, 24.9}, {19.1, 20, 22.6}}, {{6.67e6, 6.96e6, 6.32e6}, {5.91e6, 5.02e6, 4.94e6}},
+    {{1.16, 1.27, 0.588}, {1.12, 0.672, 1.14}}, {1.74, 1.51}, 0.000277, 0, 0, 0, 0, {}, 0, {}, 0, {}, 0};
 }  // namespace
 const PlanConstants& plan_constants() {
     static const PlanConstants* chosen = nullptr;
@@ -1016,6 +1026,8 @@ const PlanConstants& plan_constants() {
     return *chosen;
 }
 
+const PlanConstants& plan_constants_without_room() { return kWithoutRoom; }
+
 // Microseconds one launch takes: the workgroups run in rounds of one per CU.  A round costs the cube-root sum of its waves'
 // tiles of the longest sequence, one after the other, and of its bytes at the rate the chip streams them in this pattern: a
 // workgroup with one KV head reads half lines, and unless the batch is a multiple of 8 the other half may be fetched
@@ -1028,8 +1040,8 @@ static double bytes_per_token(int bits) { return bits == 4 ? 132.0 : 68.0; }    
 static double cube_sum(double x, double y) { return std::cbrt(x * x * x + y * y * y); }
 static int log2_of(int x) { int n = 0; while (x > 1) { x >>= 1; n++; } return n; }
 
-double decode_fused_estimate_us(int G, int num_heads, int Hk, int bits, bool allow_pairs, int hkw, int shares, double ctx, double fill) {
-    const PlanConstants& pc = plan_constants();
+double decode_fused_estimate_us(int G, int num_heads, int Hk, int bits, bool allow_pairs, int hkw, int shares, double ctx, double fill,
+                                const PlanConstants& pc) {
     const double cus = compute_units();
     const int R = Hk > 0 ? num_heads / Hk : 1;
     const int w = bits == 4 ? 0 : 1;
@@ -1037,7 +1049,8 @@ double decode_fused_estimate_us(int G, int num_heads, int Hk, int bits, bool all
     const int p = pair ? 0 : 1;
     const int parts = (pair ? 2 * kPairWaves : kFusedWaves) / hkw;          // waves that share a head's tiles
     const double units = (double)G * (Hk / hkw) * shares, full = std::floor(units / cus), rest = units - full * cus;
-    const double tiles = std::ceil(std::ceil(ctx / shares / 32.0) / parts) * pc.tile_us[p][w][group_index(R)];
+    const double share_tiles = std::ceil(ctx / shares / 32.0);            // fewer than waves: the ones that have a tile are faster
+    const double tiles = (share_tiles >= parts ? std::ceil(share_tiles / parts) : 0.5 + 0.5 * share_tiles / parts) * pc.tile_us[p][w][group_index(R)];
     const double unit_bytes = hkw * bytes_per_token(bits) * ctx / shares * fill / pc.one_bw[G % 8 == 0 ? 0 : 1][w][log2_of(hkw)];
     double us = pc.one_fixed_us[p] + pc.one_vector_us[p] * hkw * (2 + R) + pc.handover_us[log2_of(shares)];
     us += full * cube_sum(tiles, cus * unit_bytes);
@@ -1047,8 +1060,7 @@ double decode_fused_estimate_us(int G, int num_heads, int Hk, int bits, bool all
 
 // Three launches (rotation, scan, merge) for the same step: what they cost before the scan and after it, the scan's bytes
 // at its rate or the tiles of one piece of a sequence, one after the other, and the pieces through the merge.
-double decode_three_estimate_us(int G, int num_heads, int Hk, int bits, double ctx) {
-    const PlanConstants& pc = plan_constants();
+double decode_three_estimate_us(int G, int num_heads, int Hk, int bits, double ctx, const PlanConstants& pc) {
     const int w = bits == 4 ? 0 : 1, r = group_index(num_heads / Hk);
     const bool odd = (Hk & 1) != 0;
     // as plan_splits and the scans' launches cut it: 512 (sequence, chunk) items, a group of waves each
@@ -1065,20 +1077,21 @@ double decode_three_estimate_us(int G, int num_heads, int Hk, int bits, double c
 
 // KV heads per workgroup (8, 4, 2 or 1) and shares with the smallest estimate; among equals without shares the larger number
 // of heads, whose workgroups read longer contiguous pieces of a cache row.  Shares are only taken while all workgroups
-// fit the compute units in one round and a share still has a tile for every wave.
+// fit the compute units in one round and a share still has a tile for every fourth wave (for every wave: 4 bit, 4 query heads over
+// one KV head, one sequence of 2935 tokens: 16.6 us a layer with 4 shares, 14.2 with 16).
 namespace {
 std::atomic<int> g_force_hkw{0}, g_force_shares{0};
 }  // namespace
 void decode_fused_force_shape(int hkw, int shares) { g_force_hkw.store(hkw); g_force_shares.store(shares); }
 int decode_fused_forced_hkw() { return g_force_hkw.load(); }
 
-FusedShape decode_fused_shape(int G, int num_heads, int Hk, int bits, bool allow_pairs, int max_shares, double ctx) {
+FusedShape decode_fused_shape(int G, int num_heads, int Hk, int bits, bool allow_pairs, int max_shares, double ctx, const PlanConstants& pc) {
     const int R = Hk > 0 ? num_heads / Hk : 1;
     const double cus = compute_units();
     FusedShape best{1, 1, 0.0};
     for (int c = 1; c <= 8; c <<= 1) {
         if (Hk % c != 0) continue;
-        const double us = decode_fused_estimate_us(G, num_heads, Hk, bits, allow_pairs, c, 1, ctx, 1.0);
+        const double us = decode_fused_estimate_us(G, num_heads, Hk, bits, allow_pairs, c, 1, ctx, 1.0, pc);
         if (c == 1 || us <= best.us) best = FusedShape{c, 1, us};
     }
     for (int c = 1; c <= 8 && max_shares >= 2; c <<= 1) {
@@ -1087,8 +1100,8 @@ FusedShape decode_fused_shape(int G, int num_heads, int Hk, int bits, bool allow
         const int parts = (pair ? 2 * kPairWaves : kFusedWaves) / c;          // waves (parts of the context) per head
         for (int sh = 2; sh <= kMaxShares && sh <= max_shares; sh <<= 1) {
             if ((double)G * (Hk / c) * sh > cus) continue;
-            if (ctx < 32.0 * parts * sh) continue;
-            const double us = decode_fused_estimate_us(G, num_heads, Hk, bits, allow_pairs, c, sh, ctx, 1.0);
+            if (ctx < 8.0 * parts * sh) continue;
+            const double us = decode_fused_estimate_us(G, num_heads, Hk, bits, allow_pairs, c, sh, ctx, 1.0, pc);
             if (us < best.us) best = FusedShape{c, sh, us};
         }
     }

@@ -283,17 +283,19 @@ struct PlanConstants {
     double layers_both;            // this share of the smaller of (longest unit, all units) on top of the larger
 };
 const PlanConstants& plan_constants();
+const PlanConstants& plan_constants_without_room();      // the line between one launch and three where scratch has no room for partials
 bool decode_fused_usable(const AttnArgs& a, const FusedArgs& f);
 // estimated microseconds of one launch with hkw KV heads per workgroup and `shares` workgroups per sequence and head group,
 // the longest sequence at ctx tokens and the mean one at fill * ctx
 double decode_fused_estimate_us(int G, int num_heads, int num_kv_heads, int bits, bool allow_pairs, int hkw, int shares, double ctx,
-                                double fill);
+                                double fill, const PlanConstants& pc = plan_constants());
 // estimated microseconds of the same step as three launches (rotation, scan, merge), all sequences at ctx tokens
-double decode_three_estimate_us(int G, int num_heads, int num_kv_heads, int bits, double ctx);
+double decode_three_estimate_us(int G, int num_heads, int num_kv_heads, int bits, double ctx, const PlanConstants& pc = plan_constants());
 // The launch's shape when a unit's context may be shared by up to max_shares workgroups (1: the caller has no tickets
 // or no room for the shares' sums): KV heads per workgroup, shares, and the estimate for sequences of ctx tokens.
 struct FusedShape { int hkw, shares; double us; };
-FusedShape decode_fused_shape(int G, int num_heads, int num_kv_heads, int bits, bool allow_pairs, int max_shares, double ctx);
+FusedShape decode_fused_shape(int G, int num_heads, int num_kv_heads, int bits, bool allow_pairs, int max_shares, double ctx,
+                              const PlanConstants& pc = plan_constants());
 // test hook (tw_kv_debug_set_fused_shape): force hkw and / or shares (0 = automatic)
 void decode_fused_force_shape(int hkw, int shares);
 int decode_fused_forced_hkw();
