@@ -4,15 +4,19 @@
 // rotate_kernel (kv_rotate.hip) gives every wave 16 output coordinates of its vectors and nothing to share: right for the
 // few vectors of a decode step, but each vector is then fetched, transformed, measured and regrouped eight times.  Here a
 // workgroup of four waves takes a tile of 16 vectors at a time, once:
-//   - 16 lanes to a vector, 16 bytes each: RMSNorm and rotation (K), the norm, and the unit vector into LDS as fp32,
-//     regrouped for the matrix cores (coordinate 4s + kk at kk * 32 + s); K goes back to its row as the producers leave it;
-//   - wave w rotates the tile for output coordinates 16w .. 16w + 15 and 64 + 16w ...: two chains of
-//     v_mfma_f32_16x16x4_f32 in rotate_kernel's order of k, hence its bits; codes meet in LDS and leave 16 lanes to a vector.
+//   - 16 lanes to a vector, 16 bytes each: RMSNorm and rotation (K), the norm, and the vector into LDS as the halves it is;
+//     K goes back to its row as the producers leave it;
+//   - wave w rotates the tile for output coordinates 16w .. 16w + 15 and 64 + 16w ... on v_mfma_f32_16x16x32_f16 (exact products, fp32
+//     sums).  A code is taken from those sums where no boundary between buckets lies within their bound of error, which 16 of 17
+//     blocks of 16 vectors are through with; the others repeat the sum as rotate_kernel's chain of v_mfma_f32_16x16x4_f32, hence its
+//     bits.  Codes meet in LDS and leave 16 lanes to a vector.
 // One barrier per tile: tile i is rotated while tile i + 1 is transformed and the codes of tile i - 1 are stored.
-// The matrix cores bound it: 16 x 128 x 128 products per tile at 256 fp32 operations per cycle and compute unit, 14 us for
-// the 65776 vectors of 4111 tokens and 8 KV heads.  Other workgroups of the same launch transform the queries, a
-// matter of memory alone, beside them.
-// 8192 tokens, 8 KV heads, 4 bit: 47.4 us against rotate_kernel's 79.7 (2 bit 47.4 against 70.6); 4111 tokens 28.6 against 43.
+// The chain alone was bound by the matrix cores (32 of its steps take 16 of the fp16 form's time); now the issue of the transformation
+// and of the buckets bounds it.  Launches of one stream without producers, which are few tiles, keep the chain: they wait for memory, and
+// a repeated block costs more than it saves.  Other workgroups of the same launch transform the queries, a matter of memory
+// alone, beside them.
+// The prompt step of 4111 tokens (4 layers, 16 heads over 8 KV heads, 4 bit, producers; attention included): 893 us with the
+// chain, 858 with the sums; attention's own changes take it to 842.
 
 #include <algorithm>
 #include <type_traits>

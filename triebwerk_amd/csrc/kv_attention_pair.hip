@@ -5,6 +5,8 @@
 // kv_pair_scan.hpp's: at 4 bit a wave reads whole 128-byte lines (two heads) with non-temporal loads, so the waves of a
 // group (four pairs = 8 KV heads) read whole 512-byte cache rows between them and every byte is fetched once; at 2 bit
 // a pair is half a line and the loads keep the ordinary policy.
+// A launch waits for its arguments once, then for first tile, queries and lengths together, which are asked for ahead of the table; the
+// lengths' prefix and spread over the groups run on the vector ALU (DPP), not through LDS.  The loop is bound as in kv_pair_scan.hpp.
 // Contiguous and paged layout; launched between rotate_kernel (q_rot into the workspace) and merge_rotate_kernel.
 
 #include "kv_common.hpp"

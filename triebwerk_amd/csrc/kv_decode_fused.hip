@@ -13,10 +13,10 @@
 // one KV head each, described here:
 //   1. all threads fetch the unit's vectors (K heads, V heads, query heads of the new token), 16 lanes to a vector, and
 //      fill the centroid table meanwhile; the 16 lanes apply the producers' RMSNorm and rotary embedding
-//      (kernels.cu:880-961), measure the vector and leave it in LDS.  Waves 0-7 (all 16 when the unit has more than 16
-//      vectors) then rotate the vectors exactly as rotate_kernel does -- lane i16 = vector, wave = block of 16 output
-//      coordinates, the same v_mfma_f32_16x16x4_f32 chain, so the codes have the same bits -- and store the codes in
-//      the cache, the scaled q_rot in LDS;
+//      (kernels.cu:880-961), measure the vector and leave it in LDS as halves.  Waves 0-7 (all 16 when the unit has more than 16
+//      vectors) then rotate them -- lane i16 = vector, wave = block of 16 output coordinates -- on v_mfma_f32_16x16x32_f16; codes
+//      come from those sums where their bound of error allows no other, and from rotate_kernel's v_mfma_f32_16x16x4_f32
+//      chain otherwise, so they have its bits -- and store the codes in the cache, the scaled q_rot in LDS as the scan's operands;
 //   2. after the barrier wave w scans every SPLIT-th tile of the context (SPLIT = 16 / HKW, starting at tile
 //      w / HKW) for head w % HKW with the loop of attention_mfma_kernel (the table look-ups, MFMA tiling,
 //      online softmax are described there).  All its loads are issued after the barrier: the new token's row
@@ -74,10 +74,12 @@ enum { kStep = 0, kAttend = 1, kPaged = 2 };
 // hand-over uses device-scope accesses only where they are needed -- the partial sums and the ticket -- and no
 // cache-wide fence: stores with device scope are written through to where every compute unit's device-scope loads look
 // (a release / acquire pair at device scope writes back and invalidates a whole L2 and costs 20 us per launch; this costs
-// 2.9 us with 2 shares, 3.4 with 8, 4.9 with 32: what 1 sequence of 16001 tokens, 4 bit, 16 heads over 8 KV heads, pays to have
-// 128 workgroups instead of 64 single chunks, a merge launch and a rotation launch -- 19 us per layer against 38; 4 sequences
-// of 8192 tokens 20.9 against 25.3 with 8 shares merged one after the other).
-// (Tried with SHARES: the first tile requested in the middle of the prologue as in EARLY: 4 bit within 1 %, 2 bit 5 % slower.)
+// 2 to 4 us, which is what 1 sequence of 16001 tokens, 4 bit, 16 heads over 8 KV heads, pays to have 128 workgroups and
+// more instead of 64 single chunks, a merge launch and a rotation launch -- 16 us per layer against 27).
+// A share's waves have few tiles: SHARES asks for the first one in the prologue as EARLY does.  (While the prologue still waited for
+// its loads one after the other that cost 5 % at 2 bit.)  The start and end bound a step of short contexts: every argument
+// fetched in one trip, loads without branches, fp16 sums, parts merged four at a time.  28 layers of one sequence of 16001 tokens: 18.4 us
+// a layer before, 15.8 with them (300 tokens 12.0 -> 10.2).
 // MODE (PAIR, no SHARES): kAttend is attention alone, over a cache that holds the new token already (the reference's attention
 // launcher): the unit's vectors are its queries, and the first tile is asked for in the prologue, nothing being appended.  kPaged
 // is the whole step over the paged cache: a tile is two pages, whose block-table entries are fetched a tile ahead.
@@ -982,22 +984,22 @@ static bool pairs_fit(int bits, int R, int hkw) {
 }
 bool decode_fused_pairs(const AttnArgs& a, int hkw) { return pairs_fit(a.bits, a.num_heads / a.num_kv_heads, hkw); }
 
-// The measured figures behind the estimates below, fitted on MI355X.  One launch or three: 1330 steps of 1 to 256 sequences, 64 to
+// The measured figures behind the estimates below, fitted on MI355X.  One launch or three: 1870 steps of 1 to 256 sequences, 64 to
 // 16000 tokens, 1 to 16 KV heads, GQA groups of 1, 2 and 4, both widths, each in every shape of a launch with 1 to 32 shares and in
-// three launches, over as many layers as the last cache level does not hold (12 at most).  Single estimates are 6 % off (root mean
-// square); what counts is the choice: it is the fastest of the forms or within 3 % of it at 91 % of the sizes and within 10 % at
-// 99 %; fitted to 70 % of them, at 88 and 98 % of the other 30 %.  (Before the launches' starts and ends were made shorter, with the
-// figures of then and a tile for every wave of a share: 71 % and 93 %.)  A rate above what the memory gives is one the last
+// three launches, over as many layers as the last cache level does not hold (12 at most).  What counts is the choice, not the single
+// estimate: it is the fastest of the forms or within 3 % of it at 90 % of the sizes and within 10 % at 99 %; fitted to 70 % of them,
+// at 88 and 99 % of the other 30 %.  (Before the launches' starts and ends were made shorter, with the figures of then and a tile for
+// every wave of a share: 71 % and 93 %.)  A rate above what the memory gives is one the last
 // cache level helped with.  Every layer in one
 // launch: 11100 steps of 4 to 36 layers in each of the four shapes, choice within 3 % of the fastest at 91 %, 10 % at 98 %
 // of the sizes that were not fitted to (85 and 95 % before).  64 shares and ragged batches keep figures from earlier fits.
 namespace {
 constexpr PlanConstants kPlanTable[] = {
-    {"gfx950", {3.79, 4.8}, {0.231, 0.125}, {7.12, 5.02},
-     {{{2.63, 2, 2.66}, {1.38, 1.69, 1.63}}, {{2.51, 2.26, 3.47}, {1.81, 2.3, 4.19}}},
-     {{{3.18e6, 6.29e6, 7.87e6, 9e6}, {2.62e6, 4.13e6, 5.51e6, 8.74e6}},
-      {{2.78e6, 5.32e6, 8.6e6, 9e6}, {1.33e6, 3.41e6, 5.28e6, 8.97e6}}}, {0, 3.75, 3.95, 2.32, 2.14, 2.1, 4.7},
-     {{17.1, 17, 26}, {19.7, 16.7, 22.7}}, {{6.33e6, 7.06e6, 6.96e6}, {6.54e6, 4.88e6, 4.86e6}}, {{2.64, 1.69, 2.17}, {1.34, 1.41, 1.22}}, {2.56, 2.18}, 0.0004, 16.2, 0.774e-3, 0.629,
+    {"gfx950", {2.85, 4.16}, {0.178, 0.222}, {9.47, 3.73},
+     {{{2.88, 2.11, 2.92}, {1.83, 1.99, 2.39}}, {{3.1, 1.91, 3.32}, {2.65, 2.11, 3.08}}},
+     {{{3.39e6, 7.95e6, 9e6, 9e6}, {2.2e6, 4.12e6, 5.74e6, 9e6}},
+      {{2.93e6, 5.64e6, 9e6, 8.9e6}, {1.38e6, 3.05e6, 4.88e6, 9e6}}}, {0, 4.39, 6, 2.49, 2.53, 2.59, 4.7},
+     {{17.7, 20.2, 20.1}, {18.9, 15.2, 23}}, {{7.02e6, 8e6, 8e6}, {6.97e6, 4.5e6, 3.8e6}}, {{3.08, 1.54, 2.62}, {1.94, 1.8, 1.79}}, {2.39, 2.66}, 0.000465, 16.2, 0.774e-3, 0.629,
      2.5, {8.81, 7.67}, 0.01, {{1.39, 1.42, 1.29}, {1.08, 1.1, 1.09}}, 0.80, {{7.91e6, 8.52e6, 8.41e6}, {7.93e6, 8.41e6, 9.97e6}}, 0.112},
 };
 // Where scratch has no room for partials: fitted when both forms took longer, kept because the line that they draw decides

@@ -31,6 +31,14 @@
 // comes in as 4 fully used 16-byte pieces per lane, is written to LDS with the halves regrouped
 // ([kk][row][s], kv_rotate_util.hpp), and each lane reads back its 32 halves as 4 x 16 bytes.
 
+//
+// What bounds both launches of a step is the chain of trips to memory and the issue of one wave (a launch is few waves a SIMD).
+// So the arguments come in one trip (an asm statement that wants them all), positions, rows and R are asked for before any is waited
+// for, the buckets are a table of pairs instead of a search, queries for attention_pair_kernel leave as the operands of
+// its matrix instructions, and the merge asks for as many slots as there can be before it knows their number and rotates back on
+// fp16 matrix instructions (value + remainder).  With the scan's own start: 8 layers of the launchers' step, 47 ragged sequences at
+// 2 bit, 397 -> 346 us; the paged step of 64 ragged sequences 580 -> 539.
+
 #include <algorithm>
 #include <type_traits>
 
