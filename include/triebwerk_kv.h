@@ -513,7 +513,7 @@ int tw_engine_decode_step(tw_engine* e, const tw_half* q, const tw_half* k, cons
 /* When the capture or the instantiation of the step's graph fails, the step is run without a graph, one line goes
  * to stderr, and so are all later steps with the same buffers (engine.cpp:2396-2410); the next change of buffers,
  * batch, arena or producers tries again.  graph_state tells what the latest decode step did: 0 run eagerly as asked,
- * 1 graph replayed, 2 run eagerly after a failed capture.  debug_fail_captures (test hook): the next n captures
+ * 1 graph replayed (or, where all layers are a few launches, the captured ones issued again), 2 run eagerly after a failed capture.  debug_fail_captures (test hook): the next n captures
  * are treated as failed after they have been recorded. */
 int tw_engine_graph_state(const tw_engine* e);
 void tw_engine_debug_fail_captures(tw_engine* e, int n);

@@ -168,8 +168,8 @@ class Engine:
             raise RuntimeError(f"broadcast_prefix failed ({rc})")
 
     def graph_state(self) -> int:
-        """What the latest decode_step did: 0 eager as asked, 1 graph replayed, 2 eager after a failed capture
-        (generate_batch decodes without a graph when the capture fails, engine.cpp:2396-2410)."""
+        """What the latest decode_step did: 0 eager as asked, 1 graph replayed (all layers at once: its launches issued again), 2 eager after a
+        failed capture (generate_batch decodes without a graph when the capture fails, engine.cpp:2396-2410)."""
         return self._lib.tw_engine_graph_state(self._h)
 
     # ---- the single-sequence state of generate() / decode_token() (engine.cpp:322-331, 394-404, 1069-1108)
