@@ -52,9 +52,9 @@ BYTES_HEAD = {0: 256, 4: 66, 2: 34}  # per (token, kv head): fp16 row | codes + 
 # Keyed by (workload, kv_bits, kernel that ran).  Counters are not read in this run: the figures belong to
 # the kernel sources whose digest is recorded with them (`python bench.py --csrc-digest` prints the current
 # one) and are only reported while the sources are still those; otherwise `traffic` is null.
-MEASURED_TRAFFIC_CSRC_DIGEST = "61b1f4a90e3ef6ba"
-MEASURED_TRAFFIC_BYTES = {("target", 4, "every layer"): 15535.0e6, ("target", 4, "one-launch"): 555.1e6, ("target", 4, "scan"): 560.8e6,
-                          ("target", 2, "every layer"): 8017.9e6, ("target", 2, "one-launch"): 286.7e6, ("target", 2, "scan"): 292.3e6,
+MEASURED_TRAFFIC_CSRC_DIGEST = "41b45191c22320d4"
+MEASURED_TRAFFIC_BYTES = {("target", 4, "every layer"): 15532.9e6, ("target", 4, "one-launch"): 555.1e6, ("target", 4, "scan"): 560.8e6,
+                          ("target", 2, "every layer"): 8015.5e6, ("target", 2, "one-launch"): 291.4e6, ("target", 2, "scan"): 292.3e6,
                           ("target", 0, "every layer"): 60191.6e6, ("target", 0, "scan"): 2154.8e6}
 TRAFFIC_SOURCE = "profiles/scan_target_hbm_traffic_pmc.txt"
 
@@ -746,14 +746,14 @@ def decode_bench(args, kv_bits, with_probe):
     launch_bytes = algorithmic_bytes(n_tokens_prof, G * Kp, L, H, Hk, kv_bits, with_append=one_launch) / (Kp * per_step)
     frac_eager = launch_bytes / (eager_kern_ms * 1e-3) * 1e-9 / HBM_PEAK_GBS     # per-launch events, eager steps
     if one_launch and use_graph:
-        # The layer step (or the step of every layer) is this one kernel, so the timed region itself is K * per_step launches of it (plus K one-block
-        # position increments): its average duration there, the launches `value` is made of, is the events' time
+        # The layer step (or the step of every layer) is this one kernel, so the timed region itself is K * per_step launches of it (and, layer by layer
+        # or on the fp16 cache, K one-block position increments): its average duration there, the launches `value` is made of, is the events' time
         # over the region divided by the launches.  (Launched one by one with events attached the same kernel
-        # reads 1-2 % longer: a replayed graph overlaps one kernel's drain with the next one's start.)
+        # reads 1-3 % longer: a step without them overlaps one kernel's drain with the next one's start.)
         kern_ms = events_ms / (K * per_step)
         launch_bytes = algorithmic_bytes(n_tokens_timed, G * K, L, H, Hk, kv_bits, with_append=True) / (K * per_step)
-        timed = (f"HIP events on the launch stream around the {K} graph-replayed steps of the timed region / ({K} x {per_step}) launches; "
-                 f"includes 1/{per_step} of a one-block positions += 1 kernel per launch")
+        timed = (f"HIP events on the launch stream around the {K} steps of the timed region / ({K} x {per_step}) launches; "
+                 f"a step taken layer by layer, or on the fp16 cache, includes a one-block positions += 1 kernel")
     else:
         kern_ms = eager_kern_ms
         timed = (f"a pair of HIP events attached to each of {Kp * per_step} eager launches of the kernel on its stream, in steps that "
