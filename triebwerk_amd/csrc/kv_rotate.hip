@@ -290,10 +290,13 @@ void launch_rotate(const RotArgs& args, int bits, hipStream_t s) {
 // A workgroup of 8 waves takes 16 (sequence, head) vectors: all threads merge into LDS,
 // then wave w produces output coordinates [16w, 16w+16) with 8 fp16 MFMAs (A = merged vectors from LDS, B = a column block of R).
 // R lies in LDS as in memory and a wave's columns of it come out by transposing reads (four rows of 16 halves, four lanes to a row, lane ln
-// gets column ln); the merged vectors enter as fp16 value and remainder, every product exact in the fp32 accumulator.
+// gets column ln).  The merged vectors enter as fp16 value and remainder, every product exact in the fp32 accumulator: o = hi + lo / 2^11 within
+// 2^-23 of itself, and within 2^-36 where it is small.  (The remainder as it is is subnormal below 2^-14 of a value: for values of 1e-4 one output in
+// five was not the half nearest to its fp32 sum, with the remainder held 2^11 times as large one in 5000, as on fp32 matrix instructions.)
 constexpr int kMergeVecs = 16;
 constexpr int kMergeRow = 2 * kHeadDim + 16;   // bytes per LDS row of merged halves: no bank twice in 16-byte reads
 constexpr int kMergeRot = 2 * kHeadDim + 32;   // and of R
+constexpr float kLowScale = 2048.0f;           // of the remainders: at most 2^-11 of a half's range before, inside it afterwards
 
 __global__ void __launch_bounds__(8 * kWave)
 merge_rotate_kernel(AttnArgs a, int nper) {
@@ -398,7 +401,7 @@ merge_rotate_kernel(AttnArgs a, int nper) {
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             hi[i] = (half_t)o4[i];
-            lo[i] = (half_t)(o4[i] - (float)hi[i]);
+            lo[i] = (half_t)((o4[i] - (float)hi[i]) * kLowScale);
         }
         *reinterpret_cast<half4_t*>(&o_s[0][vl * kMergeRow + 2 * k4]) = hi;
         *reinterpret_cast<half4_t*>(&o_s[1][vl * kMergeRow + 2 * k4]) = lo;
@@ -410,7 +413,7 @@ merge_rotate_kernel(AttnArgs a, int nper) {
     lds_barrier();
 
     // ---- out[vector][d] = sum_k o[vector][k] R[k][d]; lane group kk owns k = 32 t + 8 kk ..
-    float4_t acc = {0.f, 0.f, 0.f, 0.f};
+    float4_t acc = {0.f, 0.f, 0.f, 0.f}, low = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int t = 0; t < 4; t++) {
         const half8_t hi = *reinterpret_cast<const half8_t*>(&o_s[0][i16 * kMergeRow + 64 * t + 16 * kk]);
@@ -422,7 +425,7 @@ merge_rotate_kernel(AttnArgs a, int nper) {
         rt.q[0] = __builtin_amdgcn_ds_read_tr16_b64_v4f16((lds_fp16x4_t)at);
         rt.q[1] = __builtin_amdgcn_ds_read_tr16_b64_v4f16((lds_fp16x4_t)(at + 4 * kMergeRot));
         acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(hi, rt.h, acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(lo, rt.h, acc, 0, 0, 0);
+        low = __builtin_amdgcn_mfma_f32_16x16x32_f16(lo, rt.h, low, 0, 0, 0);
     }
     // lane holds out[vector 4kk + r][d = 16*wave + i16]
 #pragma unroll
@@ -431,7 +434,7 @@ merge_rotate_kernel(AttnArgs a, int nper) {
         if (vv < total) {
             const int g = row_of(vv), head = vv - g * a.num_heads;
             const long long col = (long long)head * kHeadDim + 16 * wave + i16;
-            half_t h = (half_t)acc[r];
+            half_t h = (half_t)__builtin_fmaf(low[r], 1.0f / kLowScale, acc[r]);
             if (a.gate) h = gated(h, a.gate[(long long)g * a.gate_stride + col]);
             a.out[(long long)g * a.q_stride + col] = h;
         }
