@@ -931,7 +931,7 @@ decode_fused_kernel(AttnArgs a, FusedArgs f) {
             }
         }
         if (vec < nv) {
-            const float inv = 1.0f / (lsum + 1e-8f);             // kernels.cu:1746
+            const float inv = kLowScale / (lsum + 1e-8f);        // kernels.cu:1746, as split_scaled wants it
             o4 = float4{av.x * inv, av.y * inv, av.z * inv, av.w * inv};
         }
         *reinterpret_cast<float4*>(&o_s[vec][k4]) = o4;
@@ -939,11 +939,11 @@ decode_fused_kernel(AttnArgs a, FusedArgs f) {
     lds_barrier();
 
     // ---- out[vector][d] = sum_k o[vector][k] R[k][d]; lane group kk owns k in [32kk, 32kk+32).  On fp16 MFMAs: R is
-    // exact in fp16, o enters as fp16 value + rounding remainder, every product is exact in the fp32 accumulator --
+    // exact in fp16, o enters as fp16 value + enlarged rounding remainder, every product is exact in the fp32 accumulators --
     // only the order of the additions differs from the reference's chain (kernels.cu:1769-1775), far inside what the
     // fp16 result resolves -- and the chain is 8 MFMAs instead of 32.
     for (int vt = wave >> 3; back && vt * 16 < nv; vt += kRotGroups) {
-        float4_t acc = {0.f, 0.f, 0.f, 0.f};
+        float4_t acc = {0.f, 0.f, 0.f, 0.f}, low = {0.f, 0.f, 0.f, 0.f};
         const float* orow = &o_s[vt * 16 + ln][32 * kg];
 #pragma unroll
         for (int st = 0; st < 4; st++) {
@@ -954,12 +954,13 @@ decode_fused_kernel(AttnArgs a, FusedArgs f) {
             union { uint16_t u[8]; half8_t h; } bm;
 #pragma unroll
             for (int i = 0; i < 8; i++) {
-                ahi[i] = (half_t)ov[i];
-                alo[i] = (half_t)(ov[i] - (float)ahi[i]);
+                half_t hi, lo;
+                split_scaled(ov[i], hi, lo);
+                ahi[i] = hi; alo[i] = lo;
                 bm.u[i] = rb[8 * st + i];
             }
             acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi, bm.h, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo, bm.h, acc, 0, 0, 0);
+            low = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo, bm.h, low, 0, 0, 0);
         }
         // lane holds out[vector vt*16 + 4kk + r][d = 16*dblk + i16]
 #pragma unroll
@@ -968,7 +969,7 @@ decode_fused_kernel(AttnArgs a, FusedArgs f) {
             if (vec < nv) {
                 const int head = hg * HKW * R + vec;
                 const long long col = (long long)head * kHeadDim + 16 * dblk + ln;
-                half_t hv = (half_t)acc[r];
+                half_t hv = (half_t)__builtin_fmaf(low[r], 1.0f / kLowScale, acc[r]);
                 if (a.gate) hv = gated(hv, a.gate[(long long)g * a.gate_stride + col]);
                 a.out[(long long)g * a.q_stride + col] = hv;
             }

@@ -324,7 +324,7 @@ decode_layers_kernel(LayersArgs a) {
     if (kParts > 1 && !kInPlace) lds_barrier();
     pair_scan_finish<R>(L, S, 1.0f / kAlpha, [&](int, int r, const float (&o)[16]) {     // dims 16 (pn % 8) .. of head hd
         float* row = kParts > 1 ? sum_s[(part * kPairs + pair) * 2 * R + L.hd * R + r] : x_s[pair * 2 * R + L.hd * R + r];
-        const float inv = kParts > 1 ? 1.0f : 1.0f / (S.l_run[r] + 1e-8f);               // kernels.cu:1746
+        const float inv = kParts > 1 ? 1.0f : kLowScale / (S.l_run[r] + 1e-8f);          // kernels.cu:1746, as split_scaled wants it
 #pragma unroll
         for (int j4 = 0; j4 < 4; j4++)
             *reinterpret_cast<float4*>(row + 16 * (L.pn & 7) + 4 * j4) = float4{o[4 * j4] * inv, o[4 * j4 + 1] * inv, o[4 * j4 + 2] * inv, o[4 * j4 + 3] * inv};
@@ -352,13 +352,13 @@ decode_layers_kernel(LayersArgs a) {
                 o.x = __builtin_fmaf(c[p].x, fs, o.x); o.y = __builtin_fmaf(c[p].y, fs, o.y);
                 o.z = __builtin_fmaf(c[p].z, fs, o.z); o.w = __builtin_fmaf(c[p].w, fs, o.w);
             }
-            const float inv = 1.0f / (l + 1e-8f);            // kernels.cu:1746
+            const float inv = kLowScale / (l + 1e-8f);       // kernels.cu:1746
             *reinterpret_cast<float4*>(&x_s[v][k4]) = float4{o.x * inv, o.y * inv, o.z * inv, o.w * inv};
         }
         lds_barrier();
     }
 
-    // ---- rotate back (as kv_decode_fused.hip): o as fp16 value + remainder, R exact in fp16
+    // ---- rotate back (as kv_decode_fused.hip): o as fp16 value + enlarged remainder, R exact in fp16
     half_t* out = a.out + layer * a.q_layer + (long long)g * a.q_stride + (long long)hg * NQ * kHeadDim;
     half8_t ahi[4], alo[4];
     const float* orow = &x_s[ln < NQ ? ln : 0][32 * kg];
@@ -368,24 +368,25 @@ decode_layers_kernel(LayersArgs a) {
         const float o8[8] = {oa.x, oa.y, oa.z, oa.w, ob.x, ob.y, ob.z, ob.w};
 #pragma unroll
         for (int i = 0; i < 8; i++) {
-            ahi[st][i] = (half_t)o8[i];
-            alo[st][i] = (half_t)(o8[i] - (float)ahi[st][i]);
+            half_t hi, lo;
+            split_scaled(o8[i], hi, lo);
+            ahi[st][i] = hi; alo[st][i] = lo;
         }
     }
 #pragma unroll
     for (int i = 0; i < kBlocks; i++) {
-        float4_t acc = {0.f, 0.f, 0.f, 0.f};
+        float4_t acc = {0.f, 0.f, 0.f, 0.f}, low = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int st = 0; st < 4; st++) {
             union { uint4 u; half8_t h; } bm;
             bm.u = rb[i][st];
             acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(ahi[st], bm.h, acc, 0, 0, 0);
-            acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo[st], bm.h, acc, 0, 0, 0);
+            low = __builtin_amdgcn_mfma_f32_16x16x32_f16(alo[st], bm.h, low, 0, 0, 0);
         }
 #pragma unroll
         for (int r = 0; r < 4; r++) {                        // out[vector 4 kg + r][16 dblk + ln]
             const int vec = 4 * kg + r;
-            if (vec < NQ) out[(long long)vec * kHeadDim + 16 * (wave + NW * i) + ln] = (half_t)acc[r];
+            if (vec < NQ) out[(long long)vec * kHeadDim + 16 * (wave + NW * i) + ln] = (half_t)__builtin_fmaf(low[r], 1.0f / kLowScale, acc[r]);
         }
     }
     if (tid == 0 && ticket == (unsigned)(a.layers * nhg) - 1u) {

@@ -290,13 +290,10 @@ void launch_rotate(const RotArgs& args, int bits, hipStream_t s) {
 // A workgroup of 8 waves takes 16 (sequence, head) vectors: all threads merge into LDS,
 // then wave w produces output coordinates [16w, 16w+16) with 8 fp16 MFMAs (A = merged vectors from LDS, B = a column block of R).
 // R lies in LDS as in memory and a wave's columns of it come out by transposing reads (four rows of 16 halves, four lanes to a row, lane ln
-// gets column ln).  The merged vectors enter as fp16 value and remainder, every product exact in the fp32 accumulator: o = hi + lo / 2^11 within
-// 2^-23 of itself, and within 2^-36 where it is small.  (The remainder as it is is subnormal below 2^-14 of a value: for values of 1e-4 one output in
-// five was not the half nearest to its fp32 sum, with the remainder held 2^11 times as large one in 5000, as on fp32 matrix instructions.)
+// gets column ln).  The merged vectors enter as fp16 value and enlarged remainder (kLowScale), every product exact in the fp32 accumulators.
 constexpr int kMergeVecs = 16;
 constexpr int kMergeRow = 2 * kHeadDim + 16;   // bytes per LDS row of merged halves: no bank twice in 16-byte reads
 constexpr int kMergeRot = 2 * kHeadDim + 32;   // and of R
-constexpr float kLowScale = 2048.0f;           // of the remainders: at most 2^-11 of a half's range before, inside it afterwards
 
 __global__ void __launch_bounds__(8 * kWave)
 merge_rotate_kernel(AttnArgs a, int nper) {
@@ -395,13 +392,14 @@ merge_rotate_kernel(AttnArgs a, int nper) {
             merge_block(0, std::integral_constant<int, 8>{});
             for (int c0 = 8; c0 < nslots; c0 += 8) merge_block(c0, std::integral_constant<int, 8>{});
         }
-        const float inv = 1.0f / (lsum + 1e-8f);
+        const float inv = kLowScale / (lsum + 1e-8f);
         const float o4[4] = {av.x * inv, av.y * inv, av.z * inv, av.w * inv};
         half4_t hi, lo;
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            hi[i] = (half_t)o4[i];
-            lo[i] = (half_t)((o4[i] - (float)hi[i]) * kLowScale);
+            half_t h, l;
+            split_scaled(o4[i], h, l);
+            hi[i] = h; lo[i] = l;
         }
         *reinterpret_cast<half4_t*>(&o_s[0][vl * kMergeRow + 2 * k4]) = hi;
         *reinterpret_cast<half4_t*>(&o_s[1][vl * kMergeRow + 2 * k4]) = lo;

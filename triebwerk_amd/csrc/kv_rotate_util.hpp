@@ -123,6 +123,17 @@ __device__ __forceinline__ uint32_t bucket_quantize(const float2* buckets, float
     }
 }
 
+// Vectors that the forms of a step rotate back on fp16 matrix instructions are held as hi = half(x) and lo = half((x - hi) * kLowScale), whose
+// products are summed apart: hi + lo / 2^11 is within 2^-23 of x itself, and within 2^-36 where x is small.  (The remainder as it is is a
+// subnormal half below values of 2^-3: for values of 1e-4 one output in five was not the half nearest to its sum, with the enlarged one
+// it is one in 5000, as on fp32 matrix instructions.)
+constexpr float kLowScale = 2048.0f;           // a remainder is at most 2^-12 of the next power of two: no overflow
+// hi and lo of x = xs / kLowScale (one instruction each from the vector held kLowScale times as large)
+__device__ __forceinline__ void split_scaled(float xs, half_t& hi, half_t& lo) {
+    hi = (half_t)__builtin_fmaf(xs, 1.0f / kLowScale, 0.0f);
+    lo = (half_t)__builtin_fmaf((float)hi, -kLowScale, xs);
+}
+
 // K and V codes from v_mfma_f32_16x16x32_f16 -- raw fp16 coordinates, the sum scaled by 1 / |x| afterwards -- where they are sure to be those
 // of the fp32 chain, whose codes the reference's are.  How far can the two be apart, for a row of R of norm |R|?
 // The chain's fused multiply-adds lose at most 2^-24 of a partial sum s_k each, and the unit coordinates 2^-24 of |R| in all.  The
