@@ -226,12 +226,16 @@ decode_fused_kernel(AttnArgs a, FusedArgs f) {
         prod_c = reinterpret_cast<const uint4*>(roped ? f.cos_table : a.rotation)[at];
         prod_s = reinterpret_cast<const uint4*>(roped ? f.sin_table : a.rotation)[at];
     }
+    // the sequence's first cache row.  (For long contexts in scalar registers by force, as is h: the new row's address is made on the vector
+    // ALU, and with it the compiler put the base addresses of the scan there too, 8 to 12 instructions more per tile to make its
+    // descriptors.  Where waves have few tiles the start's two trips to the scalar side cost as much.)
+    const long long row0 = MODE == kPaged ? 0 : (long long)g * a.seq_stride_rows, seq_row0 = kEarly ? row0 : uniform(row0);
     // the new token's cache row
     const long long new_row = MODE == kPaged ? (long long)uniform(bt[pos / kPageTokens]) * kPageTokens + pos % kPageTokens
-                                             : (long long)g * a.seq_stride_rows + pos;
+                                             : seq_row0 + pos;
     // PAIR: wave = part * (HKW / 2) + pair; hk_local is the first head of the pair
     const int hk_local = PAIR ? 2 * (wave & ((HKW >> 1) - 1)) : wave & (HKW - 1), part = PAIR ? 2 * wave >> hkw_log2 : wave >> hkw_log2;
-    const int h = hg * HKW + hk_local;                 // (first) KV head of this wave
+    const int h = kEarly ? hg * HKW + hk_local : uniform(hg * HKW + hk_local);                 // (first) KV head of this wave
 
     // ---- tiles of 32 tokens this wave scans.  They are dealt round by round: in round r part p takes tile
     // r * SPLIT + p, so that at any moment the workgroup -- and with it the other workgroups of the sequence,
@@ -290,7 +294,6 @@ decode_fused_kernel(AttnArgs a, FusedArgs f) {
     auto lut32 = [&](uint32_t addr) -> uint32_t { return *reinterpret_cast<const uint32_t*>(tab_lane + addr); };
     auto lut64 = [&](uint32_t addr) -> uint2 { return *reinterpret_cast<const uint2*>(tab_lane + addr); };
 
-    const long long seq_row0 = (long long)g * a.seq_stride_rows;
     const char* kseq = reinterpret_cast<const char*>(a.k) + (long long)h * kHeadBytes;
     const char* vseq = reinterpret_cast<const char*>(a.v) + (long long)h * kHeadBytes;
     const char* knseq = reinterpret_cast<const char*>(a.k_norms) + (long long)h * 2;
@@ -481,7 +484,6 @@ decode_fused_kernel(AttnArgs a, FusedArgs f) {
         const uint32_t voff = L.voff_rows * kvp + L.voff_bytes;
         const uint32_t noff = (uint32_t)L.tok0 * nrow;
         // the sequence's rows of this pair: a tile is one multiplication per array away
-        const long long seq_row0 = MODE == kPaged ? 0 : (long long)g * a.seq_stride_rows;
         const char* kpair = reinterpret_cast<const char*>(a.k) + seq_row0 * kvp + (long long)h * kHeadBytes;
         const char* vpair = reinterpret_cast<const char*>(a.v) + seq_row0 * kvp + (long long)h * kHeadBytes;
         const char* knpair = reinterpret_cast<const char*>(a.k_norms) + seq_row0 * nrow + (long long)h * 2;
@@ -598,7 +600,7 @@ decode_fused_kernel(AttnArgs a, FusedArgs f) {
             }
         });
         if (!first_early) { issue_k(t); issue_n(t); issue_v(t); }
-        if (!SHARES) load_rb(); // behind the first tile's loads; the registers are there, and the epilogue need not wait
+        if (kEarly && !SHARES) load_rb();    // behind the first tile's loads; the registers are there, and the epilogue need not wait
         if (ntiles > 0) {
             S.load_query_operands(L, [&](int i, int part2, int p) { return &qop_s[query_piece(2 * (hk_local * R + i) + part2, p)]; });
             for (int it = 0; it < ntiles; it++) {
@@ -607,6 +609,9 @@ decode_fused_kernel(AttnArgs a, FusedArgs f) {
                 pair_scan_tile<R>(L, S, t, tile, n, [&]() { issue_k(t); }, [&]() { issue_n(t); }, [&]() { issue_v(t); });
             }
         }
+        // (Long contexts ask at the end: at the start these 32 two-byte loads a wave hold up the second tile.  With the scalar addresses
+        // above 64 x 8192 tokens 94.0 -> 92.7 us, 96 x 4096 79.1 -> 77.7, 112 x 8192 167.2 -> 164.5.)
+        if (!kEarly) load_rb();
         pair_scan_finish<R>(L, S, 1.0f / kAlpha, [&](int hd, int r, const float (&ov)[16]) {
             float* pr = &part_s[part * HKW + hk_local + hd][r][0];
 #pragma unroll

@@ -56,6 +56,9 @@ constexpr bool centroids_agree() {
 static_assert(centroids_agree(), "the selections give the tables' values");
 
 __device__ __forceinline__ int uniform(int x) { return __builtin_amdgcn_readfirstlane(x); }
+__device__ __forceinline__ long long uniform(long long x) {
+    return (long long)((unsigned long long)(unsigned)uniform((int)(x >> 32)) << 32 | (unsigned)uniform((int)x));
+}
 
 typedef uint32_t uint32x4_t __attribute__((ext_vector_type(4)));
 typedef uint32_t uint32x2_t __attribute__((ext_vector_type(2)));
