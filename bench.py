@@ -3,7 +3,8 @@
 
 A step = one new token for every sequence: for each layer, append K and V to the
 cache and run GQA decode attention over the whole context, then positions += 1.
-The step is captured once in a hipGraph and replayed.  Inputs (caches, q, k, v)
+The step is captured once in a hipGraph and replayed, or, where all layers are one launch,
+launched.  Inputs (caches, q, k, v)
 are resident in HBM before the timed region; every layer has its own cache, so
 nothing is re-read from a cache level between layers or steps.
 
@@ -807,7 +808,7 @@ def decode_bench(args, kv_bits, with_probe):
             "layers": L, "num_heads": H, "num_kv_heads": Hk, "head_dim": D, "batch": G,
             "context_first_timed_step": [int(ctx0.min()), int(ctx0.max())],
             "tokens_attended_per_step": n_tokens_timed / K,
-            "hipgraph": use_graph,
+            "hipgraph": use_graph and not whole_step,
             "launchers": ("tw_engine_decode_step (engine object)" + (": every layer's inputs are at hand, all layers in one launch" if whole_step else "")
                           if args.launchers == "engine" else "tw_engine_layer_step, one layer after the other" if args.launchers == "layer" else
                           "the reference's own launchers only: " +

@@ -212,8 +212,8 @@ int tw_kv_decode_step_plan2(int G, int num_heads, int num_kv_heads, int bits, in
  * launch (which they then do). */
 void tw_kv_debug_set_fused_shape(int hkw, int shares);
 /* Layer steps planned as one launch (tw_kv_decode_step_plan2) since the library was loaded, each launched or recorded into a
- * graph by itself or together with the other layers of its step (tw_engine_decode_step): lets a benchmark say which
- * kernel its figures belong to. */
+ * graph by itself or together with the other layers of its step (tw_engine_decode_step; a fixed step counts when it is fixed, not
+ * when it is repeated): lets a benchmark say which kernel its figures belong to. */
 long long tw_kv_decode_fused_launches(void);
 
 /* No counterpart in the reference.  Rate (GB/s) at which this GPU streams `bytes` of device
@@ -502,9 +502,10 @@ int tw_engine_prompt_layer(tw_engine* e, int layer, int seq, const tw_half* q, c
  * layer l's output calls tw_engine_layer_step), and all of them go into one launch where that is faster (fp16 cache: KV heads in eights)
  * -- unless `out` lies over q, k or v (fp16 with producers: q, which they transform in place, over k or v), or the producers run as
  * launches of their own (mode 2): then layer by layer, in order.
- * With use_graph != 0 the step is captured once into a hipGraph and replayed
- * (engine.cpp:2369-2412, 2480; all layers together are one to four launches, which are issued again without the graph around
- * them: that is the faster replay); the capture is dropped when the arena, G or
+ * With use_graph != 0 the step is fixed: captured once into a hipGraph and replayed
+ * (engine.cpp:2369-2412, 2480), or, where all layers go together, the same one launch (compressed) or two to four (fp16)
+ * every time, for which nothing is captured: that is faster than a replay.  On the compressed cache that one launch also advances the
+ * positions, counting a sequence's workgroups in the engine's tickets.  The capture is dropped when the arena, G or
  * the buffers change, and made again when the context lengths the host knows of have moved to where the other
  * choice of kernels (tw_kv_decode_step_plan) applies.  -8: a sequence has no row left (see
  * tw_engine_set_positions). */
@@ -513,8 +514,8 @@ int tw_engine_decode_step(tw_engine* e, const tw_half* q, const tw_half* k, cons
 /* When the capture or the instantiation of the step's graph fails, the step is run without a graph, one line goes
  * to stderr, and so are all later steps with the same buffers (engine.cpp:2396-2410); the next change of buffers,
  * batch, arena or producers tries again.  graph_state tells what the latest decode step did: 0 run eagerly as asked,
- * 1 graph replayed (or, where all layers are a few launches, the captured ones issued again), 2 run eagerly after a failed capture.  debug_fail_captures (test hook): the next n captures
- * are treated as failed after they have been recorded. */
+ * 1 as fixed (graph replayed, or all layers' launches), 2 run eagerly after a failed capture.  debug_fail_captures (test hook):
+ * the next n captures, or fixings of all layers' launches, are treated as failed. */
 int tw_engine_graph_state(const tw_engine* e);
 void tw_engine_debug_fail_captures(tw_engine* e, int n);
 /* roctx ranges (tw_engine_decode_step, tw_engine_prompt_layer, tw_engine_single_step) for a profiler's timeline,

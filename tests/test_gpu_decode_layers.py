@@ -285,3 +285,37 @@ def test_what_one_launch_does_not_take_goes_layer_by_layer(bits, why):
     torch.cuda.synchronize()
     assert torch.equal(*outs) and outs[0].abs().sum() > 0
     _same_caches(engines, L)
+
+
+@pytest.mark.parametrize("bits", [4, 2, 0])
+def test_a_step_of_every_layer_captures_nothing_itself(capfd, bits):
+    """With use_graph the few launches of all layers are issued as they are: nothing is captured for them, so inside a caller's capture
+    nothing fails, and the caller's graph replays them."""
+    import torch
+    from triebwerk_amd import kvcache
+    H, Hk, L, lens, msl = 16, 8, 6, [300, 77, 120], 512
+    G = len(lens)
+    engines, q, k, v = _pair(bits, H, Hk, L, G, msl, False)
+    outs = [torch.zeros_like(q) for _ in range(2)]
+    for e in engines:
+        e.set_positions([n - 1 for n in lens])
+    stream = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    capfd.readouterr()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream, capture_error_mode="relaxed"):
+        engines[0].decode_step(q, k, v, outs[0], use_graph=True, stream=stream)
+    assert "FAILED" not in capfd.readouterr().err
+    assert engines[0].graph_state() == 1
+    assert ("decode_layers_kernel" if bits else "attention_rows_kernel, every layer") in kvcache.last_scan_kernel()
+    for step in range(3):
+        graph.replay()
+        for l in range(L):
+            engines[1].layer_step(l, q[l], k[l], v[l], outs[1][l])
+        torch.cuda.synchronize()
+        engines[1].set_positions([n + step for n in lens])
+        assert engines[0].positions().tolist() == [n + step for n in lens]
+        got, want = (host(o).reshape(L * G, H * D) for o in outs)
+        assert rel_err(got, want) <= TOL, f"step {step}"
+        outs[0].zero_()
+    _same_caches(engines, L)

@@ -84,13 +84,13 @@ struct tw_engine {
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;
     const void* graph_key[4] = {};
-    int graph_G = 0;
-    twkv::StepPlan graph_plan{};      // what the captured launches were chosen as
+    int graph_G = 0;                  // 0: no step is fixed (use_graph), captured or not
+    twkv::StepPlan graph_plan{};      // what its launches were chosen as
     // generate_batch goes on without a graph when capture or instantiation fails (engine.cpp:2396-2410): so does
     // tw_engine_decode_step, until the buffers, the batch or the producers change
     bool graph_failed = false;
     const void* graph_failed_key[4] = {};
-    int graph_state = 0;              // of the latest decode step: 0 eager as asked, 1 graph replayed, 2 eager after a failed capture
+    int graph_state = 0;              // of the latest decode step: 0 eager as asked, 1 as fixed, 2 eager after a failed capture
     int fail_next_captures = 0;       // test hook: treat this many coming captures as failed
 
     // The stream of the latest step: reset, set_positions and everything that lets go of the arena wait for it
@@ -378,10 +378,10 @@ bool layers_together(tw_engine* e, const tw_half* q, const tw_half* k, const tw_
 }
 
 void all_layers(tw_engine* e, const twkv::StepPlan& plan, const tw_half* q, const tw_half* k, const tw_half* v, tw_half* out,
-                hipStream_t s, bool recorded = false) {
+                hipStream_t s, bool again = false) {
     if (plan.layers > 1) {
         const tw_layer_step_args p = layer_args(e, 0, q, k, v, out);
-        twkv::layers_attention_step(&p, step_layers(e), plan, s, recorded);
+        twkv::layers_attention_step(&p, step_layers(e), plan, s, again);
         if (e->kv_bits != 0) return;                         // the launch has advanced the positions
     } else {
         const size_t qs = (size_t)e->G * e->q_dim(), ks = (size_t)e->G * e->kv_dim();
@@ -803,14 +803,21 @@ int tw_engine_decode_step(tw_engine* e, const tw_half* q, const tw_half* k, cons
     // is captured again: up to 18 times on the way from 1 to 16384 tokens, 60 us of the host's time each for 28 layers.
     // (One sequence, 4 bit, 16 heads over 8 KV heads, at 16000 tokens: 18.5 us per layer in the form chosen there, 75.1 in
     // the one a step captured at 512 tokens holds.)
-    if (!e->graph_exec || e->graph_G != e->G || !(e->graph_plan == plan) || memcmp(key, e->graph_key, sizeof(key)) != 0) {
+    // All layers together are one launch (compressed) or two to four (fp16), the same ones every time: they are issued one by one, with no
+    // graph captured for them, which takes 5 us a step less on the GPU than a graph's start and end around them, and 9 of the host's 15 us
+    // (28 layers of 4 x 613 tokens at 4 bit 28.0 -> 22.9 us a step, of 1 x 100 on the fp16 cache 20.3 -> 13.2).
+    const bool launched = plan.layers > 1;
+    const bool fixed = e->graph_G == e->G && e->graph_plan == plan && memcmp(key, e->graph_key, sizeof(key)) == 0;
+    if (!fixed) {
         e->drop_graph();
         // Capture records the launches without running them, so unlike the
         // reference (engine.cpp:2414-2444) nothing has to be re-prefilled.
         int why = 0;                       // -4 begin, -5 end of capture or a launcher's error, -6 instantiation
         hipGraph_t g = nullptr;
-        hipError_t err = hipStreamBeginCapture(s, hipStreamCaptureModeRelaxed);
-        if (err != hipSuccess) {
+        hipError_t err = hipSuccess;
+        if (launched) {
+            if (e->fail_next_captures > 0) { e->fail_next_captures--; why = -6; err = hipErrorUnknown; }
+        } else if ((err = hipStreamBeginCapture(s, hipStreamCaptureModeRelaxed)) != hipSuccess) {
             why = -4;
         } else {
             all_layers(e, plan, q, k, v, out, s);
@@ -834,17 +841,15 @@ int tw_engine_decode_step(tw_engine* e, const tw_half* q, const tw_half* k, cons
         e->graph_plan = plan;
         memcpy(e->graph_key, key, sizeof(key));
     }
-    e->graph_state = 1;
-    if (plan.layers > 1) {
-        // All layers together are one to three launches, and recorded or not they are the same ones: issued one by one they take 5 us a
-        // step less on the GPU than a graph's start and end around them, and 9 of the host's 15 us (28 layers of 4 x 613 tokens at 4 bit
-        // 28.0 -> 22.9 us a step, of 1 x 100 on the fp16 cache 20.3 -> 13.2).
-        all_layers(e, plan, q, k, v, out, s, true);
+    if (launched) {
+        all_layers(e, plan, q, k, v, out, s, /*again=*/fixed);
         e->one_token_on();
+        e->graph_state = 1;
         return tw_kv_last_error();
     }
     if (hipGraphLaunch(e->graph_exec, s) != hipSuccess) return -7;
     e->one_token_on();
+    e->graph_state = 1;
     return 0;
 }
 

@@ -364,8 +364,8 @@ int rows_layers_most_pieces(int layers, int G, int num_heads, int num_kv_heads);
 int rows_layers_pieces(int layers, int G, int num_heads, int num_kv_heads, int max_seq_len, double ctx_max, double ctx_mean, size_t ws_floats);
 // Whether the buffers admit it (a plan with layers > 1 is for those that do)
 bool layers_attention_usable(const tw_layer_step_args* p, const StepLayers& layers);
-// (recorded: the launches of a captured step, issued again)
-void layers_attention_step(const tw_layer_step_args* p, const StepLayers& layers, const StepPlan& plan, hipStream_t s, bool recorded);
+// (again: the launches of a fixed step after its first time, which tw_kv_decode_fused_launches counts no more than a graph's replays)
+void layers_attention_step(const tw_layer_step_args* p, const StepLayers& layers, const StepPlan& plan, hipStream_t s, bool again);
 // allow_pairs: the kernel whose waves scan two KV heads each, where the shape admits it (false: one head per wave)
 void launch_decode_fused(const AttnArgs& a, const FusedArgs& f, hipStream_t s, bool allow_pairs, const StepPlan& plan);
 // the pair kernel (hkw KV heads a workgroup, no shares, no producers) for attention alone, or for the step over the paged cache

@@ -168,7 +168,7 @@ class Engine:
             raise RuntimeError(f"broadcast_prefix failed ({rc})")
 
     def graph_state(self) -> int:
-        """What the latest decode_step did: 0 eager as asked, 1 graph replayed (all layers at once: its launches issued again), 2 eager after a
+        """What the latest decode_step did: 0 eager as asked, 1 as fixed (graph replayed, or all layers' launches), 2 eager after a
         failed capture (generate_batch decodes without a graph when the capture fails, engine.cpp:2396-2410)."""
         return self._lib.tw_engine_graph_state(self._h)
 
