@@ -178,6 +178,9 @@ void tw_kv_debug_set_prefill_form(int form);
  * group 1, 2 or 4); 2: never; 3: as 1, with one KV head per wave also where the 4-bit kernel would give a wave two; 4: as 0.
  * tw_engine_decode_step takes every layer by itself while this is not 0, the attention variant is not 0 or a split count is set. */
 void tw_kv_debug_set_decode_fused(int mode);
+/* What the appends decide their codes from: sums[v][d] = sum over k of rotation[d][k] x[v][k] for n vectors of 128 halves on fp16 matrix
+ * instructions, and row_norms[b], their bound on the norms of rows 16 b .. 16 b + 15 of the (128, 128) rotation. */
+void tw_kv_debug_rotation_sums(const tw_half* x, int n, const tw_half* rotation, float* sums, float* row_norms, hipStream_t s);
 /* Timing of the context-scanning attention kernel alone, with HIP events attached to that kernel's launches on
  * their stream.  Enable, run eager launches (not under stream capture; at most 4096 are kept), then read the
  * summed duration and the launch count.  Reading waits for the recorded launches and resets the counter. */

@@ -65,6 +65,7 @@ SIGNATURES = {
     "tw_kv_decode_step_plan2": (I, [I, I, I, I, I, I, I, I]),
     "tw_kv_debug_set_fused_shape": (None, [I, I]),
     "tw_kv_debug_profile_attention": (None, [I]),
+    "tw_kv_debug_rotation_sums": (None, [P, I, P, P, P, P]),
     "tw_kv_debug_profile_read": (I, [C.POINTER(C.c_double), C.POINTER(I)]),
     "tw_kv_measure_read_bandwidth": (C.c_double, [P, C.c_size_t, I, P]),
     "tw_kv_broadcast_rows": (I, [P, P, P, I, I, I, I, P]),

@@ -115,7 +115,7 @@ append_tokens_kernel(AppendTokensArgs a) {
     Request next = request(x1, pos1);
     if (BITS == 4 && tid < kBuckets) bucket_s[tid] = bucket_entry(tid);
     uint4 rv[2][4];                                    // R[16 * (wave + 4 d) + i16][4s + kk], s = 8j .. 8j + 7
-    float row_norm[2];
+    float row_norm = a.row_norm;
     {
         uint32_t* mine = reinterpret_cast<uint32_t*>(x_s) + wave * kOperandTileDwords;      // this wave's own: no barrier in between
 #pragma unroll
@@ -127,9 +127,10 @@ append_tokens_kernel(AppendTokensArgs a) {
             for (int j = 0; j < 4; j++) rv[d][j] = *reinterpret_cast<const uint4*>(mine + operand_tile_dword(lane, 4 * j));
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront", "local");
             __builtin_amdgcn_wave_barrier();
-            row_norm[d] = a.row_norm == 0.0f && !a.chains ? operand_rows_norm(rv[d]) : a.row_norm;
+            if (a.row_norm == 0.0f && !a.chains) row_norm = larger_norm(row_norm, operand_rows_norm(rv[d]));
         }
     }
+    row_norm = __builtin_bit_cast(float, uniform(__builtin_bit_cast(int, row_norm)));      // (the same in every lane: no vector register)
     lds_barrier();                                     // every wave has its rows of R
 
     // coordinate 4s + kk of vector v in 16-byte piece 4kk + s / 8 of its row, which lies at that piece ^ 5v (no bank twice, written or read)
@@ -239,7 +240,7 @@ append_tokens_kernel(AppendTokensArgs a) {
 #pragma unroll
             for (int d = 0; d < 2; d++)                // lane: coordinates 16 (wave + 4d) + 4kk .. + 3 of vector i16
 #pragma unroll
-                for (int r = 0; r < 4; r++) codes[d] |= bucket_quantize_sure<BITS>(bucket_s, sums[d], r, inv, row_norm[d], doubt[d]) << (r * BITS);
+                for (int r = 0; r < 4; r++) codes[d] |= bucket_quantize_sure<BITS>(bucket_s, sums[d], r, inv, row_norm, doubt[d]) << (r * BITS);
             if (__any(doubt[0])) chains(d0, d0);
             if (__any(doubt[1])) chains(d1, d1);
         }

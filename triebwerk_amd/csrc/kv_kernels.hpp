@@ -119,6 +119,7 @@ struct AppendTokensArgs {
 bool append_tokens_usable(const AppendTokensArgs& a);
 // While one of these lives the calls of this thread have the engine's rotation, whose rows are of norm 1: the kernels need not measure them
 // (FusedArgs::row_norm).
+constexpr float kUnitRows = 1.001f;
 struct KnownRotation {
     KnownRotation();
     ~KnownRotation();
@@ -129,6 +130,8 @@ void launch_sigmoid_gate(half_t* data, long long data_stride, const half_t* gate
                          int rows, hipStream_t s);
 
 // ---------------------------------------------------------------- rotation on the matrix cores
+// test hook (tw_kv_debug_rotation_sums)
+void launch_rotation_sums(const half_t* x, int n, const half_t* rotation, float* sums, float* row_norms, hipStream_t s);
 struct RotArgs {
     // up to 3 segments: K rows, V rows (quantize), Q rows (rotate only); each 64 bytes, one scalar load of a kernel
     struct alignas(64) Segment {

@@ -283,6 +283,36 @@ void launch_rotate(const RotArgs& args, int bits, hipStream_t s) {
     }
 }
 
+// The sums that bucket_quantize_sure decides codes from, for a test of its bound: a wave per 16 vectors and 16 coordinates, operands as
+// append_tokens_kernel and the one-launch steps hold them (operand j of a lane: coordinates 4s + kk, s = 8j .. 8j + 7).
+__global__ void __launch_bounds__(kWave)
+rotation_sums_kernel(const half_t* __restrict__ x, int n, const half_t* __restrict__ rotation, float* __restrict__ sums, float* __restrict__ row_norms) {
+    const int lane = threadIdx.x, i16 = lane & 15, kk = lane >> 4, dblk = blockIdx.y, v = blockIdx.x * 16 + i16;
+    const half_t* row = rotation + (dblk * 16 + i16) * kHeadDim + kk;
+    const half_t* vec = x + (long long)min(v, n - 1) * kHeadDim + kk;
+    float4_t acc = {0.f, 0.f, 0.f, 0.f};
+    uint4 rows[4];
+    for (int j = 0; j < 4; j++) {
+        half8_t r, u;
+#pragma unroll
+        for (int e = 0; e < 8; e++) {
+            r[e] = row[4 * (8 * j + e)];
+            u[e] = vec[4 * (8 * j + e)];
+        }
+        rows[j] = __builtin_bit_cast(uint4, r);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(r, u, acc, 0, 0, 0);
+    }
+    if (v < n) {                                       // lane: coordinates 16 dblk + 4kk .. + 3 of vector v
+#pragma unroll
+        for (int r = 0; r < 4; r++) sums[(long long)v * kHeadDim + dblk * 16 + 4 * kk + r] = acc[r];
+    }
+    const float norm = operand_rows_norm(rows);
+    if (blockIdx.x == 0 && lane == 0) row_norms[dblk] = norm;
+}
+void launch_rotation_sums(const half_t* x, int n, const half_t* rotation, float* sums, float* row_norms, hipStream_t s) {
+    if (n > 0) hipLaunchKernelGGL(rotation_sums_kernel, dim3((n + 15) / 16, 8), dim3(kWave), 0, s, x, n, rotation, sums, row_norms);
+}
+
 // ---------------------------------------------------------------- split merge + rotate-back
 // out[g][head][d] = sum_k R[k][d] * o[k],  o = (sum_c f_c acc_c) / (sum_c f_c l_c + 1e-8),
 // f_c = exp(m_c - max_c m_c): the log-sum-exp merge of the split partials, the

@@ -287,6 +287,16 @@ def set_fused_shape(hkw: int = 0, shares: int = 0) -> None:
     _lib.load().tw_kv_debug_set_fused_shape(int(hkw), int(shares))
 
 
+def rotation_sums(x, rotation, stream=None):
+    """tw_kv_debug_rotation_sums: (n, 128) halves times the rows of the rotation as the appends sum them, and their bound on
+    the norms of each 16 rows (a test hook)."""
+    sums = torch.empty(x.shape, dtype=torch.float32, device=x.device)
+    norms = torch.empty(8, dtype=torch.float32, device=x.device)
+    _lib.load().tw_kv_debug_rotation_sums(_ptr(x, "f16", "x"), x.shape[0], _ptr(rotation, "f16", "rotation"), _ptr(sums, "f32", "sums"),
+                                          _ptr(norms, "f32", "row_norms"), _stream(stream))
+    return sums, norms
+
+
 def last_scan_kernel() -> str:
     """Name of the kernel that the last decode-attention call launched for the context scan (a test hook)."""
     return _lib.load().tw_kv_debug_last_scan_kernel().decode()
