@@ -129,3 +129,41 @@ def test_every_layer_at_once(oracle, bits, H, Hk, G, hkw):
             oracle.turbo_kv_quantize_batch(want[1], want[3], v[l], rot, pos, msl, G, Hk, D, Hk * D, bits)
         for got, w, what in zip(eng.cache(l), want, ("K codes", "V codes", "K norms", "V norms")):
             assert_bytes_equal(host(got)[:, :2], w[:, :2], f"layer {l} {what}")
+
+
+def _far_rows(r, n, heads):
+    """A matrix whose rows are of norm 4e5 and vectors that it takes far out, but for every 16th row and the first head, whose values lie among the
+    boundaries: there the first 56 coordinates meet the next 56 with the other sign, and the last 16 make the value.  What rounding does
+    on the way is larger than the distance of two boundaries."""
+    m = (r.uniform(20000, 65504, (D, D)) * r.choice([-1, 1], (D, D))).astype(np.float32)
+    m[::16, 56:112] = -m[::16, :56]
+    m[::16, 112:] = r.standard_normal((D // 16, 16))
+    x = r.standard_normal((n, heads, D)).astype(np.float32)
+    x[:, 0, 56:112] = x[:, 0, :56]
+    x[:, 0, 112:] *= 0.5
+    return m.astype(np.float16), x.astype(np.float16).reshape(n, heads * D)
+
+
+@pytest.mark.parametrize("scale", [1.0, 0.03, 0.001])
+@pytest.mark.parametrize("bits,T", [(4, 1366), (2, 700)])
+def test_rows_of_any_norm(oracle, bits, T, scale):
+    """The bound is wider than a bucket there, and a boundary in the next bucket within it.  One value of a block that is not far out: else
+    another one's doubt has the whole block repeated."""
+    import torch
+    from triebwerk_amd import kvcache as kvc
+    Hk = 8
+    r = gen.rng(9150 + bits)
+    rot, k = _far_rows(r, T, Hk)
+    rot = (scale * rot.astype(np.float32)).astype(np.float16)
+    v = r.standard_normal((T, Hk * D)).astype(np.float16)
+    kv_dim, msl = Hk * D, T + 1
+    pos = np.arange(T, dtype=np.int32)
+    want = [(np.zeros((msl, kv_dim * bits // 8), np.uint8), np.zeros((msl, Hk), np.float16)) for _ in range(2)]
+    got = [tuple(dev(x) for x in w) for w in want]
+    for s, (c, n) in zip((k, v), want):
+        oracle.turbo_kv_quantize(c, n, s, rot, pos, msl, T, Hk, D, kv_dim, bits)
+    kvc.tw_turbo_kv_append_tokens(*got[0], *got[1], dev(k), dev(v), dev(rot), dev(pos), msl, T, Hk, D, kv_dim, bits)
+    torch.cuda.synchronize()
+    for g, w in zip(got, want):
+        for a, b, what in zip(g, w, ("codes", "norms")):
+            assert_bytes_equal(host(a), b, what)

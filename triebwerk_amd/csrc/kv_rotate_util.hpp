@@ -149,7 +149,7 @@ __device__ __forceinline__ void split_scaled(float xs, half_t& hi, half_t& lo) {
 // 18 T + (47 + 7e-3 / |x|) |R'|.
 constexpr float kUlp = 5.9604645e-8f;                          // 2^-24
 // Code of y = S[3][r] * inv, inv = 1 / |x|, row_norm >= |R'|; doubt is set where y is not further than that from a boundary (or no number).
-static_assert(0.15 / kBucketScale > 100.0 * 175.0 * kUlp, "a value near a boundary is in its bucket, which no boundary lies near to the edge of");
+constexpr float kNextEdge = 0.149f / kBucketScale;             // a boundary that is not in a value's bucket is further off than this (edges_have_buckets)
 template <int BITS>
 __device__ __forceinline__ uint32_t bucket_quantize_sure(const float2* buckets, const float4_t (&S)[4], int r, float inv, float row_norm, bool& doubt) {
     const float val = S[3][r] * inv;
@@ -157,7 +157,7 @@ __device__ __forceinline__ uint32_t bucket_quantize_sure(const float2* buckets, 
     const float eps = __builtin_fmaf(inv, __builtin_fmaf(sums, 18.0f * kUlp, row_norm * (7e-3f * kUlp)), row_norm * (47.0f * kUlp));
     if constexpr (BITS == 4) {
         const float2 e = buckets[bucket_of(val)];
-        doubt = doubt || !(fabsf(val - e.x) > eps);
+        doubt = doubt || !(fminf(fabsf(val - e.x), kNextEdge) > eps);      // (a bound past it: long rows of R, tiny vectors)
         return __builtin_bit_cast(uint32_t, e.y) + (!(val < e.x) ? 1u : 0u);
     } else {
         doubt = doubt || !(fminf(fabsf(val), fabsf(fabsf(val) - kEdges2[2])) > eps);
