@@ -187,8 +187,8 @@ void tw_kv_debug_rotation_sums(const tw_half* x, int n, const tw_half* rotation,
 void tw_kv_debug_profile_attention(int enable);
 int tw_kv_debug_profile_read(double* total_ms, int* launches);
 /* Name of the kernel that the last attention call of this process launched (or recorded into a graph) for the
- * context: "attention_pair_kernel", "attention_mfma_kernel", "attention_rows_kernel", "attention_valu_kernel",
- * "decode_fused_kernel, two KV heads per wave", "decode_fused_kernel, one KV head per wave", a prefill kernel, or
+ * context: "attention_pair_kernel", "attention_mfma_kernel", "attention_rows_kernel", "attention_valu_kernel" (", chunks merged
+ * in the launch" where the step's tickets do that), "decode_layers_kernel, ...", "decode_fused_kernel, two KV heads per wave", "decode_fused_kernel, one KV head per wave", a prefill kernel, or
  * "none".  A static string; lets a benchmark name the kernel its figures belong to. */
 const char* tw_kv_debug_last_scan_kernel(void);
 

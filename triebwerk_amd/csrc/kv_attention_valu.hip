@@ -1057,7 +1057,7 @@ int rows_layers_pieces(int layers, int G, int num_heads, int Hk, int max_seq_len
 void launch_attention_valu(const AttnArgs& a, hipStream_t s) {
     if (a.G <= 0) return;
     if (a.even_chunks) { launch_attention_rows(a, s); return; }     // the split planner chose the whole-row kernel
-    note_scan_kernel("attention_valu_kernel");
+    note_scan_kernel(attention_valu_merges(a) ? "attention_valu_kernel, chunks merged in the launch" : "attention_valu_kernel");
     if (a.bits == 0) launch_valu_mode<0>(a, s);
     else if (a.bits == 4) launch_valu_mode<4>(a, s);
     else launch_valu_mode<2>(a, s);
