@@ -282,6 +282,7 @@ attention_pair_kernel(AttnArgs a, int total_items, int hgroups, int group_waves)
         }
         ready = false;
         S.reset();
+        S.zero_repeated_queries(L);
 
         for (int tile = t0; tile < t1; tile += 32) {
             const bool more = tile + 32 < t1;

@@ -305,6 +305,7 @@ decode_layers_kernel(LayersArgs a) {
     PairState<R> S;
     S.reset();
     S.load_query_operands(L, [&](int i, int part2, int p) { return &qop_s[query_piece(2 * (hk_local * R + i) + part2, p)]; });
+    S.zero_repeated_queries(L);
     lds_barrier();                                           // the queries have been read
     // The step's last act, positions + 1 (engine.cpp:2394): every wave of this unit has used its sequence's position by now, and the unit
     // that draws a sequence's last ticket is behind all others in that, so it writes the next one.

@@ -136,14 +136,23 @@ struct PairState {
 #pragma unroll
         for (int r = 0; r < R; r++) { m_run[r] = kNegBig; l_run[r] = 0.0f; }
     }
-    // q_rot of the pair's query heads (i = hd * R + r, 0 <= i < 2 R) from operands: piece(i, part, p) -> 16-byte piece p of the 128 halves of query head i, part 0 their fp16 values and 1 what
-    // rounding left over.  (160 instructions less per wave than making them here from floats.  The operand rows m with
-    // m % 4 >= R repeat a head, their scores are not read.)
+    // q_rot of the pair's query heads (i = hd * R + r, 0 <= i < 2 R) from operands: piece(i, part, p) -> 16-byte piece p of the 128 halves of query
+    // head i, part 0 their fp16 values and 1 what rounding left over.  (160 instructions less per wave than making them here from floats.  The
+    // operand rows m with m % 4 >= R repeat a head, their scores are not read.)
     template <class Lane, class PieceOf>
     __device__ __forceinline__ void load_query_operands(const Lane& L, PieceOf piece_of) {
         const int m = L.pn & 7, head = (m >> 2) * R + ((m & 3) < R ? (m & 3) : R - 1);
 #pragma unroll
         for (int j = 0; j < 4; j++) aq[j] = __builtin_bit_cast(half8_t, *piece_of(head, L.pn >> 3, 4 * L.pkg + j));
+    }
+    // The matrix cores multiply what the repeated rows hold, and the power that takes comes off the clock of a chip that streams: with zeros
+    // there 28 layers of 64 x 8192 tokens in one launch take 2330 us instead of 2376 (2 bit 1697 instead of 1732), layer by layer 90.3
+    // instead of 91.6.  (Launches that leave most of the chip idle do without: it only delays them.)
+    template <class Lane>
+    __device__ __forceinline__ void zero_repeated_queries(const Lane& L) {
+        if (R == 4) return;
+#pragma unroll
+        for (int j = 0; j < 4; j++) aq[j] = __builtin_bit_cast(half8_t, (L.pn & 3) < R ? __builtin_bit_cast(uint4, aq[j]) : uint4{0u, 0u, 0u, 0u});
     }
 };
 
