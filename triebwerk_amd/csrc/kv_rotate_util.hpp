@@ -149,7 +149,11 @@ __device__ __forceinline__ void split_scaled(float xs, half_t& hi, half_t& lo) {
 // 18 T + (47 + 7e-3 / |x|) |R'|.
 constexpr float kUlp = 5.9604645e-8f;                          // 2^-24
 // Code of y = S[3][r] * inv, inv = 1 / |x|, row_norm >= |R'|; doubt is set where y is not further than that from a boundary (or no number).
-constexpr float kNextEdge = 0.149f / kBucketScale;             // a boundary that is not in a value's bucket is further off than this (edges_have_buckets)
+// (A value is compared with its own bucket's boundary.  Another one is at least 0.15 of a bucket away (edges_have_buckets), which the bound
+// stays below for rows of norms up to kLongestRows and any vector, T being at most 7 |R| and 1 / |x| 1e6; matrices of longer rows, no
+// rotations, leave no value sure.  Looking at that distance for every value instead cost 1 % of a step of 4 x 613 tokens.)
+constexpr float kLongestRows = 4.0f;
+static_assert(0.149 / kBucketScale > kLongestRows * (18 * 7 + 47 + 7e-3 * 1e6) * kUlp && kUnitRows < kLongestRows, "no boundary of the next bucket within the bound");
 template <int BITS>
 __device__ __forceinline__ uint32_t bucket_quantize_sure(const float2* buckets, const float4_t (&S)[4], int r, float inv, float row_norm, bool& doubt) {
     const float val = S[3][r] * inv;
@@ -157,7 +161,7 @@ __device__ __forceinline__ uint32_t bucket_quantize_sure(const float2* buckets, 
     const float eps = __builtin_fmaf(inv, __builtin_fmaf(sums, 18.0f * kUlp, row_norm * (7e-3f * kUlp)), row_norm * (47.0f * kUlp));
     if constexpr (BITS == 4) {
         const float2 e = buckets[bucket_of(val)];
-        doubt = doubt || !(fminf(fabsf(val - e.x), kNextEdge) > eps);      // (a bound past it: long rows of R, tiny vectors)
+        doubt = doubt || !(fabsf(val - e.x) > eps);
         return __builtin_bit_cast(uint32_t, e.y) + (!(val < e.x) ? 1u : 0u);
     } else {
         doubt = doubt || !(fminf(fabsf(val), fabsf(fabsf(val) - kEdges2[2])) > eps);
@@ -169,7 +173,7 @@ __device__ __forceinline__ uint32_t bucket_quantize_sure(const float2* buckets, 
 static_assert(kUnitRows > 1.0001f + 7e-4f, "the norm of R'");
 __device__ __forceinline__ float larger_norm(float x, float y) { return x > y || x != x ? x : y; }      // (a NaN in x stays, one in y is taken)
 // |R'| of the longest of the 16 rows of R whose halves the lanes of a wave hold as operands (16 lanes a row quarter); a row that is no
-// number leaves none sure.
+// number, or longer than kLongestRows, leaves none sure.
 __device__ __forceinline__ float operand_rows_norm(const uint4 (&rows)[4]) {
     float n2 = 0.0f;
 #pragma unroll
@@ -191,7 +195,8 @@ __device__ __forceinline__ float operand_rows_norm(const uint4 (&rows)[4]) {
     n2 = larger(n2, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, n2), 0x4E, 0xf, 0xf, true));
     n2 = larger(n2, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, n2), 0x141, 0xf, 0xf, true));
     n2 = larger(n2, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, n2), 0x140, 0xf, 0xf, true));
-    return __builtin_fmaf(1.001f, __builtin_amdgcn_sqrtf(n2), 7e-4f);
+    const float n = __builtin_fmaf(1.001f, __builtin_amdgcn_sqrtf(n2), 7e-4f);
+    return n <= kLongestRows ? n : __builtin_inff();
 }
 
 }  // namespace twkv
