@@ -46,12 +46,11 @@ decode_layers_kernel(LayersArgs a) {
     constexpr int kPasses = (NV + kUnitVecs - 1) / kUnitVecs;    // of 16 vectors, 16 lanes each
     constexpr int kPairs = HKW / 2, kParts = NW / kPairs;
     constexpr int kBlocks = 8 / NW;                              // blocks of 16 output coordinates a wave rotates
-    constexpr int kRows = NW * R > kUnitVecs ? NW * R : kUnitVecs;   // the upper half of the parts leaves NW * R rows
     static_assert(NQ <= kUnitVecs && 2 * HKW <= kUnitVecs && kPairs * kParts == NW && kBlocks * NW == 8, "the unit fits its waves and LDS region");
     __shared__ __attribute__((aligned(16))) uint32_t tab_s[kTableWords];
     __shared__ __attribute__((aligned(16))) half_t p_s[NW][16][32];
     // in turn: the new token's vectors, the rotated queries, the parts' sums, the outputs
-    __shared__ __attribute__((aligned(16))) float x_s[kRows][kUnitRowFloats];
+    __shared__ __attribute__((aligned(16))) float x_s[kUnitVecs][kUnitRowFloats];
     __shared__ __attribute__((aligned(8))) float2 bucket_s[kBuckets];
     __shared__ float inv_s[kUnitVecs];                           // 1 / |vector| of the K and V vectors
     uint4* qop_s = reinterpret_cast<uint4*>(&x_s[0][0]);
@@ -320,7 +319,7 @@ decode_layers_kernel(LayersArgs a) {
 
     // ---- the parts meet in LDS: every wave leaves its sums, then 32 threads to an output merge them (in halves, the upper handed to the lower
     // until one is left, with two barriers each: 0.5 us of a unit's end)
-    constexpr bool kInPlace = NW * 2 * R <= kRows;            // else where the table was, once every wave is through with it
+    constexpr bool kInPlace = NW * 2 * R <= kUnitVecs;        // else where the table was, once every wave is through with it
     float (*sum_s)[kUnitRowFloats] = kInPlace ? x_s : reinterpret_cast<float (*)[kUnitRowFloats]>(tab_s);
     if (kParts > 1 && !kInPlace) lds_barrier();
     pair_scan_finish<R>(L, S, 1.0f / kAlpha, [&](int, int r, const float (&o)[16]) {     // dims 16 (pn % 8) .. of head hd
