@@ -12,11 +12,11 @@
 //     bits.  Codes meet in LDS and leave 16 lanes to a vector.
 // One barrier per tile: tile i is rotated while tile i + 1 is transformed and the codes of tile i - 1 are stored.
 // The chain alone was bound by the matrix cores (32 of its steps take 16 of the fp16 form's time); now the issue of the transformation
-// and of the buckets bounds it.  Launches of one stream without producers, which are few tiles, keep the chain: they wait for memory, and
-// a repeated block costs more than it saves.  Other workgroups of the same launch transform the queries, a matter of memory
+// and of the buckets bounds it.  Launches without producers whose tiles all run at once, one to a workgroup, keep the chain: they wait for
+// memory, and a repeated block costs more than the sums save.  Other workgroups of the same launch transform the queries, a matter of memory
 // alone, beside them.
 // The prompt step of 4111 tokens (4 layers, 16 heads over 8 KV heads, 4 bit, producers; attention included): 893 us with the
-// chain, 858 with the sums; attention's own changes take it to 842.
+// chain, 858 with the sums; attention's own changes take it to 836.
 
 #include <algorithm>
 #include <type_traits>

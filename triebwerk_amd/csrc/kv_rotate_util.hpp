@@ -1,5 +1,6 @@
-// kv_rotate_util.hpp -- pieces shared by the kernels that apply the 128x128 rotation with
-// v_mfma_f32_16x16x4_f32 (kv_rotate.hip, kv_decode_fused.hip).  Lane (i = lane % 16, kk = lane / 16) of a wave
+// kv_rotate_util.hpp -- pieces shared by the kernels that apply the 128x128 rotation on matrix cores: as the reference's fp32 chain with
+// v_mfma_f32_16x16x4_f32 (kv_rotate.hip), and as sums of v_mfma_f32_16x16x32_f16 that decide a code where they can, with that chain behind
+// them (kv_append_tokens.hip, kv_decode_fused.hip, kv_decode_layers.hip).  Lane (i = lane % 16, kk = lane / 16) of a wave
 // holds, for one row of R and one vector, the coordinates 4s + kk, s = 0..31.
 #pragma once
 
