@@ -603,7 +603,7 @@ decode_fused_kernel(AttnArgs a, FusedArgs f) {
         if (kEarly && !SHARES) load_rb();    // behind the first tile's loads; the registers are there, and the epilogue need not wait
         if (ntiles > 0) {
             S.load_query_operands(L, [&](int i, int part2, int p) { return &qop_s[query_piece(2 * (hk_local * R + i) + part2, p)]; });
-            if (!SHARES && MODE == kStep) S.zero_repeated_queries(L);
+            if (!kEarly) S.zero_repeated_queries(L);
             for (int it = 0; it < ntiles; it++) {
                 const int tile = next_tile;
                 set_next(it + 1);
