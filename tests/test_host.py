@@ -152,6 +152,17 @@ def test_decode_step_plan_is_the_documented_rule():
     assert plan(0, 16, 8, 4, 1024, 0, 0) == 0
 
 
+@pytest.mark.parametrize("case,one", [
+    ((260, 1, 1, 4, 262, 20, 20, 1), 0), ((407, 16, 8, 4, 262, 20, 20, 1), 0), ((667, 1, 1, 4, 240, 208, 237, 0), 0), ((751, 1, 1, 4, 248, 229, 229, 1), 0),
+    ((216, 12, 3, 4, 246, 235, 235, 0), 0), ((80, 36, 9, 4, 234, 222, 222, 1), 0), ((48, 52, 13, 4, 256, 182, 208, 1), 0), ((153, 40, 10, 2, 244, 199, 199, 1), 0),
+    ((202, 16, 16, 4, 262, 89, 89, 1), 0), ((250, 1, 1, 4, 262, 20, 20, 1), 1), ((64, 16, 8, 4, 262, 200, 200, 1), 1), ((128, 16, 8, 2, 240, 64, 64, 0), 1)])
+def test_steps_without_room_for_partials_keep_their_form(case, one):
+    """Where max_seq_len leaves scratch no room for a head's sums, three launches keep p * norm in fp32, which one launch holds as two halves (V norms
+    past 2047 overflow there).  The line between them stays where it was, whatever the other estimates are fitted to."""
+    from triebwerk_amd import _lib
+    assert _lib.load().tw_kv_decode_step_plan2(*case) == one
+
+
 def header_prototypes():
     """name -> (return kind, [parameter kinds]) for every function the header declares; a kind is 'ptr', 'int',
     'uint', 'llong', 'size', 'float', 'double', 'bool', 'void' or 'cstr'."""

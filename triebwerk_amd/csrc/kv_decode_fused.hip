@@ -1007,16 +1007,16 @@ constexpr PlanConstants kPlanTable[] = {
      {{{3.39e6, 7.95e6, 9e6, 9e6}, {2.2e6, 4.12e6, 5.74e6, 9e6}},
       {{2.93e6, 5.64e6, 9e6, 8.9e6}, {1.38e6, 3.05e6, 4.88e6, 9e6}}}, {0, 4.39, 6, 2.49, 2.53, 2.59, 4.7},
      {{17.7, 20.2, 20.1}, {18.9, 15.2, 23}}, {{7.02e6, 8e6, 8e6}, {6.97e6, 4.5e6, 3.8e6}}, {{3.08, 1.54, 2.62}, {1.94, 1.8, 1.79}}, {2.39, 2.66}, 0.000465, 16.2, 0.774e-3, 0.629,
-     2.5, {8.81, 7.67}, 0.01, {{1.39, 1.42, 1.29}, {1.08, 1.1, 1.09}}, 0.80, {{7.91e6, 8.52e6, 8.41e6}, {7.93e6, 8.41e6, 9.97e6}}, 0.112},
+     2.5, {8.81, 7.67}, 0.01, {{1.39, 1.42, 1.29}, {1.08, 1.1, 1.09}}, 0.80, {{7.91e6, 8.52e6, 8.41e6}, {7.93e6, 8.41e6, 9.97e6}}, 0.112, false},
 };
-// Where scratch has no room for partials: fitted when both forms took longer, kept because the line that they draw decides
-// which steps stay in fp32.
+// Where scratch has no room for partials: fitted when both forms took longer, kept with the count of tiles they were fitted with, because
+// the line that they draw decides which steps stay in fp32.
 constexpr PlanConstants kWithoutRoom = {
     "", {7.45, 9.43}, {0.144, 0.125}, {8.37, 8.19},
     {{{1.88, 2.05, 2.48}, {1.35, 1.48, 1.93}}, {{1.99, 2, 2.81}, {1.69, 1.77, 2.23}}},
     {{{5.02e6, 7.61e6, 7.92e6, 7.69e6}, {3.62e6, 5.33e6, 5.91e6, 6.37e6}}, {{3.39e6, 7.65e6, 6.64e6, 7.18e6}, {1.83e6, 3.96e6, 5.99e6, 5.26e6}}},
     {}, {{19.7, 21.1, 24.9}, {19.1, 20, 22.6}}, {{6.67e6, 6.96e6, 6.32e6}, {5.91e6, 5.02e6, 4.94e6}},
-    {{1.16, 1.27, 0.588}, {1.12, 0.672, 1.14}}, {1.74, 1.51}, 0.000277, 0, 0, 0, 0, {}, 0, {}, 0, {}, 0};
+    {{1.16, 1.27, 0.588}, {1.12, 0.672, 1.14}}, {1.74, 1.51}, 0.000277, 0, 0, 0, 0, {}, 0, {}, 0, {}, 0, true};
 }  // namespace
 const PlanConstants& plan_constants() {
     static const PlanConstants* chosen = nullptr;
@@ -1059,7 +1059,7 @@ double decode_fused_estimate_us(int G, int num_heads, int Hk, int bits, bool all
     const int parts = (pair ? 2 * kPairWaves : kFusedWaves) / hkw;          // waves that share a head's tiles
     const double units = (double)G * (Hk / hkw) * shares, full = std::floor(units / cus), rest = units - full * cus;
     const double share_tiles = std::ceil(ctx / shares / 32.0);            // fewer than waves: the ones that have a tile are faster
-    const double tiles = (share_tiles >= parts ? std::ceil(share_tiles / parts) : 0.5 + 0.5 * share_tiles / parts) * pc.tile_us[p][w][group_index(R)];
+    const double tiles = (share_tiles >= parts || pc.whole_tiles ? std::ceil(share_tiles / parts) : 0.5 + 0.5 * share_tiles / parts) * pc.tile_us[p][w][group_index(R)];
     const double unit_bytes = hkw * bytes_per_token(bits) * ctx / shares * fill / pc.one_bw[G % 8 == 0 ? 0 : 1][w][log2_of(hkw)];
     double us = pc.one_fixed_us[p] + pc.one_vector_us[p] * hkw * (2 + R) + pc.handover_us[log2_of(shares)];
     us += full * cube_sum(tiles, cus * unit_bytes);

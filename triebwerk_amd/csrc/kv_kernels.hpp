@@ -284,6 +284,7 @@ struct PlanConstants {
     double layers_alone;           // this share of it for a workgroup of four waves that has its compute unit for itself
     double layers_bw[2][3];        // bytes per us: [4 bit, 2 bit][2, 4, 8 KV heads per workgroup]
     double layers_both;            // this share of the smaller of (longest unit, all units) on top of the larger
+    bool whole_tiles;              // fitted with a whole tile for each wave of a unit that has fewer tiles than waves
 };
 const PlanConstants& plan_constants();
 const PlanConstants& plan_constants_without_room();      // the line between one launch and three where scratch has no room for partials
