@@ -68,3 +68,52 @@ def test_automatic_choice_away_from_the_benchmark(bits, H, Hk, lens):
     auto, one, three = (statistics.median(times[m]) for m in times)
     print(f"plan check G={G} longest={max(lens)} bits={bits} H={H} Hk={Hk}: automatic {auto:.2f} us, one launch {one:.2f}, three launches {three:.2f}", flush=True)
     assert auto <= 1.10 * min(one, three), (auto, one, three)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bits,H,Hk,lens", [(4, 2, 2, [377] * 292), (4, 8, 2, [295] * 338), (2, 4, 2, [300] * 336), (4, 16, 8, [300] * 300), (4, 32, 16, [600] * 300),
+                                            (2, 32, 8, [1500] * 400), (4, 16, 8, [2048] * 512)])
+def test_automatic_choice_past_256_sequences(bits, H, Hk, lens):
+    """Batches that take rounds of workgroups: the automatic choice against every number of heads per workgroup and the three launches."""
+    import torch
+    from triebwerk_amd import Engine, kvcache
+    G, L, steps, reps = len(lens), 3, 4, 5
+    msl = (max(lens) + steps + 2 + 255) // 256 * 256
+    eng = Engine(max_seq_len=msl, kv_bits=bits)
+    eng.set_shape(L, H, Hk, D)
+    eng.alloc_batch(G, msl)
+    gt = torch.Generator(device="cuda"); gt.manual_seed(3)
+    for l in range(L):
+        c = eng.cache(l)
+        for i in range(2):
+            c[i].copy_(torch.randint(0, 256, c[i].shape, generator=gt, device="cuda", dtype=torch.uint8))
+        for i in (2, 3):
+            c[i].copy_((11.3 + 0.7 * torch.randn(c[i].shape, generator=gt, device="cuda")).to(torch.float16))
+    q = torch.randn((L, G, H * D), generator=gt, device="cuda", dtype=torch.float16)
+    k, v = (torch.randn((L, G, Hk * D), generator=gt, device="cuda", dtype=torch.float16) for _ in range(2))
+    out = torch.zeros_like(q)
+    stream = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    forms = {"automatic": (4, 0), "three launches": (2, 0), **{f"{h} heads": (1, h) for h in (1, 2, 4, 8) if Hk % h == 0}}
+    times = {f: [] for f in forms}
+    try:
+        for _ in range(reps):
+            for form, (mode, heads) in forms.items():
+                kvcache.set_decode_fused(mode)
+                kvcache.set_fused_shape(heads, 1 if heads else 0)
+                eng.set_positions([n - 1 for n in lens])
+                with torch.cuda.stream(stream):
+                    eng.decode_step(q, k, v, out, use_graph=True, stream=stream)        # captures where the form is another
+                    e0.record(stream)
+                    for _ in range(steps):
+                        eng.decode_step(q, k, v, out, use_graph=True, stream=stream)
+                    e1.record(stream)
+                stream.synchronize()
+                times[form].append(e0.elapsed_time(e1) / steps / L * 1e3)
+    finally:
+        kvcache.set_decode_fused(0)
+        kvcache.set_fused_shape(0, 0)
+    us = {f: statistics.median(t) for f, t in times.items()}
+    print(f"plan check G={G} longest={max(lens)} bits={bits} H={H} Hk={Hk}: " + ", ".join(f"{f} {t:.2f} us" for f, t in us.items()), flush=True)
+    assert us["automatic"] <= 1.10 * min(us.values()), us

@@ -1001,14 +1001,27 @@ bool decode_fused_pairs(const AttnArgs& a, int hkw) { return pairs_fit(a.bits, a
 // launch: 11100 steps of 4 to 36 layers in each of the four shapes, choice within 3 % of the fastest at 91 %, 10 % at 98 %
 // of the sizes that were not fitted to (85 and 95 % before).  64 shares and ragged batches keep figures from earlier fits.
 namespace {
-constexpr PlanConstants kPlanTable[] = {
+// Batches past 256 sequences, every one of which takes rounds of workgroups: figures of their own, since those above, fitted without
+// such batches and with rates above the memory's, counted a further round of eight waves too high and one of sixteen too low. Fitted to 2129
+// steps of 100 to 1000 sequences of 64 to 16000 tokens, without shares, no rate above the 7.0 TB/s of the best reader: past 256 sequences
+// the choice is within 3 % of the fastest form at 97 % of the sizes and within 10 % at 99.5 %, with the figures above at 65 and
+// 78 %. us a layer, 4 bit: 300 x 600 tokens, 32 heads over 16 123 -> 94; 300 x 300, 16 over 8 42.1 -> 37.6; 292 x 377, 2 over 2 27.1 -> 20.3.
+// (One table for all of them, fitted to 5699 sizes, is 1.6 % faster in the mean, but 15 to 20 % slower at a few sizes of few long sequences.)
+constexpr int kFittedBatch = 256;
+constexpr PlanConstants kPlanTable[][2] = {{
     {"gfx950", {2.85, 4.16}, {0.178, 0.222}, {9.47, 3.73},
      {{{2.88, 2.11, 2.92}, {1.83, 1.99, 2.39}}, {{3.1, 1.91, 3.32}, {2.65, 2.11, 3.08}}},
      {{{3.39e6, 7.95e6, 9e6, 9e6}, {2.2e6, 4.12e6, 5.74e6, 9e6}},
       {{2.93e6, 5.64e6, 9e6, 8.9e6}, {1.38e6, 3.05e6, 4.88e6, 9e6}}}, {0, 4.39, 6, 2.49, 2.53, 2.59, 4.7},
      {{17.7, 20.2, 20.1}, {18.9, 15.2, 23}}, {{7.02e6, 8e6, 8e6}, {6.97e6, 4.5e6, 3.8e6}}, {{3.08, 1.54, 2.62}, {1.94, 1.8, 1.79}}, {2.39, 2.66}, 0.000465, 16.2, 0.774e-3, 0.629,
      2.5, {8.81, 7.67}, 0.01, {{1.39, 1.42, 1.29}, {1.08, 1.1, 1.09}}, 0.80, {{7.91e6, 8.52e6, 8.41e6}, {7.93e6, 8.41e6, 9.97e6}}, 0.112, false},
-};
+    {"gfx950", {9.03, 6.96}, {0.0236, 0.0398}, {6.24, 6.28},
+     {{{1.49, 1.72, 2.37}, {0.927, 1.21, 1.54}}, {{2.35, 2.98, 3.01}, {1.99, 1.9, 2.51}}},
+     {{{6.7e6, 7e6, 7e6, 6.9e6}, {5.83e6, 5.22e6, 5.37e6, 5.34e6}},
+      {{6.11e6, 6.72e6, 6.9e6, 6.66e6}, {4.16e6, 4.58e6, 5.84e6, 5.61e6}}}, {0, 4.39, 6, 2.49, 2.53, 2.59, 4.7},
+     {{14.9, 9.65, 6.55}, {12.8, 10.6, 9.25}}, {{5.37e6, 6.72e6, 7e6}, {5.86e6, 5.04e6, 6.7e6}}, {{1.52, 1.75, 1.91}, {1.61, 1.36, 1.26}}, {2.25, 1.54}, 0.00223, 16.2, 0.774e-3, 0.629,
+     2.5, {8.81, 7.67}, 0.01, {{1.39, 1.42, 1.29}, {1.08, 1.1, 1.09}}, 0.80, {{7.91e6, 8.52e6, 8.41e6}, {7.93e6, 8.41e6, 9.97e6}}, 0.112, false},
+}};
 // Where scratch has no room for partials: fitted when both forms took longer, kept with the count of tiles they were fitted with, because
 // the line that they draw decides which steps stay in fp32.
 constexpr PlanConstants kWithoutRoom = {
@@ -1018,21 +1031,21 @@ constexpr PlanConstants kWithoutRoom = {
     {}, {{19.7, 21.1, 24.9}, {19.1, 20, 22.6}}, {{6.67e6, 6.96e6, 6.32e6}, {5.91e6, 5.02e6, 4.94e6}},
     {{1.16, 1.27, 0.588}, {1.12, 0.672, 1.14}}, {1.74, 1.51}, 0.000277, 0, 0, 0, 0, {}, 0, {}, 0, {}, 0, true};
 }  // namespace
-const PlanConstants& plan_constants() {
+const PlanConstants& plan_constants(int G) {
     static const PlanConstants* chosen = nullptr;
     if (!chosen) {
-        const PlanConstants* pick = &kPlanTable[0];
+        const PlanConstants* pick = kPlanTable[0];
         int dev = 0;
         hipDeviceProp_t prop;
         if (hipGetDevice(&dev) == hipSuccess && hipGetDeviceProperties(&prop, dev) == hipSuccess) {
-            for (const PlanConstants& c : kPlanTable)
-                if (strstr(prop.gcnArchName, c.device)) { pick = &c; break; }
+            for (const auto& c : kPlanTable)
+                if (strstr(prop.gcnArchName, c[0].device)) { pick = c; break; }
         } else {
             (void)hipGetLastError();           // no device (a host-only process asking for the plan): the first entry
         }
         chosen = pick;
     }
-    return *chosen;
+    return chosen[G > kFittedBatch ? 1 : 0];
 }
 
 const PlanConstants& plan_constants_without_room() { return kWithoutRoom; }

@@ -286,7 +286,7 @@ struct PlanConstants {
     double layers_both;            // this share of the smaller of (longest unit, all units) on top of the larger
     bool whole_tiles;              // fitted with a whole tile for each wave of a unit that has fewer tiles than waves
 };
-const PlanConstants& plan_constants();
+const PlanConstants& plan_constants(int G = 0);          // of the device; batches past 256 sequences have figures of their own
 const PlanConstants& plan_constants_without_room();      // the line between one launch and three where scratch has no room for partials
 bool decode_fused_usable(const AttnArgs& a, const FusedArgs& f);
 // estimated microseconds of one launch with hkw KV heads per workgroup and `shares` workgroups per sequence and head group,
