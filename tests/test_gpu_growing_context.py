@@ -48,7 +48,8 @@ def test_replay_is_the_eager_step_at_every_length(layers_apart, bits, H, Hk, G):
 
 @pytest.mark.parametrize("bits,H,Hk,G,L", [(4, 16, 8, 1, 28), (2, 16, 8, 5, 28)])
 def test_every_layer_in_one_launch_is_captured_again_only_for_another_launch(bits, H, Hk, G, L):
-    """While every layer goes into the same one launch, what a layer by itself would take does not matter to the captured step."""
+    """While every layer goes into the same one launch, what a layer by itself would take does not matter to the fixed step: nothing is planned
+    or counted anew for it (a launch needs no capture), and it gives the very bits of the eager step."""
     import torch
     from triebwerk_amd import Engine, _lib, kvcache
     lib = _lib.load()
@@ -65,14 +66,17 @@ def test_every_layer_in_one_launch_is_captured_again_only_for_another_launch(bit
         eng.set_positions([ctx - 1] * G)
         eng.decode_step(q, k, v, out, use_graph=False)
         name = kvcache.last_scan_kernel()
+        eager = out.clone()
+        out.zero_()
         eng.set_positions([ctx - 1] * G)
         recorded = lib.tw_kv_decode_fused_launches()
         eng.decode_step(q, k, v, out, use_graph=True)
         recorded = lib.tw_kv_decode_fused_launches() - recorded
         assert eng.graph_state() == 1
+        assert kvcache.last_scan_kernel() == name and torch.equal(eager, out), f"context {ctx}: the fixed step is not the eager one"
         if name == last and "decode_layers_kernel" in name:
             same += 1
-            assert recorded == 0, f"context {ctx}: {name} captured again"
+            assert recorded == 0, f"context {ctx}: {name} fixed again"
         last = name
     torch.cuda.synchronize()
     assert same > 20
