@@ -16,7 +16,7 @@
 // memory, and a repeated block costs more than the sums save.  Other workgroups of the same launch transform the queries, a matter of memory
 // alone, beside them.
 // The prompt step of 4111 tokens (4 layers, 16 heads over 8 KV heads, 4 bit, producers; attention included): 893 us with the
-// chain, 858 with the sums; attention's own changes take it to 836.
+// chain, 858 with the sums; attention's own changes take it to 839.
 
 #include <algorithm>
 #include <type_traits>

@@ -12,9 +12,9 @@
 //
 // A unit's start and end were a third of the time of short contexts: arguments in one trip, loads without branches, K, V and q
 // rotated on fp16 matrix instructions (codes from the fp32 chain where the sums leave a doubt), the parts merged behind one
-// barrier, and no launch of its own to advance the positions.  28 layers of 4 x 613 tokens: 985 us a pass of 32 steps before, 697 now.
+// barrier, and no launch of its own to advance the positions.  28 layers of 4 x 613 tokens: 985 us a pass of 32 steps before, 697 to 714 now.
 // MI355X, us per layer, layer by layer -> all at once (16 heads over 8 KV heads, 28 layers, 4 bit unless said), before those steps: 4 x 613
-// tokens 13.8 -> 1.1 (now 0.8); 128 x 513 20.8 -> 13.8 (12.6); 64 x 8192 94.0 -> 83.2 (83.2 to 84.9, 6.5 to 6.7 TB/s); 2 bit 70.6 -> 61.1 (60.6);
+// tokens 13.8 -> 1.1 (now 0.8); 128 x 513 20.8 -> 13.8 (12.6); 64 x 8192 94.0 -> 83.2 (83 to 89 by the box, 6.2 to 6.7 TB/s); 2 bit 70.6 -> 61.1 (61 to 65);
 // 64 ragged 512..8072 75 -> 61; 32 heads, 36 layers, 2 bit, 16 x 4097 23.8 -> 10.3 (9.6).  Over 500 random steps (2 to 36 layers, 1 to 192 sequences of 64 to 16000 tokens, even and
 // ragged, both widths) 3.3 times faster in the geometric mean, the slowest 0.97.  Long contexts are bound by the streaming of the
 // cache, short ones by the units' start and end.  One workgroup of eight waves per compute unit with kv_decode_fused.hip's LDS layout
