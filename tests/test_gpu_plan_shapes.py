@@ -72,13 +72,14 @@ def test_automatic_choice_away_from_the_benchmark(bits, H, Hk, lens):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("bits,H,Hk,lens", [(4, 2, 2, [377] * 292), (4, 8, 2, [295] * 338), (2, 4, 2, [300] * 336), (4, 16, 8, [300] * 300), (4, 32, 16, [600] * 300),
-                                            (2, 32, 8, [1500] * 400), (4, 16, 8, [2048] * 512)])
+                                            (2, 32, 8, [1500] * 400), (4, 16, 8, [2048] * 512), (2, 32, 8, [231] * 129)])
 def test_automatic_choice_past_256_sequences(bits, H, Hk, lens):
-    """Batches that take rounds of workgroups: the automatic choice against every number of heads per workgroup and the three launches."""
+    """Batches that take rounds of workgroups, and one that does with fewer than eight KV heads per workgroup: the automatic choice against every
+    number of heads per workgroup and the three launches."""
     import torch
     from triebwerk_amd import Engine, kvcache
     G, L, steps, reps = len(lens), 3, 4, 5
-    msl = (max(lens) + steps + 2 + 255) // 256 * 256
+    msl = max(512, (max(lens) + steps + 2 + 255) // 256 * 256)
     eng = Engine(max_seq_len=msl, kv_bits=bits)
     eng.set_shape(L, H, Hk, D)
     eng.alloc_batch(G, msl)

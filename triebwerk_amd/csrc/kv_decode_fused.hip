@@ -1000,16 +1000,18 @@ bool decode_fused_pairs(const AttnArgs& a, int hkw) { return pairs_fit(a.bits, a
 // cache level helped with.  Every layer in one
 // launch: 11100 steps of 4 to 36 layers in each of the four shapes, choice within 3 % of the fastest at 91 %, 10 % at 98 %
 // of the sizes that were not fitted to (85 and 95 % before).  64 shares and ragged batches keep figures from earlier fits.
+// (A vector of sixteen waves was fitted as 0.222 us, which kept eight KV heads of four query heads from batches of one round: 2 bit, 129 x 231
+// tokens 23.0 us with four heads in two rounds, 19.2 with eight. As 0.208, of 4300 sizes 20 change their form, 19 of them to a faster one.)
 namespace {
-// Batches past 256 sequences, every one of which takes rounds of workgroups: figures of their own, since those above, fitted without
+// Batches past 256 sequences, every one of which takes rounds of workgroups: figures of their own, since the first ones, fitted without
 // such batches and with rates above the memory's, counted a further round of eight waves too high and one of sixteen too low. Fitted to 2129
 // steps of 100 to 1000 sequences of 64 to 16000 tokens, without shares, no rate above the 7.0 TB/s of the best reader: past 256 sequences
-// the choice is within 3 % of the fastest form at 97 % of the sizes and within 10 % at 99.5 %, with the figures above at 65 and
+// the choice is within 3 % of the fastest form at 97 % of the sizes and within 10 % at 99.5 %, with the first ones at 65 and
 // 78 %. us a layer, 4 bit: 300 x 600 tokens, 32 heads over 16 123 -> 94; 300 x 300, 16 over 8 42.1 -> 37.6; 292 x 377, 2 over 2 27.1 -> 20.3.
 // (One table for all of them, fitted to 5699 sizes, is 1.6 % faster in the mean, but 15 to 20 % slower at a few sizes of few long sequences.)
 constexpr int kFittedBatch = 256;
 constexpr PlanConstants kPlanTable[][2] = {{
-    {"gfx950", {2.85, 4.16}, {0.178, 0.222}, {9.47, 3.73},
+    {"gfx950", {2.85, 4.16}, {0.178, 0.208}, {9.47, 3.73},
      {{{2.88, 2.11, 2.92}, {1.83, 1.99, 2.39}}, {{3.1, 1.91, 3.32}, {2.65, 2.11, 3.08}}},
      {{{3.39e6, 7.95e6, 9e6, 9e6}, {2.2e6, 4.12e6, 5.74e6, 9e6}},
       {{2.93e6, 5.64e6, 9e6, 8.9e6}, {1.38e6, 3.05e6, 4.88e6, 9e6}}}, {0, 4.39, 6, 2.49, 2.53, 2.59, 4.7},
