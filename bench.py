@@ -53,7 +53,7 @@ BYTES_HEAD = {0: 256, 4: 66, 2: 34}  # per (token, kv head): fp16 row | codes + 
 # Keyed by (workload, kv_bits, kernel that ran).  Counters are not read in this run: the figures belong to
 # the kernel sources whose digest is recorded with them (`python bench.py --csrc-digest` prints the current
 # one) and are only reported while the sources are still those; otherwise `traffic` is null.
-MEASURED_TRAFFIC_CSRC_DIGEST = "754dacb9b11be622"
+MEASURED_TRAFFIC_CSRC_DIGEST = "cb3628291594b4e7"
 MEASURED_TRAFFIC_BYTES = {("target", 4, "every layer"): 15533.3e6, ("target", 4, "one-launch"): 555.2e6, ("target", 4, "scan"): 560.8e6,
                           ("target", 2, "every layer"): 8015.4e6, ("target", 2, "one-launch"): 291.4e6, ("target", 2, "scan"): 292.3e6,
                           ("target", 0, "every layer"): 60191.5e6, ("target", 0, "scan"): 2154.8e6}
